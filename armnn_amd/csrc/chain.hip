@@ -259,6 +259,7 @@ int mi355x_chain_create(uint32_t n_layers, const mi355x_conv2d_t* plans, uint32_
         delete c;
         return SetError(MI355X_ERR_OUT_OF_MEMORY, "chain: out of device memory");
     }
+    UploadScope uploads;
     rc = UploadNow(c->d_layers, c->layers.data(), c->layers.size() * sizeof(ChainLayer));
     if (!rc) rc = UploadNow(c->d_need, need.data(), need.size() * 4);
     if (!rc) rc = UploadNow(c->d_sync, zeros.data(), sync_words * 4);

@@ -1727,6 +1727,7 @@ int mi355x_conv2d_create(const mi355x_conv2d_desc* desc, const void* weights_hos
 {
     if (!desc || !plan) return SetError(MI355X_ERR_INVALID_ARGUMENT, "descriptor / plan pointer is null");
     *plan = nullptr;
+    UploadScope uploads;
     auto* p = new mi355x_conv2d_s;
     int rc = BuildPlan(*desc, weights_host, weights_quant, bias_host, bias_quant, p);
     if (rc != 0) { delete p; return rc; }
@@ -1938,6 +1939,7 @@ int mi355x_fc_create(const mi355x_fc_desc* desc, const void* weights_host, const
             for (size_t o = 0; o < O; ++o) wt[o * K + k] = w[k * O + o];
         w = wt.data();
     }
+    UploadScope uploads;
     auto* cp = new mi355x_conv2d_s;
     int rc = BuildPlan(c, w, weights_quant, bias_host, bias_quant, cp);
     if (rc != 0) { delete cp; return rc; }

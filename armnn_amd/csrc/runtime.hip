@@ -3,6 +3,7 @@
 
 #include <cmath>
 #include <mutex>
+#include <utility>
 
 namespace mi355x
 {
@@ -39,18 +40,41 @@ void NoteKernel(const char* fmt, ...)
     va_end(ap);
 }
 
+namespace
+{
+// The calling thread's upload stream: there is one while an UploadScope is open.
+thread_local hipStream_t t_upload_stream = nullptr;
+thread_local int t_upload_scopes = 0;
+
+// At most one upload stream waits here for the next plan.
+std::mutex g_idle_upload_mutex;
+hipStream_t g_idle_upload_stream = nullptr;
+
+hipStream_t SwapIdleUploadStream(hipStream_t s)
+{
+    std::lock_guard<std::mutex> lock(g_idle_upload_mutex);
+    std::swap(s, g_idle_upload_stream);
+    return s;
+}
+} // namespace
+
+UploadScope::UploadScope() { ++t_upload_scopes; }
+
+UploadScope::~UploadScope()
+{
+    if (--t_upload_scopes > 0 || !t_upload_stream) return;
+    if (const hipStream_t other = SwapIdleUploadStream(t_upload_stream)) (void)hipStreamDestroy(other);
+    t_upload_stream = nullptr;
+}
+
 int UploadNow(void* dst_dev, const void* src_host, size_t bytes)
 {
     // one stream per calling thread, so concurrent plan creations do not wait for each other
-    struct Own
-    {
-        hipStream_t s = nullptr;
-        ~Own() { if (s) (void)hipStreamDestroy(s); }
-    };
-    thread_local Own own;
-    if (!own.s) MI355X_HIP(hipStreamCreateWithFlags(&own.s, hipStreamNonBlocking));
-    MI355X_HIP(hipMemcpyAsync(dst_dev, src_host, bytes, hipMemcpyHostToDevice, own.s));
-    MI355X_HIP(hipStreamSynchronize(own.s));
+    UploadScope scope;
+    if (!t_upload_stream) t_upload_stream = SwapIdleUploadStream(nullptr);
+    if (!t_upload_stream) MI355X_HIP(hipStreamCreateWithFlags(&t_upload_stream, hipStreamNonBlocking));
+    MI355X_HIP(hipMemcpyAsync(dst_dev, src_host, bytes, hipMemcpyHostToDevice, t_upload_stream));
+    MI355X_HIP(hipStreamSynchronize(t_upload_stream));
     return 0;
 }
 
@@ -366,6 +390,8 @@ int mi355x_fill_u8(void* dst_dev, uint8_t value, size_t bytes, mi355x_stream_t s
 int mi355x_stream_create(mi355x_stream_t* stream)
 {
     if (!stream) return SetError(MI355X_ERR_INVALID_ARGUMENT, "stream is null");
+    // the new stream, not a waiting upload stream, gets the hardware queue (UploadScope)
+    if (const hipStream_t idle = SwapIdleUploadStream(nullptr)) (void)hipStreamDestroy(idle);
     hipStream_t s;
     MI355X_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));   // default priority
     *stream = reinterpret_cast<mi355x_stream_t>(s);
