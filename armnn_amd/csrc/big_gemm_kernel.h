@@ -397,12 +397,8 @@ __global__ __launch_bounds__(256) void BigGemmKernel(IgemmArgs a, int xcd_rows)
         for (int r = orow; r < BM; r += ROWS_PER_PASS)
         {
             const int m = tm * BM + r;
-            if (m >= a.M) continue;
-            for (int b = 0; b < 16; ++b)
-            {
-                const int c = c0 + b;
-                if (c < a.Co) a.y[static_cast<long long>(m) * a.Co + c] = Os[r * LDO + oc * 16 + b];
-            }
+            if (m < a.M && c0 < a.Co)
+                StoreRagged16(a.y + static_cast<long long>(m) * a.Co + c0, *reinterpret_cast<const v4i*>(Os + r * LDO + oc * 16), a.Co - c0);
         }
     }
 }

@@ -11,6 +11,7 @@
 #include "pool_softmax_items.h"
 #include "igemm_ksplit_kernel.h"
 #include "pw_gemm_kernel.h"
+#include "igemm.h"
 #include "igemm_lds_kernel.h"
 #include "big_gemm.h"
 #include "halo_conv_kernel.h"
@@ -251,12 +252,16 @@ int BuildPlan(const mi355x_conv2d_desc& d, const void* weights_host, const mi355
                          ((Kh == 3 && row_bytes <= 12) || (Kh == 7 && row_bytes <= 24) || (Kh == 1 && row_bytes <= 4) ||
                           (Kh == 5 && row_bytes <= 20));
     int32_t algo = d.algo;
+    // Channel counts that are no multiple of 16 run on the matrix cores as well, each tap padded to whole 16-byte chunks
+    // (IgemmKernel, RG).  Up to 4 channels the padding would be most of the work: those are stems, or the plain kernel.
+    const bool ragged_ok = !mfma_ok && !d.depthwise && (Ci % 16) != 0 && Ci > 4 && zw_shift >= -128 && zw_shift <= 127 && zx_shift >= -128 &&
+                           zx_shift <= 127 && p->K <= 100000 && static_cast<long long>(g.H) * g.W * Ci >= 16;
     if (algo == MI355X_ALGO_AUTO)
-        algo = mfma_ok ? MI355X_ALGO_MFMA : dw_ok ? MI355X_ALGO_DEPTHWISE : stem_ok ? MI355X_ALGO_DOT4 : MI355X_ALGO_DIRECT;
+        algo = mfma_ok || ragged_ok ? MI355X_ALGO_MFMA : dw_ok ? MI355X_ALGO_DEPTHWISE : stem_ok ? MI355X_ALGO_DOT4 : MI355X_ALGO_DIRECT;
     if (algo == MI355X_ALGO_DOT4 && !stem_ok)
         return SetError(MI355X_ERR_UNSUPPORTED, "dot4 kernel needs <= 4 input channels, symmetric int8 weights, stride 1 or 2, "
                                                 "no dilation and a 1/3/5/7-row filter");
-    if (algo == MI355X_ALGO_MFMA && !mfma_ok)
+    if (algo == MI355X_ALGO_MFMA && !mfma_ok && !(ragged_ok && d.algo == MI355X_ALGO_AUTO))
         return SetError(MI355X_ERR_UNSUPPORTED, "MFMA kernel needs a non-depthwise layer and in_c %% 16 == 0");
     if (algo == MI355X_ALGO_DEPTHWISE && !dw_ok)
         return SetError(MI355X_ERR_UNSUPPORTED, "depthwise kernel needs multiplier 1 and channels %% 4 == 0");
@@ -266,6 +271,12 @@ int BuildPlan(const mi355x_conv2d_desc& d, const void* weights_host, const mi355
     const uint8_t* wsrc = static_cast<const uint8_t*>(weights_host);
     if (algo == MI355X_ALGO_MFMA)
     {
+        const int Ck = (Ci + 15) / 16 * 16;        // bytes of K per tap
+        if (Ck != Ci)
+        {
+            p->ragged_ck = Ck;
+            p->K_pad = (Kh * Kw * Ck + 63) / 64 * 64;
+        }
         std::vector<int8_t> wp(static_cast<size_t>(p->Co_pad) * p->K_pad, 0);
         std::vector<int32_t> corr(p->Co_pad, 0);
         for (int c = 0; c < Co; ++c)
@@ -273,11 +284,12 @@ int BuildPlan(const mi355x_conv2d_desc& d, const void* weights_host, const mi355
             long long sum = 0;
             const int8_t* src = reinterpret_cast<const int8_t*>(wsrc) + static_cast<size_t>(c) * p->K;
             int8_t* dst = wp.data() + static_cast<size_t>(c) * p->K_pad;
-            for (int k = 0; k < p->K; ++k)
-            {
-                dst[k] = g.w_u8 ? static_cast<int8_t>(static_cast<uint8_t>(src[k]) ^ 0x80u) : src[k];
-                sum += dst[k];
-            }
+            for (int t = 0; t < Kh * Kw; ++t, dst += Ck)
+                for (int k = 0; k < Ci; ++k, ++src)
+                {
+                    dst[k] = g.w_u8 ? static_cast<int8_t>(static_cast<uint8_t>(*src) ^ 0x80u) : *src;
+                    sum += dst[k];
+                }
             // sum_k (x' - zx')(w - zw') = sum_k x'w - zx' sum_k w - zw' sum_k x' + K zx' zw' over the K bytes of a row, of which
             // those outside the image are zx'; the term with sum_k x' is the kernel's
             corr[c] = static_cast<int32_t>(-static_cast<long long>(zx_shift) * sum + static_cast<long long>(zw_shift) * zx_shift * p->K);
@@ -603,62 +615,6 @@ int LaunchPwKs(const mi355x_conv2d_s* p, long long M, const void* x, void* y, hi
     case 2: return LaunchPw<BN, 2>(p, M, x, y, stream, blocks_per_cu);
     default: return LaunchPw<BN, 1>(p, M, x, y, stream, blocks_per_cu);
     }
-}
-
-template <int BM, int BN, int WM, int WN, int D, int BK, bool UT, bool AW>
-int LaunchIgemmT(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, hipStream_t stream);
-
-// uniform-tap variant whenever a k-tile cannot straddle two filter taps; row sums when the weights have a zero point
-template <int BM, int BN, int WM, int WN, int D, int BK>
-int LaunchIgemm(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, hipStream_t stream)
-{
-    const bool ut = (p->geom.Ci % BK) == 0;
-    if (p->zw_neg != 0)
-        return ut ? LaunchIgemmT<BM, BN, WM, WN, D, BK, true, true>(p, batch, x, y, stream)
-                  : LaunchIgemmT<BM, BN, WM, WN, D, BK, false, true>(p, batch, x, y, stream);
-    return ut ? LaunchIgemmT<BM, BN, WM, WN, D, BK, true, false>(p, batch, x, y, stream)
-              : LaunchIgemmT<BM, BN, WM, WN, D, BK, false, false>(p, batch, x, y, stream);
-}
-
-template <int BM, int BN, int WM, int WN, int D, int BK, bool UT, bool AW>
-int LaunchIgemmT(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, hipStream_t stream)
-{
-    const ConvGeom& g = p->geom;
-    IgemmArgs a;
-    a.x = static_cast<const uint8_t*>(x);
-    a.pad16 = p->pad16;
-    a.w = p->w_mfma;
-    a.ct = ChanTab{p->chan, p->Co_pad};
-    a.corr = p->corr;
-    a.y = static_cast<uint8_t*>(y);
-    const long long M = static_cast<long long>(batch) * g.Ho * g.Wo;
-    if (M > 0x7fffffffll / 2) return SetError(MI355X_ERR_UNSUPPORTED, "too many output pixels for one launch (%lld)", M);
-    a.M = static_cast<int>(M);
-    a.H = g.H; a.W = g.W; a.Ci = g.Ci; a.Ho = g.Ho; a.Wo = g.Wo; a.Co = g.Co;
-    a.Kh = g.Kh; a.Kw = g.Kw;
-    a.pad_top = g.pad_top; a.pad_left = g.pad_left; a.stride_x = g.stride_x; a.stride_y = g.stride_y;
-    a.dil_x = g.dil_x; a.dil_y = g.dil_y;
-    a.K_pad = p->K_pad;
-    a.unit = (g.Kh == 1 && g.Kw == 1 && g.stride_x == 1 && g.stride_y == 1 && g.pad_top == 0 && g.pad_left == 0 && g.Ho == g.H &&
-              g.Wo == g.W) ? 1 : 0;
-    if (a.unit) { a.H = 1; a.W = a.M; a.Ho = 1; a.Wo = a.M; }      // one row of M pixels
-    a.tiles_m = static_cast<int>((M + BM - 1) / BM);
-    a.tiles_n = (g.Co + BN - 1) / BN;
-    a.xor_mask = p->xor_mask;
-    a.pad_word = p->pad_word;
-    a.zw_neg = p->zw_neg;
-    a.rowsum_bias = p->rowsum_bias;
-    a.rq = p->rq;
-    const int nblocks = a.tiles_m * a.tiles_n;
-    const int grid = (nblocks + 7) / 8 * 8;
-    constexpr int smem = IgemmSmemBytes<BM, BN, BK>();
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&IgemmKernel<BM, BN, WM, WN, D, BK, UT, AW>),
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-    MI355X_HIP(attr);
-    NoteKernel("IgemmKernel<%d, %d, %d, %d, %d, %d, %s, %s>", BM, BN, WM, WN, D, BK, BoolName(UT), BoolName(AW));
-    hipLaunchKernelGGL((IgemmKernel<BM, BN, WM, WN, D, BK, UT, AW>), dim3(grid), dim3(256), smem, stream, a);
-    MI355X_HIP(hipGetLastError());
-    return 0;
 }
 
 template <int BM, int BN, int WM, int WN, int ST, bool U8, bool AW>
@@ -1015,7 +971,7 @@ int RunPlan(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, hi
     switch (p->algo)
     {
     case MI355X_ALGO_MFMA:
-        if ((reinterpret_cast<uintptr_t>(x) & 15) != 0 || ((g.Co & 15) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) != 0))
+        if (p->ragged_ck == 0 && ((reinterpret_cast<uintptr_t>(x) & 15) != 0 || ((g.Co & 15) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) != 0)))
             return SetError(MI355X_ERR_INVALID_ARGUMENT, "MFMA kernel needs 16-byte aligned tensors");
     {
         const mi355x_conv2d_desc& dd = p->d;
@@ -1142,9 +1098,7 @@ int RunPlan(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, hi
             if (tile == 512) return LaunchIgemmLds<256, 256, 4, 4>(p, lds_stages, batch, x, y, stream);
             return LaunchIgemmLds<128, 128, 2, 2>(p, lds_stages, batch, x, y, stream);
         }
-        if (tile == 64) return bk128 ? LaunchIgemm<64, 64, 2, 2, 2, 128>(p, batch, x, y, stream) : LaunchIgemm<64, 64, 2, 2, 2, 64>(p, batch, x, y, stream);
-        if (g.Co <= 64 || tile == 96) return bk128 ? LaunchIgemm<128, 64, 2, 2, 2, 128>(p, batch, x, y, stream) : LaunchIgemm<128, 64, 2, 2, 2, 64>(p, batch, x, y, stream);
-        return bk128 ? LaunchIgemm<128, 128, 2, 2, 2, 128>(p, batch, x, y, stream) : LaunchIgemm<128, 128, 2, 2, 2, 64>(p, batch, x, y, stream);
+        return LaunchIgemm(p, tile, batch, x, y, stream);
     }
     case MI355X_ALGO_DOT4:
     {

@@ -4,7 +4,7 @@
 //   DepthwiseC4Kernel     depthwise, multiplier 1, channels % 4 == 0: one thread per (pixel, 4 channels).
 //   IgemmKernel<BM,BN,..> implicit GEMM on v_mfma_i32_32x32x32_i8, NHWC tiles staged in LDS, exact int32
 //                         accumulation, fused requantize/clamp epilogue, output tile staged in LDS and stored
-//                         with 16-byte coalesced writes.
+//                         with 16-byte coalesced writes.  Any channel counts (RG: channels that are no multiple of 16).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -138,6 +138,43 @@ __global__ __launch_bounds__(256) void DepthwiseC4Kernel(ConvGeom g, Requant rq,
 }
 
 // ---------------------------------------------------------------------------------------------------------
+// Pieces of rows that start at any byte.
+// ---------------------------------------------------------------------------------------------------------
+struct __attribute__((packed)) Packed16 { v4i v; };
+struct __attribute__((packed)) Packed8 { unsigned long long v; };
+struct __attribute__((packed)) Packed4 { uint32_t v; };
+struct __attribute__((packed)) Packed2 { uint16_t v; };
+
+__device__ __forceinline__ v4i LoadUnaligned16(const uint8_t* p) { return reinterpret_cast<const Packed16*>(p)->v; }
+
+// bytes n .. 15 of v, moved to the front and followed by zeros (n = 0 .. 15)
+__device__ __forceinline__ v4i ShiftDown16(const v4i& v, int n)
+{
+    v4i r = v;
+    if (n & 8) r = v4i{r[2], r[3], 0, 0};
+    if (n & 4) r = v4i{r[1], r[2], r[3], 0};
+    const uint32_t d[5] = {static_cast<uint32_t>(r[0]), static_cast<uint32_t>(r[1]), static_cast<uint32_t>(r[2]), static_cast<uint32_t>(r[3]), 0u};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = static_cast<int>(__builtin_amdgcn_alignbyte(d[i + 1], d[i], n & 3));
+    return r;
+}
+
+// the first min(n, 16) bytes of v to any address: one store where the piece is whole, else one per power of two
+__device__ __forceinline__ void StoreRagged16(uint8_t* p, const v4i& v, int n)
+{
+    if (n >= 16) { reinterpret_cast<Packed16*>(p)->v = v; return; }
+    v4i r = v;
+    if (n & 8)
+    {
+        reinterpret_cast<Packed8*>(p)->v = static_cast<uint32_t>(r[0]) | (static_cast<unsigned long long>(static_cast<uint32_t>(r[1])) << 32);
+        r[0] = r[2]; r[1] = r[3]; p += 8;
+    }
+    if (n & 4) { reinterpret_cast<Packed4*>(p)->v = static_cast<uint32_t>(r[0]); r[0] = r[1]; p += 4; }
+    if (n & 2) { reinterpret_cast<Packed2*>(p)->v = static_cast<uint16_t>(r[0]); r[0] = static_cast<int>(static_cast<uint32_t>(r[0]) >> 16); p += 2; }
+    if (n & 1) *p = static_cast<uint8_t>(r[0]);
+}
+
+// ---------------------------------------------------------------------------------------------------------
 // Implicit GEMM on MFMA.
 //
 //   GEMM view: rows m = (n, oy, ox) output pixels, columns = output channels, K = (ky, kx, ci) with ci
@@ -155,6 +192,12 @@ __global__ __launch_bounds__(256) void DepthwiseC4Kernel(ConvGeom g, Requant rq,
 //   activation fragments a lane reads for the MFMA anyway -- the two lanes that hold the halves of a pixel's k-slice
 //   add up at the end -- and enters the accumulators just before they are requantized.
 //
+//   Channel counts that are no multiple of 16 (template RG): a tap takes Ck = Ci rounded up to 16 bytes of K, its weights
+//   zero from Ci on, so a chunk of 16 bytes that reaches into the next pixel multiplies those bytes by nothing; only a
+//   chunk that would reach beyond the tensor is read from x_last16 and shifted into place, and only a row sum (AW) needs
+//   the foreign bytes replaced.  Pixels start at any byte then, which costs the loads nothing measurable against the
+//   bytes they move (3 x 3 stride 2, 9 x 75 x 75 x 72 -> 120: 321 us one thread per output, 10.4 us here).
+//
 //   Block = 256 threads = 4 waves arranged WM x WN; each wave owns (BM/WM) x (BN/WN) outputs as 32x32 MFMA
 //   tiles.  The MFMA "A" operand is the weight fragment (row = channel) and "B" the activation fragment
 //   (column = pixel), so a lane ends up with 4 consecutive channels of one pixel per accumulator quad: the
@@ -171,6 +214,8 @@ struct IgemmArgs
     uint8_t*       y;
     int M;                  // batch * Ho * Wo
     int H, W, Ci, Ho, Wo, Co;
+    int Ck = 0;             // RG: bytes of a K row per filter tap, Ci rounded up to 16 (weights are zero between Ci and Ck)
+    const uint8_t* x_last16 = nullptr;   // RG: the last address of the input from which 16 bytes can be read
     int Kh, Kw;
     int pad_top, pad_left, stride_x, stride_y, dil_x, dil_y;
     int K_pad;
@@ -183,6 +228,7 @@ struct IgemmArgs
     uint32_t pad_word;      // shifted input zero point replicated in 4 bytes
     int zw_neg;             // minus the zero point of the stored int8 weights (0: symmetric)
     int rowsum_bias;        // (K_pad - K) * zx': what the bytes beyond K add to a row sum
+    int vec_out = 0;        // IgemmKernel: output rows are whole, aligned 16-byte pieces
     Requant rq;
     const uint8_t* res = nullptr;   // direct-to-LDS kernel: the other input of an Addition fused into the write-out ([M][Co]), or null
     AddFuse add;
@@ -204,9 +250,10 @@ constexpr int IgemmSmemBytes()
 // UT ("uniform tap"): Ci is a multiple of BK, so a k-tile never straddles two filter taps.  The walk over (ky, kx, ci) is
 // then the same for every thread (scalar registers), and a thread's address is a fixed per-row pointer plus a scalar
 // tap offset: no per-load multiplications.
-template <int BM, int BN, int WM, int WN, int D, int BK, bool UT, bool AW = false>
+template <int BM, int BN, int WM, int WN, int D, int BK, bool UT, bool AW = false, bool RG = false>
 __global__ __launch_bounds__(256) void IgemmKernel(IgemmArgs a)
 {
+    static_assert(!(UT && RG), "a channel count that is a multiple of the k-tile is not ragged");
     static_assert(WM * WN == 4, "4 waves per block");
     static_assert(D >= 2 && D <= 4, "2 to 4 register slots");
     static_assert(BM % 64 == 0 && BN % 64 == 0, "tile sizes are multiples of 64");
@@ -275,19 +322,22 @@ __global__ __launch_bounds__(256) void IgemmKernel(IgemmArgs a)
         if constexpr (UT) xrow[j] += (static_cast<long long>(iy0[j]) * a.W + ix0[j]) * a.Ci + lc * 16;
     }
     // position of this thread's chunk inside K: (ky, kx, ci), advanced by BK every k-tile
+    const int tap_bytes = RG ? a.Ck : a.Ci;
     int ci, kx, ky;
     if constexpr (UT) { ci = 0; kx = 0; ky = 0; }       // of the k-tile: identical in every thread
     else
     {
         const int k0 = lc * 16;
-        const int tap = k0 / a.Ci;
-        ci = k0 - tap * a.Ci;
+        const int tap = k0 / tap_bytes;
+        ci = k0 - tap * tap_bytes;
         ky = tap / a.Kw;
         kx = tap - ky * a.Kw;
     }
     const int8_t* wrow = a.w + static_cast<long long>(tn * BN + lr) * a.K_pad + lc * 16;
 
     v4i ra[D][RA], rb[D][RB];
+    int back[RG ? D : 1][RG ? RA : 1];           // RG: bytes a chunk was read ahead of its place (0 but at the tensor's end)
+    int real[RG && AW ? D : 1];                  // RG, AW: channels of the chunk that exist
     const int xm = static_cast<int>(a.xor_mask);
 
     auto load_tile = [&](int kt, auto slot) {
@@ -307,8 +357,15 @@ __global__ __launch_bounds__(256) void IgemmKernel(IgemmArgs a)
             // waited for on the spot, which would serialise the prefetch).
             const uint8_t* in = UT ? xrow[j] + tap_off : xrow[j] + ((static_cast<long long>(iy) * a.W + ix) * a.Ci + ci);
             const uint8_t* src = ok ? in : a.pad16;
-            ra[SL][j] = *reinterpret_cast<const v4i*>(src);   // the xor waits until the value goes to LDS
+            if constexpr (RG)
+            {
+                const int over = ok && in > a.x_last16 ? static_cast<int>(in - a.x_last16) : 0;
+                back[SL][j] = over;
+                ra[SL][j] = LoadUnaligned16(src - over);
+            }
+            else ra[SL][j] = *reinterpret_cast<const v4i*>(src);   // the xor waits until the value goes to LDS
         }
+        if constexpr (RG && AW) real[SL] = min(16, a.Ci - ci);
 #pragma unroll
         for (int j = 0; j < RB; ++j)
         {
@@ -316,9 +373,9 @@ __global__ __launch_bounds__(256) void IgemmKernel(IgemmArgs a)
         }
         // advance (ky, kx, ci) by one k-tile
         ci += BK;
-        while (ci >= a.Ci)
+        while (ci >= tap_bytes)
         {
-            ci -= a.Ci;
+            ci -= tap_bytes;
             if (++kx == a.Kw) { kx = 0; ++ky; }
         }
     };
@@ -328,7 +385,27 @@ __global__ __launch_bounds__(256) void IgemmKernel(IgemmArgs a)
         uint8_t* As = smem + buf * STAGE;
         uint8_t* Bs = As + BM * LDK;
 #pragma unroll
-        for (int j = 0; j < RA; ++j) *reinterpret_cast<v4i*>(As + (lr + RP * j) * LDK + lc * 16) = ra[SL][j] ^ xm;
+        for (int j = 0; j < RA; ++j)
+        {
+            v4i v = ra[SL][j];
+            if constexpr (RG)
+            {
+                if (__builtin_expect(__builtin_amdgcn_ballot_w64(back[SL][j] != 0) != 0, 0)) v = ShiftDown16(v, back[SL][j]);
+            }
+            v ^= xm;
+            if constexpr (RG && AW)
+            {
+                // channels that do not exist count as padding in the row sum
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                {
+                    const int n = real[SL] - 4 * i;
+                    const uint32_t keep = n >= 4 ? 0xffffffffu : n <= 0 ? 0u : (1u << (8 * n)) - 1u;
+                    v[i] = static_cast<int>((static_cast<uint32_t>(v[i]) & keep) | (a.pad_word & ~keep));
+                }
+            }
+            *reinterpret_cast<v4i*>(As + (lr + RP * j) * LDK + lc * 16) = v;
+        }
 #pragma unroll
         for (int j = 0; j < RB; ++j) *reinterpret_cast<v4i*>(Bs + (lr + RP * j) * LDK + lc * 16) = rb[SL][j];
     };
@@ -452,7 +529,7 @@ __global__ __launch_bounds__(256) void IgemmKernel(IgemmArgs a)
     const int orow = tid / CHUNKS;
     const int c0 = tn * BN + oc * 16;
     const OutPtr outp = MakeOutPtr(a.y, static_cast<long long>(a.M) * a.Co);
-    if ((a.Co & 15) == 0)
+    if (a.vec_out)
     {
         if (c0 < a.Co)
         {
@@ -470,16 +547,12 @@ __global__ __launch_bounds__(256) void IgemmKernel(IgemmArgs a)
     }
     else
     {
-        // ragged channel count (e.g. 1001 classes): rows are not 16-byte aligned, store byte by byte
+        // ragged channel count (e.g. 1001 classes): rows start at any byte
         for (int r = orow; r < BM; r += ROWS_PER_PASS)
         {
             const int m = tm * BM + r;
-            if (m >= a.M) continue;
-            for (int b = 0; b < 16; ++b)
-            {
-                const int c = c0 + b;
-                if (c < a.Co) a.y[static_cast<long long>(m) * a.Co + c] = Os[r * LDO + oc * 16 + b];
-            }
+            if (m < a.M && c0 < a.Co)
+                StoreRagged16(a.y + static_cast<long long>(m) * a.Co + c0, *reinterpret_cast<const v4i*>(Os + r * LDO + oc * 16), a.Co - c0);
         }
     }
 }

@@ -278,11 +278,7 @@ __global__ __launch_bounds__(256) void HaloConvKernel(HaloArgs a)
     else
     {
         for (int r = orow; r < mt; r += ROWS_PER_PASS)
-            for (int b = 0; b < 16; ++b)
-            {
-                const int c = c0 + b;
-                if (c < a.Co) yt[static_cast<long long>(r) * a.Co + c] = Os[r * LDO + oc * 16 + b];
-            }
+            if (c0 < a.Co) StoreRagged16(yt + static_cast<long long>(r) * a.Co + c0, *reinterpret_cast<const v4i*>(Os + r * LDO + oc * 16), a.Co - c0);
     }
 }
 

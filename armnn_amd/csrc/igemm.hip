@@ -1,0 +1,84 @@
+// Launches of the register-staged implicit GEMM.
+#include "igemm.h"
+
+#include "common.h"
+#include "conv_kernels.h"
+
+using namespace mi355x;
+
+namespace
+{
+template <int BM, int BN, int WM, int WN, int D, int BK, bool UT, bool AW, bool RG>
+int LaunchIgemmT(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, hipStream_t stream)
+{
+    const ConvGeom& g = p->geom;
+    IgemmArgs a;
+    a.x = static_cast<const uint8_t*>(x);
+    a.pad16 = p->pad16;
+    a.w = p->w_mfma;
+    a.ct = ChanTab{p->chan, p->Co_pad};
+    a.corr = p->corr;
+    a.y = static_cast<uint8_t*>(y);
+    const long long M = static_cast<long long>(batch) * g.Ho * g.Wo;
+    if (M > 0x7fffffffll / 2) return SetError(MI355X_ERR_UNSUPPORTED, "too many output pixels for one launch (%lld)", M);
+    a.M = static_cast<int>(M);
+    a.H = g.H; a.W = g.W; a.Ci = g.Ci; a.Ho = g.Ho; a.Wo = g.Wo; a.Co = g.Co;
+    if (RG)
+    {
+        a.Ck = p->ragged_ck;
+        a.x_last16 = a.x + static_cast<long long>(batch) * g.H * g.W * g.Ci - 16;     // (an image has at least 16 bytes)
+    }
+    a.vec_out = (g.Co & 15) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0;
+    a.Kh = g.Kh; a.Kw = g.Kw;
+    a.pad_top = g.pad_top; a.pad_left = g.pad_left; a.stride_x = g.stride_x; a.stride_y = g.stride_y;
+    a.dil_x = g.dil_x; a.dil_y = g.dil_y;
+    a.K_pad = p->K_pad;
+    a.unit = (g.Kh == 1 && g.Kw == 1 && g.stride_x == 1 && g.stride_y == 1 && g.pad_top == 0 && g.pad_left == 0 && g.Ho == g.H &&
+              g.Wo == g.W) ? 1 : 0;
+    if (a.unit) { a.H = 1; a.W = a.M; a.Ho = 1; a.Wo = a.M; }      // one row of M pixels
+    a.tiles_m = static_cast<int>((M + BM - 1) / BM);
+    a.tiles_n = (g.Co + BN - 1) / BN;
+    a.xor_mask = p->xor_mask;
+    a.pad_word = p->pad_word;
+    a.zw_neg = p->zw_neg;
+    a.rowsum_bias = p->rowsum_bias;
+    a.rq = p->rq;
+    const int nblocks = a.tiles_m * a.tiles_n;
+    const int grid = (nblocks + 7) / 8 * 8;
+    constexpr int smem = IgemmSmemBytes<BM, BN, BK>();
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&IgemmKernel<BM, BN, WM, WN, D, BK, UT, AW, RG>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+    MI355X_HIP(attr);
+    NoteKernel("IgemmKernel<%d, %d, %d, %d, %d, %d, %s, %s, %s>", BM, BN, WM, WN, D, BK, BoolName(UT), BoolName(AW), BoolName(RG));
+    hipLaunchKernelGGL((IgemmKernel<BM, BN, WM, WN, D, BK, UT, AW, RG>), dim3(grid), dim3(256), smem, stream, a);
+    MI355X_HIP(hipGetLastError());
+    return 0;
+}
+
+// uniform-tap variant whenever a k-tile cannot straddle two filter taps; row sums when the weights have a zero point
+template <int BM, int BN, int WM, int WN, int D, int BK>
+int LaunchTile(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, hipStream_t stream)
+{
+    if constexpr (BK == 64)
+    {
+        if (p->ragged_ck != 0)
+            return p->zw_neg != 0 ? LaunchIgemmT<BM, BN, WM, WN, D, BK, false, true, true>(p, batch, x, y, stream)
+                                  : LaunchIgemmT<BM, BN, WM, WN, D, BK, false, false, true>(p, batch, x, y, stream);
+    }
+    const bool ut = (p->geom.Ci % BK) == 0;
+    if (p->zw_neg != 0)
+        return ut ? LaunchIgemmT<BM, BN, WM, WN, D, BK, true, true, false>(p, batch, x, y, stream)
+                  : LaunchIgemmT<BM, BN, WM, WN, D, BK, false, true, false>(p, batch, x, y, stream);
+    return ut ? LaunchIgemmT<BM, BN, WM, WN, D, BK, true, false, false>(p, batch, x, y, stream)
+              : LaunchIgemmT<BM, BN, WM, WN, D, BK, false, false, false>(p, batch, x, y, stream);
+}
+} // namespace
+
+int mi355x::LaunchIgemm(const mi355x_conv2d_s* p, int tile, uint32_t batch, const void* x, void* y, hipStream_t stream)
+{
+    const bool bk128 = p->bk128;
+    if (tile == 64) return bk128 ? LaunchTile<64, 64, 2, 2, 2, 128>(p, batch, x, y, stream) : LaunchTile<64, 64, 2, 2, 2, 64>(p, batch, x, y, stream);
+    if (p->geom.Co <= 64 || tile == 96)
+        return bk128 ? LaunchTile<128, 64, 2, 2, 2, 128>(p, batch, x, y, stream) : LaunchTile<128, 64, 2, 2, 2, 64>(p, batch, x, y, stream);
+    return bk128 ? LaunchTile<128, 128, 2, 2, 2, 128>(p, batch, x, y, stream) : LaunchTile<128, 128, 2, 2, 2, 64>(p, batch, x, y, stream);
+}

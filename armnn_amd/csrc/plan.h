@@ -45,6 +45,7 @@ struct mi355x_conv2d_s
     int opt_igemm_lds = 2, opt_dw_rows = 0, opt_dw_cb = 0, opt_dw_mfma = 1, opt_stem_dot4 = 0;     // the other process-wide options, as they stood at plan creation
                                    // (launches read the plan, never the mutable globals: plans may run on any host thread)
     uint32_t xor_mask = 0, pad_word = 0;
+    int ragged_ck = 0;             // MFMA plans: bytes of K per filter tap where the channel count is no multiple of 16 (else 0)
     int zw_neg = 0;                // MFMA plans: minus the zero point of the stored int8 weights (0: symmetric)
     int rowsum_bias = 0;           // ... and what the bytes between K and K_pad add to a row's sum of activations
     std::string info;

@@ -189,11 +189,14 @@ __global__ __launch_bounds__(256) void PwGemmKernel(PwArgs a)
         }
         else
         {
-            for (int j = lane; j < 32 * BN; j += 64)
+#pragma unroll
+            for (int j = lane; j < 32 * CH; j += 64)
             {
-                const int r = j / BN, c = j % BN;
+                const int r = j / CH, cc = j % CH;
                 const int row = t * 32 + r;
-                if (row < a.M && n0 + c < a.N) a.y[static_cast<long long>(row) * a.N + n0 + c] = ostage[r * LDO + c];
+                const int c0 = n0 + cc * 16;
+                if (row < a.M && c0 < a.N)
+                    StoreRagged16(a.y + static_cast<long long>(row) * a.N + c0, *reinterpret_cast<const v4i*>(ostage + r * LDO + cc * 16), a.N - c0);
             }
         }
         // and the next tile's staging writes must stay behind these reads
@@ -459,7 +462,7 @@ __device__ __forceinline__ void SmallMGemmTile(const GemvArgs& a, int n0, int m0
     else if (row < a.M)
     {
         uint8_t* dst = a.y + static_cast<long long>(row) * a.N + c;
-        if ((a.N & 3) == 0 && c + 3 < a.N) *reinterpret_cast<uint32_t*>(dst) = out;
+        if (c + 3 < a.N) reinterpret_cast<Packed4*>(dst)->v = out;
         else
         {
 #pragma unroll
