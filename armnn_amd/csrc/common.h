@@ -113,5 +113,7 @@ struct UploadScope
     UploadScope(const UploadScope&) = delete;
     UploadScope& operator=(const UploadScope&) = delete;
 };
+// The calling thread's upload stream, for work on constants that are already on the device (an UploadScope must be open).
+int UploadStream(hipStream_t* stream);
 
 } // namespace mi355x

@@ -40,6 +40,7 @@ thread_local PendingAdd* t_pending_add = nullptr;
 // unit roundoff of fp32 and the relative half-width of the requantization bracket (device_math.h)
 constexpr double kBracketUnit = 1.0 / 16777216.0;
 constexpr double kBracketRel = 16.0 / 16777216.0;
+constexpr long long kSmallConvMostTiles = 392, kSmallConvLeastSlabTiles = 128;
 
 
 void FoldCorrIntoTable(mi355x_conv2d_s* p, const std::vector<int32_t>& corr, int Co);
@@ -298,6 +299,7 @@ int BuildPlan(const mi355x_conv2d_desc& d, const void* weights_host, const mi355
         p->rowsum_bias = (p->K_pad - p->K) * zx_shift;     // kernels that walk K_pad bytes meet zx' beyond K
         if (int rc = Upload(reinterpret_cast<void**>(&p->w_mfma), wp.data(), wp.size())) return rc;
         if (int rc = Upload(reinterpret_cast<void**>(&p->corr), corr.data(), corr.size() * sizeof(int32_t))) return rc;
+        if (int rc = PackFragments(p)) return rc;
         p->xor_mask = g.in_u8 ? 0x80808080u : 0u;
         const uint32_t zb = static_cast<uint32_t>(zx_shift) & 0xffu;
         p->pad_word = zb | (zb << 8) | (zb << 16) | (zb << 24);
@@ -397,7 +399,7 @@ int BuildPlan(const mi355x_conv2d_desc& d, const void* weights_host, const mi355
     {
         const int RD = Kh == 3 ? 3 : Kh == 7 ? 6 : Kh == 5 ? 5 : 1;
         std::vector<uint32_t> wp(static_cast<size_t>(Co) * Kh * RD, 0u), wp2(static_cast<size_t>(Co) * Kh * RD, 0u);
-        std::vector<int32_t> corr(Co, 0);
+        std::vector<int32_t> corr((Co + 63) / 64 * 64, 0);     // the matrix-core kernel reads whole blocks of channels
         for (int c = 0; c < Co; ++c)
         {
             long long sum = 0;
@@ -426,7 +428,7 @@ int BuildPlan(const mi355x_conv2d_desc& d, const void* weights_host, const mi355
             const std::vector<uint8_t> padbytes(16, static_cast<uint8_t>((p->pad_word ^ p->xor_mask) & 0xffu));
             if (int rc = Upload(reinterpret_cast<void**>(&p->pad16), padbytes.data(), padbytes.size())) return rc;
         }
-        if (Co == 32 || Co == 64)
+        if (Co <= 64)
         {
             // the same rows, end to end, as the K vector of the MFMA variant
             const int kp = (Kh * RD * 4 + 31) / 32 * 32;
@@ -996,6 +998,23 @@ int RunPlan(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, hi
             MI355X_HIP(hipGetLastError());
             return 0;
         }
+        // Few rows: 32 x 32 tiles whose waves split K (small_conv_kernel.h), while they number at most one and a half per CU: at
+        // 392 of them 14 x 14 x 256 at 8 images, 3 x 3, takes 8.0 us against 9.5; from there on the larger tiles' lower traffic
+        // wins (14 x 14 x 512 -> 512 at 8 images, 784 tiles: 5.5 against 4.7).  Where the layer has a weight slab (at most 128 input
+        // channels, 1x1) from 128 tiles on: 128 -> 256 at 28 x 28, 200 tiles, 5.6 -> 3.1 us.
+        const long long small_tiles = (rows + 31) / 32 * ((g.Co + 31) / 32);
+        if (p->w_frag && p->tile_override == 0 && small_tiles <= kSmallConvMostTiles && (!p->pw_bn || small_tiles >= kSmallConvLeastSlabTiles))
+        {
+            // an Addition behind the layer joins the write-out of the layers whose larger tiles could take it as well, while the
+            // tiles are few (its 16-byte piece per lane is one more round trip of the single wave that writes)
+            const bool takes_add = (g.Ci % 128) == 0 && (g.Co & 15) == 0 && small_tiles <= 256;
+            if (!t_pending_add || takes_add || (g.Ci % 128 != 0 && !p->pw_bn))
+            {
+                const uint8_t* res = nullptr;
+                if (t_pending_add && takes_add) { res = t_pending_add->other; t_pending_add->taken = true; }
+                return LaunchSmallConv(p, batch, x, y, res, res ? &t_pending_add->fuse : nullptr, stream);
+            }
+        }
         if (unit && rows <= 64 && (g.Ci % 16) == 0 && g.Ci >= 128 && p->tile_override == 0 && p->Co_pad >= (g.Co + 31) / 32 * 32 &&
             (reinterpret_cast<uintptr_t>(y) & 3) == 0)
         {
@@ -1136,24 +1155,24 @@ int RunPlan(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, hi
                 nbm = static_cast<long long>(batch) * a.tiles_x * a.tiles_y;
             }
             const dim3 gridm(static_cast<unsigned>(nbm));
-            NoteKernel("SmallCiMfmaKernel<%d, %d, %d, %d, %s>", g.Kh, g.Kh == 3 ? 3 : 6, g.Co == 32 ? 1 : 2, th8 ? 8 : 16, BoolName(p->w_stem2 != nullptr));
+            NoteKernel("SmallCiMfmaKernel<%d, %d, %d, %d, %s>", g.Kh, g.Kh == 3 ? 3 : 6, g.Co <= 32 ? 1 : 2, th8 ? 8 : 16, BoolName(p->w_stem2 != nullptr));
             if (th8)
             {
-                if (g.Kh == 3 && g.Co == 32) hipLaunchKernelGGL((SmallCiMfmaKernel<3, 3, 1, 8>), gridm, dim3(256), 0, stream, a);
+                if (g.Kh == 3 && g.Co <= 32) hipLaunchKernelGGL((SmallCiMfmaKernel<3, 3, 1, 8>), gridm, dim3(256), 0, stream, a);
                 else if (g.Kh == 3) hipLaunchKernelGGL((SmallCiMfmaKernel<3, 3, 2, 8>), gridm, dim3(256), 0, stream, a);
-                else if (g.Co == 32) hipLaunchKernelGGL((SmallCiMfmaKernel<7, 6, 1, 8>), gridm, dim3(256), 0, stream, a);
+                else if (g.Co <= 32) hipLaunchKernelGGL((SmallCiMfmaKernel<7, 6, 1, 8>), gridm, dim3(256), 0, stream, a);
                 else hipLaunchKernelGGL((SmallCiMfmaKernel<7, 6, 2, 8>), gridm, dim3(256), 0, stream, a);
             }
             else if (p->w_stem2)
             {
-                if (g.Kh == 3 && g.Co == 32) hipLaunchKernelGGL((SmallCiMfmaKernel<3, 3, 1, 16, true>), gridm, dim3(256), 0, stream, a);
+                if (g.Kh == 3 && g.Co <= 32) hipLaunchKernelGGL((SmallCiMfmaKernel<3, 3, 1, 16, true>), gridm, dim3(256), 0, stream, a);
                 else if (g.Kh == 3) hipLaunchKernelGGL((SmallCiMfmaKernel<3, 3, 2, 16, true>), gridm, dim3(256), 0, stream, a);
-                else if (g.Co == 32) hipLaunchKernelGGL((SmallCiMfmaKernel<7, 6, 1, 16, true>), gridm, dim3(256), 0, stream, a);
+                else if (g.Co <= 32) hipLaunchKernelGGL((SmallCiMfmaKernel<7, 6, 1, 16, true>), gridm, dim3(256), 0, stream, a);
                 else hipLaunchKernelGGL((SmallCiMfmaKernel<7, 6, 2, 16, true>), gridm, dim3(256), 0, stream, a);
             }
-            else if (g.Kh == 3 && g.Co == 32) hipLaunchKernelGGL((SmallCiMfmaKernel<3, 3, 1, 16>), gridm, dim3(256), 0, stream, a);
+            else if (g.Kh == 3 && g.Co <= 32) hipLaunchKernelGGL((SmallCiMfmaKernel<3, 3, 1, 16>), gridm, dim3(256), 0, stream, a);
             else if (g.Kh == 3) hipLaunchKernelGGL((SmallCiMfmaKernel<3, 3, 2, 16>), gridm, dim3(256), 0, stream, a);
-            else if (g.Co == 32) hipLaunchKernelGGL((SmallCiMfmaKernel<7, 6, 1, 16>), gridm, dim3(256), 0, stream, a);
+            else if (g.Co <= 32) hipLaunchKernelGGL((SmallCiMfmaKernel<7, 6, 1, 16>), gridm, dim3(256), 0, stream, a);
             else hipLaunchKernelGGL((SmallCiMfmaKernel<7, 6, 2, 16>), gridm, dim3(256), 0, stream, a);
             MI355X_HIP(hipGetLastError());
             return 0;

@@ -159,6 +159,20 @@ __device__ __forceinline__ v4i ShiftDown16(const v4i& v, int n)
     return r;
 }
 
+// bytes n .. 15 of v replaced by those of the dword `pad` (n may be 16 and more)
+__device__ __forceinline__ v4i KeepBytes16(const v4i& v, int n, uint32_t pad)
+{
+    v4i r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+    {
+        const int k = n - 4 * i;
+        const uint32_t keep = k >= 4 ? 0xffffffffu : k <= 0 ? 0u : (1u << (8 * k)) - 1u;
+        r[i] = static_cast<int>((static_cast<uint32_t>(v[i]) & keep) | (pad & ~keep));
+    }
+    return r;
+}
+
 // the first min(n, 16) bytes of v to any address: one store where the piece is whole, else one per power of two
 __device__ __forceinline__ void StoreRagged16(uint8_t* p, const v4i& v, int n)
 {
@@ -395,14 +409,7 @@ __global__ __launch_bounds__(256) void IgemmKernel(IgemmArgs a)
             v ^= xm;
             if constexpr (RG && AW)
             {
-                // channels that do not exist count as padding in the row sum
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                {
-                    const int n = real[SL] - 4 * i;
-                    const uint32_t keep = n >= 4 ? 0xffffffffu : n <= 0 ? 0u : (1u << (8 * n)) - 1u;
-                    v[i] = static_cast<int>((static_cast<uint32_t>(v[i]) & keep) | (a.pad_word & ~keep));
-                }
+                v = KeepBytes16(v, real[SL], a.pad_word);       // channels that do not exist count as padding in the row sum
             }
             *reinterpret_cast<v4i*>(As + (lr + RP * j) * LDK + lc * 16) = v;
         }

@@ -528,7 +528,8 @@ __global__ __launch_bounds__(256) void SmallCiConvKernel(SmallCiArgs a)
 // holds a pixel's inputs in registers; laid end to end, the KH rows are a K vector of KH*RD*4 bytes (zero weights under
 // the padding), and 32 pixels x 32 output channels become ceil(KH*RD/8) MFMA steps instead of 32*KH*RD dot products per
 // pixel.  Both lanes of a pixel (lane, lane + 32) gather the pixel's rows from the LDS halo and keep the half of each
-// 32-byte k-step that the MFMA B operand assigns them.  A wave takes 4 of the tile's 16 rows; NT = output channels / 32.
+// 32-byte k-step that the MFMA B operand assigns them.  A wave takes 4 of the tile's 16 rows; NT = output channels / 32, rounded up (weight rows past
+// the layer's last channel are zero and store nothing).
 template <int KH, int RD, int NT, int TH, bool W2 = false>
 __global__ __launch_bounds__(256) void SmallCiMfmaKernel(SmallCiArgs a)
 {
@@ -635,11 +636,19 @@ __global__ __launch_bounds__(256) void SmallCiMfmaKernel(SmallCiArgs a)
             const uint4 v = half ? uint4{r0, o[2], r1, o[3]} : uint4{o[0], r0, o[1], r1};
             if (ox < a.Wo)
             {
-                if (a.vec16) StoreOut16(outp, (yp - a.y) + ct * 32 + 16 * half, StoreVec4{static_cast<int>(v.x), static_cast<int>(v.y), static_cast<int>(v.z), static_cast<int>(v.w)});
+                const int c0 = ct * 32 + 16 * half;
+                if (a.vec16)
+                {
+                    if (c0 < a.Co) StoreOut16(outp, (yp - a.y) + c0, StoreVec4{static_cast<int>(v.x), static_cast<int>(v.y), static_cast<int>(v.z), static_cast<int>(v.w)});
+                }
                 else
                 {
-                    uint32_t* dst = reinterpret_cast<uint32_t*>(yp + ct * 32 + 16 * half);
-                    dst[0] = v.x; dst[1] = v.y; dst[2] = v.z; dst[3] = v.w;
+                    // (channels come in fours; those past the layer's last one do not exist)
+                    uint32_t* dst = reinterpret_cast<uint32_t*>(yp + c0);
+                    if (c0 < a.Co) dst[0] = v.x;
+                    if (c0 + 4 < a.Co) dst[1] = v.y;
+                    if (c0 + 8 < a.Co) dst[2] = v.z;
+                    if (c0 + 12 < a.Co) dst[3] = v.w;
                 }
             }
         }

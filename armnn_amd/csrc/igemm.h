@@ -9,4 +9,11 @@ namespace mi355x
 // `tile`: 64, 96 (128 x 64) or anything else (128 x 128, 128 x 64 for at most 64 output channels).  `p` is a MI355X_ALGO_MFMA plan.
 int LaunchIgemm(const mi355x_conv2d_s* p, int tile, uint32_t batch, const void* x, void* y, hipStream_t stream);
 
+// w_frag of an MFMA plan from its w_mfma (PackFragKernel), queued on the calling thread's upload stream.
+int PackFragments(mi355x_conv2d_s* p);
+
+// SmallConvKernel (small_conv_kernel.h) for a plan with w_frag.  res / add: an Addition behind the layer (output channels
+// % 16 == 0, aligned tensors), or null.
+int LaunchSmallConv(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, const uint8_t* res, const AddFuse* add, hipStream_t stream);
+
 } // namespace mi355x

@@ -3,6 +3,7 @@
 
 #include "common.h"
 #include "conv_kernels.h"
+#include "small_conv_kernel.h"
 
 using namespace mi355x;
 
@@ -81,4 +82,39 @@ int mi355x::LaunchIgemm(const mi355x_conv2d_s* p, int tile, uint32_t batch, cons
     if (p->geom.Co <= 64 || tile == 96)
         return bk128 ? LaunchTile<128, 64, 2, 2, 2, 128>(p, batch, x, y, stream) : LaunchTile<128, 64, 2, 2, 2, 64>(p, batch, x, y, stream);
     return bk128 ? LaunchTile<128, 128, 2, 2, 2, 128>(p, batch, x, y, stream) : LaunchTile<128, 128, 2, 2, 2, 64>(p, batch, x, y, stream);
+}
+
+int mi355x::PackFragments(mi355x_conv2d_s* p)
+{
+    const int steps = (p->geom.Kh * p->geom.Kw * (p->ragged_ck ? p->ragged_ck : p->geom.Ci) + 63) / 64;
+    const long long pieces = static_cast<long long>(p->Co_pad / 16) * steps * 64;
+    MI355X_HIP(hipMalloc(reinterpret_cast<void**>(&p->w_frag), pieces * 16));
+    hipStream_t stream;
+    if (const int rc = UploadStream(&stream)) return rc;
+    hipLaunchKernelGGL(PackFragKernel, dim3(static_cast<unsigned>((pieces + 255) / 256)), dim3(256), 0, stream, p->w_mfma, p->w_frag, p->K_pad, steps, pieces);
+    MI355X_HIP(hipGetLastError());
+    MI355X_HIP(hipStreamSynchronize(stream));
+    return 0;
+}
+
+int mi355x::LaunchSmallConv(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, const uint8_t* res, const AddFuse* add, hipStream_t stream)
+{
+    IgemmArgs a;
+    bool unit_fast = false;
+    if (const int rc = FillIgemmLdsArgs(p, 32, 32, batch, x, y, &a, &unit_fast)) return rc;
+    a.vec_out = (p->geom.Co & 15) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0;
+    a.w = p->w_frag;
+    if (res) { a.res = res; a.add = *add; }
+    const int grid = (a.tiles_m * a.tiles_n + 7) / 8 * 8;
+    const bool aw = p->zw_neg != 0, rg = p->ragged_ck != 0;
+    if (rg)
+    {
+        a.Ck = p->ragged_ck;
+        a.x_last16 = a.x + static_cast<long long>(batch) * p->geom.H * p->geom.W * p->geom.Ci - 16;
+    }
+    NoteKernel("SmallConvKernel<%s, %s>", BoolName(aw), BoolName(rg));
+    const auto kernel = aw ? (rg ? SmallConvKernel<true, true> : SmallConvKernel<true, false>) : (rg ? SmallConvKernel<false, true> : SmallConvKernel<false, false>);
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, stream, a);
+    MI355X_HIP(hipGetLastError());
+    return 0;
 }

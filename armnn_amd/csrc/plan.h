@@ -19,6 +19,7 @@ struct mi355x_conv2d_s
     // device constants
     uint8_t* w_direct = nullptr;   // [Kh][Kw][Ci][Co] / depthwise [Kh][Kw][Co], raw codes
     int8_t*  w_mfma   = nullptr;   // [Co_pad][K_pad] signed, zero padded
+    int8_t*  w_frag   = nullptr;   // the same weights in operand order (small_conv_kernel.h), where a launch may want them
     uint8_t* pad16    = nullptr;   // 16 bytes that turn into the padding value under the kernel's input xor
     int8_t*  w_stem   = nullptr;   // small-Ci conv on MFMA: [Co rounded up to 32][stem_kp]
     int8_t*  w_stem2  = nullptr;   // ... the second halves of weight differences that need two
@@ -54,6 +55,7 @@ struct mi355x_conv2d_s
     {
         (void)hipFree(w_direct);
         (void)hipFree(w_mfma);
+        (void)hipFree(w_frag);
         (void)hipFree(pad16);
         (void)hipFree(dw_grp);
         (void)hipFree(w_stem);

@@ -67,14 +67,22 @@ UploadScope::~UploadScope()
     t_upload_stream = nullptr;
 }
 
+int UploadStream(hipStream_t* stream)
+{
+    if (!t_upload_stream) t_upload_stream = SwapIdleUploadStream(nullptr);
+    if (!t_upload_stream) MI355X_HIP(hipStreamCreateWithFlags(&t_upload_stream, hipStreamNonBlocking));
+    *stream = t_upload_stream;
+    return 0;
+}
+
 int UploadNow(void* dst_dev, const void* src_host, size_t bytes)
 {
     // one stream per calling thread, so concurrent plan creations do not wait for each other
     UploadScope scope;
-    if (!t_upload_stream) t_upload_stream = SwapIdleUploadStream(nullptr);
-    if (!t_upload_stream) MI355X_HIP(hipStreamCreateWithFlags(&t_upload_stream, hipStreamNonBlocking));
-    MI355X_HIP(hipMemcpyAsync(dst_dev, src_host, bytes, hipMemcpyHostToDevice, t_upload_stream));
-    MI355X_HIP(hipStreamSynchronize(t_upload_stream));
+    hipStream_t stream;
+    if (const int rc = UploadStream(&stream)) return rc;
+    MI355X_HIP(hipMemcpyAsync(dst_dev, src_host, bytes, hipMemcpyHostToDevice, stream));
+    MI355X_HIP(hipStreamSynchronize(stream));
     return 0;
 }
 
