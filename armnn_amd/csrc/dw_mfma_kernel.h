@@ -257,6 +257,9 @@ __global__ __launch_bounds__((DwMfmaTile<S, CB, TH, TW>::NT)) void DepthwiseMfma
         }
     };
     issue(item);
+    // the first item's constants travel beside its halo (a launch of one item per block would otherwise wait for memory twice)
+    cur_cb = decode(item).cb;
+    constants(cur_cb);
     int buf = 0;
     while (true)
     {

@@ -95,6 +95,11 @@ __global__ __launch_bounds__(256) void SmallConvKernel(IgemmArgs a)
         ky = tap / a.Kw;
         kx = tap - ky * a.Kw;
     }
+    // what this wave will requantize with (wave 2 c + p finishes channel group c of pixel group p), requested ahead of the operands
+    const int cg = wave >> 1, pg = wave & 1;
+    const int cq = tn * 32 + cg * 16 + 4 * g;
+    const v4i corr4 = *reinterpret_cast<const v4i*>(a.corr + cq);
+    const Fast4 f4 = LoadFast4(a.ct, cq);
     v4i acc[2][2];                                       // [channel group][pixel group]
 #pragma unroll
     for (int c = 0; c < 2; ++c)
@@ -176,22 +181,18 @@ __global__ __launch_bounds__(256) void SmallConvKernel(IgemmArgs a)
     if (fuse && wave == 0) other = *reinterpret_cast<const v4i*>(a.res + static_cast<long long>(min(om, a.M - 1)) * a.Co + min(c0, a.Co - 16));
     __syncthreads();
     {
-        // wave 2 c + p finishes channel group c of pixel group p
-        const int cg = wave >> 1, p = wave & 1;
-        const int c = tn * 32 + cg * 16 + 4 * g;
-        v4i v = *reinterpret_cast<const v4i*>(a.corr + c);
+        v4i v = corr4;
 #pragma unroll
         for (int w = 0; w < NW; ++w) v += part[w][wave][lane];
         if constexpr (AW)
         {
             int total = 0;
 #pragma unroll
-            for (int w = 0; w < NW; ++w) total += rowpart[w][p][j] + rowpart[w][p][j + 16] + rowpart[w][p][j + 32] + rowpart[w][p][j + 48];
+            for (int w = 0; w < NW; ++w) total += rowpart[w][pg][j] + rowpart[w][pg][j + 16] + rowpart[w][pg][j + 32] + rowpart[w][pg][j + 48];
             // what the bytes beyond K added are padding values
             v += (total - (steps * 64 - a.Kh * a.Kw * a.Ci) * static_cast<int>(static_cast<int8_t>(a.pad_word & 0xffu))) * a.zw_neg;
         }
-        const Fast4 f4 = LoadFast4(a.ct, c);
-        stage[p * 16 + j][cg * 4 + g] = Requant4Dev(v[0], v[1], v[2], v[3], f4, a.ct, c, a.rq);
+        stage[pg * 16 + j][cg * 4 + g] = Requant4Dev(v[0], v[1], v[2], v[3], f4, a.ct, cq, a.rq);
     }
     __syncthreads();
     if (wave == 0 && om < a.M && c0 < a.Co)
