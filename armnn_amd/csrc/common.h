@@ -88,7 +88,7 @@ struct Options
     int pwdw_mf = 0;                   // 32-pixel fragments per block of the whole-image kernels (1x1 convolution + depthwise / + pooling): 0 automatic, 2, 4 or 7 forced
     int pool_small = 1;                // 0: pooling over a whole image of at most 64 pixels runs on the LDS-staged kernel (tests compare the two)
     int pwpool_auto = 1;               // 1: mi355x_conv2d_pool_fusion_pays may recommend a 1x1 convolution + the global pooling behind it
-    int dwpw_panel = 1;                // 0: fused depthwise + pointwise launches never take the one-block-per-tile-over-all-channels kernel
+    int dwpw_panel = 1;                // 0: fused depthwise + pointwise launches never take the kernel that keeps a tile of the layer between in LDS
     int chain_stages = 2;              // LDS stages of the matrix-core tiles inside a layer chain (2, 3 or 4), read at mi355x_chain_create
     int chain_defer_signal = 0;        // 1: layer chains count a tile as finished behind the next tile's loads (no wait for its stores)
     int chain_panel = 0;               // 1: layer chains run 1x1 convolutions with 256 or 512 input channels and many rows as one work item per

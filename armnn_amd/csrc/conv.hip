@@ -5,7 +5,7 @@
 #include "dw_stem_kernels.h"
 #include "dw_mfma_kernel.h"
 #include "dwpw_kernel.h"
-#include "dwpw_panel_kernel.h"
+#include "dwpw_panel.h"
 #include "dwpw_stream_kernel.h"
 #include "pwdw_kernel.h"
 #include "pool_softmax_items.h"
@@ -372,6 +372,29 @@ int BuildPlan(const mi355x_conv2d_desc& d, const void* weights_host, const mi355
                 for (int r = 0; r < 4; ++r) std::memcpy(&gdst[(4 + r) * 4], &p->chan_host[static_cast<size_t>(2 + r) * CP + c], 4);
             }
             if (int rc = Upload(reinterpret_cast<void**>(&p->dw_grp), grp.data(), grp.size() * sizeof(uint32_t))) return rc;
+            // blocks of 64 channels: rows of [16][4] dwords, entry [j][e] for channel 16 e + j of the block: corr, m+, b+, m-, b-,
+            // filter taps 0..3, 4..7, 8, and those of the second halves.  Channels past the last one have the code 0 in int8.
+            const int rows = 11;
+            const float past = 128.0f;
+            std::vector<uint32_t> blk(static_cast<size_t>((Co + 63) / 64) * rows * 64, 0u);
+            for (int c = 0; c < (Co + 63) / 64 * 64; ++c)
+            {
+                uint32_t* bdst = blk.data() + static_cast<size_t>(c / 64) * rows * 64 + (c % 16) * 4 + c % 64 / 16;
+                if (c >= Co)
+                {
+                    std::memcpy(&bdst[2 * 64], &past, 4);
+                    std::memcpy(&bdst[4 * 64], &past, 4);
+                    continue;
+                }
+                bdst[0] = static_cast<uint32_t>(corr[c]);
+                for (int r = 0; r < 4; ++r) std::memcpy(&bdst[(1 + r) * 64], &p->chan_host[static_cast<size_t>(2 + r) * CP + c], 4);
+                for (int t = 0; t < 9; ++t)
+                {
+                    bdst[(5 + t / 4) * 64] |= (wp[static_cast<size_t>(c) * 4 + t / 3] >> (8 * (t % 3)) & 0xffu) << (8 * (t % 4));
+                    if (!dw3_fits) bdst[(8 + t / 4) * 64] |= (wp2[static_cast<size_t>(c) * 4 + t / 3] >> (8 * (t % 3)) & 0xffu) << (8 * (t % 4));
+                }
+            }
+            if (int rc = Upload(reinterpret_cast<void**>(&p->dw_blk), blk.data(), blk.size() * sizeof(uint32_t))) return rc;
             const std::vector<uint8_t> padbytes(16, static_cast<uint8_t>((zb ^ (g.in_u8 ? 0x80u : 0u)) & 0xffu));
             if (int rc = Upload(reinterpret_cast<void**>(&p->pad16), padbytes.data(), padbytes.size())) return rc;
         }
@@ -1361,94 +1384,6 @@ int LaunchDwPwStream(const mi355x_conv2d_s* dw, const mi355x_conv2d_s* pw, int w
     return LaunchDwPwStreamT<1, 128, 128, 8, 8>(a, g, stream);
 }
 
-// ---- depthwise 3x3 stride 1 + pointwise over 256 / 512 channels: one block per 8 x 8 tile over all channels ---------------
-// KT = channels between the layers / 128, NQ = output channels / 256; 0 when the pair does not fit that kernel
-bool DwPwPanelShape(const mi355x_conv2d_s* dw, const mi355x_conv2d_s* pw, int* kt, int* nq)
-{
-    const mi355x_conv2d_desc& a = dw->d;
-    if (dw->algo != MI355X_ALGO_DEPTHWISE || dw->variant != 1 || dw->w_dot4b || a.stride_x != a.stride_y || a.stride_x > 2) return false;
-    if (a.out_c != a.in_c || (a.out_c != 256 && a.out_c != 512)) return false;
-    // stride 2 (a 17 x 17 halo per 128 channels): built for 256 -> 512 channels
-    if (a.stride_x == 2 && (a.out_c != 256 || pw->d.out_c != 512)) return false;
-    if (pw->zw_neg != 0 || pw->K_pad != static_cast<int>(a.out_c) || !pw->bk128 || !pw->w_mfma || pw->pw_bn != 0) return false;
-    if (pw->d.out_c != 256 && pw->d.out_c != 512) return false;
-    if (static_cast<long long>(a.in_h) * a.in_w * a.in_c >= (1ll << 31)) return false;
-    *kt = static_cast<int>(a.out_c) / 128;
-    *nq = static_cast<int>(pw->d.out_c) / 256;
-    return true;
-}
-
-template <int KT, int NQ, int S = 1>
-int LaunchDwPwPanelT(const DwPwPanelArgs& a, hipStream_t stream)
-{
-    constexpr int smem = DwPwPanelGeom<KT, NQ, S>::SMEM;
-    static_assert(smem <= 156 * 1024, "LDS of one CU");
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&DwPwPanelKernel<KT, NQ, S>), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-    MI355X_HIP(attr);
-    NoteKernel("DwPwPanelKernel<%d, %d, %d>", KT, NQ, S);
-    hipLaunchKernelGGL((DwPwPanelKernel<KT, NQ, S>), dim3(static_cast<unsigned>(a.xcd_chunk) * 8u), dim3(512), smem, stream, a);
-    MI355X_HIP(hipGetLastError());
-    return 0;
-}
-
-int LaunchDwPwPanel(const mi355x_conv2d_s* dw, const mi355x_conv2d_s* pw, int kt, int nq, uint32_t batch, const void* x, void* y, hipStream_t stream)
-{
-    const ConvGeom& g = dw->geom;
-    DwPwPanelArgs a;
-    a.x = static_cast<const uint8_t*>(x); a.pad16 = dw->pad16; a.wpack = dw->w_dot4; a.dw_ct = ChanTab{dw->chan, dw->Co_pad}; a.dw_corr = dw->corr;
-    a.N = static_cast<int>(batch); a.H = g.H; a.W = g.W; a.C = g.Co; a.Ho = g.Ho; a.Wo = g.Wo;
-    a.pad_top = g.pad_top; a.pad_left = g.pad_left;
-    a.tiles_x = (g.Wo + 7) / 8; a.tiles_y = (g.Ho + 7) / 8;
-    const long long nb = static_cast<long long>(batch) * a.tiles_x * a.tiles_y;
-    if (nb > 0x7fffffffll - 8) return SetError(MI355X_ERR_UNSUPPORTED, "grid too large");
-    a.total_tiles = static_cast<int>(nb); a.xcd_chunk = static_cast<int>((nb + 7) / 8);
-    a.dw_xor = dw->xor_mask; a.dw_rq = dw->rq;
-    a.w = pw->w_mfma; a.K_pad = pw->K_pad; a.pw_ct = ChanTab{pw->chan, pw->Co_pad}; a.pw_corr = pw->corr;
-    a.y = static_cast<uint8_t*>(y); a.Co = pw->geom.Co; a.mid_xor = pw->xor_mask; a.pw_rq = pw->rq;
-#ifdef MI355X_DWPW_STAMPS
-    // measurement build: the first 40 launches record wave 0's shader-clock stamps per block and print the average durations
-    // between consecutive stamps, over all blocks
-    static unsigned long long* d_stamps = nullptr;
-    static int launches = 0;
-    a.stamps = nullptr;
-    if (launches < 40)
-    {
-        if (!d_stamps) MI355X_HIP(hipMalloc(reinterpret_cast<void**>(&d_stamps), 65536 * 16 * 8));
-        a.stamps = a.total_tiles <= 65536 - 8 ? d_stamps : nullptr;
-    }
-    int rc = dw->d.stride_x == 2 ? LaunchDwPwPanelT<2, 2, 2>(a, stream)
-             : kt == 2 ? (nq == 1 ? LaunchDwPwPanelT<2, 1>(a, stream) : LaunchDwPwPanelT<2, 2>(a, stream))
-                       : (nq == 1 ? LaunchDwPwPanelT<4, 1>(a, stream) : LaunchDwPwPanelT<4, 2>(a, stream));
-    if (a.stamps && rc == 0 && ++launches == 40)
-    {
-        MI355X_HIP(hipStreamSynchronize(stream));
-        const int nblk = a.xcd_chunk * 8;
-        std::vector<unsigned long long> h(static_cast<size_t>(nblk) * 16);
-        MI355X_HIP(hipMemcpy(h.data(), d_stamps, h.size() * 8, hipMemcpyDeviceToHost));
-        const int ns = 3 + 3 * kt + 1;
-        std::vector<double> sum(ns, 0.0);
-        int used = 0;
-        unsigned long long tmin = ~0ull, tmax = 0;
-        for (int b = 0; b < a.total_tiles; ++b)
-        {
-            const unsigned long long* s = &h[static_cast<size_t>(b) * 16];
-            if (s[0] == 0) continue;
-            ++used;
-            for (int i = 1; i < ns; ++i) sum[i] += static_cast<double>(s[i] - s[i - 1]);
-            tmin = std::min(tmin, s[0]); tmax = std::max(tmax, s[ns - 1]);
-        }
-        std::fprintf(stderr, "DwPwPanelKernel<%d, %d> stamps over %d blocks (cycles): prologue %.0f", kt, nq, used, sum[1] / used);
-        for (int k = 0; k < kt; ++k) std::fprintf(stderr, " | dw%d %.0f wait %.0f gemm %.0f", k, sum[2 + 3 * k] / used, sum[3 + 3 * k] / used, sum[4 + 3 * k] / used);
-        std::fprintf(stderr, " | requant %.0f stores %.0f | first start to last end %llu\n", sum[2 + 3 * kt] / used, sum[3 + 3 * kt] / used, tmax - tmin);
-    }
-    return rc;
-#else
-    if (dw->d.stride_x == 2) return LaunchDwPwPanelT<2, 2, 2>(a, stream);
-    if (kt == 2) return nq == 1 ? LaunchDwPwPanelT<2, 1>(a, stream) : LaunchDwPwPanelT<2, 2>(a, stream);
-    return nq == 1 ? LaunchDwPwPanelT<4, 1>(a, stream) : LaunchDwPwPanelT<4, 2>(a, stream);
-#endif
-}
-
 // ---- pointwise 1x1 followed by depthwise 3x3, whole images per block ---------------------------------------------------
 constexpr int kPwDwMF = 7;       // 224 pixel rows per block: one 14x14 image, four 7x7 images
 // Two LDS stages and eight waves: with a K of 256 .. 512 bytes the k-loop is bound by what a CU's vector L1 delivers, not
@@ -1743,6 +1678,29 @@ int mi355x_conv2d_run_add(mi355x_conv2d_t plan, uint32_t batch, const void* inpu
     return mi355x_add_run(n, &plan->d.output, other_quant, sum_quant, activation, a, b, output_dev, other_dev, output_dev, stream);
 }
 
+namespace
+{
+// Depthwise + pointwise pairs go to the kernel with resident weights where it is built for the shape (DwPwStreamShape), else to
+// the one with the layer between in LDS; what either option switches off, and nothing else, is left to DwPwKernel.
+bool PanelRuns(const mi355x_conv2d_s* dw, const mi355x_conv2d_s* pw)
+{
+    return GlobalOptions().dwpw_panel != 0 && DwPwStreamShape(dw, pw) == 0 && DwPwPanelTakes(dw, pw);
+}
+
+int DwPwTileCheck(const mi355x_conv2d_s* dw, const mi355x_conv2d_s* pw)
+{
+    const mi355x_conv2d_desc& a = dw->d;
+    if (!dw->dw_grp || dw->w_dot4b || (a.out_c % 32) != 0)
+        return SetError(MI355X_ERR_UNSUPPORTED, "first plan is not a 3x3 depthwise layer on the v_dot4 kernel");
+    if (pw->zw_neg != 0) return SetError(MI355X_ERR_UNSUPPORTED, "fused kernel needs pointwise weights without a zero point");
+    if ((pw->d.out_c % 64) != 0) return SetError(MI355X_ERR_UNSUPPORTED, "fused kernel needs output channels %% 64 == 0");
+    const int smem = a.stride_x == 1 ? DwPwSmemBytes<1, 2>(static_cast<int>(a.out_c)) : DwPwSmemBytes<2, 2>(static_cast<int>(a.out_c));
+    if (smem > 160 * 1024) return SetError(MI355X_ERR_UNSUPPORTED, "fused kernel: %d channels need %d bytes of LDS", a.out_c, smem);
+    if (static_cast<long long>(a.in_h) * a.in_w * a.in_c >= (1ll << 31)) return SetError(MI355X_ERR_UNSUPPORTED, "image too large for 32-bit offsets");
+    return 0;
+}
+} // namespace
+
 int mi355x_conv2d_fusable(mi355x_conv2d_t dw, mi355x_conv2d_t pw)
 {
     if (!dw || !pw) return SetError(MI355X_ERR_INVALID_ARGUMENT, "plan is null");
@@ -1750,20 +1708,16 @@ int mi355x_conv2d_fusable(mi355x_conv2d_t dw, mi355x_conv2d_t pw)
     if (!dw->d.depthwise && pw->d.depthwise) return PwDwCheck(dw, pw, nullptr);
     const mi355x_conv2d_desc& a = dw->d;
     const mi355x_conv2d_desc& b = pw->d;
-    if (dw->algo != MI355X_ALGO_DEPTHWISE || dw->variant != 1 || !dw->dw_grp || dw->w_dot4b || (dw->d.out_c % 32) != 0)
-        return SetError(MI355X_ERR_UNSUPPORTED, "first plan is not a 3x3 depthwise layer on the v_dot4 kernel");
+    if (dw->algo != MI355X_ALGO_DEPTHWISE || dw->variant != 1)
+        return SetError(MI355X_ERR_UNSUPPORTED, "first plan is not a 3x3 depthwise layer on the matrix-core kernel");
     const bool pointwise = pw->algo == MI355X_ALGO_MFMA && !b.depthwise && b.kernel_h == 1 && b.kernel_w == 1 && b.stride_x == 1 &&
                            b.stride_y == 1 && b.pad_top == 0 && b.pad_left == 0 && b.out_h == b.in_h && b.out_w == b.in_w;
     if (!pointwise) return SetError(MI355X_ERR_UNSUPPORTED, "second plan is not an unpadded 1x1 stride-1 convolution on the MFMA kernel");
-    if (pw->zw_neg != 0) return SetError(MI355X_ERR_UNSUPPORTED, "fused kernel needs pointwise weights without a zero point");
     if (a.out_c != b.in_c || a.out_h != b.in_h || a.out_w != b.in_w) return SetError(MI355X_ERR_INVALID_ARGUMENT, "the layers' shapes do not chain");
     if (a.output.dtype != b.input.dtype || a.output.scale != b.input.scale || a.output.offset != b.input.offset)
         return SetError(MI355X_ERR_INVALID_ARGUMENT, "the first layer's output quantization is not the second layer's input quantization");
-    if ((b.out_c % 64) != 0) return SetError(MI355X_ERR_UNSUPPORTED, "fused kernel needs output channels %% 64 == 0");
-    const int smem = a.stride_x == 1 ? DwPwSmemBytes<1, 2>(static_cast<int>(a.out_c)) : DwPwSmemBytes<2, 2>(static_cast<int>(a.out_c));
-    if (smem > 160 * 1024) return SetError(MI355X_ERR_UNSUPPORTED, "fused kernel: %d channels need %d bytes of LDS", a.out_c, smem);
-    if (static_cast<long long>(a.in_h) * a.in_w * a.in_c >= (1ll << 31)) return SetError(MI355X_ERR_UNSUPPORTED, "image too large for 32-bit offsets");
-    return 0;
+    if (PanelRuns(dw, pw)) return 0;
+    return DwPwTileCheck(dw, pw);
 }
 
 int mi355x_conv2d_fusion_pays(mi355x_conv2d_t first, mi355x_conv2d_t second, uint32_t batch)
@@ -1780,17 +1734,18 @@ int mi355x_conv2d_fusion_pays(mi355x_conv2d_t first, mi355x_conv2d_t second, uin
     if (!first->d.depthwise || second->d.depthwise) return 0;
     if (GlobalOptions().dwpw_stream != 0 && DwPwStreamShape(first, second) != 0 && mi355x_conv2d_fusable(first, second) == 0)
     {
-        // persistent blocks: a few items each are needed to overlap anything
-        const long long items = static_cast<long long>(batch) * ((first->d.out_w + 7) / 8) * ((first->d.out_h + 7) / 8);
-        return items >= 1024 ? 1 : 0;
+        // persistent blocks overlap items, and want a few each: 1024 items are four per CU.  One launch of few items is still shorter
+        // than two launches (MobileNetV1, its four such pairs: one image 104 -> 98 us, four images 137 -> 123 us a pass): up to one
+        // item per CU, and up to 1024 on maps of 16 tiles and more, where it was measured
+        const long long tiles = static_cast<long long>((first->d.out_w + 7) / 8) * ((first->d.out_h + 7) / 8), items = batch * tiles;
+        return items >= 1024 || (items >= 16 && (items <= 256 || tiles >= 16)) ? 1 : 0;
     }
-    int kt = 0, nq = 0;
-    if (GlobalOptions().dwpw_panel == 0 || !DwPwPanelShape(first, second, &kt, &nq)) return 0;
-    if (mi355x_conv2d_fusable(first, second) != 0) return 0;
-    // a block takes a CU to itself: below about a hundred tiles per launch most of the device would idle (measured on
-    // MobileNetV1: a gain at 32 images per launch, a loss at 16)
-    const long long tiles = static_cast<long long>(batch) * ((first->d.out_w + 7) / 8) * ((first->d.out_h + 7) / 8);
-    return tiles >= 100 ? 1 : 0;
+    if (mi355x_conv2d_fusable(first, second) != 0 || !PanelRuns(first, second)) return 0;
+    // 7 x 7 maps: from 8 images on the 1x1 convolution is worth more with a pooling behind it (mi355x_conv2d_pool_fusion_pays), and
+    // from 64 on with the depthwise layer behind it (above); beyond 512 channels every block's own copy of the depthwise layer
+    // costs what the launch saves (1024 -> 1024, one image: 6.9 us against 7.4)
+    if (first->d.out_c > 512) return 0;
+    return first->d.out_h > 7 || first->d.out_w > 7 || batch < (first->d.stride_x == 1 ? 8u : 64u) ? 1 : 0;
 }
 
 int mi355x_conv2d_run_fused(mi355x_conv2d_t dw, mi355x_conv2d_t pw, uint32_t batch, const void* input_dev, void* output_dev,
@@ -1809,10 +1764,7 @@ int mi355x_conv2d_run_fused(mi355x_conv2d_t dw, mi355x_conv2d_t pw, uint32_t bat
     }
     if (GlobalOptions().dwpw_stream != 0)
         if (const int which = DwPwStreamShape(dw, pw)) return LaunchDwPwStream(dw, pw, which, batch, input_dev, output_dev, ToHip(stream));
-    {
-        int kt = 0, nq = 0;
-        if (GlobalOptions().dwpw_panel != 0 && DwPwPanelShape(dw, pw, &kt, &nq)) return LaunchDwPwPanel(dw, pw, kt, nq, batch, input_dev, output_dev, ToHip(stream));
-    }
+    if (PanelRuns(dw, pw)) return LaunchDwPwPanel(dw, pw, batch, input_dev, output_dev, ToHip(stream));
     if (dw->d.stride_x == 2) return LaunchDwPw<2, 2>(dw, pw, batch, input_dev, output_dev, ToHip(stream));
     // stride 1: the wide tile (8 x 16 pixels) while it still yields two blocks per CU, else the narrow one (8 x 8)
     const long long wide = static_cast<long long>(batch) * ((dw->d.out_w + 15) / 16) * ((dw->d.out_h + 7) / 8);

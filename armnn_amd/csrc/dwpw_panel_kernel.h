@@ -1,26 +1,26 @@
-// Depthwise 3x3 (stride 1 or 2) + the pointwise 1x1 convolution that consumes it as ONE kernel, for 256 or 512 channels between
-// them: a block of eight waves owns an 8 x 8 pixel tile of one image over ALL channels, and a CU holds one block.
+// Depthwise 3x3 (stride 1 or 2) + the pointwise 1x1 convolution that consumes it as ONE kernel: a block owns TH x TW pixels of
+// one image over all channels between the layers, and 16 NW CG of the output channels.
 //
-//   The intermediate tensor never leaves the CU, and it is produced in exactly the pieces the GEMM consumes: the
-//   depthwise layer's channel block kt (128 channels) of the 64 pixels IS k-tile kt of the GEMM's activation operand.
-//   The kernel alternates, once per k-tile, between
-//     a depthwise phase   the eight waves run the matrix-core arithmetic of DepthwiseMfmaKernel on channel block kt (wave =
-//                         16 channels, four groups of 16 pixels: three v_mfma_i32_16x16x64_i8 per group over diagonal weight
-//                         operands; a third of the VALU work of the v_dot4 formulation, which bounded this phase),
-//                         requantize with the depthwise layer's own constants and write the codes -- the bytes the
-//                         separate layer would have stored, shifted to int8 where they are uint8 -- into k-tile kt of the
-//                         activation panel in LDS (the xor-swizzled image the MFMA fragment reads expect), and
-//     a GEMM phase        all eight waves multiply k-tile kt into accumulators for ALL output channels: wave (wm, wq) keeps
-//                         the 32 pixel rows wm x 64 NQ channels wq of the output in 32 NQ registers for the whole kernel.
-//   What keeps the phases short is that nothing in them waits for memory: the weights of k-tile kt (64 KB for 512 output
-//   channels) and the input halo of channel block kt + 1 are requested at the start of depthwise phase kt -- the halo and
-//   the phase's constants first, the weights behind them, because a wave's vector memory operations complete in issue order
-//   -- and are first touched after it.  One wait and one barrier per phase.
-//   The write-out requantizes from a copy of the pointwise layer's bracket rows in LDS (accumulators start at zero: the
-//   zero-point correction is part of rows 6 / 7), stages the 64 x Co output bytes over the weight ring and stores whole
-//   rows of Co bytes per pixel.
-//   Both layers' arithmetic is untouched -- exact int32 sums, the same requantization routine with the same constants -- so
-//   the bytes are those of the two layers run one after the other.
+//   * The halo of the tile, all channels, is requested at once (one round trip), with the constants of both layers, and lies in
+//     LDS as [channels / 16][halo pixel][16 bytes]: the depthwise operands are 16-byte reads of neighbouring pixels, and an odd
+//     number of pieces per channel group keeps the staging writes on different banks.
+//   * Depthwise: v_mfma_i32_16x16x64_i8 with pixels as rows and channels as columns, the weights of a tap diagonal (a column keeps
+//     one byte of the 16).  A wave takes 64 channels as four groups: tap slots 0 .. 3 and 4 .. 7 are one operand read per group,
+//     the ninth taps of the four groups share a third (lane group g reads group g, and only that group's weights are not zero).
+//     A lane then holds one channel of four pixels in each group, so its constants are one 16-byte row entry for four groups;
+//     four channels per lane, as DepthwiseMfmaKernel has them, took five reads per group and made LDS bandwidth the bound (14 x
+//     14 x 512, one image 6.0 -> 5.5 us).  Its four codes of a pixel -- channels j, 16 + j, 32 + j, 48 + j -- are one dword, which
+//     goes back to LDS over the halo just read; the pointwise weights are packed with their channels in that order.
+//   * Pointwise: a wave owns 16 CG output channels of all pixels and reads its weights in operand order straight from L2 (runs of
+//     1 KB; 55 bytes a clock and CU were measured for that, 14 to 20 for 128-byte rows through LDS with a wait per k-tile), the
+//     first k-steps requested ahead of the depthwise phase.  No barrier inside: two after the halo, two around the write-out.
+//   * The outputs meet in LDS and leave as 16 bytes per lane.
+// At many tiles VALU work bounds it, most of that the requantization of both layers (25 instructions per four values); at few,
+// the chain of round trips.  Times against the kernel with a k-tile loop it replaces (64 images | 256): 14 x 14 x 512 -> 512
+// 15.4 -> 12.8 | 54.2 -> 35.7 us, 28 x 28 x 256 -> 256 20.2 -> 17.7 | 68.9 -> 61.3, 28 x 28 x 256 -> 14 x 14 x 512 11.2 -> 10.7 | 43.1 ->
+// 34.8; against two launches, one image | eight: 14 x 14 x 512 7.6 -> 5.5 | 9.3 -> 7.5, 28 x 28 x 256 7.2 -> 4.6 | 8.6 -> 6.3.
+// Both layers' arithmetic is untouched -- exact int32 sums, the same requantization routine with the same constants -- so the
+// bytes are those of the two layers run one after the other.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -28,289 +28,366 @@
 #include "common.h"
 #include "conv_kernels.h"
 #include "device_math.h"
-#include "dw_stem_kernels.h"
-#include "igemm_lds_kernel.h"
+#include "dw_mfma_kernel.h"
 
 namespace mi355x
 {
 
 struct DwPwPanelArgs
 {
-    // depthwise 3x3, multiplier 1, C % 128 == 0
+    // depthwise 3x3, multiplier 1, C % 16 == 0
     const uint8_t*  x;
     const uint8_t*  pad16;      // 16 bytes that become the depthwise padding value under dw_xor
-    const uint32_t* wpack;      // [C][4] dwords, rows of the 3x3 filter per channel (Dw3x3Args::wpack)
+    const uint32_t* dw_blk;     // constants per block of 64 channels: 11 rows of [16][4] dwords
     ChanTab         dw_ct;
-    const int32_t*  dw_corr;
-    int N, H, W, C, Ho, Wo;
+    int H, W, C, Ho, Wo;
     int pad_top, pad_left;
-    int tiles_x, tiles_y;
-    int total_tiles, xcd_chunk;
+    int tiles_x, tiles_y, nb;   // nb: blocks per tile (output channels / (16 NW CG), rounded up)
+    int total_items, xcd_chunk;
+    uint32_t rcp_tiles_x, rcp_tiles_y, rcp_nb, rcp_ng;      // ceil(2^32 / d) of tiles_x, tiles_y, nb and C / 16
     uint32_t dw_xor;
     Requant dw_rq;
-    // pointwise 1x1: K = C, Co = 256 NQ
-    const int8_t*  w;           // [Co_pad][K_pad], K_pad == C
-    int            K_pad;
+    // pointwise 1x1 over C channels
+    const int8_t*  w;           // operand order (PackFragKernel)
+    int            co_groups;   // groups of 16 channels w holds
     ChanTab        pw_ct;
     const int32_t* pw_corr;
     uint8_t*       y;
+    long long      y_bytes;
     int            Co;
+    int            zw_neg;      // AW: minus the zero point of the weights
     uint32_t       mid_xor;     // 0x80808080 when the tensor between the layers is uint8: the panel holds the int8-shifted codes
     Requant        pw_rq;
-#ifdef MI355X_DWPW_STAMPS
-    unsigned long long* stamps; // [blocks][16] shader-clock stamps of wave 0
-#endif
 };
 
-template <int KT, int NQ, int S = 1>
+template <int S, int TH, int TW, int NW, int CG>
 struct DwPwPanelGeom
 {
-    static constexpr int NCOL = 256 * NQ;             // output channels
-    static constexpr int NT = 4 * NQ;                 // 64-channel weight tiles per k-tile
-    static constexpr int HR = 7 * S + 3, HC = 7 * S + 3;   // halo of an 8 x 8 tile of outputs: 10 x 10 or 17 x 17 input pixels
-    static constexpr int NCHUNK = HR * HC * 8;        // 16-byte pieces of a halo (128 channels per pixel)
-    static constexpr int HPITCH = 144;                // bytes per halo pixel in LDS: 128 + 16, so that the 16-byte reads of 8
-                                                      // neighbouring pixels fall on different bank quads (stride 1)
-    static constexpr int HROWP = S == 1 ? 1664 : HC * HPITCH;   // bytes per halo row; at stride 1 >= 10 pixels and 128 mod 256, so that
-                                                      // the reads of the pixel group's second row take the quads the first row's leave free
-    static constexpr int HALO = HR * HROWP;
-    static constexpr int LDO = NCOL + 16;
-    static constexpr int PANEL = KT * 64 * 128;
-    static constexpr int TAB = 4 * NCOL * 4;
-    static constexpr int RING = NT * 64 * 128;
-    static constexpr int OUT = 64 * LDO;
-    static constexpr int WORK = HALO + RING > OUT ? HALO + RING : OUT;   // halo buffer + weight ring; the output staging reuses them
-    static constexpr int SMEM = PANEL + TAB + WORK;
+    static_assert(TW == 4 || TW == 8 || TW == 16, "a group of 16 pixels is whole tile rows");
+    static constexpr int NT = 64 * NW;
+    static constexpr int PX = TH * TW, PG = PX / 16;
+    static constexpr int HR = (TH - 1) * S + 3, HC = (TW - 1) * S + 3, HPX = HR * HC;
+    static constexpr int GP = (HPX | 1) * 16;            // bytes per group of 16 channels in LDS: an odd number of 16-byte pieces
+    static constexpr int NCOL = 16 * NW * CG;            // output channels of a block
+    static constexpr int OP = NCOL + 16;                 // bytes per pixel of the output staging
+    static constexpr int Panel(int C)                    // halo and panel, later the output staging
+    {
+        const int in = (C + 63) / 64 * 4 * GP, out = PX * OP;
+        return in > out ? in : out;
+    }
+    // behind it the depthwise layer's constants and four rows of NCOL floats of the pointwise layer's
+    static constexpr int TB(bool u) { return u ? 2816 : 2048; }        // bytes per 64 channels
+    static constexpr int Smem(int C, bool u) { return Panel(C) + (C + 63) / 64 * TB(u) + 16 * NCOL; }
 };
 
-// KT = C / 128 (2 or 4), NQ = Co / 256 (1 or 2), S = depthwise stride.  512 threads.
-template <int KT, int NQ, int S = 1>
-__global__ __launch_bounds__(512) void DwPwPanelKernel(DwPwPanelArgs a)
+// KS: k-steps of 64 channels where the instance fixes them (64 (KS - 1) < C <= 64 KS), 0: a.C decides.  U: depthwise weights in two
+// halves, pointwise weights with a zero point.
+template <int S, int TH, int TW, int NW, int CG, int KS, bool U>
+__global__ __launch_bounds__(64 * NW, 4) void DwPwPanelKernel(DwPwPanelArgs a)
 {
-    using G = DwPwPanelGeom<KT, NQ, S>;
-    constexpr int NCHUNK = G::NCHUNK, NHS = (G::NCHUNK + 511) / 512;     // halo pieces, and pieces per thread
-    constexpr int NCOL = G::NCOL, NT = G::NT, HC = G::HC, HALO = G::HALO, LDO = G::LDO, HPITCH = G::HPITCH, HROWP = G::HROWP;
-    constexpr int NTHR = 512;
-    typedef __attribute__((address_space(3))) void* LdsPtr;
-    typedef const __attribute__((address_space(1))) void* GlobalPtr;
-    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    uint8_t* const panel = smem;                                           // [KT][64 pixels][128 B]
-    float* const tab = reinterpret_cast<float*>(smem + G::PANEL);          // [4][NCOL]: m+, b+ (corr folded in), m-, b- (corr folded in)
-    uint8_t* const halo = smem + G::PANEL + G::TAB;                        // [10 rows of HROWP bytes][10 pixels of HPITCH bytes]
-    uint8_t* const ring = halo + HALO;                                 // [NT][64 channels][128 B]
-    uint8_t* const Os = halo;                                              // [64][LDO], after the last GEMM phase
+    using G = DwPwPanelGeom<S, TH, TW, NW, CG>;
+    constexpr int NT = G::NT, PG = G::PG, HC = G::HC, HPX = G::HPX, GP = G::GP, OP = G::OP;
+    constexpr int RPG = 16 / TW;                         // tile rows per group of 16 pixels
+    constexpr int DEPTH = CG >= 4 ? 2 : CG == 2 ? 4 : 8;
+    constexpr int RD = KS != 0 && KS < DEPTH ? KS : DEPTH;   // k-steps of weights in flight
+    constexpr int HS = KS != 0 ? (HPX * KS * 4 + NT - 1) / NT : 6;   // halo pieces of a thread in flight
+    // depthwise work: blocks of 64 channels go to the waves in turn, all PG groups of 16 pixels of a block to one wave (UC at a
+    // time); with fewer blocks than waves, WPB waves share a block
+    constexpr int WPB = KS != 0 && NW / KS >= 2 ? (NW / KS < PG ? NW / KS : PG) : 1;
+    constexpr int UW = PG / WPB, UC = WPB > 1 ? UW : UW < 2 || U ? 1 : 2;
+    static_assert(PG % WPB == 0 && UW % UC == 0, "whole shares");
+    constexpr bool EARLY = PG == 1 || (PG == 2 && !U);                      // registers for weights requested ahead of the depthwise phase
+    constexpr int TB = G::TB(U);
+    constexpr int TS = KS != 0 ? (KS * (TB / 16) + G::NCOL + NT - 1) / NT : 4;      // ... and table pieces
+    extern __shared__ __attribute__((aligned(16))) uint8_t panel_lds[];   // [C / 16][GP]: halo pixels, then panel pixels, of 16 bytes
 
     int b = XcdContiguousWorkItem(blockIdx.x, a.xcd_chunk);
-    if ((static_cast<int>(blockIdx.x) >> 3) >= a.xcd_chunk || b >= a.total_tiles) return;
-    const int tx = b % a.tiles_x; b /= a.tiles_x;
-    const int ty = b % a.tiles_y;
-    const int n = b / a.tiles_y;
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
-#ifdef MI355X_DWPW_STAMPS
-    int stamp_i = 0;
-#define DWPW_STAMP() do { if (tid == 0 && a.stamps) a.stamps[static_cast<size_t>(blockIdx.x) * 16 + stamp_i++] = clock64(); } while (0)
-#else
-#define DWPW_STAMP() do { } while (0)
-#endif
-    DWPW_STAMP();
+    if ((static_cast<int>(blockIdx.x) >> 3) >= a.xcd_chunk || b >= a.total_items) return;
+    int q = DivByInvariant(b, a.nb, a.rcp_nb);
+    const int bn = b - q * a.nb; b = q;
+    q = DivByInvariant(b, a.tiles_x, a.rcp_tiles_x);
+    const int tx = b - q * a.tiles_x; b = q;
+    const int n = DivByInvariant(b, a.tiles_y, a.rcp_tiles_y);
+    const int ty = b - n * a.tiles_y;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int j = lane & 15, g = lane >> 4;
+    const int ng = a.C >> 4;                             // groups of 16 channels between the layers
+    const int steps = KS != 0 ? KS : (a.C + 63) >> 6;
 
-    // ---- depthwise roles: wave = 16 channels of the current 128-channel block; lane (j, g): pixel j of a group of 16 (two
-    // tile rows) and tap slot g as an MFMA operand, channel quad g of pixel j as a result
-    const int dj = lane & 15, dg = lane >> 4;
-    const int drj = dj >> 3, dcj = dj & 7;
-    int dtap[3], dwrow[3], dwshift[3];
+    // ---- weights of the wave's CG groups of output channels ---------------------------------------------------------------------
+    v4i wv[RD][CG];
+    auto load_weights = [&](int ks, int r) {
 #pragma unroll
-    for (int m = 0; m < 3; ++m)
-    {
-        const int t = 4 * m + dg;
-        const int tc = min(t, 8);                      // slots past the ninth tap read the ninth; their weights are zero
-        dtap[m] = (drj * S + tc / 3) * HROWP + (dcj * S + tc % 3) * HPITCH + wave * 16;
-        dwrow[m] = tc / 3;
-        dwshift[m] = t < 9 ? 8 * (tc % 3) : 24;        // shift 24: the zero byte of a packed filter row
-    }
-    // ---- staging of a halo: NCHUNK pieces of 16 bytes, NHS per thread at most; only the channel block moves from phase to phase
-    const int iy_org = ty * 8 * S - a.pad_top;
-    const int ix_org = tx * 8 * S - a.pad_left;
-    const uint8_t* const xn = a.x + static_cast<long long>(n) * a.H * a.W * a.C;
-    const int dxm = static_cast<int>(a.dw_xor);
-    int hoff[NHS], hlds[NHS];                              // offset within the image (-1: outside, reads the padding), place in LDS (-1: none)
-#pragma unroll
-    for (int k = 0; k < NHS; ++k)
-    {
-        const int i = min(tid + k * NTHR, NCHUNK - 1);
-        const int part = i & 7, pix = i >> 3;
-        const int col = pix % HC, hrow = pix / HC;
-        const int iy = iy_org + hrow, ix = ix_org + col;
-        const bool ok = static_cast<unsigned>(iy) < static_cast<unsigned>(a.H) && static_cast<unsigned>(ix) < static_cast<unsigned>(a.W);
-        hoff[k] = ok ? (iy * a.W + ix) * a.C + part * 16 : -1;
-        hlds[k] = tid + k * NTHR < NCHUNK ? hrow * HROWP + col * HPITCH + part * 16 : -1;
-    }
-    auto load_halo = [&](int kt, v4i (&h)[NHS]) {
-#pragma unroll
-        for (int k = 0; k < NHS; ++k) h[k] = *reinterpret_cast<const v4i*>(hoff[k] >= 0 ? xn + hoff[k] + kt * 128 : a.pad16);
+        for (int c = 0; c < CG; ++c)
+            wv[r][c] = *reinterpret_cast<const v4i*>(a.w + static_cast<long long>(min((bn * NW + wave) * CG + c, a.co_groups - 1) * steps + ks) * 1024 + lane * 16);
     };
-    auto store_halo = [&](const v4i (&h)[NHS]) {
-#pragma unroll
-        for (int k = 0; k < NHS; ++k)
-            if (hlds[k] >= 0) *reinterpret_cast<v4i*>(halo + hlds[k]) = h[k] ^ dxm;
+    // ---- tables ---------------------------------------------------------------------------------------------------------------------
+    uint8_t* const tab = panel_lds + G::Panel(64 * steps);
+    uint8_t* const ptab = tab + steps * TB;
+    const int dw_pieces = steps * (TB / 16), tab_pieces = dw_pieces + G::NCOL;
+    auto tab_src = [&](int i) -> const void* {
+        if (i < dw_pieces) return a.dw_blk + (U ? i * 4 : (i >> 7) * 704 + (i & 127) * 4);
+        i -= dw_pieces;
+        const int r = i / (G::NCOL / 4), c4 = (i - r * (G::NCOL / 4)) * 4;
+        const int row = U ? r + 2 : r == 0 ? 2 : r == 1 ? 6 : r == 2 ? 4 : 7;
+        return a.pw_ct.p + row * a.pw_ct.stride + min(bn * G::NCOL + c4, a.co_groups * 16 - 4);
     };
 
-    // ---- GEMM roles: wave (wm, wq) owns pixel rows [32 wm, 32 wm + 32) x output channels [64 NQ wq, 64 NQ (wq + 1)) ----------
-    const int wm = wave & 1, wq = wave >> 1;
-    const int frag_row = lane & 31, frag_half = lane >> 5;
-    const int lane_c = 4 * (lane >> 5);
-    // weights of k-tile kt: tile tn (64 channels x 128 B) into ring slot tn; wave w fetches rows [8w, 8w + 8) of every tile,
-    // lane l the chunk that belongs in slot (l & 7) of row 8w + (l >> 3)  (chunk c of row r sits at slot c ^ ((r >> 1) & 7))
-    const int lrow = lane >> 3;
-    const int wrow = 8 * wave + lrow;
-    const uint32_t boff = static_cast<uint32_t>(wrow) * static_cast<uint32_t>(a.K_pad) + (((lane & 7) ^ ((wrow >> 1) & 7)) * 16);
-    auto load_weights = [&](int kt) {
-#pragma unroll
-        for (int tn = 0; tn < NT; ++tn)
-            __builtin_amdgcn_global_load_lds((GlobalPtr)(a.w + static_cast<long long>(tn) * 64 * a.K_pad + kt * 128 + boff),
-                                             (LdsPtr)(ring + tn * 8192 + wave * 1024), 16, 0, 0);
-    };
-
-    // ---- prologue: the pointwise layer's bracket rows and the first halo --------------------------------------------------
+    // ---- the halo of the tile, all channels ---------------------------------------------------------------------------------------
     {
-        constexpr int TABV = NCOL / NTHR + (NCOL % NTHR ? 1 : 0);          // float4 pieces per thread ([4][NCOL / 4] in all)
-        float4 tv[TABV];
-#pragma unroll
-        for (int i = 0; i < TABV; ++i)
+        const int iy_org = ty * TH * S - a.pad_top, ix_org = tx * TW * S - a.pad_left;
+        const uint8_t* const xn = a.x + static_cast<long long>(n) * a.H * a.W * a.C;
+        const int xm = static_cast<int>(a.dw_xor);
+        const int pieces = HPX * ng;
+        for (int i0 = 0; KS != 0 ? i0 == 0 : i0 < pieces; i0 += NT * HS)
         {
-            const int e = min(tid + i * NTHR, NCOL - 1);
-            const int r = e / (NCOL / 4), col4 = e - r * (NCOL / 4);
-            const int src_row = r == 0 ? 2 : r == 1 ? 6 : r == 2 ? 4 : 7;
-            tv[i] = *reinterpret_cast<const float4*>(a.pw_ct.p + src_row * a.pw_ct.stride + col4 * 4);
-        }
-        v4i h0[NHS];
-        load_halo(0, h0);
+            v4i h[HS];
+            int at[HS];
 #pragma unroll
-        for (int i = 0; i < TABV; ++i)
-            if (tid + i * NTHR < NCOL) *reinterpret_cast<float4*>(tab + (tid + i * NTHR) * 4) = tv[i];
-        store_halo(h0);
+            for (int k = 0; k < HS; ++k)
+            {
+                at[k] = -1;
+                if (i0 + k * NT >= pieces) continue;
+                const int i = min(i0 + k * NT + tid, pieces - 1);
+                const int px = DivByInvariant(i, ng, a.rcp_ng);
+                const int part = i - px * ng;
+                const int row = px / HC, col = px - row * HC;
+                const int iy = iy_org + row, ix = ix_org + col;
+                const bool ok = static_cast<unsigned>(iy) < static_cast<unsigned>(a.H) && static_cast<unsigned>(ix) < static_cast<unsigned>(a.W);
+                h[k] = *reinterpret_cast<const v4i*>(ok ? xn + (iy * a.W + ix) * a.C + part * 16 : a.pad16);
+                if (i0 + k * NT + tid < pieces) at[k] = part * GP + px * 16;
+            }
+            if (i0 == 0)
+            {
+                v4i t[TS];
+#pragma unroll
+                for (int k = 0; k < TS; ++k)
+                    if (KS != 0 || k * NT < tab_pieces) t[k] = *reinterpret_cast<const v4i*>(tab_src(min(tid + k * NT, tab_pieces - 1)));
+                if constexpr (EARLY)
+                {
+#pragma unroll
+                    for (int r = 0; r < RD; ++r)
+                        if (r < steps) load_weights(r, r);
+                }
+#pragma unroll
+                for (int k = 0; k < TS; ++k)
+                    if (tid + k * NT < tab_pieces) *reinterpret_cast<v4i*>(tab + (tid + k * NT) * 16) = t[k];
+            }
+#pragma unroll
+            for (int k = 0; k < HS; ++k)
+                if (at[k] >= 0) *reinterpret_cast<v4i*>(panel_lds + at[k]) = h[k] ^ xm;
+        }
+        if (KS == 0)
+            for (int i = tid + TS * NT; i < tab_pieces; i += NT) *reinterpret_cast<v4i*>(tab + i * 16) = *reinterpret_cast<const v4i*>(tab_src(i));
     }
     __syncthreads();
-    DWPW_STAMP();
 
-    v16i acc[NQ][2];
-#pragma unroll
-    for (int t = 0; t < NQ; ++t)
-#pragma unroll
-        for (int s = 0; s < 2; ++s) acc[t][s] = v16i{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-
-#pragma unroll
-    for (int kt = 0; kt < KT; ++kt)
+    // ---- depthwise: a wave takes 64 channels and writes their codes over the halo it has just read ------------------------------
     {
-        // ---- requests of this phase, in the order they will be needed: constants, next halo, weights ----------------------
-        const int c0 = kt * 128 + wave * 16;
-        const uint4 w4 = *reinterpret_cast<const uint4*>(a.wpack + (c0 + dj) * 4);
-        const int cq = c0 + 4 * dg;                        // the four channels this lane requantizes
-        const v4i corr4 = *reinterpret_cast<const v4i*>(a.dw_corr + cq);
-        const Fast4 f4 = LoadFast4(a.dw_ct, cq);
-        v4i hn[NHS];
-        if (kt + 1 < KT) load_halo(kt + 1, hn);
-        load_weights(kt);
-
-        // ---- depthwise phase: channel block kt of the 8 x 8 tile --------------------------------------------------------
-        // weight operands: byte dj of the lane's 16 is w[tap][c0 + dj], the others are zero
-        v4i wa[3];
+        const int rj = j / TW, cj = j % TW;
+        int dtap[3];
+#pragma unroll
+        for (int m = 0; m < 3; ++m)
         {
-            const int dw = dj >> 2, sh = 8 * (dj & 3);
+            const int t = m < 2 ? 4 * m + g : 8;
+            dtap[m] = ((rj * S + t / 3) * HC + cj * S + t % 3) * 16;
+        }
+        // weight operand: byte j of the lane's 16 is byte b of `taps`, the others are zero
+        uint32_t sel[4], sel8[4];
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+        {
+            sel[d] = (j >> 2) == d ? 0x0c0c0c0cu ^ (static_cast<uint32_t>(0x0c ^ g) << (8 * (j & 3))) : 0x0c0c0c0cu;
+            sel8[d] = (j >> 2) == d ? 0x0c0c0c0cu ^ (0x0cu << (8 * (j & 3))) : 0x0c0c0c0cu;
+        }
+        auto operand = [&](uint32_t taps, const uint32_t (&s)[4]) {
+            v4i o;
+#pragma unroll
+            for (int d = 0; d < 4; ++d) o[d] = static_cast<int>(__builtin_amdgcn_perm(0u, taps, s[d]));
+            return o;
+        };
+        // exact sums of UC pixel groups from u0 on, channel 64 blk + 16 e + j of pixels 4 g .. 4 g + 3 in acc[e]
+        auto sums = [&](int blk, int u0, v4i (&acc)[4][UC]) {
+            const uint8_t* const tb = tab + blk * TB + j * 16;
+            const uint8_t* const hu = panel_lds + blk * (4 * GP) + u0 * (RPG * S * HC * 16);
+            const v4i corr = *reinterpret_cast<const v4i*>(tb);
+            v4i w[3], w2[3];
 #pragma unroll
             for (int m = 0; m < 3; ++m)
             {
-                const uint32_t ra = dwrow[m] == 0 ? w4.x : dwrow[m] == 1 ? w4.y : w4.z;
-                const int ba = static_cast<int>(((ra >> dwshift[m]) & 0xffu) << sh);
-                wa[m] = v4i{dw == 0 ? ba : 0, dw == 1 ? ba : 0, dw == 2 ? ba : 0, dw == 3 ? ba : 0};
+                w[m] = *reinterpret_cast<const v4i*>(tb + (5 + m) * 256);
+                if constexpr (U) w2[m] = *reinterpret_cast<const v4i*>(tb + (8 + m) * 256);
             }
-        }
-        const uint8_t* hb = halo;
+            // the ninth tap of the four channel groups shares one operand: lane group g reads it from channel group g
+            v4i x8[UC];
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-        {
-            const v4i b0 = *reinterpret_cast<const v4i*>(hb + dtap[0] + u * 2 * S * HROWP);
-            const v4i b1 = *reinterpret_cast<const v4i*>(hb + dtap[1] + u * 2 * S * HROWP);
-            const v4i b2 = *reinterpret_cast<const v4i*>(hb + dtap[2] + u * 2 * S * HROWP);
-            v4i dacc = corr4;
-            dacc = __builtin_amdgcn_mfma_i32_16x16x64_i8(wa[0], b0, dacc, 0, 0, 0);
-            dacc = __builtin_amdgcn_mfma_i32_16x16x64_i8(wa[1], b1, dacc, 0, 0, 0);
-            dacc = __builtin_amdgcn_mfma_i32_16x16x64_i8(wa[2], b2, dacc, 0, 0, 0);
-            // the codes of pixel r = 16 u + dj, channels cq .. cq + 3: chunk `wave` of panel row r, at its swizzled slot
-            const uint32_t q = Requant4Dev(dacc[0], dacc[1], dacc[2], dacc[3], f4, a.dw_ct, cq, a.dw_rq) ^ a.mid_xor;
-            const int r = 16 * u + dj;
-            *reinterpret_cast<uint32_t*>(panel + kt * 8192 + r * 128 + ((wave ^ ((r >> 1) & 7)) * 16) + dg * 4) = q;
-        }
-        DWPW_STAMP();
-        __builtin_amdgcn_s_waitcnt(VmcntImm(0));          // this wave's share of the weights (and of the next halo) has landed
-        __syncthreads();                                   // k-tile kt of the panel and all weight tiles are in LDS; the halo has been read
-        if (kt + 1 < KT) store_halo(hn);                   // (the barrier behind the GEMM phase orders it before the next phase's reads)
-        DWPW_STAMP();
-
-        // ---- GEMM phase: k-tile kt into every accumulator ------------------------------------------------------------------
-        const uint8_t* As = panel + kt * 8192;
+            for (int u = 0; u < UC; ++u) x8[u] = *reinterpret_cast<const v4i*>(hu + g * GP + dtap[2] + u * (RPG * S * HC * 16));
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks)
-        {
-            const int sl = ((ks * 2 + frag_half) ^ ((frag_row >> 1) & 7)) * 16;
-            const v4i fa = *reinterpret_cast<const v4i*>(As + (wm * 32 + frag_row) * 128 + sl);
-#pragma unroll
-            for (int t = 0; t < NQ; ++t)
+            for (int e = 0; e < 4; ++e)
             {
-                const uint8_t* Bs = ring + (wq * NQ + t) * 8192;
+                const v4i w03 = operand(w[0][e], sel), w47 = operand(w[1][e], sel), w8 = operand(g == e ? w[2][e] : 0, sel8);
+                v4i v03, v47, v8;
+                if constexpr (U) { v03 = operand(w2[0][e], sel); v47 = operand(w2[1][e], sel); v8 = operand(g == e ? w2[2][e] : 0, sel8); }
 #pragma unroll
-                for (int s = 0; s < 2; ++s)
+                for (int u = 0; u < UC; ++u)
                 {
-                    const v4i fw = *reinterpret_cast<const v4i*>(Bs + (s * 32 + frag_row) * 128 + sl);
-                    acc[t][s] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fw, fa, acc[t][s], 0, 0, 0);
+                    const v4i x0 = *reinterpret_cast<const v4i*>(hu + e * GP + dtap[0] + u * (RPG * S * HC * 16));
+                    const v4i x1 = *reinterpret_cast<const v4i*>(hu + e * GP + dtap[1] + u * (RPG * S * HC * 16));
+                    v4i v = v4i{corr[e], corr[e], corr[e], corr[e]};
+                    v = __builtin_amdgcn_mfma_i32_16x16x64_i8(x0, w03, v, 0, 0, 0);
+                    v = __builtin_amdgcn_mfma_i32_16x16x64_i8(x1, w47, v, 0, 0, 0);
+                    v = __builtin_amdgcn_mfma_i32_16x16x64_i8(x8[u], w8, v, 0, 0, 0);
+                    if constexpr (U)
+                    {
+                        v = __builtin_amdgcn_mfma_i32_16x16x64_i8(x0, v03, v, 0, 0, 0);
+                        v = __builtin_amdgcn_mfma_i32_16x16x64_i8(x1, v47, v, 0, 0, 0);
+                        v = __builtin_amdgcn_mfma_i32_16x16x64_i8(x8[u], v8, v, 0, 0, 0);
+                    }
+                    acc[e][u] = v;
                 }
             }
+        };
+        auto codes = [&](int blk, int u0, const v4i (&acc)[4][UC]) {
+            const uint8_t* const tb = tab + blk * TB + j * 16;
+            Fast4 f;
+            f.mp = *reinterpret_cast<const float4*>(tb + 256);
+            f.bp = *reinterpret_cast<const float4*>(tb + 512);
+            f.mm = *reinterpret_cast<const float4*>(tb + 768);
+            f.bm = *reinterpret_cast<const float4*>(tb + 1024);
+            uint8_t* const out = panel_lds + blk * (4 * GP) + (j >> 2) * GP + (16 * u0 + 4 * g) * 16 + (j & 3) * 4;
+#pragma unroll
+            for (int u = 0; u < UC; ++u)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    *reinterpret_cast<uint32_t*>(out + (16 * u + r) * 16) =
+                        Requant4Core(acc[0][u][r], acc[1][u][r], acc[2][u][r], acc[3][u][r], f.mp, f.bp, f.mm, f.bm, a.dw_rq,
+                                     [&](float4& m, float4& b, int4& cr) {
+                                         float mv[4], bv[4];
+#pragma unroll
+                                         for (int e = 0; e < 4; ++e)
+                                         {
+                                             const int c = min(blk * 64 + 16 * e + j, a.C - 1);
+                                             mv[e] = a.dw_ct.p[c];
+                                             bv[e] = a.dw_ct.p[a.dw_ct.stride + c];
+                                         }
+                                         m = float4{mv[0], mv[1], mv[2], mv[3]};
+                                         b = float4{bv[0], bv[1], bv[2], bv[3]};
+                                         cr = int4{0, 0, 0, 0};
+                                     }) ^ a.mid_xor;
+        };
+        if constexpr (WPB > 1)
+        {
+            const int blk = wave / WPB, u0 = wave % WPB * UW;
+            v4i acc[4][UC];
+            if (blk < KS) sums(blk, u0, acc);
+            __syncthreads();                             // all have read the halo
+            if (blk < KS) codes(blk, u0, acc);
         }
-        __syncthreads();                                   // the ring may be refilled; the next halo is in LDS
-        DWPW_STAMP();
+        else
+        {
+            // A pixel group's codes go to pixels 16 u .. 16 u + 15 of the block, and the later groups read halo pixels from
+            // (u + 1) RPG S HC on, behind them: a wave may write before it reads on.
+            static_assert(RPG * S * HC >= 16, "a later pixel group reads behind what an earlier one writes");
+            for (int blk = wave; blk < steps; blk += NW)
+#pragma unroll
+                for (int u0 = 0; u0 < UW; u0 += UC)
+                {
+                    v4i acc[4][UC];
+                    sums(blk, u0, acc);
+                    codes(blk, u0, acc);
+                }
+        }
+        if constexpr (!EARLY)
+        {
+#pragma unroll
+            for (int r = 0; r < RD; ++r)
+                if (r < steps) load_weights(r, r);
+        }
+    }
+    __syncthreads();
+
+    // ---- pointwise ------------------------------------------------------------------------------------------------------------------
+    v4i acc[CG][PG];
+    int xs[PG];
+#pragma unroll
+    for (int p = 0; p < PG; ++p)
+    {
+        xs[p] = 0;
+#pragma unroll
+        for (int c = 0; c < CG; ++c) acc[c][p] = v4i{0, 0, 0, 0};
+    }
+    const uint8_t* const pb = panel_lds + g * GP + j * 16;
+    for (int k0 = 0; k0 < steps; k0 += RD)
+    {
+#pragma unroll
+        for (int r = 0; r < RD; ++r)
+        {
+            const int ks = k0 + r;
+            if (ks >= steps) break;
+            v4i xb[PG];
+#pragma unroll
+            for (int p = 0; p < PG; ++p) xb[p] = *reinterpret_cast<const v4i*>(pb + ks * 4 * GP + p * 256);
+#pragma unroll
+            for (int c = 0; c < CG; ++c)
+#pragma unroll
+                for (int p = 0; p < PG; ++p) acc[c][p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wv[r][c], xb[p], acc[c][p], 0, 0, 0);
+            if constexpr (U)
+            {
+#pragma unroll
+                for (int p = 0; p < PG; ++p)
+#pragma unroll
+                    for (int d = 0; d < 4; ++d) xs[p] = __builtin_amdgcn_sdot4(xb[p][d], 0x01010101, xs[p], false);
+            }
+            if (ks + RD < steps) load_weights(ks + RD, r);
+        }
     }
 
-    // ---- write-out ---------------------------------------------------------------------------------------------------------
+    // ---- write-out --------------------------------------------------------------------------------------------------------------------
+    if constexpr (U)
+    {
 #pragma unroll
-    for (int t = 0; t < NQ; ++t)
+        for (int p = 0; p < PG; ++p)
+        {
+            xs[p] += __shfl_xor(xs[p], 16);
+            xs[p] += __shfl_xor(xs[p], 32);
+            xs[p] *= a.zw_neg;
+        }
+    }
+    __syncthreads();                                     // the panel has been read; the outputs take its place
 #pragma unroll
-        for (int s = 0; s < 2; ++s)
+    for (int c = 0; c < CG; ++c)
+    {
+        const uint8_t* const tc = ptab + ((wave * CG + c) * 16 + 4 * g) * 4;
+        Fast4 f;
+        f.mp = *reinterpret_cast<const float4*>(tc);
+        f.bp = *reinterpret_cast<const float4*>(tc + 4 * G::NCOL);
+        f.mm = *reinterpret_cast<const float4*>(tc + 8 * G::NCOL);
+        f.bm = *reinterpret_cast<const float4*>(tc + 12 * G::NCOL);
+        const int cq = min((bn * NW + wave) * CG + c, a.co_groups - 1) * 16 + 4 * g;
+        v4i corr = {0, 0, 0, 0};
+        if constexpr (U) corr = *reinterpret_cast<const v4i*>(a.pw_corr + cq);
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-            {
-                const int cl = (wq * NQ + t) * 64 + s * 32 + 8 * q + lane_c;
-                const float4 mp = *reinterpret_cast<const float4*>(tab + cl);
-                const float4 bp = *reinterpret_cast<const float4*>(tab + NCOL + cl);
-                const float4 mm = *reinterpret_cast<const float4*>(tab + 2 * NCOL + cl);
-                const float4 bm = *reinterpret_cast<const float4*>(tab + 3 * NCOL + cl);
-                const v16i& v = acc[t][s];
-                const uint32_t out = Requant4Dev(v[4 * q + 0], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3], mp, bp, mm, bm, a.pw_ct, a.pw_corr, cl, a.pw_rq);
-                *reinterpret_cast<uint32_t*>(Os + (wm * 32 + frag_row) * LDO + cl) = out;
-            }
+        for (int p = 0; p < PG; ++p)
+        {
+            v4i v = acc[c][p];
+            if constexpr (U) v += corr + xs[p];
+            *reinterpret_cast<uint32_t*>(panel_lds + (16 * p + j) * OP + (wave * CG + c) * 16 + 4 * g) =
+                Requant4Dev(v[0], v[1], v[2], v[3], f.mp, f.bp, f.mm, f.bm, a.pw_ct, U ? nullptr : a.pw_corr, cq, a.pw_rq);
+        }
+    }
     __syncthreads();
-    DWPW_STAMP();
-    const OutPtr outp = MakeOutPtr(a.y, static_cast<long long>(a.N) * a.Ho * a.Wo * a.Co);
-    constexpr int CHUNKS = NCOL / 16;                      // 16-byte pieces per pixel
-    constexpr int NP = 64 * CHUNKS / NTHR;
+    const OutPtr outp = MakeOutPtr(a.y, a.y_bytes);
+    constexpr int CHUNKS = NW * CG;                      // 16-byte pieces per pixel
+    constexpr int NP = (G::PX * CHUNKS + NT - 1) / NT;
 #pragma unroll
     for (int i = 0; i < NP; ++i)
     {
-        const int idx = tid + i * NTHR;
+        const int idx = tid + i * NT;
         const int r = idx / CHUNKS, chunk = idx - r * CHUNKS;
-        const int oy = ty * 8 + (r >> 3), ox = tx * 8 + (r & 7);
-        if (oy < a.Ho && ox < a.Wo && chunk * 16 < a.Co)
-        {
-            const v4i ov = *reinterpret_cast<const v4i*>(Os + r * LDO + chunk * 16);
-            StoreOut16(outp, ((static_cast<long long>(n) * a.Ho + oy) * a.Wo + ox) * a.Co + chunk * 16, ov);
-        }
+        const int oy = ty * TH + r / TW, ox = tx * TW + r % TW, c0 = bn * G::NCOL + chunk * 16;
+        if (r < G::PX && oy < a.Ho && ox < a.Wo && c0 < a.Co)
+            StoreOut16(outp, ((static_cast<long long>(n) * a.Ho + oy) * a.Wo + ox) * a.Co + c0, *reinterpret_cast<const v4i*>(panel_lds + r * OP + chunk * 16));
     }
-#ifdef MI355X_DWPW_STAMPS
-    __builtin_amdgcn_s_waitcnt(0);
-    DWPW_STAMP();
-#endif
-#undef DWPW_STAMP
 }
 
 } // namespace mi355x

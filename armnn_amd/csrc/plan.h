@@ -20,11 +20,13 @@ struct mi355x_conv2d_s
     uint8_t* w_direct = nullptr;   // [Kh][Kw][Ci][Co] / depthwise [Kh][Kw][Co], raw codes
     int8_t*  w_mfma   = nullptr;   // [Co_pad][K_pad] signed, zero padded
     int8_t*  w_frag   = nullptr;   // the same weights in operand order (small_conv_kernel.h), where a launch may want them
+    int8_t*  w_panel  = nullptr;   // 1x1: in operand order with the channels of a k-step interleaved as a depthwise layer before it leaves them
     uint8_t* pad16    = nullptr;   // 16 bytes that turn into the padding value under the kernel's input xor
     int8_t*  w_stem   = nullptr;   // small-Ci conv on MFMA: [Co rounded up to 32][stem_kp]
     int8_t*  w_stem2  = nullptr;   // ... the second halves of weight differences that need two
     int      stem_kp  = 0;
     uint32_t* dw_grp  = nullptr;   // depthwise 3x3: constants per group of 4 channels for the fused dw+pw kernel
+    uint32_t* dw_blk  = nullptr;   // depthwise 3x3: constants per block of 64 channels for the fused kernel with the layer between in LDS
     uint32_t* w_dot4  = nullptr;   // depthwise 3x3: [C][4] dwords; small-Ci conv: [Co][Kh][RD] dwords
     uint32_t* w_dot4b = nullptr;   // depthwise 3x3 / small-Ci conv whose weight differences need two int8 halves: the second halves
     int variant = 0;               // kernel variant within an algo (see RunPlan)
@@ -58,6 +60,8 @@ struct mi355x_conv2d_s
         (void)hipFree(w_frag);
         (void)hipFree(pad16);
         (void)hipFree(dw_grp);
+        (void)hipFree(dw_blk);
+        (void)hipFree(w_panel);
         (void)hipFree(w_stem);
         (void)hipFree(w_stem2);
         (void)hipFree(w_dot4);

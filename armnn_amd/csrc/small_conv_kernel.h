@@ -29,7 +29,8 @@ namespace mi355x
 
 // Weights in the order the kernel below loads them: [Co / 16][steps][64 lanes][16 bytes], lane l of a step = bytes
 // 64 step + 16 (l / 16) .. + 15 of row l % 16.  `steps` = K / 64 rounded up; bytes beyond K_pad are zero.
-static __global__ __launch_bounds__(256) void PackFragKernel(const int8_t* __restrict__ w, int8_t* __restrict__ out, int K_pad, int steps, long long pieces)
+// interleave: byte 4 i + e of those 16 is byte 64 step + 16 e + 4 (l / 16) + i of the row instead (dwpw_panel_kernel.h).
+static __global__ __launch_bounds__(256) void PackFragKernel(const int8_t* __restrict__ w, int8_t* __restrict__ out, int K_pad, int steps, long long pieces, int interleave)
 {
     const long long i = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
     if (i >= pieces) return;
@@ -39,7 +40,16 @@ static __global__ __launch_bounds__(256) void PackFragKernel(const int8_t* __res
     const long long row = gs / steps * 16 + (l & 15);
     const int k = s * 64 + (l >> 4) * 16;
     v4i v = {0, 0, 0, 0};
-    if (k < K_pad) v = *reinterpret_cast<const v4i*>(w + row * K_pad + k);
+    if (interleave != 0)
+    {
+        for (int e = 0; e < 4; ++e)
+            for (int b = 0; b < 4; ++b)
+            {
+                const int kb = s * 64 + 16 * e + 4 * (l >> 4) + b;
+                if (kb < K_pad) v[b] |= static_cast<int>(static_cast<uint32_t>(static_cast<uint8_t>(w[row * K_pad + kb])) << (8 * e));
+            }
+    }
+    else if (k < K_pad) v = *reinterpret_cast<const v4i*>(w + row * K_pad + k);
     *reinterpret_cast<v4i*>(out + i * 16) = v;
 }
 

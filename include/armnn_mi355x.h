@@ -133,9 +133,9 @@ int  mi355x_abi_version(void);
  *   bytes.
  *   "pwpool_auto" = 1 | 0: mi355x_conv2d_pool_fusion_pays may (1) or may not (0) recommend a 1x1 convolution + the global
  *   pooling behind it (tests and tuning).
- *   "dwpw_panel" = 1 | 0: mi355x_conv2d_run_fused may (1) or may not (0) run a depthwise layer of 256 or 512
- *   channels and a pointwise layer of 256 or 512 output channels on the kernel that gives a block an 8 x 8 pixel tile over
- *   all channels (identical bytes; lets tests compare it with the older fused kernel).
+ *   "dwpw_panel" = 1 | 0: mi355x_conv2d_run_fused may (1) or may not (0) run the other depthwise + pointwise pairs on the
+ *   kernel that keeps a tile of the layer between, over all its channels, in on-chip memory (identical bytes; lets tests
+ *   compare it with the older fused kernel).
  *   "chain_stages" = 2 | 3 | 4: LDS stages of the matrix-core tiles inside a layer chain; "chain_blocks_per_cu" = 0 .. 16:
  *   persistent blocks per CU of a layer chain (0: as many as fit); "chain_panel" = 0 | 1: 1x1 convolutions with 256 or 512
  *   input channels and at least 96 row blocks run as one work item per 64 output rows with the activation panel resident
@@ -259,9 +259,9 @@ int mi355x_conv2d_run_add(mi355x_conv2d_t plan, uint32_t batch, const void* inpu
  * there, so the intermediate tensor is never written.  The bytes produced equal mi355x_conv2d_run(depthwise) followed
  * by mi355x_conv2d_run(pointwise) -- in the reference these are two workloads in sequence
  * (RefDepthwiseConvolution2dWorkload.cpp:38-62, then RefConvolution2dWorkload.cpp:38-58).
- * mi355x_conv2d_fusable returns 0 when the pair qualifies (3x3 depthwise with channels % 32 == 0, multiplier 1,
- * stride 1 or 2; pointwise with output channels % 64 == 0; chaining shapes and identical quantization of the shared
- * tensor), else MI355X_ERR_UNSUPPORTED / MI355X_ERR_INVALID_ARGUMENT with the reason in mi355x_last_error().
+ * mi355x_conv2d_fusable returns 0 when the pair qualifies (3x3 depthwise with channels % 16 == 0, multiplier 1,
+ * stride 1 or 2; pointwise with output channels % 16 == 0; at most 1024 channels between; chaining shapes and identical
+ * quantization of the shared tensor), else MI355X_ERR_UNSUPPORTED / MI355X_ERR_INVALID_ARGUMENT with the reason in mi355x_last_error().
  * The other order is accepted as well: first = the unpadded 1x1 stride-1 Convolution2d, second = the 3x3 depthwise layer
  * that consumes it (stride 1 or 2, multiplier 1).  A block then computes whole images of the intermediate tensor for 64
  * of its channels, keeps them on chip and runs the depthwise filter there; it qualifies when one image has at most 224
@@ -270,10 +270,10 @@ int mi355x_conv2d_run_add(mi355x_conv2d_t plan, uint32_t batch, const void* inpu
 int mi355x_conv2d_fusable(mi355x_conv2d_t first, mi355x_conv2d_t second);
 /* 1 when running the pair as one launch is what the library recommends at this batch, else 0; never an error.  Today:
  * a depthwise layer over 32, 64 (stride 2) or 128 channels and the pointwise layer behind it (64, 128, 128 or -- at stride
- * 2 -- 256 output channels) in launches of at least 1024 tiles of 8 x 8 output pixels, which run on the persistent kernel
- * that keeps the pointwise weights on chip; and a depthwise layer over 256 or 512 channels (stride 1, or stride 2 from 256
- * to 512 channels) and the pointwise layer of 256 or 512 output channels behind it in launches of at least 100 such tiles,
- * which run on the kernel that gives a block an 8 x 8 pixel tile over all channels; and, in the other order, a 1x1
+ * 2 -- 256 output channels), which run on the persistent kernel that keeps the pointwise weights on chip, in launches of at
+ * least 1024 tiles of 8 x 8 output pixels, of 16 to 256 such tiles, and of 16 or more on maps of at least 16 tiles; any other
+ * depthwise layer of at most 512 channels and the pointwise layer behind it, which run on the kernel that keeps a tile of
+ * the layer between on chip, except on maps of at most 7 x 7 pixels from 8 images (stride 2: 64) on; and, in the other order, a 1x1
  * convolution and the depthwise layer behind it on maps of at most 7 x 7 pixels in launches of at least 64 images (option
  * "pwdw_auto" = 0 turns this one off).  No counterpart in the reference, which has no fused workloads on CpuRef. */
 int mi355x_conv2d_fusion_pays(mi355x_conv2d_t first, mi355x_conv2d_t second, uint32_t batch);

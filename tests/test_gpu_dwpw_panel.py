@@ -1,0 +1,65 @@
+"""Depthwise 3x3 + pointwise 1x1 in one launch with the layer between in LDS: the bytes of the two layers run apart, over the
+kernel's instances, maps that are no whole tiles, channel counts that are no whole blocks, weights with a zero point."""
+import numpy as np
+import pytest
+
+from armnn_amd import shim
+from armnn_amd.tensor import numpy_dtype
+from tests import cases
+
+pytestmark = pytest.mark.gpu
+U8, S8 = cases.U8, cases.S8
+
+# n, h, w, channels, output channels, stride: the tile that the launch's size asks for
+PAIRS = [
+    (1, 3, 5, 16, 16, 1, "4, 4, 8, 1, 0"),
+    (1, 9, 6, 48, 80, 2, "4, 4, 8, 1, 0"),
+    (1, 7, 7, 1024, 1024, 1, "4, 4, 8, 1, 0"),
+    (4, 14, 14, 512, 512, 1, "4, 4, 16, 1, 0"),
+    (13, 27, 30, 192, 208, 2, "4, 8, 8, 2, 0"),
+    (8, 20, 22, 192, 192, 1, "4, 8, 8, 2, 0"),
+    (5, 28, 28, 256, 256, 1, "4, 8, 8, 2, 4"),
+    (7, 14, 14, 512, 512, 1, "4, 8, 8, 2, 8"),
+    (14, 28, 27, 256, 512, 2, "4, 8, 8, 4, 4"),
+    (14, 14, 14, 512, 512, 1, "4, 8, 8, 4, 8"),
+    (27, 14, 13, 512, 1024, 2, "4, 8, 8, 4, 8"),
+    (14, 28, 28, 256, 256, 1, "8, 8, 8, 2, 4"),
+    (52, 13, 14, 256, 512, 1, "8, 8, 8, 4, 4"),
+    (52, 14, 14, 512, 512, 1, "8, 8, 8, 4, 8"),
+    (4, 60, 50, 16, 48, 1, "8, 16, 4, 1, 1"),
+    (9, 65, 70, 48, 96, 2, "8, 16, 4, 2, 1"),
+    (4, 41, 44, 96, 96, 1, "8, 8, 4, 2, 2"),
+    (8, 60, 61, 112, 192, 2, "8, 8, 4, 4, 2"),
+]
+
+
+@pytest.mark.parametrize("general", [False, True], ids=["symmetric", "zero_points"])
+@pytest.mark.parametrize("n,h,w,c,co,s,tile", PAIRS, ids=[f"{p[0]}x{p[1]}x{p[2]}x{p[3]}_{p[4]}_s{p[5]}" for p in PAIRS])
+def test_pair_equals_the_layers_run_apart(n, h, w, c, co, s, tile, general):
+    dt, mid_zp = (U8, 0) if (c + h) % 2 else (S8, -128)
+    wq = dict(w_dtype=U8, w_offset=101, per_axis=False) if general else {}
+    dw = cases.make_conv_case("dw", 61000 + c + h, n=n, h=h, w=w, ci=c, depthwise=True, stride=(s, s), in_dtype=dt, in_scale=0.0235,
+                              in_offset=120 if dt == U8 else -8, out_scale=0.0235, out_offset=mid_zp, act=cases.RELU6,
+                              **(dict(wq, w_scale_range=(0.01, 0.02)) if general else dict(w_scale_range=(0.01, 0.05))))
+    ho, wo = dw.out_info.shape[1:3]
+    pw = cases.make_conv_case("pw", 62000 + co + h, n=n, h=ho, w=wo, ci=c, co=co, kh=1, kw=1, in_dtype=dt, in_scale=0.0235, in_offset=mid_zp,
+                              out_scale=0.03, out_offset=mid_zp + 5, act=cases.RELU6 if h % 2 else (0, 0.0, 0.0), **wq)
+    dev = shim.Device()
+
+    def plan(case):
+        return shim.Conv2dPlan(case.x.info, case.w, case.b, case.out_info, activation=case.act[0], act_a=case.act[1], act_b=case.act[2], **case.params)
+    first, second = plan(dw), plan(pw)
+    assert first.fusable_with(second), shim.load_library().mi355x_last_error().decode()
+    x = shim.DeviceBuffer(dw.x.data.nbytes).upload(dw.x.data)
+    mid = shim.DeviceBuffer(dw.out_info.num_elements)
+    apart, one = shim.DeviceBuffer(pw.out_info.num_elements), shim.DeviceBuffer(pw.out_info.num_elements)
+    first.run_fused(second, n, x.ptr, one.ptr)
+    kernel = shim.last_kernel()
+    print(kernel, flush=True)
+    assert kernel == f"DwPwPanelKernel<{s}, {tile}, {'true' if general else 'false'}>", kernel
+    first.run(n, x.ptr, mid.ptr)
+    second.run(n, mid.ptr, apart.ptr)
+    dev.synchronize()
+    got, want = (b.download(pw.out_info.shape, numpy_dtype(dt)) for b in (one, apart))
+    assert len(np.unique(want)) > 8
+    np.testing.assert_array_equal(got, want)
