@@ -1681,10 +1681,16 @@ int mi355x_conv2d_run_add(mi355x_conv2d_t plan, uint32_t batch, const void* inpu
 namespace
 {
 // Depthwise + pointwise pairs go to the kernel with resident weights where it is built for the shape (DwPwStreamShape), else to
-// the one with the layer between in LDS; what either option switches off, and nothing else, is left to DwPwKernel.
-bool PanelRuns(const mi355x_conv2d_s* dw, const mi355x_conv2d_s* pw)
+// the one with the layer between in LDS; what either option switches off, and nothing else, is left to DwPwKernel.  Over 128
+// channels the resident weights leave a CU one or two blocks, and large launches are faster on the other kernel: 56 x 56 x 128 ->
+// 128, 64 images 28.5 -> 23.8 us, 256 88.8 -> 80.7; -> 28 x 28 x 256 19.2 -> 16.2, 61.6 -> 50.2 (from four items per CU on; 28 x 28
+// x 256 at 8 images, 128 items, 6.4 against 7.8).  Below, and over 32 and 64 channels at any size, it is the other way round.
+bool PanelRuns(const mi355x_conv2d_s* dw, const mi355x_conv2d_s* pw, uint32_t batch)
 {
-    return GlobalOptions().dwpw_panel != 0 && DwPwStreamShape(dw, pw) == 0 && DwPwPanelTakes(dw, pw);
+    if (GlobalOptions().dwpw_panel == 0 || !DwPwPanelTakes(dw, pw)) return false;
+    if (DwPwStreamShape(dw, pw) == 0) return true;
+    const long long items = static_cast<long long>(batch) * ((dw->d.out_w + 7) / 8) * ((dw->d.out_h + 7) / 8);
+    return dw->d.out_c >= 128 && items >= 1024;
 }
 
 int DwPwTileCheck(const mi355x_conv2d_s* dw, const mi355x_conv2d_s* pw)
@@ -1716,7 +1722,7 @@ int mi355x_conv2d_fusable(mi355x_conv2d_t dw, mi355x_conv2d_t pw)
     if (a.out_c != b.in_c || a.out_h != b.in_h || a.out_w != b.in_w) return SetError(MI355X_ERR_INVALID_ARGUMENT, "the layers' shapes do not chain");
     if (a.output.dtype != b.input.dtype || a.output.scale != b.input.scale || a.output.offset != b.input.offset)
         return SetError(MI355X_ERR_INVALID_ARGUMENT, "the first layer's output quantization is not the second layer's input quantization");
-    if (PanelRuns(dw, pw)) return 0;
+    if (PanelRuns(dw, pw, 0)) return 0;
     return DwPwTileCheck(dw, pw);
 }
 
@@ -1740,7 +1746,7 @@ int mi355x_conv2d_fusion_pays(mi355x_conv2d_t first, mi355x_conv2d_t second, uin
         const long long tiles = static_cast<long long>((first->d.out_w + 7) / 8) * ((first->d.out_h + 7) / 8), items = batch * tiles;
         return items >= 1024 || (items >= 16 && (items <= 256 || tiles >= 16)) ? 1 : 0;
     }
-    if (mi355x_conv2d_fusable(first, second) != 0 || !PanelRuns(first, second)) return 0;
+    if (mi355x_conv2d_fusable(first, second) != 0 || !PanelRuns(first, second, batch)) return 0;
     // 7 x 7 maps: from 8 images on the 1x1 convolution is worth more with a pooling behind it (mi355x_conv2d_pool_fusion_pays), and
     // from 64 on with the depthwise layer behind it (above); beyond 512 channels every block's own copy of the depthwise layer
     // costs what the launch saves (1024 -> 1024, one image: 6.9 us against 7.4)
@@ -1762,9 +1768,9 @@ int mi355x_conv2d_run_fused(mi355x_conv2d_t dw, mi355x_conv2d_t pw, uint32_t bat
         if (int rc = PwDwCheck(dw, pw, &sh)) return rc;
         return LaunchPwDw(dw, pw, sh, batch, input_dev, output_dev, ToHip(stream));
     }
+    if (PanelRuns(dw, pw, batch)) return LaunchDwPwPanel(dw, pw, batch, input_dev, output_dev, ToHip(stream));
     if (GlobalOptions().dwpw_stream != 0)
         if (const int which = DwPwStreamShape(dw, pw)) return LaunchDwPwStream(dw, pw, which, batch, input_dev, output_dev, ToHip(stream));
-    if (PanelRuns(dw, pw)) return LaunchDwPwPanel(dw, pw, batch, input_dev, output_dev, ToHip(stream));
     if (dw->d.stride_x == 2) return LaunchDwPw<2, 2>(dw, pw, batch, input_dev, output_dev, ToHip(stream));
     // stride 1: the wide tile (8 x 16 pixels) while it still yields two blocks per CU, else the narrow one (8 x 8)
     const long long wide = static_cast<long long>(batch) * ((dw->d.out_w + 15) / 16) * ((dw->d.out_h + 7) / 8);

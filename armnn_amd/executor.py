@@ -4,6 +4,9 @@ the whole forward pass launched kernel by kernel or captured into a HIP graph an
 from __future__ import annotations
 
 import ctypes as C
+import os
+import threading
+import weakref
 from dataclasses import dataclass
 from typing import Dict, List, Optional, Tuple
 
@@ -99,7 +102,7 @@ class DeviceNetwork:
         self.dev = shim.Device()
         self.lib = shim.load_library()
         self.stream = self.dev.stream()
-        self.side_streams = [self.dev.stream() for _ in range(lanes - 1)]
+        self._side_streams: Optional[List] = None
         self.buffers: Dict[str, shim.DeviceBuffer] = {}
         self.steps: List = []          # (layer, callable(stream))
         self._step_plans: List = []    # plan of each step (None for plan-less layers), parallel to self.steps
@@ -110,7 +113,7 @@ class DeviceNetwork:
         self.lanes_after_chain = lanes_after_chain
         self._pinned, self._staging_busy = None, False
         self.join_for_fused = join_for_fused      # fused pairs run on the whole batch: the lanes join in front of the first one
-        self.graph = None
+        self.graphs: Dict[bool, List] = {}                  # of a pass in its lanes / as one lane, captured when first replayed
         self.use_graph = use_graph
         algo_overrides = algo_overrides or {}
 
@@ -425,37 +428,45 @@ class DeviceNetwork:
         forked = False
         single_from_here = False
 
-        def fork():
-            ev = self._sync_event()
-            self.dev.event_record(ev, self.stream)
-            for side in self.side_streams:
-                self.dev.stream_wait_event(side, ev)
-
-        def join():
-            for side in self.side_streams:
-                ev = self._sync_event()
-                self.dev.event_record(ev, side)
-                self.dev.stream_wait_event(self.stream, ev)
-
         self._sync_next = 0
         # lanes interleaved layer by layer, so launches next to each other in submission order can overlap
         for _, fn in self.steps:
             if getattr(fn, "whole_batch", False) or single_from_here:
                 if forked:
-                    join()
+                    self._join()
                     forked = False
                 fn(self.stream, 0, 1)
                 if getattr(fn, "whole_batch", False) and not self.lanes_after_chain:
                     single_from_here = True
                 continue
             if not forked:
-                fork()
+                self._fork()
                 forked = True
             fn(self.stream, 0, self.lanes)
             for k, side in enumerate(self.side_streams, start=1):
                 fn(side, k, self.lanes)
         if forked:
-            join()
+            self._join()
+
+    @property
+    def side_streams(self):
+        """The streams of the lanes behind the first, created at the first pass that runs in lanes: a stream that exists takes part
+        in the sharing of hardware queues whether it is used or not."""
+        if self._side_streams is None:
+            self._side_streams = [self.dev.stream() for _ in range(self.lanes - 1)]
+        return self._side_streams
+
+    def _fork(self):
+        ev = self._sync_event()
+        self.dev.event_record(ev, self.stream)
+        for side in self.side_streams:
+            self.dev.stream_wait_event(side, ev)
+
+    def _join(self):
+        for side in self.side_streams:
+            ev = self._sync_event()
+            self.dev.event_record(ev, side)
+            self.dev.stream_wait_event(self.stream, ev)
 
     def _sync_event(self):
         """Events for forks and joins, one per use within a forward pass (a captured graph keeps them)."""
@@ -467,14 +478,64 @@ class DeviceNetwork:
         self._sync_next += 1
         return ev
 
+    # The networks of the process that have run, and how many hardware queues the streams of a process share.
+    _running_lock = threading.Lock()
+    _running: "weakref.WeakSet[DeviceNetwork]" = weakref.WeakSet()
+    _hardware_queues = int(os.environ.get("GPU_MAX_HW_QUEUES", "4"))
+
+    def _one_lane_now(self) -> bool:
+        """Whether this pass runs as one lane: where the lanes of all networks outnumber the hardware queues, streams share them
+        and a lane waits behind another network's, or behind its own sibling (three of ResNet-50 side by side, 32 images in
+        two lanes each, 605 us a pass; as one lane each 525; one alone 720 in its lanes, 870 as one, 1130 with the two on one
+        queue)."""
+        with self._running_lock:
+            self._running.add(self)
+            lanes = sum(n.lanes for n in self._running)
+        return lanes > max(self._hardware_queues, self.lanes) and not self.chains and not self.tails
+
+    def _capture(self, one_lane: bool):
+        """The graphs of a pass: one per lane, because a chain of kernels is replayed without the host (57 launches of ResNet-50 in
+        45 us of host time) while a graph with branches is taken apart node by node (430 us at two lanes, more than the device
+        needs); one for everything where a step works on the whole batch."""
+        graphs = []
+        if one_lane and self.lanes > 1:
+            for p in self.plans:
+                if isinstance(p, shim.Conv2dPlan):
+                    p.set_concurrency(1)
+            self.dev.graph_begin(self.stream)
+            for _, fn in self.steps:
+                fn(self.stream, 0, 1)
+            graphs.append(self.dev.graph_end(self.stream))
+            for p in self.plans:
+                if isinstance(p, shim.Conv2dPlan):
+                    p.set_concurrency(self.lanes)
+            return graphs
+        if self.lanes == 1 or any(getattr(fn, "whole_batch", False) for _, fn in self.steps):
+            self.dev.graph_begin(self.stream)
+            self._enqueue_lanes()
+            return [self.dev.graph_end(self.stream)]
+        for lane, stream in enumerate([self.stream] + self.side_streams):
+            self.dev.graph_begin(stream)
+            for _, fn in self.steps:
+                fn(stream, lane, self.lanes)
+            graphs.append(self.dev.graph_end(stream))
+        return graphs
+
     def enqueue(self):
         """One forward pass on self.stream (asynchronous)."""
         if self.use_graph:
-            if self.graph is None:
-                self.dev.graph_begin(self.stream)
-                self._enqueue_lanes()
-                self.graph = self.dev.graph_end(self.stream)
-            self.dev.graph_launch(self.graph, self.stream)
+            one_lane = self.lanes > 1 and self._one_lane_now()
+            if one_lane not in self.graphs:
+                self.graphs[one_lane] = self._capture(one_lane)
+            graphs = self.graphs[one_lane]
+            if len(graphs) == 1:
+                self.dev.graph_launch(graphs[0], self.stream)
+                return
+            self._sync_next = 0
+            self._fork()
+            for graph, stream in zip(graphs, [self.stream] + self.side_streams):
+                self.dev.graph_launch(graph, stream)
+            self._join()
         else:
             self._enqueue_lanes()
 
@@ -573,9 +634,9 @@ class DeviceNetwork:
         return out
 
     def close(self):
-        if self.graph is not None:
-            self.dev.graph_destroy(self.graph)
-            self.graph = None
+        for g in [g for graphs in self.graphs.values() for g in graphs]:
+            self.dev.graph_destroy(g)
+        self.graphs = {}
         for ch in self.chains:
             ch.destroy()
         self.chains = []
@@ -584,6 +645,8 @@ class DeviceNetwork:
         self.tails = []
         for p in self.plans:
             p.destroy()
+        with self._running_lock:
+            self._running.discard(self)
         for b in set(self.buffers.values()):
             b.free()
         if self._pinned is not None:
@@ -591,6 +654,6 @@ class DeviceNetwork:
             for p in self._pinned:
                 shim._chk(self.lib.mi355x_host_free(p))
             self._pinned = None
-        for side in self.side_streams:
+        for side in self._side_streams or []:
             self.dev.stream_destroy(side)
         self.dev.stream_destroy(self.stream)

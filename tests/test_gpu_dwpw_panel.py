@@ -30,6 +30,8 @@ PAIRS = [
     (9, 65, 70, 48, 96, 2, "8, 16, 4, 2, 1"),
     (4, 41, 44, 96, 96, 1, "8, 8, 4, 2, 2"),
     (8, 60, 61, 112, 192, 2, "8, 8, 4, 4, 2"),
+    (1024, 7, 8, 128, 128, 1, "8, 8, 4, 2, 2"),
+    (1024, 13, 15, 128, 256, 2, "8, 8, 4, 4, 2"),
 ]
 
 
