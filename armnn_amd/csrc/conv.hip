@@ -1021,6 +1021,22 @@ int RunPlan(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, hi
             MI355X_HIP(hipGetLastError());
             return 0;
         }
+        // 1x1 layers of many rows: whole rows in LDS, weights from L2 (row_panel_kernel.h), from the number of 64 x 128 tiles that fills
+        // the chip on.  Up to 256 channels that is seven tiles for eight CUs (128 -> 512 at 28 x 28, 8 images, 392 tiles: 6.1 ->
+        // 4.5 us); beyond, a tile takes long enough to want one and a half (512 -> 256: 196 tiles 5.4 against 5.6, 392 7.7 -> 6.6), and
+        // with more than 1024 output channels the 256-row tiles, where they fill the chip, read the rows less often (4096 rows, 512
+        // -> 2048: 12.0 against 12.4).  Up to 64 channels the kernel with resident weights is faster for launches of more than 2048
+        // (64 -> 256 at 56 x 56, 16 images, 1568 tiles: 8.4 -> 7.7; 32 images: 12.6 against 13.4).
+        if (unit && p->w_frag && p->ragged_ck == 0 && (g.Co & 15) == 0 && p->tile_override == 0 && p->opt_igemm_lds != 0)
+        {
+            const long long tiles = (rows + 63) / 64 * ((g.Co + 127) / 128);
+            if (g.Ci <= 256 ? tiles >= 224 && (g.Ci > 64 || tiles <= 2048) : g.Ci <= 768 && tiles >= 384 && (g.Co <= 1024 || tiles < 896))
+            {
+                const uint8_t* res = nullptr;
+                if (t_pending_add) { res = t_pending_add->other; t_pending_add->taken = true; }
+                return LaunchRowPanel(p, batch, x, y, res, res ? &t_pending_add->fuse : nullptr, stream);
+            }
+        }
         // Few rows: 32 x 32 tiles whose waves split K (small_conv_kernel.h), while they number at most one and a half per CU: at
         // 392 of them 14 x 14 x 256 at 8 images, 3 x 3, takes 8.0 us against 9.5; from there on the larger tiles' lower traffic
         // wins (14 x 14 x 512 -> 512 at 8 images, 784 tiles: 5.5 against 4.7).  Where the layer has a weight slab (at most 128 input

@@ -16,4 +16,7 @@ int PackFragments(mi355x_conv2d_s* p);
 // % 16 == 0, aligned tensors), or null.
 int LaunchSmallConv(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, const uint8_t* res, const AddFuse* add, hipStream_t stream);
 
+// RowPanelKernel (row_panel_kernel.h) for a 1x1 plan with w_frag; res / add as above, any output channels % 16 == 0.
+int LaunchRowPanel(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, const uint8_t* res, const AddFuse* add, hipStream_t stream);
+
 } // namespace mi355x

@@ -3,6 +3,7 @@
 
 #include "common.h"
 #include "conv_kernels.h"
+#include "row_panel_kernel.h"
 #include "small_conv_kernel.h"
 
 using namespace mi355x;
@@ -130,4 +131,37 @@ int mi355x::LaunchSmallConv(const mi355x_conv2d_s* p, uint32_t batch, const void
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, stream, a);
     MI355X_HIP(hipGetLastError());
     return 0;
+}
+
+template <int CG, int KB, bool AW>
+static int LaunchRowPanelT(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, const uint8_t* res, const AddFuse* add, hipStream_t stream)
+{
+    IgemmArgs a;
+    bool unit_fast = false;
+    if (const int rc = FillIgemmLdsArgs(p, 64, 64 * CG, batch, x, y, &a, &unit_fast)) return rc;
+    a.w = p->w_frag;
+    if (res) { a.res = res; a.add = *add; }
+    const long long nblocks = static_cast<long long>(a.tiles_m) * a.tiles_n;
+    if (nblocks * a.tiles_n >= (1ll << 32) || nblocks > 0x7fffffffll - 8) return SetError(MI355X_ERR_UNSUPPORTED, "grid too large");
+    const uint32_t rcp = static_cast<uint32_t>(((1ull << 32) + static_cast<uint32_t>(a.tiles_n) - 1) / static_cast<uint32_t>(a.tiles_n));
+    const int grid = static_cast<int>((nblocks + 7) / 8 * 8);
+    NoteKernel("RowPanelKernel<%d, %d, %s>", CG, KB, BoolName(AW));
+    hipLaunchKernelGGL((RowPanelKernel<CG, KB, AW>), dim3(grid), dim3(256), RowPanelSmem<CG>(a.Ci), stream, a, p->Co_pad / 16, rcp);
+    MI355X_HIP(hipGetLastError());
+    return 0;
+}
+
+template <int CG, bool AW>
+static int LaunchRowPanelK(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, const uint8_t* res, const AddFuse* add, hipStream_t stream)
+{
+    return p->geom.Ci <= 128 ? LaunchRowPanelT<CG, 128, AW>(p, batch, x, y, res, add, stream)
+           : p->geom.Ci <= 256 ? LaunchRowPanelT<CG, 256, AW>(p, batch, x, y, res, add, stream)
+                               : LaunchRowPanelT<CG, kRowPanelK, AW>(p, batch, x, y, res, add, stream);
+}
+
+int mi355x::LaunchRowPanel(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, const uint8_t* res, const AddFuse* add, hipStream_t stream)
+{
+    const bool aw = p->zw_neg != 0;
+    if (p->geom.Co <= 64) return aw ? LaunchRowPanelK<1, true>(p, batch, x, y, res, add, stream) : LaunchRowPanelK<1, false>(p, batch, x, y, res, add, stream);
+    return aw ? LaunchRowPanelK<2, true>(p, batch, x, y, res, add, stream) : LaunchRowPanelK<2, false>(p, batch, x, y, res, add, stream);
 }
