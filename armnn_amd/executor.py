@@ -103,6 +103,8 @@ class DeviceNetwork:
         self.lib = shim.load_library()
         self.stream = self.dev.stream()
         self._side_streams: Optional[List] = None
+        with self._blocks_lock:
+            self._open.add(self)
         self.buffers: Dict[str, shim.DeviceBuffer] = {}
         self.steps: List = []          # (layer, callable(stream))
         self._step_plans: List = []    # plan of each step (None for plan-less layers), parallel to self.steps
@@ -111,7 +113,6 @@ class DeviceNetwork:
         self.tails: List = []
         self._pool_descs = {}
         self.lanes_after_chain = lanes_after_chain
-        self._pinned, self._staging_busy = None, False
         self.join_for_fused = join_for_fused      # fused pairs run on the whole batch: the lanes join in front of the first one
         self.graphs: Dict[bool, List] = {}                  # of a pass in its lanes / as one lane, captured when first replayed
         self.use_graph = use_graph
@@ -570,19 +571,32 @@ class DeviceNetwork:
         self.synchronize()
         return QTensor(info, self.buffers[name].download(info.shape, numpy_dtype(info.dtype), self.stream))
 
-    # host arrays pass through pinned memory of the network's own, up to this many bytes of images
-    _STAGED_BYTES = 64 << 20
+    # Pinned memory that host arrays pass through: blocks shared by the networks of the process, at most this many kept while no
+    # call uses them, and none once the last network is closed.
+    _BLOCK_BYTES, _BLOCKS_KEPT = 2 << 20, 32
+    _blocks_lock = threading.Lock()
+    _blocks: List[int] = []
+    _open: "weakref.WeakSet[DeviceNetwork]" = weakref.WeakSet()
 
-    def _staging(self, nbytes_in: int, nbytes_out: int):
-        """(address of pinned memory for the images, for the results), allocated at the first call."""
-        if self._pinned is None:
-            ptrs = []
-            for n in (nbytes_in, nbytes_out):
-                p = C.c_void_p()
-                shim._chk(self.lib.mi355x_host_alloc(C.byref(p), n))
-                ptrs.append(p.value)
-            self._pinned = tuple(ptrs)
-        return self._pinned
+    def _take_blocks(self, n: int) -> List[int]:
+        with self._blocks_lock:
+            taken, self._blocks[:] = self._blocks[:n], self._blocks[n:]
+        while len(taken) < n:
+            p = C.c_void_p()
+            rc = self.lib.mi355x_host_alloc(C.byref(p), self._BLOCK_BYTES)
+            if rc != 0:
+                self._give_blocks(taken)
+                shim._chk(rc)
+            taken.append(p.value)
+        return taken
+
+    def _give_blocks(self, blocks: List[int]):
+        with self._blocks_lock:
+            self._blocks.extend(blocks)
+            keep = self._BLOCKS_KEPT if len(self._open) > 0 else 0
+            extra, self._blocks[:] = self._blocks[keep:], self._blocks[:keep]
+        for p in extra:
+            shim._chk(self.lib.mi355x_host_free(p))
 
     def run(self, x: QTensor) -> QTensor:
         """One forward pass over host arrays.  The images are copied to pinned memory a part at a time, each part on its way
@@ -593,26 +607,30 @@ class DeviceNetwork:
         info = self.net.info(self.net.output, self.batch)
         src = np.ascontiguousarray(x.data)
         dst = np.empty(info.shape, dtype=numpy_dtype(info.dtype))
-        if src.nbytes > self._STAGED_BYTES or dst.nbytes > self._STAGED_BYTES:
+        part = min(max(src.nbytes // 4 + 0xffff & ~0xffff, 512 << 10), self._BLOCK_BYTES)
+        parts = -(-src.nbytes // part)
+        if parts > self._BLOCKS_KEPT or dst.nbytes > self._BLOCK_BYTES:
             self.upload_input(x)
             self.enqueue()
             return self.download()
         assert x.info.shape == self.net.info(self.net.input, self.batch).shape and src.nbytes <= self.buffers[self.net.input].nbytes
-        pin_in, pin_out = self._staging(src.nbytes, dst.nbytes)
-        if self._staging_busy:                             # an earlier call failed half way: its transfers may still be under way
+        blocks = self._take_blocks(parts + 1)
+        try:
+            at, dev = src.ctypes.data, self.buffers[self.net.input].ptr
+            for k in range(parts):
+                o = k * part
+                n = min(part, src.nbytes - o)
+                C.memmove(blocks[k], at + o, n)
+                shim._chk(self.lib.mi355x_memcpy_h2d_async(dev + o, blocks[k], n, self.stream))
+            self.enqueue()
+            shim._chk(self.lib.mi355x_memcpy_d2h_async(blocks[parts], self.buffers[self.net.output].ptr, dst.nbytes, self.stream))
             self.synchronize()
-        self._staging_busy = True
-        at, dev = src.ctypes.data, self.buffers[self.net.input].ptr
-        part = min(max(src.nbytes // 4 + 0xffff & ~0xffff, 512 << 10), 2 << 20)
-        for o in range(0, src.nbytes, part):
-            n = min(part, src.nbytes - o)
-            C.memmove(pin_in + o, at + o, n)
-            shim._chk(self.lib.mi355x_memcpy_h2d_async(dev + o, pin_in + o, n, self.stream))
-        self.enqueue()
-        shim._chk(self.lib.mi355x_memcpy_d2h_async(pin_out, self.buffers[self.net.output].ptr, dst.nbytes, self.stream))
-        self.synchronize()
-        self._staging_busy = False
-        C.memmove(dst.ctypes.data, pin_out, dst.nbytes)
+            C.memmove(dst.ctypes.data, blocks[parts], dst.nbytes)
+        except BaseException:
+            self.synchronize()                             # no transfer may still use the blocks
+            raise
+        finally:
+            self._give_blocks(blocks)
         return QTensor(info, dst)
 
     def time_layers(self, iters: int = 20, warmup: int = 3):
@@ -647,13 +665,11 @@ class DeviceNetwork:
             p.destroy()
         with self._running_lock:
             self._running.discard(self)
+        with self._blocks_lock:
+            self._open.discard(self)
+        self._give_blocks([])
         for b in set(self.buffers.values()):
             b.free()
-        if self._pinned is not None:
-            self.synchronize()
-            for p in self._pinned:
-                shim._chk(self.lib.mi355x_host_free(p))
-            self._pinned = None
         for side in self._side_streams or []:
             self.dev.stream_destroy(side)
         self.dev.stream_destroy(self.stream)
