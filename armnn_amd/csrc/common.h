@@ -19,8 +19,32 @@ int SetError(int code, const char* fmt, ...);
 
 // Records the name of the kernel the calling thread is about to launch, as a profiler would list it (without the
 // namespace and the argument list); mi355x_last_kernel() returns it.  Measurement support: lets a benchmark label its
-// per-layer timings with kernel symbols.
-void NoteKernel(const char* fmt, ...);
+// per-layer timings with kernel symbols.  Only the format and its arguments are kept at a launch -- integers and strings that
+// outlive it -- and written out when asked for: formatting took a twentieth of the host's share of a small layer's call.
+struct KernelNote
+{
+    static constexpr int kMostArgs = 10;
+    const char* format;
+    long long   number[kMostArgs];
+    const char* text[kMostArgs];     // of a %s; null for a %d
+};
+KernelNote& CurrentKernelNote();     // the calling thread's
+
+inline void SetNoteArg(KernelNote& n, int i, const char* s) { n.text[i] = s; }
+inline void SetNoteArg(KernelNote& n, int i, long long v) { n.text[i] = nullptr; n.number[i] = v; }
+inline void SetNoteArg(KernelNote& n, int i, int v) { SetNoteArg(n, i, static_cast<long long>(v)); }
+inline void SetNoteArg(KernelNote& n, int i, unsigned v) { SetNoteArg(n, i, static_cast<long long>(v)); }
+
+template <typename... A>
+void NoteKernel(const char* format, A... args)
+{
+    static_assert(sizeof...(A) <= KernelNote::kMostArgs, "KernelNote::kMostArgs");
+    KernelNote& n = CurrentKernelNote();
+    n.format = format;
+    [[maybe_unused]] int i = 0;
+    (SetNoteArg(n, i++, args), ...);
+}
+
 inline const char* BoolName(bool b) { return b ? "true" : "false"; }
 
 inline int HipFail(hipError_t e, const char* what)

@@ -24,21 +24,10 @@ int SetError(int code, const char* fmt, ...)
     return code;
 }
 
-namespace
+KernelNote& CurrentKernelNote()
 {
-char* KernelNameBuffer()
-{
-    static thread_local char buf[192] = {0};
-    return buf;
-}
-} // namespace
-
-void NoteKernel(const char* fmt, ...)
-{
-    va_list ap;
-    va_start(ap, fmt);
-    vsnprintf(KernelNameBuffer(), 192, fmt, ap);
-    va_end(ap);
+    static thread_local KernelNote note{};
+    return note;
 }
 
 namespace
@@ -161,7 +150,25 @@ extern "C" {
 
 const char* mi355x_last_error(void) { return ErrorBuffer(); }
 
-const char* mi355x_last_kernel(void) { return KernelNameBuffer(); }
+const char* mi355x_last_kernel(void)
+{
+    static thread_local char buf[192];
+    const KernelNote& n = CurrentKernelNote();
+    size_t at = 0;
+    int arg = 0;
+    for (const char* f = n.format; f && *f && at + 24 < sizeof(buf); ++f)
+    {
+        if (*f != '%') { buf[at++] = *f; continue; }
+        ++f;                                             // the d or s of a conversion
+        if (arg == KernelNote::kMostArgs) break;
+        const int left = static_cast<int>(sizeof(buf) - at);
+        const int w = n.text[arg] ? snprintf(buf + at, left, "%s", n.text[arg]) : snprintf(buf + at, left, "%lld", n.number[arg]);
+        at += static_cast<size_t>(std::min(w, left - 1));
+        ++arg;
+    }
+    buf[at] = 0;
+    return buf;
+}
 
 int mi355x_abi_version(void) { return MI355X_ABI_VERSION; }
 

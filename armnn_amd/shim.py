@@ -6,6 +6,8 @@ returns an error: there is no CPU fallback anywhere in this package.
 from __future__ import annotations
 
 import ctypes as C
+import importlib.machinery
+import importlib.util
 import os
 from typing import Optional, Sequence
 
@@ -15,6 +17,7 @@ from .tensor import DataType, QTensor, TensorInfo, numpy_dtype
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libarmnn_mi355x.so")
+CALLS_PATH = os.path.join(_HERE, "lib", "_calls.so")
 
 ALGO_AUTO, ALGO_DIRECT, ALGO_MFMA, ALGO_DEPTHWISE, ALGO_DOT4 = 0, 1, 2, 3, 4
 ACT_NONE, ACT_RELU, ACT_BOUNDED_RELU = 0, 1, 2
@@ -85,16 +88,23 @@ class ShimError(RuntimeError):
 
 
 _lib = None
+_calls = None                          # the launch entry points without ctypes (csrc/pycalls.cpp), and their addresses
+_conv2d_run_at = _fc_run_at = 0
 
 
 def load_library(path: str = LIB_PATH) -> C.CDLL:
     """dlopen the device library (no GPU needed for loading)."""
-    global _lib
+    global _lib, _calls, _conv2d_run_at, _fc_run_at
     if _lib is None:
-        if not os.path.exists(path):
-            raise FileNotFoundError(f"{path} not found: build it with `make -C armnn_amd/csrc` "
-                                    f"(or __graft_entry__.build()); there is no fallback path")
+        for p in (path, CALLS_PATH):
+            if not os.path.exists(p):
+                raise FileNotFoundError(f"{p} not found: build it with `make -C armnn_amd/csrc` "
+                                        f"(or __graft_entry__.build()); there is no fallback path")
+        loader = importlib.machinery.ExtensionFileLoader("_calls", CALLS_PATH)
+        _calls = importlib.util.module_from_spec(importlib.util.spec_from_loader("_calls", loader))
+        loader.exec_module(_calls)
         _lib = C.CDLL(path)
+        _conv2d_run_at, _fc_run_at = (C.cast(fn, C.c_void_p).value for fn in (_lib.mi355x_conv2d_run, _lib.mi355x_fc_run))
         _lib.mi355x_last_error.restype = C.c_char_p
         _lib.mi355x_last_kernel.restype = C.c_char_p
         V = C.c_void_p
@@ -311,7 +321,12 @@ class Conv2dPlan:
         return a.value, buf.value.decode()
 
     def run(self, batch: int, x_dev: int, y_dev: int, stream=None):
-        _chk(self.lib.mi355x_conv2d_run(self.plan, batch, x_dev, y_dev, stream))
+        try:
+            rc = _calls.run(_conv2d_run_at, self.plan, batch, x_dev, y_dev, stream)
+        except TypeError:                                  # an argument that is no plain int: ctypes' own conversions decide
+            rc = self.lib.mi355x_conv2d_run(self.plan, batch, x_dev, y_dev, stream)
+        if rc != 0:
+            _chk(rc)
 
     def fusable_with(self, second: "Conv2dPlan") -> bool:
         """True when this plan and `second`, the layer consuming its output, can run as one kernel: 3x3 depthwise + 1x1
@@ -451,7 +466,12 @@ class FullyConnectedPlan:
         return a.value, buf.value.decode()
 
     def run(self, batch: int, x_dev: int, y_dev: int, stream=None):
-        _chk(self.lib.mi355x_fc_run(self.plan, batch, x_dev, y_dev, stream))
+        try:
+            rc = _calls.run(_fc_run_at, self.plan, batch, x_dev, y_dev, stream)
+        except TypeError:
+            rc = self.lib.mi355x_fc_run(self.plan, batch, x_dev, y_dev, stream)
+        if rc != 0:
+            _chk(rc)
 
     def destroy(self):
         if self.plan:
