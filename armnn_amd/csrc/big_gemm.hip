@@ -16,6 +16,8 @@ int SetLimit()
 {
     MI355X_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&BigGemmKernel<BM, BN, ST, U8, AW, true>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                    BigGemmSmemBytes<BM, BN, ST>()));
+    MI355X_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&BigGemmKernel<BM, BN, ST, U8, AW, true, true>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   BigGemmSmemBytes<BM, BN, ST>()));
     MI355X_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&BigGemmKernel<BM, BN, ST, U8, AW, false>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                    BigGemmSmemBytes<BM, BN, ST>()));
     return 0;
@@ -42,8 +44,10 @@ int Launch(IgemmArgs a, hipStream_t stream)
     xcd_rows = std::max(1, std::min(xcd_rows, a.tiles_m));
     const int grid = (nblocks + 7) / 8 * 8;
     constexpr int smem = BigGemmSmemBytes<BM, BN, ST>();
-    NoteKernel("BigGemmKernel<%d, %d, %d, %s, %s, %s>", BM, BN, ST, BoolName(U8), BoolName(AW), BoolName(a.unit != 0));
-    if (a.unit) hipLaunchKernelGGL((BigGemmKernel<BM, BN, ST, U8, AW, true>), dim3(grid), dim3(256), smem, stream, a, xcd_rows);
+    const bool tail = (a.Ci % 128) != 0;
+    NoteKernel("BigGemmKernel<%d, %d, %d, %s, %s, %s, %s>", BM, BN, ST, BoolName(U8), BoolName(AW), BoolName(a.unit != 0), BoolName(tail));
+    if (tail) hipLaunchKernelGGL((BigGemmKernel<BM, BN, ST, U8, AW, true, true>), dim3(grid), dim3(256), smem, stream, a, xcd_rows);
+    else if (a.unit) hipLaunchKernelGGL((BigGemmKernel<BM, BN, ST, U8, AW, true>), dim3(grid), dim3(256), smem, stream, a, xcd_rows);
     else hipLaunchKernelGGL((BigGemmKernel<BM, BN, ST, U8, AW, false>), dim3(grid), dim3(256), smem, stream, a, xcd_rows);
     MI355X_HIP(hipGetLastError());
     return 0;
@@ -71,7 +75,7 @@ int PrepareBigGemm()
 
 int LaunchBigGemm(IgemmArgs a, int bm, int bn, hipStream_t stream)
 {
-    if ((a.Ci % 128) != 0 || (a.K_pad % 128) != 0) return SetError(MI355X_ERR_INVALID_ARGUMENT, "large-tile GEMM needs channels %% 128 == 0");
+    if ((!a.unit && (a.Ci % 128) != 0) || (a.Ci % 16) != 0 || (a.K_pad % 128) != 0) return SetError(MI355X_ERR_INVALID_ARGUMENT, "large-tile GEMM needs channels %% 128 == 0");
     if (!a.unit && a.Kh * a.Kw > 32) return SetError(MI355X_ERR_UNSUPPORTED, "large-tile GEMM: filters of more than 32 taps are not supported");
     if (a.M <= 0) return 0;
     if (int rc = PrepareBigGemm()) return rc;

@@ -40,7 +40,8 @@ constexpr int BigGemmSmemBytes()
 // UNIT: 1x1 kernel, stride 1, no padding (and FullyConnected): a row's k-tiles are consecutive in memory, so a request's
 // address is a per-row constant plus a scalar.  Otherwise every row carries a bit mask of the filter taps that fall inside
 // the image for it (Kh * Kw <= 32), and a tap outside fetches 16 prepared padding bytes.
-template <int BM, int BN, int ST, bool U8, bool AW, bool UNIT>
+// TAIL (with UNIT): the channels are no multiple of 128 (but of 16): the last k-tile fetches prepared bytes beyond K.
+template <int BM, int BN, int ST, bool U8, bool AW, bool UNIT, bool TAIL = false>
 __global__ __launch_bounds__(256) void BigGemmKernel(IgemmArgs a, int xcd_rows)
 {
     static_assert(ST >= 2 && ST <= 4, "2 to 4 LDS stages");
@@ -126,9 +127,13 @@ __global__ __launch_bounds__(256) void BigGemmKernel(IgemmArgs a, int xcd_rows)
         if constexpr (UNIT)
         {
             const uint8_t* xk = a.x + kt * BK;
+            const bool in_even = !TAIL || lchunk_even * 16 < a.Ci - kt * BK, in_odd = !TAIL || lchunk_odd * 16 < a.Ci - kt * BK;
 #pragma unroll
             for (int j = 0; j < RA; ++j)
-                __builtin_amdgcn_global_load_lds((GlobalPtr)(xk + xoff[j]), (LdsPtr)(As + j * 8 * BK), 16, 0, 0);
+            {
+                const uint8_t* src = ((j & 1) ? in_odd : in_even) ? xk + xoff[j] : a.pad16;
+                __builtin_amdgcn_global_load_lds((GlobalPtr)(src), (LdsPtr)(As + j * 8 * BK), 16, 0, 0);
+            }
         }
         else
         {

@@ -145,6 +145,11 @@ int BuildPlan(const mi355x_conv2d_desc& d, const void* weights_host, const mi355
     p->halo_ok = !d.depthwise && (d.in_c == 64 || d.in_c == 128 || d.in_c == 256) && d.kernel_h * d.kernel_w > 1 && d.kernel_h <= 3 &&
                  d.kernel_w <= 3 && d.stride_x == 1 && d.stride_y == 1 && d.dilation_x == 1 && d.dilation_y == 1 && d.out_w <= 224;
     if (p->halo_ok) p->K_pad = (p->K + 127) / 128 * 128;
+    // 1x1 and FullyConnected over more than 128 channels, no multiple of 128 but of 16: rows still are whole lines but for the last,
+    // and the direct-to-LDS kernels take them with a last k-tile that ends early
+    p->k_tail = !d.depthwise && (d.in_c % 16) == 0 && d.in_c > 128 && (d.in_c % 128) != 0 && d.kernel_h == 1 && d.kernel_w == 1 && d.stride_x == 1 &&
+                d.stride_y == 1 && d.pad_top == 0 && d.pad_left == 0 && d.out_h == d.in_h && d.out_w == d.in_w;
+    if (p->k_tail) p->K_pad = (p->K + 127) / 128 * 128;
 
     // ---- per-channel requantization constants, in fp32 exactly as the reference's decoders produce them ----
     std::vector<float> mult(p->Co_pad, 0.0f), biasf(p->Co_pad, 0.0f);
@@ -670,8 +675,21 @@ int LaunchIgemmLdsT(const mi355x_conv2d_s* p, uint32_t batch, const void* x, voi
             static const hipError_t uattr = hipFuncSetAttribute(reinterpret_cast<const void*>(&IgemmLdsKernel<BM, BN, WM, WN, ST, U8, false, true>),
                                                                 hipFuncAttributeMaxDynamicSharedMemorySize, smem);
             MI355X_HIP(uattr);
-            NoteKernel("IgemmLdsKernel<%d, %d, %d, %d, %d, %s, false, true>", BM, BN, WM, WN, ST, BoolName(U8));
+            NoteKernel("IgemmLdsKernel<%d, %d, %d, %d, %d, %s, false, true, false>", BM, BN, WM, WN, ST, BoolName(U8));
             hipLaunchKernelGGL((IgemmLdsKernel<BM, BN, WM, WN, ST, U8, false, true>), dim3(grid), dim3(64 * WM * WN), smem, stream, a);
+            MI355X_HIP(hipGetLastError());
+            return 0;
+        }
+    }
+    if constexpr (BM <= 128)
+    {
+        if (p->k_tail)
+        {
+            static const hipError_t tattr = hipFuncSetAttribute(reinterpret_cast<const void*>(&IgemmLdsKernel<BM, BN, WM, WN, ST, U8, AW, false, true>),
+                                                                hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+            MI355X_HIP(tattr);
+            NoteKernel("IgemmLdsKernel<%d, %d, %d, %d, %d, %s, %s, false, true>", BM, BN, WM, WN, ST, BoolName(U8), BoolName(AW));
+            hipLaunchKernelGGL((IgemmLdsKernel<BM, BN, WM, WN, ST, U8, AW, false, true>), dim3(grid), dim3(64 * WM * WN), smem, stream, a);
             MI355X_HIP(hipGetLastError());
             return 0;
         }
@@ -679,7 +697,7 @@ int LaunchIgemmLdsT(const mi355x_conv2d_s* p, uint32_t batch, const void* x, voi
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&IgemmLdsKernel<BM, BN, WM, WN, ST, U8, AW>),
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, smem);
     MI355X_HIP(attr);
-    NoteKernel("IgemmLdsKernel<%d, %d, %d, %d, %d, %s, %s, false>", BM, BN, WM, WN, ST, BoolName(U8), BoolName(AW));
+    NoteKernel("IgemmLdsKernel<%d, %d, %d, %d, %d, %s, %s, false, false>", BM, BN, WM, WN, ST, BoolName(U8), BoolName(AW));
     hipLaunchKernelGGL((IgemmLdsKernel<BM, BN, WM, WN, ST, U8, AW>), dim3(grid), dim3(64 * WM * WN), smem, stream, a);
     MI355X_HIP(hipGetLastError());
     return 0;
@@ -1117,25 +1135,30 @@ int RunPlan(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, hi
                        : big < 400 ? 64 : (huge >= 192 && g.Co >= 256) ? 512 : 128;
         // channel counts that are multiples of 128: k-tiles go from global memory straight into LDS
         const int lds_stages = p->opt_igemm_lds;
-        if (lds_stages != 0 && bk128 && (g.Ci % 128) == 0)
+        if (lds_stages != 0 && ((bk128 && (g.Ci % 128) == 0) || (p->k_tail && p->tile_override == 0)))
         {
             // Launches that fill the device with 256-row tiles: one wave per SIMD with a 128 x 128 (or 128 x 64) wave tile.
             // A CU's L1 delivers 30 to 45 bytes per clock from L2; only these tiles ask for less than that per MFMA clock.
             if (p->tile_override == 0 || p->tile_override >= 1000)
             {
                 const long long rows256 = (M + 255) / 256;
+                // (Where K ends inside a k-tile they have to fill the last round of CUs as well, and K has to be long: 2537 x 1712 ->
+                // 3548, 280 tiles, 43 us against 34 on 128 x 128 tiles, 6826 x 400 -> 2137 26 against 24.)
+                const auto fills = [&](long long blocks) {
+                    return blocks >= 224 && (!p->k_tail || (p->K >= 1024 && blocks * 100 >= (blocks + 255) / 256 * 256 * 85));
+                };
                 int bm = 0, bn = 0;
                 if (p->tile_override == 2256) { bm = 256; bn = 256; }
                 else if (p->tile_override == 2128) { bm = 256; bn = 128; }
                 else if (p->tile_override == 1256) { bm = 128; bn = 256; }
-                else if ((p->Co_pad % 256) == 0 && rows256 * (p->Co_pad / 256) >= 224) { bm = 256; bn = 256; }
-                else if (rows256 * (p->Co_pad / 128) >= 224) { bm = 256; bn = 128; }
+                else if ((p->Co_pad % 256) == 0 && fills(rows256 * (p->Co_pad / 256))) { bm = 256; bn = 256; }
+                else if (fills(rows256 * (p->Co_pad / 128))) { bm = 256; bn = 128; }
                 // the large-tile kernel walks a filter's taps through a 32-bit mask per row: filters of more than 32 taps
                 // (6 x 6, 7 x 7 ...) stay on the tiles below, also when a test forces the large tile
                 if (bm != 0 && (unit || g.Kh * g.Kw <= 32)) return LaunchBig(p, bm, bn, batch, x, y, stream);
             }
             if ((tile == 4064 || tile == 2064) && p->zw_neg == 0) return LaunchIgemmKSplit(p, tile == 4064 ? 4 : 2, batch, x, y, stream);
-            if (tile == 64 && p->tile_override == 0 && p->zw_neg == 0 && p->K_pad >= 16 * 128)
+            if (tile == 64 && p->tile_override == 0 && p->zw_neg == 0 && p->K_pad >= 16 * 128 && !p->k_tail)
             {
                 // At most one block per CU and a long K: a SIMD would hold one wave and the k-loop run at that wave's issue
                 // rate.  K split over groups of waves inside the block: 17.4 -> 13.5 us for 7 x 7 x 512 -> 512, 3 x 3, 16 images.
@@ -1145,6 +1168,9 @@ int RunPlan(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, hi
                 // 64 x 64 blocks of 256 threads co-run better: ResNet-50 b32 in two lanes, 6.3 us per step for five layers)
                 if (blocks64 <= 256 && !shared_device) return LaunchIgemmKSplit(p, 2, batch, x, y, stream);
             }
+            // 128 x 128 tiles over a long K with such an end: the register-staged kernel is as fast, and faster from 1024 on (2080: 47 us
+            // against 51 for 5040 rows -> 2112; 400: 26 against 23 for 6826 -> 2137)
+            if (p->k_tail && tile != 64 && p->K >= 1024) return LaunchIgemm(p, tile, batch, x, y, stream);
             if (tile == 64)
             {
                 // at most one block per CU: nothing else hides a k-tile's round trip, so keep two tiles on their way
@@ -1153,7 +1179,7 @@ int RunPlan(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, hi
             }
             if (g.Co <= 64 || tile == 96) return LaunchIgemmLds<128, 64, 2, 2>(p, lds_stages, batch, x, y, stream);
             if (tile == 256) return LaunchIgemmLds<256, 128, 4, 2>(p, lds_stages, batch, x, y, stream);
-            if (tile == 512) return LaunchIgemmLds<256, 256, 4, 4>(p, lds_stages, batch, x, y, stream);
+            if (tile == 512 && !p->k_tail) return LaunchIgemmLds<256, 256, 4, 4>(p, lds_stages, batch, x, y, stream);
             return LaunchIgemmLds<128, 128, 2, 2>(p, lds_stages, batch, x, y, stream);
         }
         return LaunchIgemm(p, tile, batch, x, y, stream);

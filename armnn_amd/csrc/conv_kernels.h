@@ -242,6 +242,7 @@ struct IgemmArgs
     uint32_t pad_word;      // shifted input zero point replicated in 4 bytes
     int zw_neg;             // minus the zero point of the stored int8 weights (0: symmetric)
     int rowsum_bias;        // (K_pad - K) * zx': what the bytes beyond K add to a row sum
+    int k_tiles = 0;        // IgemmKernel: k-tiles to walk where they are fewer than K_pad holds
     int vec_out = 0;        // IgemmKernel: output rows are whole, aligned 16-byte pieces
     Requant rq;
     const uint8_t* res = nullptr;   // direct-to-LDS kernel: the other input of an Addition fused into the write-out ([M][Co]), or null
@@ -440,7 +441,7 @@ __global__ __launch_bounds__(256) void IgemmKernel(IgemmArgs a)
         for (int tp = 0; tp < TP; ++tp) acc[tc][tp] = init;
     }
 
-    const int nk = a.K_pad / BK;
+    const int nk = a.k_tiles != 0 ? a.k_tiles : a.K_pad / BK;
     const int frag_row = lane & 31;
     const int frag_k = (lane >> 5) * 16;
     using std::integral_constant;

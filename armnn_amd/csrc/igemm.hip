@@ -44,6 +44,12 @@ int LaunchIgemmT(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* 
     a.pad_word = p->pad_word;
     a.zw_neg = p->zw_neg;
     a.rowsum_bias = p->rowsum_bias;
+    if (p->k_tail)
+    {
+        // K_pad is a multiple of 128 for the kernels with such k-tiles; here it need not be
+        a.k_tiles = (p->K + BK - 1) / BK;
+        a.rowsum_bias = (a.k_tiles * BK - p->K) * static_cast<int>(static_cast<int8_t>(p->pad_word & 0xffu));
+    }
     a.rq = p->rq;
     const int nblocks = a.tiles_m * a.tiles_n;
     const int grid = (nblocks + 7) / 8 * 8;

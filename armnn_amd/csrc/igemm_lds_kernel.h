@@ -54,7 +54,8 @@ struct NoTileHook
     __device__ __forceinline__ void operator()() const {}
 };
 
-template <int BM, int BN, int WM, int WN, int ST, bool U8, bool AW = false, bool UNIT = false, typename Hook = NoTileHook>
+// TAIL: 1x1 or FullyConnected whose channels are no multiple of 128 (but of 16): the last k-tile fetches prepared bytes beyond K.
+template <int BM, int BN, int WM, int WN, int ST, bool U8, bool AW = false, bool UNIT = false, typename Hook = NoTileHook, bool TAIL = false>
 __device__ __forceinline__ void IgemmLdsTile(const IgemmArgs& a, const int tile, uint8_t* const smem, Hook after_loads = Hook())
 {
     static_assert(ST >= 2 && ST <= 8, "2 to 8 LDS stages");
@@ -155,7 +156,8 @@ __device__ __forceinline__ void IgemmLdsTile(const IgemmArgs& a, const int tile,
         {
             const int iy = iy0[j] + dy;
             const int ix = ix0[j] + dx;
-            const bool ok = mvalid[j] && static_cast<unsigned>(iy) < static_cast<unsigned>(a.H) && static_cast<unsigned>(ix) < static_cast<unsigned>(a.W);
+            bool ok = mvalid[j] && static_cast<unsigned>(iy) < static_cast<unsigned>(a.H) && static_cast<unsigned>(ix) < static_cast<unsigned>(a.W);
+            if constexpr (TAIL) ok = ok && ci + ((j & 1) ? lchunk_odd : lchunk_even) * 16 < a.Ci;
             // padding and rows past the end fetch 16 prepared bytes instead: every lane always delivers its slot
             const uint8_t* src = ok ? xrow[j] + tap_off : a.pad16;
             __builtin_amdgcn_global_load_lds((GlobalPtr)(src), (LdsPtr)(As + j * 8 * BK), 16, 0, 0);
@@ -394,7 +396,7 @@ __host__ __device__ inline int IgemmLdsBlocksPerXcd(int tiles_m, int tiles_n, in
     return (tiles_m * tiles_n + 7) / 8;
 }
 
-template <int BM, int BN, int WM, int WN, int ST, bool U8, bool AW = false, bool UNIT = false>
+template <int BM, int BN, int WM, int WN, int ST, bool U8, bool AW = false, bool UNIT = false, bool TAIL = false>
 __global__ __launch_bounds__(64 * WM * WN) void IgemmLdsKernel(IgemmArgs a)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];   // IgemmLdsSmemBytes<BM, BN, ST>()
@@ -414,7 +416,7 @@ __global__ __launch_bounds__(64 * WM * WN) void IgemmLdsKernel(IgemmArgs a)
         tile = x * per_xcd + i;
         if (i >= per_xcd || tile >= nblocks) return;
     }
-    IgemmLdsTile<BM, BN, WM, WN, ST, U8, AW, UNIT>(a, tile, smem);
+    IgemmLdsTile<BM, BN, WM, WN, ST, U8, AW, UNIT, NoTileHook, TAIL>(a, tile, smem);
 }
 
 } // namespace mi355x

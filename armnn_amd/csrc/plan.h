@@ -41,6 +41,7 @@ struct mi355x_conv2d_s
     std::vector<double> fast_cw;           // bracket (negative: no fast path), kept until the table is uploaded
     int pw_bn = 0, pw_ks = 0;      // pointwise GEMM kernel configuration (0: not applicable)
     bool bk128 = false;            // implicit GEMM walks K in 128-byte tiles
+    bool k_tail = false;           // 1x1 plan whose K ends inside a 128-byte k-tile, zero padded to whole ones
     bool halo_ok = false;          // shape fits the resident-tile kernel (weights without a zero point are checked at launch)
     unsigned concurrency = 1;      // launches of the plan's network that run side by side (mi355x_conv2d_set_concurrency)
     int tile_override = 0;         // 0: choose the MFMA tile per launch; 64 / 96 (= 128x64) / 128: the "igemm_tile" option at plan creation
