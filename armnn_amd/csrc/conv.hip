@@ -378,19 +378,13 @@ int BuildPlan(const mi355x_conv2d_desc& d, const void* weights_host, const mi355
             }
             if (int rc = Upload(reinterpret_cast<void**>(&p->dw_grp), grp.data(), grp.size() * sizeof(uint32_t))) return rc;
             // blocks of 64 channels: rows of [16][4] dwords, entry [j][e] for channel 16 e + j of the block: corr, m+, b+, m-, b-,
-            // filter taps 0..3, 4..7, 8, and those of the second halves.  Channels past the last one have the code 0 in int8.
+            // filter taps 0..3, 4..7, 8, and those of the second halves.  Channels past the last one are all zero: a bracket that
+            // closes, some code that no weight and no row sum counts.
             const int rows = 11;
-            const float past = 128.0f;
             std::vector<uint32_t> blk(static_cast<size_t>((Co + 63) / 64) * rows * 64, 0u);
-            for (int c = 0; c < (Co + 63) / 64 * 64; ++c)
+            for (int c = 0; c < Co; ++c)
             {
                 uint32_t* bdst = blk.data() + static_cast<size_t>(c / 64) * rows * 64 + (c % 16) * 4 + c % 64 / 16;
-                if (c >= Co)
-                {
-                    std::memcpy(&bdst[2 * 64], &past, 4);
-                    std::memcpy(&bdst[4 * 64], &past, 4);
-                    continue;
-                }
                 bdst[0] = static_cast<uint32_t>(corr[c]);
                 for (int r = 0; r < 4; ++r) std::memcpy(&bdst[(1 + r) * 64], &p->chan_host[static_cast<size_t>(2 + r) * CP + c], 4);
                 for (int t = 0; t < 9; ++t)

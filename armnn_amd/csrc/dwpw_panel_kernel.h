@@ -317,6 +317,10 @@ __global__ __launch_bounds__(64 * NW, 4) void DwPwPanelKernel(DwPwPanelArgs a)
         for (int c = 0; c < CG; ++c) acc[c][p] = v4i{0, 0, 0, 0};
     }
     const uint8_t* const pb = panel_lds + g * GP + j * 16;
+    // The sum of a pixel's codes is over the channels that exist.  Those that complete the last block of 64 hold whatever the
+    // activation between the layers makes of them (their weights are zero, so the products do not mind); they are the high bytes
+    // of each dword of the last k-step.
+    const int last_ones = static_cast<int>(0x01010101u >> (8 * (-ng & 3)));
     for (int k0 = 0; k0 < steps; k0 += RD)
     {
 #pragma unroll
@@ -333,10 +337,11 @@ __global__ __launch_bounds__(64 * NW, 4) void DwPwPanelKernel(DwPwPanelArgs a)
                 for (int p = 0; p < PG; ++p) acc[c][p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wv[r][c], xb[p], acc[c][p], 0, 0, 0);
             if constexpr (U)
             {
+                const int ones = ks == steps - 1 ? last_ones : 0x01010101;
 #pragma unroll
                 for (int p = 0; p < PG; ++p)
 #pragma unroll
-                    for (int d = 0; d < 4; ++d) xs[p] = __builtin_amdgcn_sdot4(xb[p][d], 0x01010101, xs[p], false);
+                    for (int d = 0; d < 4; ++d) xs[p] = __builtin_amdgcn_sdot4(xb[p][d], ones, xs[p], false);
             }
             if (ks + RD < steps) load_weights(ks + RD, r);
         }

@@ -4,8 +4,9 @@ import numpy as np
 import pytest
 
 from armnn_amd import shim
-from armnn_amd.tensor import numpy_dtype
+from armnn_amd.tensor import QTensor, numpy_dtype
 from tests import cases
+from tests.helpers import lsb_diff
 
 pytestmark = pytest.mark.gpu
 U8, S8 = cases.U8, cases.S8
@@ -65,3 +66,53 @@ def test_pair_equals_the_layers_run_apart(n, h, w, c, co, s, tile, general):
     got, want = (b.download(pw.out_info.shape, numpy_dtype(dt)) for b in (one, apart))
     assert len(np.unique(want)) > 8
     np.testing.assert_array_equal(got, want)
+
+
+# n, h, w, channels, output channels, stride, and the layer between's type, scale, zero point and activation, whose lowest or highest code
+# lies inside the type: the last block of 64 channels is no whole one in any of them
+CLAMPED = [
+    (1, 7, 9, 16, 32, 1, U8, 0.1, 0, cases.RELU6),
+    (1, 9, 6, 48, 80, 2, S8, 0.05, 20, cases.RELU),
+    (8, 20, 22, 176, 192, 1, U8, 0.05, 140, cases.RELU),
+    (5, 28, 28, 208, 256, 1, S8, 0.1, -100, cases.RELU6),
+    (14, 14, 14, 464, 512, 1, U8, 0.1, 0, cases.RELU6),
+    (4, 60, 50, 32, 48, 1, S8, 0.05, 20, cases.RELU),
+    (9, 65, 70, 48, 96, 2, U8, 0.05, 140, cases.RELU),
+    (8, 60, 61, 112, 192, 2, S8, 0.05, 20, cases.RELU),
+]
+
+
+@pytest.mark.parametrize("n,h,w,c,co,s,dt,scale,zp,act", CLAMPED, ids=[f"{p[0]}x{p[1]}x{p[2]}x{p[3]}_{p[4]}_s{p[5]}" for p in CLAMPED])
+def test_channels_that_do_not_exist_count_for_nothing_under_a_clamp(port, n, h, w, c, co, s, dt, scale, zp, act):
+    """Weights with a zero point need the sum of a pixel's codes: those past the last channel must not be in it, whatever code
+    the activation between the layers turns them into."""
+    wq = dict(w_dtype=U8, w_offset=101, per_axis=False)
+    dw = cases.make_conv_case("dw", 63000 + c + h, n=n, h=h, w=w, ci=c, depthwise=True, stride=(s, s), in_dtype=dt, in_scale=0.0235,
+                              in_offset=120 if dt == U8 else -8, out_scale=scale, out_offset=zp, act=act, w_scale_range=(0.01, 0.02), **wq)
+    ho, wo = dw.out_info.shape[1:3]
+    pw = cases.make_conv_case("pw", 64000 + co + h, n=n, h=ho, w=wo, ci=c, co=co, kh=1, kw=1, in_dtype=dt, in_scale=scale, in_offset=zp,
+                              out_scale=0.3, out_offset=100 if dt == U8 else -20, **wq)
+    dev = shim.Device()
+
+    def plan(case):
+        return shim.Conv2dPlan(case.x.info, case.w, case.b, case.out_info, activation=case.act[0], act_a=case.act[1], act_b=case.act[2], **case.params)
+    first, second = plan(dw), plan(pw)
+    assert first.fusable_with(second), shim.load_library().mi355x_last_error().decode()
+    x = shim.DeviceBuffer(dw.x.data.nbytes).upload(dw.x.data)
+    mid = shim.DeviceBuffer(dw.out_info.num_elements)
+    apart, one = shim.DeviceBuffer(pw.out_info.num_elements), shim.DeviceBuffer(pw.out_info.num_elements)
+    first.run_fused(second, n, x.ptr, one.ptr)
+    kernel = shim.last_kernel()
+    print(kernel, flush=True)
+    assert kernel.startswith(f"DwPwPanelKernel<{s}, ") and kernel.endswith("true>"), kernel
+    first.run(n, x.ptr, mid.ptr)
+    second.run(n, mid.ptr, apart.ptr)
+    dev.synchronize()
+    got, want = (b.download(pw.out_info.shape, numpy_dtype(dt)) for b in (one, apart))
+    assert len(np.unique(want)) > 8
+    np.testing.assert_array_equal(got, want)
+    if n == 1:
+        between = port.activation(port.conv2d(dw.x, dw.w, dw.b, dw.out_info, **dw.params), dw.out_info, *dw.act)
+        ref = port.conv2d(QTensor(pw.x.info, between.data), pw.w, pw.b, pw.out_info, **pw.params)
+        mx, exact = lsb_diff(got, ref.data)
+        assert mx <= 1 and exact >= 0.99, (mx, exact)
