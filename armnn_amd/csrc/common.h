@@ -125,7 +125,7 @@ Options& GlobalOptions();
 // legacy default stream: that one may not be touched while any thread captures a graph.
 int UploadNow(void* dst_dev, const void* src_host, size_t bytes);
 
-// Keeps the calling thread's upload stream across several UploadNow calls; at the end it waits for the next plan, until
+// Keeps the calling thread's upload stream across several UploadNow calls; at the end it waits for the next plan on its device, until
 // mi355x_stream_create destroys it.  A stream that stayed would hold one of the process's four hardware queues for good:
 // the third network loaded then shared a queue with another one and ran behind it instead of beside it (three MobileNetV1
 // at one image each, replayed in turn: 99 us per pass with a stream kept per thread, 53 us without; ResNet-50 279 and

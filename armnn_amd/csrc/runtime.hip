@@ -1,10 +1,9 @@
 // Device runtime part of the C ABI: device selection, memory, streams, events, graphs.
 #include "common.h"
+#include "idle_stream.h"
 
 #include <algorithm>
 #include <cmath>
-#include <mutex>
-#include <utility>
 
 namespace mi355x
 {
@@ -32,20 +31,13 @@ KernelNote& CurrentKernelNote()
 
 namespace
 {
-// The calling thread's upload stream: there is one while an UploadScope is open.
+// The calling thread's upload stream and the device it belongs to: there is one while an UploadScope is open.
 thread_local hipStream_t t_upload_stream = nullptr;
+thread_local int t_upload_device = 0;
 thread_local int t_upload_scopes = 0;
 
-// At most one upload stream waits here for the next plan.
-std::mutex g_idle_upload_mutex;
-hipStream_t g_idle_upload_stream = nullptr;
-
-hipStream_t SwapIdleUploadStream(hipStream_t s)
-{
-    std::lock_guard<std::mutex> lock(g_idle_upload_mutex);
-    std::swap(s, g_idle_upload_stream);
-    return s;
-}
+// At most one upload stream waits here for the next plan of its device.
+IdleStream<hipStream_t> g_idle_upload_stream;
 } // namespace
 
 UploadScope::UploadScope() { ++t_upload_scopes; }
@@ -53,13 +45,17 @@ UploadScope::UploadScope() { ++t_upload_scopes; }
 UploadScope::~UploadScope()
 {
     if (--t_upload_scopes > 0 || !t_upload_stream) return;
-    if (const hipStream_t other = SwapIdleUploadStream(t_upload_stream)) (void)hipStreamDestroy(other);
+    if (const hipStream_t other = g_idle_upload_stream.Put(t_upload_device, t_upload_stream)) (void)hipStreamDestroy(other);
     t_upload_stream = nullptr;
 }
 
 int UploadStream(hipStream_t* stream)
 {
-    if (!t_upload_stream) t_upload_stream = SwapIdleUploadStream(nullptr);
+    if (!t_upload_stream)
+    {
+        MI355X_HIP(hipGetDevice(&t_upload_device));
+        t_upload_stream = g_idle_upload_stream.Take(t_upload_device);
+    }
     if (!t_upload_stream) MI355X_HIP(hipStreamCreateWithFlags(&t_upload_stream, hipStreamNonBlocking));
     *stream = t_upload_stream;
     return 0;
@@ -427,7 +423,7 @@ int mi355x_stream_create(mi355x_stream_t* stream)
 {
     if (!stream) return SetError(MI355X_ERR_INVALID_ARGUMENT, "stream is null");
     // the new stream, not a waiting upload stream, gets the hardware queue (UploadScope)
-    if (const hipStream_t idle = SwapIdleUploadStream(nullptr)) (void)hipStreamDestroy(idle);
+    if (const hipStream_t idle = g_idle_upload_stream.TakeAny()) (void)hipStreamDestroy(idle);
     hipStream_t s;
     MI355X_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));   // default priority
     *stream = reinterpret_cast<mi355x_stream_t>(s);
