@@ -3,9 +3,10 @@ the whole forward pass launched kernel by kernel or captured into a HIP graph an
 (DeviceNetwork.choose_submission measures which is faster for the network and batch at hand)."""
 from __future__ import annotations
 
+import collections
 import ctypes as C
+import itertools
 import os
-import threading
 import weakref
 from dataclasses import dataclass
 from typing import Dict, List, Optional, Tuple
@@ -80,6 +81,30 @@ class FusedTail:
         return self.parts[1].macs_per_image
 
 
+class _OpenNetworks:
+    """The open networks of the process, held weakly.  There is no lock in what networks share: any allocation may run the garbage
+    collector and with it a __del__ that closes a network, on the thread that is in here, and a lock would make that thread wait for
+    itself.  Each operation is one call on a dict with whole numbers as keys, which nothing interrupts."""
+
+    def __init__(self):
+        self._refs: Dict[int, weakref.ref] = {}
+        self._keys = itertools.count()
+
+    def add(self, network: "DeviceNetwork") -> int:
+        key, refs = next(self._keys), self._refs
+        refs[key] = weakref.ref(network, lambda _: refs.pop(key, None))
+        return key
+
+    def remove(self, key: int):
+        self._refs.pop(key, None)
+
+    def __len__(self):
+        return len(self._refs)
+
+    def __iter__(self):
+        return iter([n for n in (ref() for ref in list(self._refs.values())) if n is not None])
+
+
 class DeviceNetwork:
     def __init__(self, net: Network, batch: int, algo_overrides: Optional[Dict[str, int]] = None, use_graph: bool = True,
                  fuse: bool = False, lanes: int = 1, fuse_add: bool = True, chain: bool = False, lanes_after_chain: bool = False,
@@ -103,8 +128,7 @@ class DeviceNetwork:
         self.lib = shim.load_library()
         self.stream = self.dev.stream()
         self._side_streams: Optional[List] = None
-        with self._blocks_lock:
-            self._open.add(self)
+        self._register()
         self.buffers: Dict[str, shim.DeviceBuffer] = {}
         self.steps: List = []          # (layer, callable(stream))
         self._step_plans: List = []    # plan of each step (None for plan-less layers), parallel to self.steps
@@ -192,6 +216,10 @@ class DeviceNetwork:
             self._fuse_tail()
         if fuse_pool or (fuse_pool is None and fuse == "auto"):
             self._fuse_conv_pool(only_where_it_pays=not fuse_pool)
+
+    def _register(self):
+        self._has_run = False
+        self._key = self._open.add(self)
 
     def _fuse_conv_pool(self, only_where_it_pays):
         """A 1x1 convolution whose output only feeds the pooling launched right behind it, where the library runs the two
@@ -479,9 +507,8 @@ class DeviceNetwork:
         self._sync_next += 1
         return ev
 
-    # The networks of the process that have run, and how many hardware queues the streams of a process share.
-    _running_lock = threading.Lock()
-    _running: "weakref.WeakSet[DeviceNetwork]" = weakref.WeakSet()
+    # The networks of the process, and how many hardware queues the streams of a process share.
+    _open = _OpenNetworks()
     _hardware_queues = int(os.environ.get("GPU_MAX_HW_QUEUES", "4"))
 
     def _one_lane_now(self) -> bool:
@@ -489,9 +516,8 @@ class DeviceNetwork:
         and a lane waits behind another network's, or behind its own sibling (three of ResNet-50 side by side, 32 images in
         two lanes each, 605 us a pass; as one lane each 525; one alone 720 in its lanes, 870 as one, 1130 with the two on one
         queue)."""
-        with self._running_lock:
-            self._running.add(self)
-            lanes = sum(n.lanes for n in self._running)
+        self._has_run = True
+        lanes = sum(n.lanes for n in self._open if n._has_run)
         return lanes > max(self._hardware_queues, self.lanes) and not self.chains and not self.tails
 
     def _capture(self, one_lane: bool):
@@ -574,28 +600,30 @@ class DeviceNetwork:
     # Pinned memory that host arrays pass through: blocks shared by the networks of the process, at most this many kept while no
     # call uses them, and none once the last network is closed.
     _BLOCK_BYTES, _BLOCKS_KEPT = 2 << 20, 32
-    _blocks_lock = threading.Lock()
-    _blocks: List[int] = []
-    _open: "weakref.WeakSet[DeviceNetwork]" = weakref.WeakSet()
+    _blocks: "collections.deque[int]" = collections.deque()      # (append and pop are one call each: see _OpenNetworks)
 
     def _take_blocks(self, n: int) -> List[int]:
-        with self._blocks_lock:
-            taken, self._blocks[:] = self._blocks[:n], self._blocks[n:]
-        while len(taken) < n:
-            p = C.c_void_p()
-            rc = self.lib.mi355x_host_alloc(C.byref(p), self._BLOCK_BYTES)
-            if rc != 0:
-                self._give_blocks(taken)
-                shim._chk(rc)
-            taken.append(p.value)
+        taken = []
+        try:
+            while len(taken) < n:
+                try:
+                    taken.append(self._blocks.pop())
+                except IndexError:
+                    p = C.c_void_p()
+                    shim._chk(self.lib.mi355x_host_alloc(C.byref(p), self._BLOCK_BYTES))
+                    taken.append(p.value)
+        except BaseException:
+            self._give_blocks(taken)
+            raise
         return taken
 
     def _give_blocks(self, blocks: List[int]):
-        with self._blocks_lock:
-            self._blocks.extend(blocks)
-            keep = self._BLOCKS_KEPT if len(self._open) > 0 else 0
-            extra, self._blocks[:] = self._blocks[keep:], self._blocks[:keep]
-        for p in extra:
+        self._blocks.extend(blocks)
+        while len(self._blocks) > (self._BLOCKS_KEPT if len(self._open) > 0 else 0):
+            try:
+                p = self._blocks.pop()
+            except IndexError:                                 # another thread took it
+                break
             shim._chk(self.lib.mi355x_host_free(p))
 
     def run(self, x: QTensor) -> QTensor:
@@ -663,10 +691,7 @@ class DeviceNetwork:
         self.tails = []
         for p in self.plans:
             p.destroy()
-        with self._running_lock:
-            self._running.discard(self)
-        with self._blocks_lock:
-            self._open.discard(self)
+        self._open.remove(self._key)
         self._give_blocks([])
         for b in set(self.buffers.values()):
             b.free()
