@@ -597,9 +597,10 @@ class DeviceNetwork:
         self.synchronize()
         return QTensor(info, self.buffers[name].download(info.shape, numpy_dtype(info.dtype), self.stream))
 
-    # Pinned memory that host arrays pass through: blocks shared by the networks of the process, at most this many kept while no
-    # call uses them, and none once the last network is closed.
-    _BLOCK_BYTES, _BLOCKS_KEPT = 2 << 20, 32
+    # Pinned memory that host arrays pass through: blocks shared by the networks of the process.  Freeing one waits for the device, so
+    # all that calls have used side by side are kept: at most what one call of each open network takes (_MOST_PARTS and the
+    # results), fewer where calls follow each other, and none once the last network is closed.
+    _BLOCK_BYTES, _MOST_PARTS = 2 << 20, 32
     _blocks: "collections.deque[int]" = collections.deque()      # (append and pop are one call each: see _OpenNetworks)
 
     def _take_blocks(self, n: int) -> List[int]:
@@ -619,7 +620,7 @@ class DeviceNetwork:
 
     def _give_blocks(self, blocks: List[int]):
         self._blocks.extend(blocks)
-        while len(self._blocks) > (self._BLOCKS_KEPT if len(self._open) > 0 else 0):
+        while len(self._blocks) > (self._MOST_PARTS + 1) * len(self._open):
             try:
                 p = self._blocks.pop()
             except IndexError:                                 # another thread took it
@@ -637,7 +638,7 @@ class DeviceNetwork:
         dst = np.empty(info.shape, dtype=numpy_dtype(info.dtype))
         part = min(max(src.nbytes // 4 + 0xffff & ~0xffff, 512 << 10), self._BLOCK_BYTES)
         parts = -(-src.nbytes // part)
-        if parts > self._BLOCKS_KEPT or dst.nbytes > self._BLOCK_BYTES:
+        if parts > self._MOST_PARTS or dst.nbytes > self._BLOCK_BYTES:
             self.upload_input(x)
             self.enqueue()
             return self.download()

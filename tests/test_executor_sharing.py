@@ -84,3 +84,22 @@ def test_close_from_a_garbage_collection_inside_the_sharing_code():
     gc.collect()
     keeper.close()
     assert not lib.live                                    # nothing is kept once the last network is closed
+
+
+def test_repeated_calls_allocate_no_pinned_memory():
+    """The largest call takes a block for each of its parts and one for the results; two networks may be in a call at once."""
+    lib = FakeLibrary()
+    a, b = bare_network(lib), bare_network(lib)
+    for _ in range(3):
+        a._give_blocks(a._take_blocks(DeviceNetwork._MOST_PARTS + 1))
+        assert (lib.allocated, lib.freed) == (33, 0)
+    for _ in range(3):
+        first, second = a._take_blocks(20), b._take_blocks(20)
+        assert not set(first) & set(second)
+        a._give_blocks(first)
+        b._give_blocks(second)
+        assert (lib.allocated, lib.freed) == (40, 0)
+    b.close()
+    assert len(lib.live) == 33                             # what one network's call takes
+    a.close()
+    assert not lib.live
