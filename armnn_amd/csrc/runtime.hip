@@ -383,6 +383,20 @@ static __global__ __launch_bounds__(256) void PinnedCopyKernel(const int4* __res
         reinterpret_cast<uint8_t*>(dst + pieces)[threadIdx.x] = reinterpret_cast<const uint8_t*>(src + pieces)[threadIdx.x];
 }
 
+// Whether `bytes` from `p` on lie inside one allocation that the runtime knows.
+static bool WithinAllocation(const void* p, size_t bytes)
+{
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    if (hipMemGetAddressRange(&base, &size, const_cast<void*>(p)) != hipSuccess)
+    {
+        (void)hipGetLastError();
+        return false;
+    }
+    const uintptr_t at = reinterpret_cast<uintptr_t>(p), from = reinterpret_cast<uintptr_t>(base);
+    return at >= from && at - from <= size && bytes <= size - (at - from);
+}
+
 static int CopyAsync(void* dst, const void* src, const void* host, size_t bytes, hipMemcpyKind kind, mi355x_stream_t stream)
 {
     constexpr size_t kMostByKernel = 4u << 20;
@@ -391,10 +405,11 @@ static int CopyAsync(void* dst, const void* src, const void* host, size_t bytes,
     void* device_alias = nullptr;
     int is_device = 0;
     if (int rc = mi355x_host_device_pointer(host, &device_alias, &is_device)) return rc;
-    if (bytes <= kMostByKernel && ((reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(device_alias)) & 15) == 0)
+    const void* from = kind == hipMemcpyHostToDevice ? device_alias : src;
+    void* to = kind == hipMemcpyHostToDevice ? dst : device_alias;
+    // The kernel takes what is aligned for it and certain to be there; everything else is the runtime's to check and to move.
+    if (bytes <= kMostByKernel && ((reinterpret_cast<uintptr_t>(from) | reinterpret_cast<uintptr_t>(to)) & 15) == 0 && WithinAllocation(from, bytes) && WithinAllocation(to, bytes))
     {
-        const void* from = kind == hipMemcpyHostToDevice ? device_alias : src;
-        void* to = kind == hipMemcpyHostToDevice ? dst : device_alias;
         const unsigned pieces = static_cast<unsigned>(bytes / 16), blocks = std::min(64u, pieces / 256 + 1);
         hipLaunchKernelGGL(PinnedCopyKernel, dim3(blocks), dim3(256), 0, ToHip(stream), static_cast<const int4*>(from), static_cast<int4*>(to), pieces, static_cast<unsigned>(bytes & 15));
         MI355X_HIP(hipGetLastError());

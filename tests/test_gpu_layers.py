@@ -247,6 +247,38 @@ def test_async_copies_need_memory_the_device_reaches_and_keep_stream_order():
     dev.stream_destroy(stream)
 
 
+@pytest.mark.parametrize("shift", [0, 16, 5])
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 4095, 4096 + 3, (1 << 20) + 8, (4 << 20) - 1, 4 << 20, (4 << 20) + 19])
+def test_pinned_transfers_move_these_bytes_and_no_others(n, shift):
+    """Transfers of up to 4 MiB at addresses that are multiples of 16 are a kernel's (whole pieces of 16 bytes and a rest), all others
+    the copy engine's; up to the last byte of both allocations."""
+    import ctypes as C
+    lib = shim.load_library()
+    dev = shim.Device()
+    stream = dev.stream()
+    before, total = 64, 64 + shift + n
+    p, q = C.c_void_p(), C.c_void_p()
+    shim._chk(lib.mi355x_host_alloc(C.byref(p), total))
+    shim._chk(lib.mi355x_host_alloc(C.byref(q), total))
+    up, down = (np.frombuffer((C.c_uint8 * total).from_address(v.value), dtype=np.uint8) for v in (p, q))
+    up[:] = np.random.default_rng(n + shift).integers(0, 256, total, dtype=np.uint8)
+    down[:] = 0xa5
+    buf = shim.DeviceBuffer(total)
+    shim._chk(lib.mi355x_fill_u8(buf.ptr, 0x5a, total, stream))
+    o = before + shift
+    shim._chk(lib.mi355x_memcpy_h2d_async(buf.ptr + o, p.value + o, n, stream))
+    shim._chk(lib.mi355x_memcpy_d2h_async(q.value + o, buf.ptr + o, n, stream))
+    dev.stream_sync(stream)
+    on_device = buf.download((total,), np.uint8)
+    np.testing.assert_array_equal(on_device[o:], up[o:])
+    np.testing.assert_array_equal(down[o:], up[o:])
+    assert (on_device[:o] == 0x5a).all() and (down[:o] == 0xa5).all()
+    del up, down
+    shim._chk(lib.mi355x_host_free(p))
+    shim._chk(lib.mi355x_host_free(q))
+    dev.stream_destroy(stream)
+
+
 @pytest.mark.parametrize("chunk", range(4))
 def test_random_pooling_add_softmax_pad(port, chunk):
     """Seeded draws over the bandwidth-bound layers: window, stride, padding (also wider than the window), padding method,
