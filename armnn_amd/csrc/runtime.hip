@@ -498,6 +498,20 @@ int mi355x_event_synchronize(mi355x_event_t event)
     return 0;
 }
 
+int mi355x_event_query(mi355x_event_t event, int* done)
+{
+    if (!done) return SetError(MI355X_ERR_INVALID_ARGUMENT, "done is null");
+    const hipError_t e = hipEventQuery(reinterpret_cast<hipEvent_t>(event));
+    *done = e == hipSuccess;
+    if (e == hipErrorNotReady)
+    {
+        (void)hipGetLastError();      // an answer, not an error
+        return 0;
+    }
+    MI355X_HIP(e);
+    return 0;
+}
+
 int mi355x_event_elapsed_ms(mi355x_event_t start, mi355x_event_t stop, float* ms)
 {
     if (!ms) return SetError(MI355X_ERR_INVALID_ARGUMENT, "ms is null");

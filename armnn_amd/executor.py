@@ -6,7 +6,6 @@ from __future__ import annotations
 import collections
 import ctypes as C
 import itertools
-import os
 import weakref
 from dataclasses import dataclass
 from typing import Dict, List, Optional, Tuple
@@ -103,6 +102,26 @@ class _OpenNetworks:
 
     def __iter__(self):
         return iter([n for n in (ref() for ref in list(self._refs.values())) if n is not None])
+
+
+class _PassEnd:
+    """A point in a stream.  Networks on other threads may be asking for it while its own network closes, so it lives until the last
+    of them has let go."""
+
+    def __init__(self, dev: shim.Device):
+        self._dev, self._event = dev, dev.event()
+
+    def record(self, stream):
+        self._dev.event_record(self._event, stream)
+
+    def done(self) -> bool:
+        return self._dev.event_done(self._event)
+
+    def __del__(self):
+        try:
+            self._dev.event_destroy(self._event)
+        except Exception:
+            pass
 
 
 class DeviceNetwork:
@@ -218,7 +237,7 @@ class DeviceNetwork:
             self._fuse_conv_pool(only_where_it_pays=not fuse_pool)
 
     def _register(self):
-        self._has_run = False
+        self._pass_end: Optional[_PassEnd] = None              # behind the last replayed pass, for other networks to ask
         self._key = self._open.add(self)
 
     def _fuse_conv_pool(self, only_where_it_pays):
@@ -507,18 +526,17 @@ class DeviceNetwork:
         self._sync_next += 1
         return ev
 
-    # The networks of the process, and how many hardware queues the streams of a process share.
-    _open = _OpenNetworks()
-    _hardware_queues = int(os.environ.get("GPU_MAX_HW_QUEUES", "4"))
+    _open = _OpenNetworks()                    # of the process
+
+    def _under_way(self) -> bool:
+        """Whether the device still works on a replayed pass of this network (one that may run in lanes)."""
+        return self._pass_end is not None and not self._pass_end.done()
 
     def _one_lane_now(self) -> bool:
-        """Whether this pass runs as one lane: where the lanes of all networks outnumber the hardware queues, streams share them
-        and a lane waits behind another network's, or behind its own sibling (three of ResNet-50 side by side, 32 images in
-        two lanes each, 605 us a pass; as one lane each 525; one alone 720 in its lanes, 870 as one, 1130 with the two on one
-        queue)."""
-        self._has_run = True
-        lanes = sum(n.lanes for n in self._open if n._has_run)
-        return lanes > max(self._hardware_queues, self.lanes) and not self.chains and not self.tails
+        """Whether this pass runs as one lane: while another network's pass is under way the two fill each other's gaps, and lanes on
+        top of that wait behind one another in the device's few hardware queues.  ResNet-50, 32 images in two lanes each, us a pass:
+        three networks in turn 552 in lanes, 439 as one lane each; two 662 and 511; one by itself 646 and 751."""
+        return any(n is not self and n._under_way() for n in self._open)
 
     def _capture(self, one_lane: bool):
         """The graphs of a pass: one per lane, because a chain of kernels is replayed without the host (57 launches of ResNet-50 in
@@ -541,30 +559,35 @@ class DeviceNetwork:
             self.dev.graph_begin(self.stream)
             self._enqueue_lanes()
             return [self.dev.graph_end(self.stream)]
-        for lane, stream in enumerate([self.stream] + self.side_streams):
-            self.dev.graph_begin(stream)
+        for lane in range(self.lanes):
+            self.dev.graph_begin(self.stream)
             for _, fn in self.steps:
-                fn(stream, lane, self.lanes)
-            graphs.append(self.dev.graph_end(stream))
+                fn(self.stream, lane, self.lanes)
+            graphs.append(self.dev.graph_end(self.stream))
         return graphs
 
     def enqueue(self):
         """One forward pass on self.stream (asynchronous)."""
-        if self.use_graph:
-            one_lane = self.lanes > 1 and self._one_lane_now()
+        if not self.use_graph:
+            self._enqueue_lanes()
+            return
+        may_choose = self.lanes > 1 and not self.chains and not self.tails
+        for one_lane in (False, True) if may_choose else (False,):     # (all at the first pass: no later one captures)
             if one_lane not in self.graphs:
                 self.graphs[one_lane] = self._capture(one_lane)
-            graphs = self.graphs[one_lane]
-            if len(graphs) == 1:
-                self.dev.graph_launch(graphs[0], self.stream)
-                return
+        graphs = self.graphs[may_choose and self._one_lane_now()]
+        if len(graphs) == 1:
+            self.dev.graph_launch(graphs[0], self.stream)
+        else:
             self._sync_next = 0
             self._fork()
             for graph, stream in zip(graphs, [self.stream] + self.side_streams):
                 self.dev.graph_launch(graph, stream)
             self._join()
-        else:
-            self._enqueue_lanes()
+        if may_choose:
+            if self._pass_end is None:
+                self._pass_end = _PassEnd(self.dev)
+            self._pass_end.record(self.stream)
 
     def choose_submission(self, passes: int = 40, rounds: int = 2):
         """Times `passes` forward passes launched kernel by kernel and the same number of replays of the captured graph,

@@ -28,7 +28,7 @@ EXPORTS = [
     "mi355x_device_props", "mi355x_malloc", "mi355x_free", "mi355x_host_alloc", "mi355x_host_device_pointer", "mi355x_host_free",
     "mi355x_memcpy_h2d", "mi355x_memcpy_d2h", "mi355x_memcpy_d2d", "mi355x_memcpy_h2d_async", "mi355x_memcpy_d2h_async", "mi355x_fill_u8", "mi355x_stream_create",
     "mi355x_stream_destroy", "mi355x_stream_synchronize", "mi355x_device_synchronize", "mi355x_event_create",
-    "mi355x_event_destroy", "mi355x_event_record", "mi355x_stream_wait_event", "mi355x_event_synchronize", "mi355x_event_elapsed_ms",
+    "mi355x_event_destroy", "mi355x_event_record", "mi355x_stream_wait_event", "mi355x_event_synchronize", "mi355x_event_query", "mi355x_event_elapsed_ms",
     "mi355x_graph_capture_begin", "mi355x_graph_capture_end", "mi355x_graph_launch", "mi355x_graph_destroy",
     "mi355x_conv2d_create", "mi355x_conv2d_run", "mi355x_conv2d_destroy", "mi355x_conv2d_algo",
     "mi355x_conv2d_fusable", "mi355x_conv2d_fusion_pays", "mi355x_conv2d_run_fused", "mi355x_conv2d_pool_fusable",
@@ -118,7 +118,7 @@ def load_library(path: str = LIB_PATH) -> C.CDLL:
             "mi355x_stream_create": [C.POINTER(V)], "mi355x_stream_destroy": [V], "mi355x_stream_synchronize": [V],
             "mi355x_event_create": [C.POINTER(V)], "mi355x_event_destroy": [V], "mi355x_event_record": [V, V],
             "mi355x_stream_wait_event": [V, V],
-            "mi355x_event_synchronize": [V], "mi355x_event_elapsed_ms": [V, V, C.POINTER(C.c_float)],
+            "mi355x_event_synchronize": [V], "mi355x_event_query": [V, C.POINTER(C.c_int)], "mi355x_event_elapsed_ms": [V, V, C.POINTER(C.c_float)],
             "mi355x_graph_capture_begin": [V], "mi355x_graph_capture_end": [V, C.POINTER(V)],
             "mi355x_graph_launch": [V, V], "mi355x_graph_destroy": [V],
             "mi355x_conv2d_create": [C.POINTER(Conv2dDesc), V, C.POINTER(ConstQuant), V, C.POINTER(ConstQuant), C.POINTER(V)],
@@ -265,6 +265,14 @@ class Device:
 
     def event_sync(self, e):
         _chk(self.lib.mi355x_event_synchronize(e))
+
+    def event_destroy(self, e):
+        _chk(self.lib.mi355x_event_destroy(e))
+
+    def event_done(self, e) -> bool:
+        done = C.c_int()
+        _chk(self.lib.mi355x_event_query(e, C.byref(done)))
+        return done.value != 0
 
     def elapsed_ms(self, e0, e1) -> float:
         ms = C.c_float()

@@ -184,6 +184,8 @@ int  mi355x_event_record(mi355x_event_t event, mi355x_stream_t stream);
  * capture this is how a second stream joins the capture (fork) and how its work is joined back. */
 int  mi355x_stream_wait_event(mi355x_stream_t stream, mi355x_event_t event);
 int  mi355x_event_synchronize(mi355x_event_t event);
+/* *done = 1 when the work in front of the last record of `event` is complete, or there is no record; else 0.  Does not wait. */
+int  mi355x_event_query(mi355x_event_t event, int* done);
 int  mi355x_event_elapsed_ms(mi355x_event_t start, mi355x_event_t stop, float* ms);
 
 /* Capture everything launched on `stream` between begin and end into an executable graph, then replay it

@@ -25,13 +25,34 @@ class FakeLibrary:
 
 
 class FakeDevice:
-    def stream_destroy(self, s):
-        pass
+    """Streams, events and graphs that only note what was asked of them; an event is done when the test says so."""
+
+    def __init__(self):
+        self.handles, self.log, self.done = 0, [], set()
+
+    def stream(self):
+        self.handles += 1
+        return self.handles
+
+    event = stream
+
+    def event_done(self, e):
+        return e in self.done
+
+    def event_destroy(self, e):
+        self.log.append(("event_destroy", e))
+
+    def graph_end(self, stream):
+        return self.stream()
+
+    def __getattr__(self, name):
+        return lambda *a: self.log.append((name,) + a)
 
 
-def bare_network(lib, lanes=1):
+def bare_network(lib, lanes=1, dev=None):
     n = object.__new__(DeviceNetwork)
-    n.lib, n.dev, n.stream, n.lanes = lib, FakeDevice(), 1, lanes
+    n.lib, n.dev, n.stream, n.lanes, n.use_graph = lib, dev or FakeDevice(), 1, lanes, True
+    n.steps = [("layer", lambda stream, lane=0, lanes=1: n.dev.log.append(("launch", lane, lanes)))]
     n.graphs, n.chains, n.tails, n.plans, n.buffers, n._side_streams = {}, [], [], [], {}, None
     n._register()
     return n
@@ -103,3 +124,43 @@ def test_repeated_calls_allocate_no_pinned_memory():
     assert len(lib.live) == 33                             # what one network's call takes
     a.close()
     assert not lib.live
+
+
+def test_a_pass_runs_as_one_lane_only_while_another_networks_pass_is_under_way():
+    """What networks that are merely open have done before does not matter."""
+    lib, dev = FakeLibrary(), FakeDevice()
+    a, b, c = (bare_network(lib, lanes=2, dev=dev) for _ in range(3))
+
+    def passes(network):
+        """Lanes that a pass of the network replays a graph for."""
+        dev.log.clear()
+        network.enqueue()
+        return [e[0] for e in dev.log].count("graph_launch")
+
+    assert passes(a) == 2 and passes(a) == 2               # by itself, again and again
+    assert passes(b) == 1                                  # a's pass is under way
+    dev.done.update((a._pass_end._event, b._pass_end._event))
+    assert passes(c) == 2                                  # a and b are open, have run, and are idle
+    assert passes(a) == 1
+    dev.done.add(a._pass_end._event)
+    assert passes(c) == 2
+    c.close()
+    dev.done.discard(b._pass_end._event)
+    assert passes(a) == 1
+    b.close()
+    assert passes(a) == 2
+    a.close()
+
+
+def test_only_the_first_pass_captures():
+    lib, dev = FakeLibrary(), FakeDevice()
+    a, b = (bare_network(lib, lanes=2, dev=dev) for _ in range(2))
+    a.enqueue()
+    assert [e[1:] for e in dev.log if e[0] == "launch"] == [(0, 2), (1, 2), (0, 1)]
+    b.enqueue()
+    dev.log.clear()
+    for _ in range(2):
+        a.enqueue()                                        # as one lane: b's pass is under way
+        b.close()
+    assert not [e for e in dev.log if e[0] in ("launch", "graph_begin")]
+    a.close()

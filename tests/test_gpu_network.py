@@ -191,6 +191,32 @@ def test_the_measured_choice_between_launching_and_replaying_changes_no_byte(whi
     dn.close()
 
 
+def test_two_networks_in_lanes_give_the_same_bytes_in_turn_and_apart():
+    """A pass runs as one lane while another network's is under way, in its lanes otherwise; the bytes are the eager launches'."""
+    net = nets.resnet50(resolution=64)
+    a, b = (DeviceNetwork(net, 8, lanes=2) for _ in range(2))
+    eager = DeviceNetwork(net, 8, use_graph=False)
+    inputs = [nets.synthetic_input(net, 8, seed=s) for s in (71, 72)]
+    want = [eager.run(x).data for x in inputs]
+    for dn, x in zip((a, b), inputs):
+        dn.upload_input(x)
+    ways = {True: 0, False: 0}
+    for _ in range(3):
+        for apart in (True, False):
+            for _ in range(1 if apart else 20):
+                for dn, out in zip((a, b), want):
+                    ways[dn._one_lane_now()] += 1
+                    dn.enqueue()
+                    if apart:
+                        assert np.array_equal(dn.download().data, out)
+            for dn, out in zip((a, b), want):
+                assert np.array_equal(dn.download().data, out)
+            assert not a._one_lane_now() and not b._one_lane_now()
+    assert ways[True] >= 3 and ways[False] >= 6, ways
+    for dn in (a, b, eager):
+        dn.close()
+
+
 def test_mobilenet_v1_batch64_in_one_lane_rows_equal_batch2_runs():
     # 64 images per launch: the largest launches of the benchmark (persistent blocks walk the most tiles here)
     _rows_equal_small_batch_runs(nets.mobilenet_v1(), 64, (0, 20, 42, 62), lanes=1)
