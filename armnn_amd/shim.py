@@ -88,7 +88,7 @@ class ShimError(RuntimeError):
 
 
 _lib = None
-_calls = None                          # the launch entry points without ctypes (csrc/pycalls.cpp), and their addresses
+_calls = None                          # the launch entry points without ctypes (csrc/pycalls.cpp) where they load, and their addresses
 _conv2d_run_at = _fc_run_at = 0
 
 
@@ -96,13 +96,15 @@ def load_library(path: str = LIB_PATH) -> C.CDLL:
     """dlopen the device library (no GPU needed for loading)."""
     global _lib, _calls, _conv2d_run_at, _fc_run_at
     if _lib is None:
-        for p in (path, CALLS_PATH):
-            if not os.path.exists(p):
-                raise FileNotFoundError(f"{p} not found: build it with `make -C armnn_amd/csrc` "
-                                        f"(or __graft_entry__.build()); there is no fallback path")
-        loader = importlib.machinery.ExtensionFileLoader("_calls", CALLS_PATH)
-        _calls = importlib.util.module_from_spec(importlib.util.spec_from_loader("_calls", loader))
-        loader.exec_module(_calls)
+        if not os.path.exists(path):
+            raise FileNotFoundError(f"{path} not found: build it with `make -C armnn_amd/csrc` "
+                                    f"(or __graft_entry__.build()); there is no fallback path")
+        try:
+            loader = importlib.machinery.ExtensionFileLoader("_calls", CALLS_PATH)
+            _calls = importlib.util.module_from_spec(importlib.util.spec_from_loader("_calls", loader))
+            loader.exec_module(_calls)
+        except ImportError:                                # not built, or built for another Python: ctypes makes the same calls
+            _calls = None
         _lib = C.CDLL(path)
         _conv2d_run_at, _fc_run_at = (C.cast(fn, C.c_void_p).value for fn in (_lib.mi355x_conv2d_run, _lib.mi355x_fc_run))
         _lib.mi355x_last_error.restype = C.c_char_p
@@ -331,7 +333,7 @@ class Conv2dPlan:
     def run(self, batch: int, x_dev: int, y_dev: int, stream=None):
         try:
             rc = _calls.run(_conv2d_run_at, self.plan, batch, x_dev, y_dev, stream)
-        except TypeError:                                  # an argument that is no plain int: ctypes' own conversions decide
+        except (TypeError, AttributeError):                # an argument that is no plain int, or no _calls: ctypes' own conversions
             rc = self.lib.mi355x_conv2d_run(self.plan, batch, x_dev, y_dev, stream)
         if rc != 0:
             _chk(rc)
@@ -476,7 +478,7 @@ class FullyConnectedPlan:
     def run(self, batch: int, x_dev: int, y_dev: int, stream=None):
         try:
             rc = _calls.run(_fc_run_at, self.plan, batch, x_dev, y_dev, stream)
-        except TypeError:
+        except (TypeError, AttributeError):
             rc = self.lib.mi355x_fc_run(self.plan, batch, x_dev, y_dev, stream)
         if rc != 0:
             _chk(rc)
