@@ -41,7 +41,7 @@ thread_local PendingAdd* t_pending_add = nullptr;
 constexpr double kBracketUnit = 1.0 / 16777216.0;
 constexpr double kBracketRel = 16.0 / 16777216.0;
 constexpr long long kSmallConvMostTiles = 392, kSmallConvLeastSlabTiles = 128;
-
+constexpr int kRowPanelMostChannels = 768;
 
 void FoldCorrIntoTable(mi355x_conv2d_s* p, const std::vector<int32_t>& corr, int Co);
 void ChoosePointwiseConfig(mi355x_conv2d_s* p);
@@ -304,7 +304,6 @@ int BuildPlan(const mi355x_conv2d_desc& d, const void* weights_host, const mi355
         p->rowsum_bias = (p->K_pad - p->K) * zx_shift;     // kernels that walk K_pad bytes meet zx' beyond K
         if (int rc = Upload(reinterpret_cast<void**>(&p->w_mfma), wp.data(), wp.size())) return rc;
         if (int rc = Upload(reinterpret_cast<void**>(&p->corr), corr.data(), corr.size() * sizeof(int32_t))) return rc;
-        if (int rc = PackFragments(p)) return rc;
         p->xor_mask = g.in_u8 ? 0x80808080u : 0u;
         const uint32_t zb = static_cast<uint32_t>(zx_shift) & 0xffu;
         p->pad_word = zb | (zb << 8) | (zb << 16) | (zb << 24);
@@ -313,6 +312,8 @@ int BuildPlan(const mi355x_conv2d_desc& d, const void* weights_host, const mi355
             if (int rc = Upload(reinterpret_cast<void**>(&p->pad16), padbytes.data(), padbytes.size())) return rc;
         }
         p->tile_override = GlobalOptions().igemm_tile;
+        if (FragmentsWanted(p))
+            if (int rc = PackFragments(p, false, &p->w_frag)) return rc;
         if (p->bk128 && (Ci % 128) == 0)
             if (int rc = PrepareBigGemm()) return rc;
         FoldCorrIntoTable(p, corr, Co);
@@ -377,23 +378,6 @@ int BuildPlan(const mi355x_conv2d_desc& d, const void* weights_host, const mi355
                 for (int r = 0; r < 4; ++r) std::memcpy(&gdst[(4 + r) * 4], &p->chan_host[static_cast<size_t>(2 + r) * CP + c], 4);
             }
             if (int rc = Upload(reinterpret_cast<void**>(&p->dw_grp), grp.data(), grp.size() * sizeof(uint32_t))) return rc;
-            // blocks of 64 channels: rows of [16][4] dwords, entry [j][e] for channel 16 e + j of the block: corr, m+, b+, m-, b-,
-            // filter taps 0..3, 4..7, 8, and those of the second halves.  Channels past the last one are all zero: a bracket that
-            // closes, some code that no weight and no row sum counts.
-            const int rows = 11;
-            std::vector<uint32_t> blk(static_cast<size_t>((Co + 63) / 64) * rows * 64, 0u);
-            for (int c = 0; c < Co; ++c)
-            {
-                uint32_t* bdst = blk.data() + static_cast<size_t>(c / 64) * rows * 64 + (c % 16) * 4 + c % 64 / 16;
-                bdst[0] = static_cast<uint32_t>(corr[c]);
-                for (int r = 0; r < 4; ++r) std::memcpy(&bdst[(1 + r) * 64], &p->chan_host[static_cast<size_t>(2 + r) * CP + c], 4);
-                for (int t = 0; t < 9; ++t)
-                {
-                    bdst[(5 + t / 4) * 64] |= (wp[static_cast<size_t>(c) * 4 + t / 3] >> (8 * (t % 3)) & 0xffu) << (8 * (t % 4));
-                    if (!dw3_fits) bdst[(8 + t / 4) * 64] |= (wp2[static_cast<size_t>(c) * 4 + t / 3] >> (8 * (t % 3)) & 0xffu) << (8 * (t % 4));
-                }
-            }
-            if (int rc = Upload(reinterpret_cast<void**>(&p->dw_blk), blk.data(), blk.size() * sizeof(uint32_t))) return rc;
             const std::vector<uint8_t> padbytes(16, static_cast<uint8_t>((zb ^ (g.in_u8 ? 0x80u : 0u)) & 0xffu));
             if (int rc = Upload(reinterpret_cast<void**>(&p->pad16), padbytes.data(), padbytes.size())) return rc;
         }
@@ -1042,7 +1026,7 @@ int RunPlan(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, hi
         if (unit && p->w_frag && p->ragged_ck == 0 && (g.Co & 15) == 0 && p->tile_override == 0 && p->opt_igemm_lds != 0)
         {
             const long long tiles = (rows + 63) / 64 * ((g.Co + 127) / 128);
-            if (g.Ci <= 256 ? tiles >= 224 && (g.Ci > 64 || tiles <= 2048) : g.Ci <= 768 && tiles >= 384 && (g.Co <= 1024 || tiles < 896))
+            if (g.Ci <= 256 ? tiles >= 224 && (g.Ci > 64 || tiles <= 2048) : g.Ci <= kRowPanelMostChannels && tiles >= 384 && (g.Co <= 1024 || tiles < 896))
             {
                 const uint8_t* res = nullptr;
                 if (t_pending_add) { res = t_pending_add->other; t_pending_add->taken = true; }
@@ -1592,6 +1576,18 @@ int LaunchPwPool(const mi355x_conv2d_s* pw, const mi355x_pool2d_desc* pool, int 
 
 namespace mi355x
 {
+// A plan does not know the batches it will run: the smallest number of rows decides for the kernel of few rows (RunPlan; up to four
+// rows of a 1x1 layer are GemvKernel's, one or five make one tile), any large one may come for the kernel of many.
+bool FragmentsWanted(const mi355x_conv2d_s* p)
+{
+    const ConvGeom& g = p->geom;
+    if (p->tile_override != 0) return false;
+    const long long least_tiles = (static_cast<long long>(g.Ho) * g.Wo + 31) / 32 * ((g.Co + 31) / 32);
+    if (least_tiles <= kSmallConvMostTiles) return true;
+    const bool unit = g.Kh == 1 && g.Kw == 1 && g.stride_x == 1 && g.stride_y == 1 && g.pad_top == 0 && g.pad_left == 0 && g.Ho == g.H && g.Wo == g.W;
+    return unit && p->ragged_ck == 0 && (g.Co & 15) == 0 && g.Ci <= kRowPanelMostChannels && p->opt_igemm_lds != 0;
+}
+
 int FillIgemmLdsArgs(const mi355x_conv2d_s* p, int bm, int bn, uint32_t batch, const void* x, void* y, IgemmArgs* out, bool* unit_fast)
 {
     const ConvGeom& g = p->geom;
@@ -1780,14 +1776,16 @@ int mi355x_conv2d_fusion_pays(mi355x_conv2d_t first, mi355x_conv2d_t second, uin
         // than two launches (MobileNetV1, its four such pairs: one image 104 -> 98 us, four images 137 -> 123 us a pass): up to one
         // item per CU, and up to 1024 on maps of 16 tiles and more, where it was measured
         const long long tiles = static_cast<long long>((first->d.out_w + 7) / 8) * ((first->d.out_h + 7) / 8), items = batch * tiles;
-        return items >= 1024 || (items >= 16 && (items <= 256 || tiles >= 16)) ? 1 : 0;
+        if (items < 1024 && (items < 16 || (items > 256 && tiles < 16))) return 0;
+        return !PanelRuns(first, second, batch) || PrepareDwPwPanel(first, second) == 0 ? 1 : 0;
     }
     if (mi355x_conv2d_fusable(first, second) != 0 || !PanelRuns(first, second, batch)) return 0;
     // 7 x 7 maps: from 8 images on the 1x1 convolution is worth more with a pooling behind it (mi355x_conv2d_pool_fusion_pays), and
     // from 64 on with the depthwise layer behind it (above); beyond 512 channels every block's own copy of the depthwise layer
     // costs what the launch saves (1024 -> 1024, one image: 6.9 us against 7.4)
     if (first->d.out_c > 512) return 0;
-    return first->d.out_h > 7 || first->d.out_w > 7 || batch < (first->d.stride_x == 1 ? 8u : 64u) ? 1 : 0;
+    if (first->d.out_h <= 7 && first->d.out_w <= 7 && batch >= (first->d.stride_x == 1 ? 8u : 64u)) return 0;
+    return PrepareDwPwPanel(first, second) == 0 ? 1 : 0;
 }
 
 int mi355x_conv2d_run_fused(mi355x_conv2d_t dw, mi355x_conv2d_t pw, uint32_t batch, const void* input_dev, void* output_dev,
@@ -1804,7 +1802,11 @@ int mi355x_conv2d_run_fused(mi355x_conv2d_t dw, mi355x_conv2d_t pw, uint32_t bat
         if (int rc = PwDwCheck(dw, pw, &sh)) return rc;
         return LaunchPwDw(dw, pw, sh, batch, input_dev, output_dev, ToHip(stream));
     }
-    if (PanelRuns(dw, pw, batch)) return LaunchDwPwPanel(dw, pw, batch, input_dev, output_dev, ToHip(stream));
+    if (PanelRuns(dw, pw, batch))
+    {
+        if (int rc = PrepareDwPwPanel(dw, pw)) return rc;
+        return LaunchDwPwPanel(dw, pw, batch, input_dev, output_dev, ToHip(stream));
+    }
     if (GlobalOptions().dwpw_stream != 0)
         if (const int which = DwPwStreamShape(dw, pw)) return LaunchDwPwStream(dw, pw, which, batch, input_dev, output_dev, ToHip(stream));
     if (dw->d.stride_x == 2) return LaunchDwPw<2, 2>(dw, pw, batch, input_dev, output_dev, ToHip(stream));

@@ -5,6 +5,7 @@
 
 #include "common.h"
 #include "dwpw_panel_kernel.h"
+#include "igemm.h"
 
 using namespace mi355x;
 
@@ -17,7 +18,7 @@ int LaunchT(const mi355x_conv2d_s* dw, const mi355x_conv2d_s* pw, uint32_t batch
     const ConvGeom& g = dw->geom;
     const auto rcp = [](int d) { return static_cast<uint32_t>(((1ull << 32) + static_cast<uint32_t>(d) - 1) / static_cast<uint32_t>(d)); };
     DwPwPanelArgs a;
-    a.x = static_cast<const uint8_t*>(x); a.pad16 = dw->pad16; a.dw_blk = dw->dw_blk;
+    a.x = static_cast<const uint8_t*>(x); a.pad16 = dw->pad16; a.dw_blk = dw->dw_blk.load(std::memory_order_acquire);
     a.dw_ct = ChanTab{dw->chan, dw->Co_pad};
     a.H = g.H; a.W = g.W; a.C = g.Co; a.Ho = g.Ho; a.Wo = g.Wo;
     a.pad_top = g.pad_top; a.pad_left = g.pad_left;
@@ -31,7 +32,7 @@ int LaunchT(const mi355x_conv2d_s* dw, const mi355x_conv2d_s* pw, uint32_t batch
     a.total_items = static_cast<int>(items); a.xcd_chunk = static_cast<int>((items + 7) / 8);
     a.rcp_tiles_x = rcp(a.tiles_x); a.rcp_tiles_y = rcp(a.tiles_y); a.rcp_nb = rcp(a.nb); a.rcp_ng = rcp(a.C / 16);
     a.dw_xor = dw->xor_mask; a.dw_rq = dw->rq;
-    a.w = pw->w_panel; a.co_groups = pw->Co_pad / 16;
+    a.w = pw->w_panel.load(std::memory_order_acquire); a.co_groups = pw->Co_pad / 16;
     a.pw_ct = ChanTab{pw->chan, pw->Co_pad}; a.pw_corr = pw->corr;
     a.y = static_cast<uint8_t*>(y);
     a.y_bytes = static_cast<long long>(batch) * g.Ho * g.Wo * a.Co;
@@ -88,10 +89,82 @@ bool mi355x::DwPwPanelTakes(const mi355x_conv2d_s* dw, const mi355x_conv2d_s* pw
 {
     const mi355x_conv2d_desc& a = dw->d;
     if (dw->algo != MI355X_ALGO_DEPTHWISE || dw->variant != 1 || a.out_c != a.in_c || (a.out_c & 15) != 0) return false;
-    if (!pw->w_panel || (pw->d.out_c & 15) != 0 || pw->geom.Ci != static_cast<int>(a.out_c)) return false;
+    const ConvGeom& g = pw->geom;
+    const bool unit = g.Kh == 1 && g.Kw == 1 && g.stride_x == 1 && g.stride_y == 1 && g.Ho == g.H && g.Wo == g.W && g.H * g.W > 1;
+    if (!pw->w_mfma || !unit || pw->ragged_ck != 0 || g.Ci > 1024 || (g.Co & 15) != 0 || g.Ci != static_cast<int>(a.out_c)) return false;
     if (static_cast<long long>(a.in_h) * a.in_w * a.in_c >= (1ll << 31)) return false;
     const int smem = a.stride_x == 1 ? DwPwPanelGeom<1, 4, 8, 8, 2>::Smem(static_cast<int>(a.out_c), true) : DwPwPanelGeom<2, 4, 8, 8, 2>::Smem(static_cast<int>(a.out_c), true);
     return smem <= 160 * 1024;
+}
+
+namespace
+{
+// Blocks of 64 channels: 11 rows of [16][4] dwords, entry [j][e] for channel 16 e + j of the block: corr, m+, b+, m-, b-, filter taps
+// 0..3, 4..7, 8, and those of the second halves.  Channels past the last one are all zero: a bracket that closes, some code that no
+// weight and no row sum counts.  `grp`, `second`: the plan's dw_grp and w_dot4b (or null).
+__global__ __launch_bounds__(256) void PackDwBlkKernel(const uint32_t* __restrict__ grp, const uint32_t* __restrict__ second, uint32_t* __restrict__ blk, int C, int dwords)
+{
+    const int i = static_cast<int>(blockIdx.x) * 256 + static_cast<int>(threadIdx.x);
+    if (i >= dwords) return;
+    const int b = i / 704, row = i % 704 / 64, c = b * 64 + i % 4 * 16 + i % 64 / 4;
+    uint32_t v = 0;
+    if (c < C)
+    {
+        const uint32_t* const of = grp + (c / 4) * 32 + c % 4;         // rows of four: weights 0 .. 2, corr, m+, b+, m-, b-
+        if (row < 5) v = of[(3 + row) * 4];
+        else
+            for (int t = (row - (row < 8 ? 5 : 8)) * 4, n = 0; n < 4 && t < 9; ++t, ++n)
+            {
+                const uint32_t taps = row < 8 ? of[t / 3 * 4] : second ? second[c * 4 + t / 3] : 0u;
+                v |= (taps >> (8 * (t % 3)) & 0xffu) << (8 * n);
+            }
+    }
+    blk[i] = v;
+}
+
+int PackDwBlk(const mi355x_conv2d_s* dw, uint32_t** out)
+{
+    const int C = dw->geom.Co, dwords = (C + 63) / 64 * 704;
+    hipStream_t stream;
+    if (const int rc = UploadStream(&stream)) return rc;
+    MI355X_HIP(hipMalloc(reinterpret_cast<void**>(out), static_cast<size_t>(dwords) * 4));
+    hipLaunchKernelGGL(PackDwBlkKernel, dim3(static_cast<unsigned>((dwords + 255) / 256)), dim3(256), 0, stream, dw->dw_grp, dw->w_dot4b, *out, C, dwords);
+    MI355X_HIP(hipGetLastError());
+    MI355X_HIP(hipStreamSynchronize(stream));
+    return 0;
+}
+
+// While one is open, the thread may allocate and wait although it captures a graph.
+struct OutsideCapture
+{
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    OutsideCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~OutsideCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+} // namespace
+
+int mi355x::PrepareDwPwPanel(const mi355x_conv2d_s* dw, const mi355x_conv2d_s* pw)
+{
+    if (dw->dw_blk.load(std::memory_order_acquire) && pw->w_panel.load(std::memory_order_acquire)) return 0;
+    OutsideCapture outside;
+    UploadScope uploads;
+    {
+        std::lock_guard<std::mutex> lock(dw->panel_mutex);
+        if (!dw->dw_blk.load(std::memory_order_relaxed))
+        {
+            uint32_t* blk = nullptr;
+            if (const int rc = PackDwBlk(dw, &blk)) { (void)hipFree(blk); return rc; }
+            dw->dw_blk.store(blk, std::memory_order_release);
+        }
+    }
+    std::lock_guard<std::mutex> lock(pw->panel_mutex);
+    if (!pw->w_panel.load(std::memory_order_relaxed))
+    {
+        int8_t* w = nullptr;
+        if (const int rc = PackFragments(pw, true, &w)) { (void)hipFree(w); return rc; }
+        pw->w_panel.store(w, std::memory_order_release);
+    }
+    return 0;
 }
 
 int mi355x::LaunchDwPwPanel(const mi355x_conv2d_s* dw, const mi355x_conv2d_s* pw, uint32_t batch, const void* x, void* y, hipStream_t stream)

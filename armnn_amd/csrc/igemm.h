@@ -9,8 +9,11 @@ namespace mi355x
 // `tile`: 64, 96 (128 x 64) or anything else (128 x 128, 128 x 64 for at most 64 output channels).  `p` is a MI355X_ALGO_MFMA plan.
 int LaunchIgemm(const mi355x_conv2d_s* p, int tile, uint32_t batch, const void* x, void* y, hipStream_t stream);
 
-// w_frag of an MFMA plan from its w_mfma (PackFragKernel), queued on the calling thread's upload stream.
-int PackFragments(mi355x_conv2d_s* p);
+// The weights of an MFMA plan in operand order (PackFragKernel) as a new device array; waits for it (an UploadScope must be open).
+int PackFragments(const mi355x_conv2d_s* p, bool interleave, int8_t** out);
+
+// Whether a launch of some batch reads an MFMA plan's w_frag.
+bool FragmentsWanted(const mi355x_conv2d_s* p);
 
 // SmallConvKernel (small_conv_kernel.h) for a plan with w_frag.  res / add: an Addition behind the layer (output channels
 // % 16 == 0, aligned tensors), or null.

@@ -91,28 +91,15 @@ int mi355x::LaunchIgemm(const mi355x_conv2d_s* p, int tile, uint32_t batch, cons
     return bk128 ? LaunchTile<128, 128, 2, 2, 2, 128>(p, batch, x, y, stream) : LaunchTile<128, 128, 2, 2, 2, 64>(p, batch, x, y, stream);
 }
 
-// 1x1 layers that may follow a depthwise layer in one launch (dwpw_panel_kernel.h)
-static bool PanelWeights(const mi355x_conv2d_s* p)
-{
-    const ConvGeom& g = p->geom;
-    return g.Kh == 1 && g.Kw == 1 && g.stride_x == 1 && g.stride_y == 1 && g.Ho == g.H && g.Wo == g.W && g.H * g.W > 1 && p->ragged_ck == 0 && g.Ci <= 1024;
-}
-
-int mi355x::PackFragments(mi355x_conv2d_s* p)
+int mi355x::PackFragments(const mi355x_conv2d_s* p, bool interleave, int8_t** out)
 {
     const int steps = (p->geom.Kh * p->geom.Kw * (p->ragged_ck ? p->ragged_ck : p->geom.Ci) + 63) / 64;
     const long long pieces = static_cast<long long>(p->Co_pad / 16) * steps * 64;
-    MI355X_HIP(hipMalloc(reinterpret_cast<void**>(&p->w_frag), pieces * 16));
     hipStream_t stream;
     if (const int rc = UploadStream(&stream)) return rc;
-    hipLaunchKernelGGL(PackFragKernel, dim3(static_cast<unsigned>((pieces + 255) / 256)), dim3(256), 0, stream, p->w_mfma, p->w_frag, p->K_pad, steps, pieces, 0);
+    MI355X_HIP(hipMalloc(reinterpret_cast<void**>(out), pieces * 16));
+    hipLaunchKernelGGL(PackFragKernel, dim3(static_cast<unsigned>((pieces + 255) / 256)), dim3(256), 0, stream, p->w_mfma, *out, p->K_pad, steps, pieces, interleave ? 1 : 0);
     MI355X_HIP(hipGetLastError());
-    if (PanelWeights(p))
-    {
-        MI355X_HIP(hipMalloc(reinterpret_cast<void**>(&p->w_panel), pieces * 16));
-        hipLaunchKernelGGL(PackFragKernel, dim3(static_cast<unsigned>((pieces + 255) / 256)), dim3(256), 0, stream, p->w_mfma, p->w_panel, p->K_pad, steps, pieces, 1);
-        MI355X_HIP(hipGetLastError());
-    }
     MI355X_HIP(hipStreamSynchronize(stream));
     return 0;
 }

@@ -3,6 +3,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -19,14 +21,17 @@ struct mi355x_conv2d_s
     // device constants
     uint8_t* w_direct = nullptr;   // [Kh][Kw][Ci][Co] / depthwise [Kh][Kw][Co], raw codes
     int8_t*  w_mfma   = nullptr;   // [Co_pad][K_pad] signed, zero padded
-    int8_t*  w_frag   = nullptr;   // the same weights in operand order (small_conv_kernel.h), where a launch may want them
-    int8_t*  w_panel  = nullptr;   // 1x1: in operand order with the channels of a k-step interleaved as a depthwise layer before it leaves them
+    int8_t*  w_frag   = nullptr;   // the same weights in operand order (small_conv_kernel.h), where a launch of some batch wants them
+    // What only the fused kernel with the layer between in LDS reads (dwpw_panel_kernel.h): nothing until the first pair that the
+    // plan is part of goes to that kernel (PrepareDwPwPanel), under `panel_mutex`.
+    mutable std::mutex panel_mutex;
+    mutable std::atomic<int8_t*>   w_panel{nullptr};   // 1x1: weights in operand order, the channels of a k-step interleaved as the depthwise layer leaves them
+    mutable std::atomic<uint32_t*> dw_blk{nullptr};    // depthwise 3x3: constants per block of 64 channels
     uint8_t* pad16    = nullptr;   // 16 bytes that turn into the padding value under the kernel's input xor
     int8_t*  w_stem   = nullptr;   // small-Ci conv on MFMA: [Co rounded up to 32][stem_kp]
     int8_t*  w_stem2  = nullptr;   // ... the second halves of weight differences that need two
     int      stem_kp  = 0;
     uint32_t* dw_grp  = nullptr;   // depthwise 3x3: constants per group of 4 channels for the fused dw+pw kernel
-    uint32_t* dw_blk  = nullptr;   // depthwise 3x3: constants per block of 64 channels for the fused kernel with the layer between in LDS
     uint32_t* w_dot4  = nullptr;   // depthwise 3x3: [C][4] dwords; small-Ci conv: [Co][Kh][RD] dwords
     uint32_t* w_dot4b = nullptr;   // depthwise 3x3 / small-Ci conv whose weight differences need two int8 halves: the second halves
     int variant = 0;               // kernel variant within an algo (see RunPlan)

@@ -13,8 +13,9 @@
  *   - tensors are dense NHWC (Convolution2d / DepthwiseConvolution2d / Pooling2d) or row-major [M,K]
  *     (FullyConnected), 8-bit quantized, exactly as the reference's workloads see them.
  *   - a "plan" owns device copies of the constant operands (weights re-laid-out for the kernel, per-channel
- *     requantization multipliers, bias, zero-point corrections).  Plans are immutable after creation and may
- *     be run concurrently on different streams.
+ *     requantization multipliers, bias, zero-point corrections).  Plans do not change after creation, but for
+ *     constants that only some launches read and the first of them builds, and may be run concurrently on different
+ *     streams and from different threads.
  *   - results equal the reference's CpuRef workloads to within 1 LSB (the accumulation is exact int32 where
  *     the reference accumulates in fp32); the requantization uses the reference's float formula.
  *

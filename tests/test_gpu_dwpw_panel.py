@@ -116,3 +116,94 @@ def test_channels_that_do_not_exist_count_for_nothing_under_a_clamp(port, n, h, 
         ref = port.conv2d(QTensor(pw.x.info, between.data), pw.w, pw.b, pw.out_info, **pw.params)
         mx, exact = lsb_diff(got, ref.data)
         assert mx <= 1 and exact >= 0.99, (mx, exact)
+
+
+def _pair(seed, n, h, c, co, **wq):
+    scales = dict(w_scale_range=(0.01, 0.02)) if wq else dict(w_scale_range=(0.01, 0.05))
+    dw = cases.make_conv_case("dw", seed, n=n, h=h, w=h, ci=c, depthwise=True, in_dtype=U8, in_scale=0.0235, in_offset=120, out_scale=0.0235,
+                              out_offset=0, act=cases.RELU6, **scales, **wq)
+    pw = cases.make_conv_case("pw", seed + 9, n=n, h=h, w=h, ci=c, co=co, kh=1, kw=1, in_dtype=U8, in_scale=0.0235, in_offset=0, out_scale=0.03,
+                              out_offset=5, **wq)
+    plans = [shim.Conv2dPlan(q.x.info, q.w, q.b, q.out_info, activation=q.act[0], act_a=q.act[1], act_b=q.act[2], **q.params) for q in (dw, pw)]
+    return dw, pw, plans
+
+
+@pytest.mark.parametrize("asked", [False, True], ids=["first_run", "after_fusion_pays"])
+def test_constants_of_the_pair_are_built_at_first_use_also_under_capture_and_from_two_threads(asked):
+    import threading
+    dev = shim.Device()
+    n, h, c, co = 3, 14, 208, 192
+    dw, pw, (first, second) = _pair(65000, n, h, c, co, w_dtype=U8, w_offset=101, per_axis=False)
+    streams = [dev.stream(), dev.stream()]
+    x = shim.DeviceBuffer(dw.x.data.nbytes).upload(dw.x.data)
+    mid, apart = shim.DeviceBuffer(dw.out_info.num_elements), shim.DeviceBuffer(pw.out_info.num_elements)
+    first.run(n, x.ptr, mid.ptr)
+    second.run(n, mid.ptr, apart.ptr)
+    dev.synchronize()
+    want = apart.download(pw.out_info.shape, numpy_dtype(U8))
+    # captured: the building does not go into the graph
+    one = shim.DeviceBuffer(pw.out_info.num_elements)
+    if asked:
+        assert first.fusion_pays(second, n)
+    dev.graph_begin(streams[0])
+    first.run_fused(second, n, x.ptr, one.ptr, streams[0])
+    assert shim.last_kernel().startswith("DwPwPanelKernel<1, ")
+    graph = dev.graph_end(streams[0])
+    for fill in (0, 255, 7):
+        shim._chk(one.lib.mi355x_fill_u8(one.ptr, fill, pw.out_info.num_elements, streams[0]))
+        dev.graph_launch(graph, streams[0])
+        np.testing.assert_array_equal(one.download(pw.out_info.shape, numpy_dtype(U8), streams[0]), want)
+    dev.graph_destroy(graph)
+    # two threads meet at the same fresh plans
+    _, _, (first, second) = _pair(65000, n, h, c, co, w_dtype=U8, w_offset=101, per_axis=False)
+    outs, errors, start = [shim.DeviceBuffer(pw.out_info.num_elements) for _ in range(2)], [], threading.Barrier(2)
+
+    def work(k):
+        try:
+            start.wait()
+            if asked:
+                first.fusion_pays(second, n)
+            first.run_fused(second, n, x.ptr, outs[k].ptr, streams[k])
+            dev.stream_sync(streams[k])
+        except Exception as e:                             # pragma: no cover
+            errors.append(e)
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+    for o in outs:
+        np.testing.assert_array_equal(o.download(pw.out_info.shape, numpy_dtype(U8)), want)
+
+
+def test_plans_hold_what_their_launches_read_and_no_more():
+    """Device memory of plans: a 1x1 layer has its weights twice where launches of few or many rows read them in operand order, a third
+    copy only once it runs behind a depthwise layer; a layer that no such launch comes from has them once."""
+    import ctypes as C
+    dev = shim.Device()
+
+    def free():
+        dev.synchronize()
+        left, total = C.c_size_t(), C.c_size_t()
+        assert dev.lib.hipMemGetInfo(C.byref(left), C.byref(total)) == 0
+        return left.value
+
+    def taken(make):
+        make(-1).destroy()                                 # (what the runtime allocates for itself at first)
+        before = free()
+        keep = [make(k) for k in range(4)]
+        used = before - free()
+        for p in keep:
+            p.destroy()
+        return used / 4
+
+    def conv(k, h, ci, co, taps):
+        c = cases.make_conv_case("memory", 66000, n=1, h=2, w=2, ci=ci, co=co, kh=taps, kw=taps, in_dtype=U8, in_offset=3, out_offset=0)
+        from armnn_amd.tensor import TensorInfo
+        xin, yout = (TensorInfo((1, h, h, n), U8, (0.0235,), 3) for n in (ci, co))
+        return shim.Conv2dPlan(xin, c.w, c.b, yout, pad_top=taps // 2, pad_left=taps // 2)
+    twice = taken(lambda k: conv(k, 28, 768, 8192, 1)) / (768 * 8192)
+    once = [taken(lambda k: conv(k, 28, 1024, 8192, 1)) / (1024 * 8192), taken(lambda k: conv(k, 224, 1024, 1024, 3)) / (9 * 1024 * 1024)]
+    print(f"times the weights: {twice:.2f}, {once}", flush=True)
+    assert twice < 2.6 and max(once) < 1.6
