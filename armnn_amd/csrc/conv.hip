@@ -1772,14 +1772,11 @@ int mi355x_conv2d_fusion_pays(mi355x_conv2d_t first, mi355x_conv2d_t second, uin
     if (!first->d.depthwise || second->d.depthwise) return 0;
     if (GlobalOptions().dwpw_stream != 0 && DwPwStreamShape(first, second) != 0 && mi355x_conv2d_fusable(first, second) == 0)
     {
-        // In items of 8 x 8 output pixels, of which a CU has four at 1024.  One launch of few items is shorter than two launches: one
-        // image of MobileNetV1 has 16 in the smallest of its four such pairs (104 -> 98 us a pass with them, four images 137 -> 123).
-        // Between 256 and 1024 items on maps of 1 to 16 of them it takes 0.65 to 1.0 of the time of the two launches (64 -> 128
-        // 0.64 to 0.77, 128 -> 128 0.65 to 0.92, 128 -> 256 0.82 to 1.0, 32 -> 64 0.84 to 1.01), but for 32 -> 64 on maps of a
-        // single item: its tiles are 16 x 16, three quarters of them outside the map (256 items 6.7 against 6.7 us, 512 7.9
-        // against 7.2, 1023 11.7 against 8.6).
+        // persistent blocks overlap items, and want a few each: 1024 items are four per CU.  One launch of few items is still shorter
+        // than two launches (MobileNetV1, its four such pairs: one image 104 -> 98 us, four images 137 -> 123 us a pass): up to one
+        // item per CU, and up to 1024 on maps of 16 tiles and more, where it was measured
         const long long tiles = static_cast<long long>((first->d.out_w + 7) / 8) * ((first->d.out_h + 7) / 8), items = batch * tiles;
-        if (items < 16 || (first->d.out_c == 32 && tiles == 1 && items > 256)) return 0;
+        if (items < 1024 && (items < 16 || (items > 256 && tiles < 16))) return 0;
         return !PanelRuns(first, second, batch) || PrepareDwPwPanel(first, second) == 0 ? 1 : 0;
     }
     if (mi355x_conv2d_fusable(first, second) != 0 || !PanelRuns(first, second, batch)) return 0;

@@ -274,7 +274,7 @@ int mi355x_conv2d_fusable(mi355x_conv2d_t first, mi355x_conv2d_t second);
 /* 1 when running the pair as one launch is what the library recommends at this batch, else 0; never an error.  Today:
  * a depthwise layer over 32, 64 (stride 2) or 128 channels and the pointwise layer behind it (64, 128, 128 or -- at stride
  * 2 -- 256 output channels), which run on the persistent kernel that keeps the pointwise weights on chip, in launches of at
- * least 16 tiles of 8 x 8 output pixels (over 32 channels not in launches of more than 256 images of one such tile); any other
+ * least 1024 tiles of 8 x 8 output pixels, of 16 to 256 such tiles, and of 16 or more on maps of at least 16 tiles; any other
  * depthwise layer of at most 512 channels and the pointwise layer behind it, which run on the kernel that keeps a tile of
  * the layer between on chip, except on maps of at most 7 x 7 pixels from 8 images (stride 2: 64) on; and, in the other order, a 1x1
  * convolution and the depthwise layer behind it on maps of at most 7 x 7 pixels in launches of at least 64 images (option
