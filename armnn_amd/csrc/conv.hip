@@ -1033,10 +1033,12 @@ int RunPlan(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, hi
                 return LaunchRowPanel(p, batch, x, y, res, res ? &t_pending_add->fuse : nullptr, stream);
             }
         }
-        // Few rows: 32 x 32 tiles whose waves split K (small_conv_kernel.h), while they number at most one and a half per CU: at
-        // 392 of them 14 x 14 x 256 at 8 images, 3 x 3, takes 8.0 us against 9.5; from there on the larger tiles' lower traffic
-        // wins (14 x 14 x 512 -> 512 at 8 images, 784 tiles: 5.5 against 4.7).  Where the layer has a weight slab (at most 128 input
-        // channels, 1x1) from 128 tiles on: 128 -> 256 at 28 x 28, 200 tiles, 5.6 -> 3.1 us.
+        // Few rows: 32 x 32 tiles whose waves split K (small_conv_kernel.h), while they number at most what 14 x 14 x 256 makes at 8
+        // images.  Tiles run in rounds of one per CU, and a round takes its time whole: 14 x 14 x 256, 3 x 3, 248 tiles 6.1 us, 344 to
+        // 496 8.5 to 8.8, 592 11.1, where the larger tiles take 9.0 to 9.3 for all of them.  So the line belongs between one round and
+        // two, and inside the second it decides little: there the small tiles take 0.94 to 0.97 of the others' time over 512 and
+        // 1024 channels, 0.6 over 72, 96 and 128, and 0.98 to 1.06 in 1x1 layers of 2048 to 4096.  Where the layer has a weight slab (at
+        // most 128 input channels, 1x1) from 128 tiles on: 128 -> 256 at 28 x 28, 200 tiles, 5.6 -> 3.1 us.
         const long long small_tiles = (rows + 31) / 32 * ((g.Co + 31) / 32);
         if (p->w_frag && p->tile_override == 0 && small_tiles <= kSmallConvMostTiles && (!p->pw_bn || small_tiles >= kSmallConvLeastSlabTiles))
         {
@@ -1774,7 +1776,8 @@ int mi355x_conv2d_fusion_pays(mi355x_conv2d_t first, mi355x_conv2d_t second, uin
     {
         // persistent blocks overlap items, and want a few each: 1024 items are four per CU.  One launch of few items is still shorter
         // than two launches (MobileNetV1, its four such pairs: one image 104 -> 98 us, four images 137 -> 123 us a pass): up to one
-        // item per CU, and up to 1024 on maps of 16 tiles and more, where it was measured
+        // item per CU, and up to 1024 on maps of 16 tiles and more.  (On smaller maps two launches are kept between 257 and 1023 items,
+        // where one takes 0.64 to 1.0 of their time in three of the shapes and up to 1.35 in 32 -> 64 over maps of one tile.)
         const long long tiles = static_cast<long long>((first->d.out_w + 7) / 8) * ((first->d.out_h + 7) / 8), items = batch * tiles;
         if (items < 1024 && (items < 16 || (items > 256 && tiles < 16))) return 0;
         return !PanelRuns(first, second, batch) || PrepareDwPwPanel(first, second) == 0 ? 1 : 0;
