@@ -15,8 +15,9 @@
 //     1 KB; 55 bytes a clock and CU were measured for that, 14 to 20 for 128-byte rows through LDS with a wait per k-tile), the
 //     first k-steps requested ahead of the depthwise phase.  No barrier inside: two after the halo, two around the write-out.
 //   * The outputs meet in LDS and leave as 16 bytes per lane.
-// At many tiles VALU work bounds it, most of that the requantization of both layers (25 instructions per four values); at few,
-// the chain of round trips.  Times against the kernel with a k-tile loop it replaces (64 images | 256): 14 x 14 x 512 -> 512
+// At many tiles VALU work is the largest share, most of it the requantization of both layers (25 instructions per four values): 14 x 14 x
+// 512, 64 images, 12 k of a SIMD's 27 k cycles issue VALU and 5.6 k matrix instructions, the rest of a wave's life is waits, at barriers
+// and for the weights (82 MB through the CUs' L1s).  At few tiles it is the chain of round trips.  Times against the kernel with a k-tile loop it replaces (64 images | 256): 14 x 14 x 512 -> 512
 // 15.4 -> 12.8 | 54.2 -> 35.7 us, 28 x 28 x 256 -> 256 20.2 -> 17.7 | 68.9 -> 61.3, 28 x 28 x 256 -> 14 x 14 x 512 11.2 -> 10.7 | 43.1 ->
 // 34.8; against two launches, one image | eight: 14 x 14 x 512 7.6 -> 5.5 | 9.3 -> 7.5, 28 x 28 x 256 7.2 -> 4.6 | 8.6 -> 6.3.
 // Both layers' arithmetic is untouched -- exact int32 sums, the same requantization routine with the same constants -- so the

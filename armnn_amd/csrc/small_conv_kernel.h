@@ -8,9 +8,10 @@
 //     its way after a quarter as many round trips and no LDS staging or barrier lies in between;
 //   * the partial tiles meet in LDS, where the waves add them up in a fixed order, requantize four channels per lane, and
 //     one wave writes the tile in 16-byte pieces (with a following Addition on the way, if there is one).
-// What bounds it then is the CU's address unit, which takes an instruction's cache lines one after the other: hence
-// v_mfma_i32_16x16x64_i8, whose activation operand is 16 pixels x 64 contiguous bytes (32x32x32: 32 pixels x 32), and weights
-// stored in operand order (PackFragKernel), so that a wave's weight load is one run of 1 KB instead of 32 rows.
+// What is left is latency: waves wait 63 % of their cycles (3 x 3 over 14 x 14 x 256, one image), and of the 14 k cycles of a block the
+// CU's address unit, which takes an instruction's cache lines one after the other, is busy for 4.3 k.  Hence v_mfma_i32_16x16x64_i8,
+// whose activation operand is 16 pixels x 64 contiguous bytes (32x32x32: 32 pixels x 32), and weights stored in operand order
+// (PackFragKernel), so that a wave's weight load is one run of 1 KB instead of 32 rows.
 // Launches back to back, before -> here (one image unless said): 3 x 3 over 28 x 28 x 128 7.2 -> 4.5 us, 14 x 14 x 256 9.1 ->
 // 5.5, 7 x 7 x 512 13.3 -> 7.4, 56 x 56 x 64 5.9 -> 3.7, 28 x 28 x 96 7.2 -> 3.8; 1 x 1 over 14 x 14 x 1024 -> 256 5.7 -> 4.0, 28 x 28 x
 // 128 -> 256 5.6 -> 3.1; FullyConnected 4096 -> 4096 of 64 rows 12.9 -> 9.6.  An empty kernel takes 2.75 us in such a row.

@@ -191,6 +191,43 @@ def test_the_measured_choice_between_launching_and_replaying_changes_no_byte(whi
     dn.close()
 
 
+def test_two_threads_pass_host_arrays_through_the_shared_pinned_blocks():
+    """Two networks in two threads, each call in more than half as many parts as the largest may have, so that both together take more blocks
+    than one call; the bytes are those of one call at a time, and all blocks are given back."""
+    import threading
+
+    nets_ = [nets.mobilenet_v1(resolution=224, width=0.25, classes=20) for _ in range(2)]
+    batch = 256                                            # 38.5 MB of images: 19 parts of 2 MB
+    dns = [DeviceNetwork(n, batch, fuse="auto") for n in nets_]
+    inputs = [nets.synthetic_input(n, batch, seed=90 + k) for k, n in enumerate(nets_)]
+    want = []
+    for dn, x in zip(dns, inputs):
+        dn.upload_input(x)
+        dn.enqueue()
+        want.append(dn.download().data.copy())
+    errors, start, before = [], threading.Barrier(2), len(DeviceNetwork._blocks)
+
+    def work(k):
+        try:
+            start.wait()
+            for _ in range(4):
+                np.testing.assert_array_equal(dns[k].run(inputs[k]).data, want[k])
+        except Exception as e:                             # pragma: no cover
+            errors.append(e)
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+    assert 20 <= len(DeviceNetwork._blocks) <= max(before, 40)
+    assert len(set(DeviceNetwork._blocks)) == len(DeviceNetwork._blocks)
+    others = len(DeviceNetwork._open) - 2
+    for dn in dns:
+        dn.close()
+    assert len(DeviceNetwork._blocks) <= 33 * others
+
+
 def test_two_networks_in_lanes_give_the_same_bytes_in_turn_and_apart():
     """A pass runs as one lane while another network's is under way, in its lanes otherwise; the bytes are the eager launches'."""
     net = nets.resnet50(resolution=64)
