@@ -32,7 +32,7 @@ constexpr int BigGemmSmemBytes()
 {
     constexpr int stages = ST * (BM + BN) * 128;
     constexpr int out = BM * (BN + 16);
-    return (stages > out ? stages : out) + 4 * BN * 4;       // + the block's slice of the per-channel table
+    return (stages > out ? stages : out) + 2 * BN * 4;       // + the block's slice of the per-channel table
 }
 
 // 2 x 2 waves, wave tile (BM / 2) x (BN / 2).  Needs Ci % 128 == 0 (a k-tile is 128 bytes of one filter tap) and
@@ -162,7 +162,7 @@ __global__ __launch_bounds__(256) void BigGemmKernel(IgemmArgs a, int xcd_rows)
             __builtin_amdgcn_global_load_lds((GlobalPtr)(wk + j * wstep + ((j & 1) ? lchunk_odd : lchunk_even) * 16), (LdsPtr)(Bs + j * 8 * BK), 16, 0, 0);
     };
 
-    // ---- accumulators start at the zero-point correction
+    // ---- accumulators start from the plan's constants (zero-point correction, Requant::acc_base)
     const int lane_c = 4 * (lane >> 5);
     const int cbase = tn * BN + wn * WTN;
     v16i acc[TC][TP];
@@ -252,13 +252,13 @@ __global__ __launch_bounds__(256) void BigGemmKernel(IgemmArgs a, int xcd_rows)
     constexpr int LAST = (KS - 1) & 1;           // fragment buffer of a tile's last k-step
     constexpr int PRE = NM / 4;                  // MFMAs of the last k-step issued ahead of the barrier
 
-    // ---- the block's slice of the per-channel table (rows 2 .. 5: the fast path's bracket, BN channels) goes to LDS behind
+    // ---- the block's slice of the per-channel table (rows 2 and 3, BN channels) goes to LDS behind
     // the stages: with one wave per SIMD nothing would hide the epilogue's table reads from global memory, one round trip
     // per channel quad.  The rare exact path reads its two rows from global memory.
     constexpr int TAB = (ST * STAGE > BM * LDO ? ST * STAGE : BM * LDO);
     float* tab_lds = reinterpret_cast<float*>(smem + TAB);
     {
-        constexpr int N4 = 4 * BN / 4;                     // float4 pieces
+        constexpr int N4 = 2 * BN / 4;                     // float4 pieces
         v4i piece[(N4 + 255) / 256];
 #pragma unroll
         for (int i = 0; i < (N4 + 255) / 256; ++i)
@@ -355,6 +355,7 @@ __global__ __launch_bounds__(256) void BigGemmKernel(IgemmArgs a, int xcd_rows)
 #pragma unroll
         for (int tp = 0; tp < TP; ++tp) rowsum[tp] = (rowsum[tp] + __shfl_xor(rowsum[tp], 32) - a.rowsum_bias) * a.zw_neg;
     }
+    WithBits(a.rq, [&](auto bits) {
 #pragma unroll
     for (int tc = 0; tc < TC; ++tc)
     {
@@ -362,21 +363,17 @@ __global__ __launch_bounds__(256) void BigGemmKernel(IgemmArgs a, int xcd_rows)
         for (int q = 0; q < 4; ++q)
         {
             const int cl = wn * WTN + tc * 32 + 8 * q + lane_c;
-            const float4 mp = *reinterpret_cast<const float4*>(tab_lds + 0 * BN + cl);
-            const float4 bp = *reinterpret_cast<const float4*>(tab_lds + 1 * BN + cl);
-            const float4 mm = *reinterpret_cast<const float4*>(tab_lds + 2 * BN + cl);
-            const float4 bm = *reinterpret_cast<const float4*>(tab_lds + 3 * BN + cl);
+            const Fast4 f4 = {*reinterpret_cast<const float4*>(tab_lds + cl), *reinterpret_cast<const float4*>(tab_lds + BN + cl)};
+            v4i v[TP];
+            uint32_t out[TP];
 #pragma unroll
-            for (int tp = 0; tp < TP; ++tp)
-            {
-                const v16i& c = acc[tc][tp];
-                const int rt = AW ? rowsum[tp] : 0;
-                const uint32_t out = Requant4Dev(c[4 * q + 0] + rt, c[4 * q + 1] + rt, c[4 * q + 2] + rt, c[4 * q + 3] + rt, mp, bp, mm, bm, a.ct, nullptr, tn * BN + cl, a.rq);
-                const int pl = wm * WTM + tp * 32 + (lane & 31);
-                *reinterpret_cast<uint32_t*>(Os + pl * LDO + cl) = out;
-            }
+            for (int tp = 0; tp < TP; ++tp) v[tp] = Quad(acc[tc][tp], q) + (AW ? rowsum[tp] : 0);
+            RequantPixels<decltype(bits)::value, TP>(v, out, f4, a.ct, tn * BN + cl, a.rq);
+#pragma unroll
+            for (int tp = 0; tp < TP; ++tp) *reinterpret_cast<uint32_t*>(Os + (wm * WTM + tp * 32 + (lane & 31)) * LDO + cl) = out[tp];
         }
     }
+    });
     __syncthreads();
     constexpr int CHUNKS = BN / 16;
     constexpr int ROWS_PER_PASS = 256 / CHUNKS;

@@ -69,6 +69,13 @@ int32_t QuantizeHost(float value, float scale, int32_t offset, int32_t dtype);
 // q2 = clamp(q1, Quantize(b), Quantize(a)) for BoundedReLu, clamp(q1, Quantize(0), type max) for ReLu.
 void ActivationClamp(int32_t activation, float a, float b, const mi355x_quant& out, int32_t* lo, int32_t* hi);
 
+// dwords per group of 4 channels of a 3x3 depthwise plan's grouped constants: six rows of four
+constexpr int kDwGrpDwords = 24;
+
+// 1.5 * 2^23 as a float: the bits of this plus a small integer are the float 1.5 * 2^23 + that integer
+constexpr int32_t kAccBaseBits = 0x4b400000;
+constexpr float kAccBaseValue = 12582912.0f;
+
 // Parameters of the shared requantization epilogue
 struct Requant
 {
@@ -84,13 +91,16 @@ struct Requant
     float   inv_scale;
     float   act_lo_f, act_hi_f;
     int32_t fast_ok;
-    // Convolution / FullyConnected epilogue: codes are produced as unsigned bytes with v_cvt_pk_u8_f32 (converts,
-    // saturates to 0..255 and packs in one instruction).  Signed outputs are computed 128 higher (pk_bias is folded into
-    // the per-channel constant fb on the host) and the finished dword is xor-ed with 0x80808080.
+    // Codes are produced as unsigned bytes by saturating conversions.  Signed outputs are computed 128 higher (pk_bias is folded
+    // into the constants on the host) and the finished dword is xor-ed with 0x80808080.
     int32_t  pk_bias;       // 128 for QAsymmS8 outputs, 0 for QAsymmU8
     uint32_t pk_xor;        // 0x80808080 or 0
     float    pk_lo_f, pk_hi_f;   // activation clamp in the biased domain
     int32_t  pk_full;       // the clamp is 0..255: the instruction's own saturation does it
+    // Convolution / FullyConnected epilogue (device_math.h), per plan
+    float    two_c;              // width of the bracket
+    int32_t  acc_base;           // kAccBaseBits where the bits of an accumulator are a float, else 0: sums are raised by this much
+    uint32_t pk_lo2, pk_hi2;     // the clamp, for two codes at a time in 16 bits each
 };
 
 Requant MakeRequant(const mi355x_quant& out, int32_t activation, float a, float b);

@@ -37,13 +37,10 @@ struct PendingAdd
 };
 thread_local PendingAdd* t_pending_add = nullptr;
 
-// unit roundoff of fp32 and the relative half-width of the requantization bracket (device_math.h)
-constexpr double kBracketUnit = 1.0 / 16777216.0;
-constexpr double kBracketRel = 16.0 / 16777216.0;
 constexpr long long kSmallConvMostTiles = 392, kSmallConvLeastSlabTiles = 128;
 constexpr int kRowPanelMostChannels = 768;
 
-void FoldCorrIntoTable(mi355x_conv2d_s* p, const std::vector<int32_t>& corr, int Co);
+void FinishTable(mi355x_conv2d_s* p, std::vector<int32_t>& corr);
 void ChoosePointwiseConfig(mi355x_conv2d_s* p);
 int PreparePointwise(mi355x_conv2d_s* p);
 
@@ -131,7 +128,8 @@ int BuildPlan(const mi355x_conv2d_desc& d, const void* weights_host, const mi355
             const int wv = g.w_u8 ? static_cast<int>(wb[i]) : static_cast<int>(static_cast<int8_t>(wb[i]));
             wmax = std::max<long long>(wmax, std::abs(wv - g.zw));
         }
-        if (static_cast<long long>(p->K) * xmax * wmax >= (1ll << 31))
+        p->acc_most = static_cast<long long>(p->K) * xmax * wmax;
+        if (p->acc_most >= (1ll << 31))
             return SetError(MI355X_ERR_UNSUPPORTED, "%d taps of up to %lld x %lld could overflow the 32-bit accumulator", p->K, xmax, wmax);
     }
     p->Co_pad = (Co + 127) / 128 * 128;
@@ -171,49 +169,9 @@ int BuildPlan(const mi355x_conv2d_desc& d, const void* weights_host, const mi355
             }
         }
     }
-    // fast-path coefficients: the bracket r- < f / s_out + offset' < r+ of device_math.h, one FMA per side.  A channel
-    // whose constants do not qualify gets a bracket that never closes (bytes 255 and 0), so it always takes the exact path.
-    {
-        const int CP = p->Co_pad;
-        std::vector<float> tab(static_cast<size_t>(8) * CP, 0.0f);
-        const float inv = 1.0f / d.output.scale;
-        // the fast path works 128 codes higher for signed outputs (Requant::pk_bias), so that is its offset
-        const float zp_f = static_cast<float>(d.output.offset + (d.output.dtype == MI355X_QASYMM_U8 ? 0 : 128));
-        const double max_acc = static_cast<double>(p->K) * 65025.0;
-        const bool base_ok = !GlobalOptions().exact_division_epilogue && std::isnormal(inv) && std::isnormal(d.output.scale) &&
-                             d.output.offset >= -255 && d.output.offset <= 255 && p->rq.fast_ok;
-        p->fast_fm.assign(CP, 0.0f);
-        p->fast_fb.assign(CP, 0.0f);
-        p->fast_cw.assign(CP, -1.0);
-        for (int c = 0; c < CP; ++c)
-        {
-            tab[c] = mult[c];
-            tab[CP + c] = biasf[c];
-            if (c >= Co) continue;                    // padding: both sides give byte 0, nothing is ever redone or stored
-            tab[3 * CP + c] = tab[6 * CP + c] = 255.0f;
-            if (!base_ok) continue;
-            const float fm = mult[c] * inv;
-            const float fb = biasf[c] * inv + zp_f;
-            const double bq = std::fabs(static_cast<double>(biasf[c])) * inv;
-            // constant half-width (device_math.h): 1.5 * 2^-24 * (14 |biasf/s_out| + 10 |offset'| + 64) + 2 e; the part
-            // proportional to the value is the factor 1 +- e on both constants
-            const double cw = 1.5 * kBracketUnit * (14.0 * bq + 10.0 * std::fabs(static_cast<double>(zp_f)) + 64.0) + 2.0 * kBracketRel;
-            const bool ok = std::isfinite(fm) && std::isfinite(fb) && std::isfinite(cw) && cw < 0.125 &&
-                            max_acc * std::fabs(static_cast<double>(fm)) < 268435456.0;
-            if (!ok) continue;
-            tab[2 * CP + c] = static_cast<float>(static_cast<double>(fm) * (1.0 + kBracketRel));
-            tab[3 * CP + c] = static_cast<float>(static_cast<double>(fb) * (1.0 + kBracketRel) + cw);
-            tab[4 * CP + c] = static_cast<float>(static_cast<double>(fm) * (1.0 - kBracketRel));
-            tab[5 * CP + c] = static_cast<float>(static_cast<double>(fb) * (1.0 - kBracketRel) - cw);
-            // until a kernel folds its zero-point correction in, rows 6/7 never close either
-            tab[6 * CP + c] = 255.0f;
-            tab[7 * CP + c] = 0.0f;
-            p->fast_fm[c] = fm;
-            p->fast_fb[c] = fb;
-            p->fast_cw[c] = cw;
-        }
-        p->chan_host = tab;
-    }
+    p->chan_host.assign(static_cast<size_t>(4) * p->Co_pad, 0.0f);
+    std::copy(mult.begin(), mult.end(), p->chan_host.begin());
+    std::copy(biasf.begin(), biasf.end(), p->chan_host.begin() + p->Co_pad);
 
     // ---- kernel selection ----------------------------------------------------------------------------------
     const int zx_shift = g.in_u8 ? g.zx - 128 : g.zx;
@@ -302,6 +260,7 @@ int BuildPlan(const mi355x_conv2d_desc& d, const void* weights_host, const mi355
         }
         p->zw_neg = -zw_shift;
         p->rowsum_bias = (p->K_pad - p->K) * zx_shift;     // kernels that walk K_pad bytes meet zx' beyond K
+        FinishTable(p, corr);
         if (int rc = Upload(reinterpret_cast<void**>(&p->w_mfma), wp.data(), wp.size())) return rc;
         if (int rc = Upload(reinterpret_cast<void**>(&p->corr), corr.data(), corr.size() * sizeof(int32_t))) return rc;
         p->xor_mask = g.in_u8 ? 0x80808080u : 0u;
@@ -316,7 +275,6 @@ int BuildPlan(const mi355x_conv2d_desc& d, const void* weights_host, const mi355
             if (int rc = PackFragments(p, false, &p->w_frag)) return rc;
         if (p->bk128 && (Ci % 128) == 0)
             if (int rc = PrepareBigGemm()) return rc;
-        FoldCorrIntoTable(p, corr, Co);
         ChoosePointwiseConfig(p);
         if (p->tile_override != 0) p->pw_bn = 0;     // a forced tile also forces the LDS-tiled implicit GEMM
         if (int rc = PreparePointwise(p)) return rc;
@@ -358,6 +316,7 @@ int BuildPlan(const mi355x_conv2d_desc& d, const void* weights_host, const mi355
             }
             corr[c] = static_cast<int32_t>(-static_cast<long long>(zx_shift) * sum);
         }
+        FinishTable(p, corr);
         if (int rc = Upload(reinterpret_cast<void**>(&p->w_dot4), wp.data(), wp.size() * sizeof(uint32_t))) return rc;
         if (!dw3_fits)
             if (int rc = Upload(reinterpret_cast<void**>(&p->w_dot4b), wp2.data(), wp2.size() * sizeof(uint32_t))) return rc;
@@ -367,15 +326,15 @@ int BuildPlan(const mi355x_conv2d_desc& d, const void* weights_host, const mi355
         p->pad_word = zb | (zb << 8) | (zb << 16) | (zb << 24);
         p->variant = 1;
         {
-            // [C/4][8][4] dwords: weight rows 0..2, corr, m+, b+, m-, b- (rows 2..5 of the channel table)
+            // [C/4][6][4] dwords: weight rows 0..2, corr, m, b (rows 2 and 3 of the channel table)
             const int CP = p->Co_pad;
-            std::vector<uint32_t> grp(static_cast<size_t>(Co / 4) * 32, 0u);
+            std::vector<uint32_t> grp(static_cast<size_t>(Co / 4) * kDwGrpDwords, 0u);
             for (int c = 0; c < Co; ++c)
             {
-                uint32_t* gdst = grp.data() + static_cast<size_t>(c / 4) * 32 + (c % 4);
+                uint32_t* gdst = grp.data() + static_cast<size_t>(c / 4) * kDwGrpDwords + (c % 4);
                 for (int r = 0; r < 3; ++r) gdst[r * 4] = wp[static_cast<size_t>(c) * 4 + r];
                 gdst[3 * 4] = static_cast<uint32_t>(corr[c]);
-                for (int r = 0; r < 4; ++r) std::memcpy(&gdst[(4 + r) * 4], &p->chan_host[static_cast<size_t>(2 + r) * CP + c], 4);
+                for (int r = 0; r < 2; ++r) std::memcpy(&gdst[(4 + r) * 4], &p->chan_host[static_cast<size_t>(2 + r) * CP + c], 4);
             }
             if (int rc = Upload(reinterpret_cast<void**>(&p->dw_grp), grp.data(), grp.size() * sizeof(uint32_t))) return rc;
             const std::vector<uint8_t> padbytes(16, static_cast<uint8_t>((zb ^ (g.in_u8 ? 0x80u : 0u)) & 0xffu));
@@ -398,6 +357,8 @@ int BuildPlan(const mi355x_conv2d_desc& d, const void* weights_host, const mi355
     }
     else if (algo == MI355X_ALGO_DEPTHWISE)
     {
+        std::vector<int32_t> none;
+        FinishTable(p, none);
         if (int rc = Upload(reinterpret_cast<void**>(&p->w_direct), wsrc, static_cast<size_t>(Kh) * Kw * Co)) return rc;
         p->info = "depthwise_c4_valu";
     }
@@ -423,6 +384,7 @@ int BuildPlan(const mi355x_conv2d_desc& d, const void* weights_host, const mi355
                 }
             corr[c] = static_cast<int32_t>(-static_cast<long long>(zx_shift) * sum);
         }
+        FinishTable(p, corr);
         if (int rc = Upload(reinterpret_cast<void**>(&p->w_dot4), wp.data(), wp.size() * sizeof(uint32_t))) return rc;
         if (!stem_fits)
             if (int rc = Upload(reinterpret_cast<void**>(&p->w_dot4b), wp2.data(), wp2.size() * sizeof(uint32_t))) return rc;
@@ -450,7 +412,6 @@ int BuildPlan(const mi355x_conv2d_desc& d, const void* weights_host, const mi355
             }
             p->stem_kp = kp;
         }
-        FoldCorrIntoTable(p, corr, Co);
         char buf[96];
         snprintf(buf, sizeof(buf), "smallci_dot4_lds %dx%dx%d stride %u, tile 32x16", Kh, Kw, Ci, d.stride_x);
         p->info = buf;
@@ -458,6 +419,8 @@ int BuildPlan(const mi355x_conv2d_desc& d, const void* weights_host, const mi355
     }
     else
     {
+        std::vector<int32_t> none;
+        FinishTable(p, none);
         if (d.depthwise)
         {
             if (int rc = Upload(reinterpret_cast<void**>(&p->w_direct), wsrc, static_cast<size_t>(Kh) * Kw * Co)) return rc;
@@ -476,30 +439,53 @@ int BuildPlan(const mi355x_conv2d_desc& d, const void* weights_host, const mi355
     if (int rc = Upload(reinterpret_cast<void**>(&p->chan), p->chan_host.data(), p->chan_host.size() * sizeof(float))) return rc;
     p->chan_host.clear();
     p->chan_host.shrink_to_fit();
-    p->fast_fm = std::vector<float>();
-    p->fast_fb = std::vector<float>();
-    p->fast_cw = std::vector<double>();
     return 0;
 }
 
-// Rows 6/7 of the channel table: the bracket with the zero-point correction folded in,
-//   bc+- = (fb + corr * fm) (1 +- e) +- (c + 1.5 * 2^-24 * 5 |corr * fm|)
-// (the accumulator then starts at zero and only the rare exact path adds corr as an integer; the wider constant covers
-// the roundings of corr * fm and of the two conversions of an accumulator beyond 2^24).
-void FoldCorrIntoTable(mi355x_conv2d_s* p, const std::vector<int32_t>& corr, int Co)
+// Rows 2 and 3 of the channel table, Requant::two_c and Requant::acc_base; `corr` (may be empty), the zero-point correction, becomes
+// what accumulators of raw products start from.  What the bracket encloses is told in device_math.h.
+void FinishTable(mi355x_conv2d_s* p, std::vector<int32_t>& corr)
 {
-    const int CP = p->Co_pad;
+    constexpr double u = 1.0 / 16777216.0;            // unit roundoff of fp32
+    constexpr double unit = 256.0 / 65535.0;          // a code on the scale of m and b
+    constexpr double whole = 1 << 22;                 // 1.5 * 2^23 + sum steps in ones up to here
+    const mi355x_conv2d_desc& d = p->d;
+    const int CP = p->Co_pad, Co = static_cast<int>(d.out_c);
     std::vector<float>& tab = p->chan_host;
-    for (int c = 0; c < Co && c < static_cast<int>(p->fast_cw.size()); ++c)
+    const double s_out = d.output.scale;
+    // the fast path works 128 codes higher for signed outputs (Requant::pk_bias), so that is its offset
+    const double zp = d.output.offset + p->rq.pk_bias;
+    // |t - offset'| of a value that is not saturated
+    const double most_t = std::max(std::fabs(257.5 - zp), std::fabs(-1.5 - zp));
+    std::vector<uint8_t> fast(Co, 0);
+    bool bits = p->acc_most < (1ll << 29);
+    double c_codes = 1024.0 * u;                      // (enough to tell p from q anywhere)
+    for (int c = 0; c < Co; ++c)
     {
-        if (p->fast_cw[c] < 0.0) continue;            // fast path disabled for this channel
-        const double cq = static_cast<double>(corr[c]) * static_cast<double>(p->fast_fm[c]);
-        const double fbc = static_cast<double>(p->fast_fb[c]) + cq;
-        const double cw = p->fast_cw[c] + 1.5 * kBracketUnit * 5.0 * std::fabs(cq);
-        if (!std::isfinite(fbc) || !(cw < 0.125) || std::fabs(static_cast<double>(corr[c])) >= 16777216.0) continue;
-        tab[6 * CP + c] = static_cast<float>(fbc * (1.0 + kBracketRel) + cw);
-        tab[7 * CP + c] = static_cast<float>(fbc * (1.0 - kBracketRel) - cw);
+        const double fm = static_cast<double>(tab[c]) / s_out, fb = static_cast<double>(tab[CP + c]) / s_out, bias = std::fabs(fb);
+        // Half-width in codes: the reference converts the sum (sums beyond 2^24 round), multiplies, adds the bias and divides, the first
+        // two on values of up to |t| + |bias| codes, the others of up to |t|; here a conversion and m round |t| + |bias|, b rounds
+        // |bias| + |offset'| + 1, and p and q round on a scale where 256 codes are 1 (128 each).  1.05 for the second order.
+        const double w = 1.05 * u * (2.0 * (most_t + bias) + 2.0 * most_t + 2.0 * (most_t + bias) + bias + std::fabs(zp) + 1.0 + 256.0);
+        fast[c] = p->rq.fast_ok != 0 && std::isfinite(fm) && std::isfinite(fb) && (fm == 0.0 || (std::isnormal(tab[c]) && std::isnormal(static_cast<float>(fm * unit)))) &&
+                  w < 0.0625 && static_cast<double>(p->acc_most) * std::fabs(fm) < 268435456.0;
+        if (!fast[c]) continue;
+        c_codes = std::max(c_codes, w);
+        // where the steps are not ones, codes must be saturated
+        if (static_cast<double>(p->acc_most) > whole && whole * std::fabs(fm) - std::fabs(fb + zp) < 300.0) bits = false;
     }
+    const double c_x = c_codes * unit;
+    for (int c = 0; c < Co; ++c)
+    {
+        const double fm = static_cast<double>(tab[c]) / s_out, fb = static_cast<double>(tab[CP + c]) / s_out;
+        // (a channel without a fast path: a byte's edge whatever the sum, p gives 128 and q 127)
+        const double code = fast[c] ? fb + zp + 0.5 : 128.0;
+        tab[2 * CP + c] = fast[c] ? static_cast<float>(fm * unit) : 0.0f;
+        tab[3 * CP + c] = static_cast<float>((256.0 * code - 0.5) / 65535.0 + c_x);
+    }
+    p->rq.two_c = std::nextafterf(static_cast<float>(2.0 * c_x), 1.0f);
+    p->rq.acc_base = bits ? kAccBaseBits : 0;
+    for (int32_t& v : corr) v += p->rq.acc_base;
 }
 
 // Configuration of the weight-stationary pointwise GEMM kernel, or bn == 0 when it does not apply.

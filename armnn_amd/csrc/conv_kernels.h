@@ -17,9 +17,6 @@
 namespace mi355x
 {
 
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v16i __attribute__((ext_vector_type(16)));
-
 struct ConvGeom
 {
     int H, W, Ci, Ho, Wo, Co;
@@ -82,7 +79,7 @@ __global__ __launch_bounds__(256) void ConvDirectKernel(ConvGeom g, Requant rq, 
             }
         }
     }
-    y[idx] = static_cast<uint8_t>(Requant1Dev(acc, ct, co, rq));
+    y[idx] = static_cast<uint8_t>(Requant1Dev(acc + rq.acc_base, ct, co, rq));
 }
 
 // ---------------------------------------------------------------------------------------------------------
@@ -134,7 +131,8 @@ __global__ __launch_bounds__(256) void DepthwiseC4Kernel(ConvGeom g, Requant rq,
         }
     }
     const Fast4 f4 = LoadFast4(ct, c);
-    *reinterpret_cast<uint32_t*>(y + idx * 4) = Requant4Dev(acc[0], acc[1], acc[2], acc[3], f4, ct, c, rq);
+    const int base = rq.acc_base;
+    *reinterpret_cast<uint32_t*>(y + idx * 4) = Requant4Any(acc[0] + base, acc[1] + base, acc[2] + base, acc[3] + base, f4, ct, c, rq);
 }
 
 // ---------------------------------------------------------------------------------------------------------
@@ -418,7 +416,7 @@ __global__ __launch_bounds__(256) void IgemmKernel(IgemmArgs a)
         for (int j = 0; j < RB; ++j) *reinterpret_cast<v4i*>(Bs + (lr + RP * j) * LDK + lc * 16) = rb[SL][j];
     };
 
-    // ---- accumulators, initialised with the zero-point correction -------------------------------------
+    // ---- accumulators start from the plan's constants (zero-point correction, Requant::acc_base) -------------------------------------
     // lane owns pixel (lane & 31) of each pixel sub-tile and channels 8*(v/4) + 4*(lane/32) + v%4 of each
     // channel sub-tile.
     const int lane_c = 4 * (lane >> 5);
@@ -509,6 +507,7 @@ __global__ __launch_bounds__(256) void IgemmKernel(IgemmArgs a)
 #pragma unroll
         for (int tp = 0; tp < TP; ++tp) rowsum[tp] = (rowsum[tp] + __shfl_xor(rowsum[tp], 32) - a.rowsum_bias) * a.zw_neg;
     }
+    WithBits(a.rq, [&](auto bits) {
 #pragma unroll
     for (int tc = 0; tc < TC; ++tc)
     {
@@ -517,17 +516,16 @@ __global__ __launch_bounds__(256) void IgemmKernel(IgemmArgs a)
         {
             const int cl = wn * WTN + tc * 32 + 8 * q + lane_c;           // channel within the block tile
             const Fast4 f4 = LoadFast4(a.ct, tn * BN + cl);
+            v4i v[TP];
+            uint32_t out[TP];
 #pragma unroll
-            for (int tp = 0; tp < TP; ++tp)
-            {
-                const v16i& c = acc[tc][tp];
-                const int rt = AW ? rowsum[tp] : 0;
-                const uint32_t out = Requant4Dev(c[4 * q + 0] + rt, c[4 * q + 1] + rt, c[4 * q + 2] + rt, c[4 * q + 3] + rt, f4, a.ct, tn * BN + cl, a.rq);
-                const int pl = wm * WTM + tp * 32 + (lane & 31);          // pixel within the block tile
-                *reinterpret_cast<uint32_t*>(Os + pl * LDO + cl) = out;
-            }
+            for (int tp = 0; tp < TP; ++tp) v[tp] = Quad(acc[tc][tp], q) + (AW ? rowsum[tp] : 0);
+            RequantPixels<decltype(bits)::value, TP>(v, out, f4, a.ct, tn * BN + cl, a.rq);
+#pragma unroll
+            for (int tp = 0; tp < TP; ++tp) *reinterpret_cast<uint32_t*>(Os + (wm * WTM + tp * 32 + (lane & 31)) * LDO + cl) = out[tp];
         }
     }
+    });
     __syncthreads();
 
     // ---- coalesced write-out ----------------------------------------------------------------------------

@@ -4,11 +4,15 @@
 #include <hip/hip_runtime.h>
 
 #include <cmath>
+#include <type_traits>
 
 #include "common.h"
 
 namespace mi355x
 {
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v16i __attribute__((ext_vector_type(16)));
 
 // float value -> output code, exactly armnn::Quantize (src/armnn/TypesUtils.cpp:29-45):
 //   clamp(float(offset) + round(value / scale), lowest, max), round = half away from zero, fp32 division,
@@ -33,35 +37,46 @@ __device__ __forceinline__ int RequantExactDev(int acc, float mult, float biasf,
     return QuantizeDev(__fadd_rn(__fmul_rn(static_cast<float>(acc), mult), biasf), rq);
 }
 
-// Per-channel constants, eight rows of `stride` floats, built on the host (conv.hip):
+// Per-channel constants, four rows of `stride` floats, built on the host (conv.hip, FinishTable):
 //   row 0 mult   s_in * s_w[c]                      row 1 biasf  float(bias[c]) * s_b[c]
-//   rows 2..5    m+, b+, m-, b-   the bracket of the fast path (below); b carries offset' = offset + Requant::pk_bias
-//                                 (codes as unsigned bytes)
-//   rows 6, 7    bc+, bc-         b+ and b- with corr * m+ / corr * m- added
-// Rows 6/7 serve kernels whose accumulators start at zero: the zero-point correction corr[c] is then part of the
-// fast-path constants, and only the exact path adds it to the accumulator as an integer.
+//   row 2 m, row 3 b   the fast path (below)
+// A kernel's accumulators start from the plan's `corr` array (or get it added before the requantization): the zero-point
+// correction of a sum of raw products, raised by Requant::acc_base.
 struct ChanTab
 {
     const float* p;
     int stride;
 };
 
+// four accumulators of a 32 x 32 result: channels 8 q + 4 (lane / 32) + 0 .. 3
+__device__ __forceinline__ v4i Quad(const v16i& v, int q)
+{
+    return v4i{v[4 * q + 0], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+}
+
 // Fast path with an exact fallback.
-//   With rho = float(acc) * fm + fb in real arithmetic (fm = fl(mult * fl(1/s_out)), fb = fl(fl(biasf * fl(1/s_out)) + offset'))
-//   and t = fl(f / s_out) + offset' the reference's value before rounding (f = fl(fl(float(acc) * mult) + biasf)), counting
-//   every rounding on both sides (three in the reference, five in the constants) gives
-//       |t - rho|  <=  2^-24 * (5 |rho| + 10 |biasf / s_out| + 6 |offset'|),
-//   two more |rho| where a kernel converts an accumulator beyond 2^24 without its zero-point correction.
-//   The host widens that to a bracket r- < t < r+ that costs one FMA per side,
-//       r+ = fma(float(acc), m+, b+),   m+ = fm (1 + e),  b+ = fb (1 + e) + c
-//       r- = fma(float(acc), m-, b-),   m- = fm (1 - e),  b- = fb (1 - e) - c
-//   with e = 16 * 2^-24 and c a per-channel constant that also covers the roundings of m+-, b+- and of the FMA itself
-//   (conv.hip, 1.5x margin on every term; valid while -1 <= rho <= 257, and beyond that range both sides saturate).
-//   v_cvt_pk_u8_f32 rounds to nearest (ties to even) and saturates to 0..255, both monotone, so when r- and r+ convert
-//   to the same byte, t -- strictly between them -- rounds to that byte under any tie rule, the reference's half-away-
-//   from-zero included.  Values whose two bytes differ (about two in 10^4: r lies that close to a half-integer) are
-//   recomputed with the reference's own sequence.  A channel without a fast path has m+ = m- = 0, b+ = 255, b- = 0.
-//   The activation's clamp, where it is narrower than 0..255, is applied to both sides before converting.
+//   t = float(acc) * mult / s_out + biasf / s_out + offset' is the reference's value before rounding, with its roundings (offset': 128
+//   higher for signed outputs, codes as unsigned bytes).  The fast path works on a scale on which v_cvt_pknorm_u16_f32 (two values
+//   per instruction: rint(65535 x), saturated to 0 .. 65535) leaves the code in the high byte of its 16 bits,
+//       65535 x = 256 (t + 0.5) - 0.5,
+//   so that x crosses from one high byte to the next where t is a half-integer.  The host chooses c above every rounding on both
+//   sides (the reference's four; those of m, b, the conversion, the fma and the subtraction: FinishTable has the sum), so that
+//       p = fma(float(acc), m, b)  and  q = p - 2c     enclose the reference's x:   q < x(t) < p.
+//   When both give the same high byte, t -- strictly between them -- rounds to that code under any tie rule, the reference's
+//   half-away-from-zero included.  Values whose two bytes differ (about two in 10^4) are recomputed with the reference's own
+//   sequence.  A channel without a fast path has m = 0 and a b on a byte's edge, so that its bytes always differ.
+//   Where Requant::acc_base is not zero, accumulators run that much higher than the sums, and their bits are the float 1.5 * 2^23 +
+//   sum: one subtraction instead of a conversion.  That is exact up to 2^22; beyond, the steps are larger or smaller than one,
+//   but still in order, and the host has checked that no sum gets there or that all codes are saturated.  (Not so in a
+//   4096-wide FullyConnected with small scales.)
+//   What instructions cost here was measured pair by pair: conversions, permutes and packed integers take a SIMD four cycles a wave,
+//   float additions two, and fma and additions issue beside the conversions of another wave.  Four values: 4 subtract, 4 fma, 4
+//   subtract, 4 conversions, 2 permutes, xor, compare -- where the form before (v_cvt_f32_i32, one fma and one
+//   v_cvt_pk_u8_f32 per side) had 12 conversions.  A loop of little else: 10.8 against 7.9 T values/s on the whole device, 9.3
+//   with the accumulators converted.
+//   Passes (RequantCore's batches included): MobileNetV1 at 64 images 177.3 -> 170.2 us, at 256 647.8 -> 615.1, ResNet-50 at 32 459.6 ->
+//   454.0, FullyConnected 8192 x 4096 x 4096 130.3 -> 125.1, depthwise 64 x 112 x 112 x 32 15.3 -> 14.4.
+//   The activation's clamp, where it is narrower than 0..255, is applied to the codes.
 
 // Stores of layer outputs.  An ordinary store leaves its line dirty in the XCD's L2 until the end-of-kernel write-back,
 // which then moves the whole output tensor (up to the 32 MB the eight L2s hold) after the last wave has finished, with
@@ -115,111 +130,144 @@ __device__ __forceinline__ uint32_t Pack4(int q0, int q1, int q2, int q3)
 
 struct Fast4
 {
-    float4 mp, bp, mm, bm;   // rows 2..5: the bracket (the rare exact path fetches rows 0 / 1 when it is entered)
+    float4 m, b;   // rows 2 and 3 (the rare exact path fetches rows 0 and 1 when it is entered)
 };
 
 __device__ __forceinline__ Fast4 LoadFast4(const ChanTab& ct, int c)
 {
     Fast4 f;
-    f.mp = *reinterpret_cast<const float4*>(ct.p + 2 * ct.stride + c);
-    f.bp = *reinterpret_cast<const float4*>(ct.p + 3 * ct.stride + c);
-    f.mm = *reinterpret_cast<const float4*>(ct.p + 4 * ct.stride + c);
-    f.bm = *reinterpret_cast<const float4*>(ct.p + 5 * ct.stride + c);
+    f.m = *reinterpret_cast<const float4*>(ct.p + 2 * ct.stride + c);
+    f.b = *reinterpret_cast<const float4*>(ct.p + 3 * ct.stride + c);
     return f;
 }
 
-// Four consecutive channels c..c+3 of one pixel -> packed dword.
-// Five VALU instructions per value on the fast path (convert, two FMAs, two converting packs; two v_med3 more when the
-// activation clamps inside 0..255) and one compare and scalar branch per quad.  When some lane of the wave has a byte
-// that differs between the two sides, the wave redoes that position of the quad with the reference's sequence on every
-// lane (always right, and cheaper than sorting out which lanes need it); LOAD_EXACT supplies rows 0 / 1 of the table
-// and, for kernels whose accumulators start at zero, the zero-point correction that only the exact path adds as an
-// integer.  The constants are finite (the host checks them and the accumulator range), so no NaN reaches a conversion.
-template <typename LoadExact>
-__device__ __forceinline__ uint32_t Requant4Core(int a0, int a1, int a2, int a3, const float4& mp, const float4& bp,
-                                                 const float4& mm, const float4& bm, const Requant& rq, LoadExact load_exact)
+// The sum in an accumulator as a float; BITS: Requant::acc_base is not zero.
+template <bool BITS>
+__device__ __forceinline__ float AccValue(int acc)
 {
-    const float f0 = static_cast<float>(a0), f1 = static_cast<float>(a1), f2 = static_cast<float>(a2), f3 = static_cast<float>(a3);
-    float p0 = __fmaf_rn(f0, mp.x, bp.x), p1 = __fmaf_rn(f1, mp.y, bp.y), p2 = __fmaf_rn(f2, mp.z, bp.z), p3 = __fmaf_rn(f3, mp.w, bp.w);
-    float q0 = __fmaf_rn(f0, mm.x, bm.x), q1 = __fmaf_rn(f1, mm.y, bm.y), q2 = __fmaf_rn(f2, mm.z, bm.z), q3 = __fmaf_rn(f3, mm.w, bm.w);
-    if (!rq.pk_full)
-    {
-        p0 = __builtin_amdgcn_fmed3f(p0, rq.pk_lo_f, rq.pk_hi_f); q0 = __builtin_amdgcn_fmed3f(q0, rq.pk_lo_f, rq.pk_hi_f);
-        p1 = __builtin_amdgcn_fmed3f(p1, rq.pk_lo_f, rq.pk_hi_f); q1 = __builtin_amdgcn_fmed3f(q1, rq.pk_lo_f, rq.pk_hi_f);
-        p2 = __builtin_amdgcn_fmed3f(p2, rq.pk_lo_f, rq.pk_hi_f); q2 = __builtin_amdgcn_fmed3f(q2, rq.pk_lo_f, rq.pk_hi_f);
-        p3 = __builtin_amdgcn_fmed3f(p3, rq.pk_lo_f, rq.pk_hi_f); q3 = __builtin_amdgcn_fmed3f(q3, rq.pk_lo_f, rq.pk_hi_f);
-    }
-    // round to nearest, saturate to 0..255 and pack, one instruction per value
-    uint32_t out = __builtin_amdgcn_cvt_pk_u8_f32(p0, 0, 0u);
-    out = __builtin_amdgcn_cvt_pk_u8_f32(p1, 1, out);
-    out = __builtin_amdgcn_cvt_pk_u8_f32(p2, 2, out);
-    out = __builtin_amdgcn_cvt_pk_u8_f32(p3, 3, out);
-    uint32_t low = __builtin_amdgcn_cvt_pk_u8_f32(q0, 0, 0u);
-    low = __builtin_amdgcn_cvt_pk_u8_f32(q1, 1, low);
-    low = __builtin_amdgcn_cvt_pk_u8_f32(q2, 2, low);
-    low = __builtin_amdgcn_cvt_pk_u8_f32(q3, 3, low);
-    const uint32_t differ = out ^ low;
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(differ != 0u) != 0, 0))
-    {
-        float4 m, b;
-        int4 cr;
-        load_exact(m, b, cr);
-        // usually one value of the wave's 256 is flagged: only its position is redone (on every lane: the exact result is
-        // always the right one)
-        if (__builtin_amdgcn_ballot_w64((differ & 0x000000ffu) != 0u) != 0)
-            out = (out & 0xffffff00u) | (static_cast<uint32_t>(RequantExactDev(a0 + cr.x, m.x, b.x, rq) + rq.pk_bias) & 0xffu);
-        if (__builtin_amdgcn_ballot_w64((differ & 0x0000ff00u) != 0u) != 0)
-            out = (out & 0xffff00ffu) | ((static_cast<uint32_t>(RequantExactDev(a1 + cr.y, m.y, b.y, rq) + rq.pk_bias) & 0xffu) << 8);
-        if (__builtin_amdgcn_ballot_w64((differ & 0x00ff0000u) != 0u) != 0)
-            out = (out & 0xff00ffffu) | ((static_cast<uint32_t>(RequantExactDev(a2 + cr.z, m.z, b.z, rq) + rq.pk_bias) & 0xffu) << 16);
-        if (__builtin_amdgcn_ballot_w64((differ & 0xff000000u) != 0u) != 0)
-            out = (out & 0x00ffffffu) | ((static_cast<uint32_t>(RequantExactDev(a3 + cr.w, m.w, b.w, rq) + rq.pk_bias) & 0xffu) << 24);
-    }
-    return out ^ rq.pk_xor;
+    if constexpr (BITS) return __fsub_rn(__builtin_bit_cast(float, acc), kAccBaseValue);
+    else return static_cast<float>(acc);
 }
 
-// Bracket constants given row by row (kernels that keep rows 2, 6, 4, 7 -- the corr-folded bracket -- in LDS or registers).
-// `corr` (may be null) is an integer added to the accumulator on the exact path only.
-__device__ __forceinline__ uint32_t Requant4Dev(int a0, int a1, int a2, int a3, const float4& mp, const float4& bp,
-                                                const float4& mm, const float4& bm, const ChanTab& ct, const int32_t* corr, int c,
-                                                const Requant& rq)
+typedef unsigned short U16x2 __attribute__((ext_vector_type(2)));
+
+// the high bytes of four 16-bit values -> one dword
+__device__ __forceinline__ uint32_t HighBytes4(U16x2 v01, U16x2 v23)
 {
-    return Requant4Core(a0, a1, a2, a3, mp, bp, mm, bm, rq, [&](float4& m, float4& b, int4& cr) {
+    return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, v23), __builtin_bit_cast(uint32_t, v01), 0x07050301u);
+}
+
+// N times four values -> N packed dwords; their constants: f[n], or f[0] for all.
+// The N are independent chains of arithmetic with one test at their end, so that a wave has all of them to issue from: a test
+// per four values is a branch, which the compiler moves nothing across.  When some lane of the wave has a byte that differs between
+// the two sides, the wave redoes that position of those four with the reference's sequence on every lane (always right, and
+// cheaper than sorting out which lanes need it); load_exact(n, mult, biasf) supplies rows 0 and 1 of the table.  The constants are
+// finite (the host checks them and the accumulator range), so no NaN reaches a conversion.
+template <bool BITS, int N, int NF, typename LoadExact>
+__device__ __forceinline__ void RequantCore(const v4i (&acc)[N], uint32_t (&out)[N], const Fast4 (&f)[NF], const Requant& rq, LoadExact load_exact)
+{
+    static_assert(NF == 1 || NF == N, "one set of constants, or one each");
+    uint32_t differ[N], any = 0u;
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+    {
+        const Fast4& c = f[NF == 1 ? 0 : n];
+        const float p0 = __fmaf_rn(AccValue<BITS>(acc[n][0]), c.m.x, c.b.x), p1 = __fmaf_rn(AccValue<BITS>(acc[n][1]), c.m.y, c.b.y);
+        const float p2 = __fmaf_rn(AccValue<BITS>(acc[n][2]), c.m.z, c.b.z), p3 = __fmaf_rn(AccValue<BITS>(acc[n][3]), c.m.w, c.b.w);
+        const U16x2 hi01 = __builtin_amdgcn_cvt_pknorm_u16(p0, p1), hi23 = __builtin_amdgcn_cvt_pknorm_u16(p2, p3);
+        const U16x2 lo01 = __builtin_amdgcn_cvt_pknorm_u16(__fsub_rn(p0, rq.two_c), __fsub_rn(p1, rq.two_c));
+        const U16x2 lo23 = __builtin_amdgcn_cvt_pknorm_u16(__fsub_rn(p2, rq.two_c), __fsub_rn(p3, rq.two_c));
+        out[n] = HighBytes4(hi01, hi23);
+        differ[n] = out[n] ^ HighBytes4(lo01, lo23);
+        any |= differ[n];
+    }
+    if (!rq.pk_full)
+    {
+        // the clamp, two codes at a time
+        const U16x2 least = __builtin_bit_cast(U16x2, rq.pk_lo2), most = __builtin_bit_cast(U16x2, rq.pk_hi2);
+#pragma unroll
+        for (int n = 0; n < N; ++n)
+        {
+            const U16x2 even = __builtin_elementwise_min(__builtin_elementwise_max(__builtin_bit_cast(U16x2, out[n] & 0x00ff00ffu), least), most);
+            const U16x2 odd = __builtin_elementwise_min(__builtin_elementwise_max(__builtin_bit_cast(U16x2, (out[n] >> 8) & 0x00ff00ffu), least), most);
+            out[n] = __builtin_bit_cast(uint32_t, even) | (__builtin_bit_cast(uint32_t, odd) << 8);
+        }
+    }
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(any != 0u) != 0, 0))
+    {
+        constexpr int base = BITS ? kAccBaseBits : 0;
+        // usually one value of the wave's 256 N is flagged: only its position is redone (on every lane: the exact result is
+        // always the right one)
+#pragma unroll
+        for (int n = 0; n < N; ++n)
+        {
+            if (N > 1 && __builtin_amdgcn_ballot_w64(differ[n] != 0u) == 0) continue;
+            float4 m, b;
+            load_exact(n, m, b);
+            const float ms[4] = {m.x, m.y, m.z, m.w}, bs[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (__builtin_amdgcn_ballot_w64((differ[n] & (0xffu << (8 * k))) != 0u) != 0)
+                    out[n] = (out[n] & ~(0xffu << (8 * k))) | ((static_cast<uint32_t>(RequantExactDev(acc[n][k] - base, ms[k], bs[k], rq) + rq.pk_bias) & 0xffu) << (8 * k));
+        }
+    }
+#pragma unroll
+    for (int n = 0; n < N; ++n) out[n] ^= rq.pk_xor;
+}
+
+// N pixels, channels c .. c + 3 of each
+template <bool BITS, int N>
+__device__ __forceinline__ void RequantPixels(const v4i (&acc)[N], uint32_t (&out)[N], const Fast4& f, const ChanTab& ct, int c, const Requant& rq)
+{
+    const Fast4 fs[1] = {f};
+    RequantCore<BITS, N, 1>(acc, out, fs, rq, [&](int, float4& m, float4& b) {
         m = *reinterpret_cast<const float4*>(ct.p + c);
         b = *reinterpret_cast<const float4*>(ct.p + ct.stride + c);
-        cr = int4{0, 0, 0, 0};
-        if (corr) cr = *reinterpret_cast<const int4*>(corr + c);
     });
 }
 
-// constants of rows 2..5 (accumulator already contains the zero-point correction)
-__device__ __forceinline__ uint32_t Requant4Dev(int a0, int a1, int a2, int a3, const Fast4& f, const ChanTab& ct, int c,
-                                                const Requant& rq)
+// one pixel, channels c + STEP n .. c + STEP n + 3
+template <bool BITS, int N, int STEP>
+__device__ __forceinline__ void RequantChannels(const v4i (&acc)[N], uint32_t (&out)[N], const Fast4 (&f)[N], const ChanTab& ct, int c, const Requant& rq)
 {
-    return Requant4Dev(a0, a1, a2, a3, f.mp, f.bp, f.mm, f.bm, ct, nullptr, c, rq);
+    RequantCore<BITS, N, N>(acc, out, f, rq, [&](int n, float4& m, float4& b) {
+        m = *reinterpret_cast<const float4*>(ct.p + c + STEP * n);
+        b = *reinterpret_cast<const float4*>(ct.p + ct.stride + c + STEP * n);
+    });
 }
 
-// one channel (scalar kernels): the same bracket, compared after rounding
-__device__ __forceinline__ int RequantBracket1(int acc, int exact_acc, float mp, float bp, float mm, float bm, float m0, float b0, const Requant& rq)
+// channels c .. c + 3 of one pixel; BITS must say whether Requant::acc_base is not zero (in a 3x3 depthwise plan it never is zero)
+template <bool BITS>
+__device__ __forceinline__ uint32_t Requant4Dev(int a0, int a1, int a2, int a3, const Fast4& f, const ChanTab& ct, int c, const Requant& rq)
 {
-    const float f = static_cast<float>(acc);
-    const float kp = __builtin_rintf(__builtin_amdgcn_fmed3f(__fmaf_rn(f, mp, bp), rq.pk_lo_f, rq.pk_hi_f));
-    const float km = __builtin_rintf(__builtin_amdgcn_fmed3f(__fmaf_rn(f, mm, bm), rq.pk_lo_f, rq.pk_hi_f));
-    if (__builtin_expect(!(kp == km), 0)) return RequantExactDev(exact_acc, m0, b0, rq);
-    return static_cast<int>(kp) - rq.pk_bias;
+    const v4i acc[1] = {{a0, a1, a2, a3}};
+    uint32_t out[1];
+    RequantPixels<BITS, 1>(acc, out, f, ct, c, rq);
+    return out[0];
 }
 
+// ... where the kernel is not worth two copies of its write-out
+__device__ __forceinline__ uint32_t Requant4Any(int a0, int a1, int a2, int a3, const Fast4& f, const ChanTab& ct, int c, const Requant& rq)
+{
+    return rq.acc_base != 0 ? Requant4Dev<true>(a0, a1, a2, a3, f, ct, c, rq) : Requant4Dev<false>(a0, a1, a2, a3, f, ct, c, rq);
+}
+
+// ... and where it is: `write_out` is called with std::true_type or std::false_type for BITS
+template <typename F>
+__device__ __forceinline__ void WithBits(const Requant& rq, F write_out)
+{
+    if (rq.acc_base != 0) write_out(std::true_type{});
+    else write_out(std::false_type{});
+}
+
+// one channel (scalar kernels): the same bracket
 __device__ __forceinline__ int Requant1Dev(int acc, const ChanTab& ct, int c, const Requant& rq)
 {
-    return RequantBracket1(acc, acc, ct.p[2 * ct.stride + c], ct.p[3 * ct.stride + c], ct.p[4 * ct.stride + c], ct.p[5 * ct.stride + c],
-                           ct.p[c], ct.p[ct.stride + c], rq);
-}
-
-// one channel, accumulator started at zero: rows 2/6/4/7 on the fast path, `corr[c]` joins the accumulator on the exact path
-__device__ __forceinline__ int Requant1FoldedDev(int acc, const ChanTab& ct, const int32_t* corr, int c, const Requant& rq)
-{
-    return RequantBracket1(acc, acc + corr[c], ct.p[2 * ct.stride + c], ct.p[6 * ct.stride + c], ct.p[4 * ct.stride + c], ct.p[7 * ct.stride + c],
-                           ct.p[c], ct.p[ct.stride + c], rq);
+    const float p = __fmaf_rn(rq.acc_base != 0 ? AccValue<true>(acc) : AccValue<false>(acc), ct.p[2 * ct.stride + c], ct.p[3 * ct.stride + c]);
+    const U16x2 v = __builtin_amdgcn_cvt_pknorm_u16(p, __fsub_rn(p, rq.two_c));
+    const int hi = v.x >> 8, lo = v.y >> 8;
+    if (__builtin_expect(hi != lo, 0)) return RequantExactDev(acc - rq.acc_base, ct.p[c], ct.p[ct.stride + c], rq);
+    return min(max(hi - rq.pk_bias, rq.act_lo), rq.act_hi);
 }
 
 // value already in float (pooling, add, ...): reciprocal fast path with the exact fallback near ties.

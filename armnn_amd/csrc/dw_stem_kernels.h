@@ -235,7 +235,7 @@ __device__ __forceinline__ void Depthwise3x3Block(const Dw3x3Args& a, int b, uin
             const int ox = tx * TW + xg * P + j;
             if (ox < a.Wo && c < a.C)
             {
-                const uint32_t q = Requant4Dev(acc[o][j][0], acc[o][j][1], acc[o][j][2], acc[o][j][3], f4, a.ct, c, a.rq);
+                const uint32_t q = Requant4Dev<true>(acc[o][j][0], acc[o][j][1], acc[o][j][2], acc[o][j][3], f4, a.ct, c, a.rq);
                 if constexpr (THROUGH)
                     __builtin_amdgcn_raw_buffer_store_b32(q, yrsrc, static_cast<int>(yrow - a.y) + ox * a.C, 0, kStoreAuxSc1);
                 else
@@ -271,7 +271,7 @@ struct SmallCiArgs
     const uint8_t*  x;
     const uint32_t* wpack;    // [Co][KH][RD] dwords: row r of filter co as consecutive (kx, ci) bytes, zero padded
     const uint32_t* wpack2;   // W2: the second halves, same layout
-    ChanTab         ct;       // rows 2, 5, 6 on the fast path (accumulators start at zero), rows 0, 1 on the exact path
+    ChanTab         ct;
     const int32_t*  corr;     // [Co]
     uint8_t*        y;
     int N, H, W, Ci, Ho, Wo, Co;
@@ -465,6 +465,7 @@ __global__ __launch_bounds__(256) void SmallCiConvKernel(SmallCiArgs a)
     const uint32_t MI355X_CONST_AS* wc = AsConstant(a.wpack);
     const uint32_t MI355X_CONST_AS* wc2 = AsConstant(W2 ? a.wpack2 : a.wpack);
     const float MI355X_CONST_AS* tab = AsConstant(a.ct.p);
+    const int32_t MI355X_CONST_AS* corr = AsConstant(a.corr);
     const int ts = a.ct.stride;
     for (int co = 0; co < a.Co; co += 16)
     {
@@ -481,7 +482,7 @@ __global__ __launch_bounds__(256) void SmallCiConvKernel(SmallCiArgs a)
             {
                 const uint32_t MI355X_CONST_AS* w = wc + (c + u) * (KH * RD);
 #pragma unroll
-                for (int p = 0; p < P; ++p) acc[p][u] = 0;
+                for (int p = 0; p < P; ++p) acc[p][u] = corr[c + u];
 #pragma unroll
                 for (int r = 0; r < KH; ++r)
 #pragma unroll
@@ -498,13 +499,11 @@ __global__ __launch_bounds__(256) void SmallCiConvKernel(SmallCiArgs a)
                         }
                     }
             }
-            const float4 mp = {tab[2 * ts + c], tab[2 * ts + c + 1], tab[2 * ts + c + 2], tab[2 * ts + c + 3]};
-            const float4 bp = {tab[6 * ts + c], tab[6 * ts + c + 1], tab[6 * ts + c + 2], tab[6 * ts + c + 3]};
-            const float4 mm = {tab[4 * ts + c], tab[4 * ts + c + 1], tab[4 * ts + c + 2], tab[4 * ts + c + 3]};
-            const float4 bm = {tab[7 * ts + c], tab[7 * ts + c + 1], tab[7 * ts + c + 2], tab[7 * ts + c + 3]};
+            const Fast4 f4 = {{tab[2 * ts + c], tab[2 * ts + c + 1], tab[2 * ts + c + 2], tab[2 * ts + c + 3]},
+                              {tab[3 * ts + c], tab[3 * ts + c + 1], tab[3 * ts + c + 2], tab[3 * ts + c + 3]}};
 #pragma unroll
             for (int p = 0; p < P; ++p)
-                o[p][g4] = Requant4Dev(acc[p][0], acc[p][1], acc[p][2], acc[p][3], mp, bp, mm, bm, a.ct, a.corr, c, a.rq);
+                o[p][g4] = Requant4Any(acc[p][0], acc[p][1], acc[p][2], acc[p][3], f4, a.ct, c, a.rq);
         }
         if (groups == 4 && a.vec16)
         {
@@ -538,7 +537,7 @@ __global__ __launch_bounds__(256) void SmallCiMfmaKernel(SmallCiArgs a)
     constexpr int NDWP = KH * RD;                 // patch dwords per pixel
     constexpr int KST = (NDWP + 7) / 8;           // MFMA k-steps of 32 bytes
     __shared__ __attribute__((aligned(16))) uint32_t tile[SmallCiTile<KH, TH>::DWORDS];
-    __shared__ __attribute__((aligned(16))) float cst[4][NT * 32];      // the corr-folded bracket: m+, bc+, m-, bc-
+    __shared__ __attribute__((aligned(16))) float cst[3][NT * 32];      // m, b and (as integers) what the accumulators start from
 
     int b = blockIdx.x;
     const int tx = b % a.tiles_x; b /= a.tiles_x;
@@ -548,10 +547,10 @@ __global__ __launch_bounds__(256) void SmallCiMfmaKernel(SmallCiArgs a)
     const int S = a.stride;
     int iy_org, ix_org, mis;
     StageSmallCiHalo<KH, TH>(a, tile, tx, ty, n, tid, iy_org, ix_org, mis);
-    for (int i = tid; i < 4 * NT * 32; i += 256)
+    for (int i = tid; i < 3 * NT * 32; i += 256)
     {
         const int row = i / (NT * 32), c = i - row * (NT * 32);
-        cst[row][c] = a.ct.p[(row == 0 ? 2 : row == 1 ? 6 : row == 2 ? 4 : 7) * a.ct.stride + c];
+        cst[row][c] = row < 2 ? a.ct.p[(row + 2) * a.ct.stride + c] : __builtin_bit_cast(float, a.corr[c]);
     }
 
     const int lane = tid & 63, wave = tid >> 6;
@@ -609,8 +608,14 @@ __global__ __launch_bounds__(256) void SmallCiMfmaKernel(SmallCiArgs a)
 #pragma unroll
         for (int ct = 0; ct < NT; ++ct)
         {
-            const v16i zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-            v16i acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(wfrag[ct][0], bfrag[0], zero, 0, 0, 0);
+            v16i acc;
+#pragma unroll
+            for (int qd = 0; qd < 4; ++qd)
+            {
+                const v4i c4 = *reinterpret_cast<const v4i*>(&cst[2][ct * 32 + 8 * qd + 4 * half]);
+                acc[4 * qd + 0] = c4[0]; acc[4 * qd + 1] = c4[1]; acc[4 * qd + 2] = c4[2]; acc[4 * qd + 3] = c4[3];
+            }
+            acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(wfrag[ct][0], bfrag[0], acc, 0, 0, 0);
 #pragma unroll
             for (int t = 1; t < KST; ++t) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(wfrag[ct][t], bfrag[t], acc, 0, 0, 0);
             if constexpr (W2)
@@ -619,16 +624,16 @@ __global__ __launch_bounds__(256) void SmallCiMfmaKernel(SmallCiArgs a)
                 for (int t = 0; t < KST; ++t) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(wfrag2[ct][t], bfrag[t], acc, 0, 0, 0);
             }
             uint32_t o[4];
+            v4i q4[4];
+            Fast4 f[4];
+            const int cl = ct * 32 + 4 * half;
 #pragma unroll
             for (int qd = 0; qd < 4; ++qd)
             {
-                const int cl = ct * 32 + 8 * qd + 4 * half;
-                const float4 mp = *reinterpret_cast<const float4*>(&cst[0][cl]);
-                const float4 bp = *reinterpret_cast<const float4*>(&cst[1][cl]);
-                const float4 mm = *reinterpret_cast<const float4*>(&cst[2][cl]);
-                const float4 bm = *reinterpret_cast<const float4*>(&cst[3][cl]);
-                o[qd] = Requant4Dev(acc[4 * qd + 0], acc[4 * qd + 1], acc[4 * qd + 2], acc[4 * qd + 3], mp, bp, mm, bm, a.ct, a.corr, cl, a.rq);
+                q4[qd] = Quad(acc, qd);
+                f[qd] = {*reinterpret_cast<const float4*>(&cst[0][cl + 8 * qd]), *reinterpret_cast<const float4*>(&cst[1][cl + 8 * qd])};
             }
+            WithBits(a.rq, [&](auto bits) { RequantChannels<decltype(bits)::value, 4, 8>(q4, o, f, a.ct, cl, a.rq); });
             // lane and lane + 32 hold interleaved 4-channel groups of one pixel; trading two dwords gives each of them
             // 16 contiguous channels (the low lane 0..15, the high lane 16..31) and one 16-byte store
             const uint32_t r0 = __shfl_xor(half ? o[0] : o[2], 32);

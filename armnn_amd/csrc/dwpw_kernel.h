@@ -31,7 +31,7 @@ struct DwPwArgs
     // depthwise stage
     const uint8_t*  x;
     const uint8_t*  pad16;      // 16 bytes that become the depthwise padding value under dw_xor
-    const uint32_t* dw_grp;     // [C/4][8][4] dwords per group of 4 channels: w row 0, w row 1, w row 2, corr, m+, b+, m-, b-
+    const uint32_t* dw_grp;     // per group of 4 channels, kDwGrpDwords: rows of four, w row 0, w row 1, w row 2, corr, m, b
     ChanTab         dw_ct;      // exact-path constants of the depthwise layer
     int N, H, W, C, Ho, Wo;
     int pad_top, pad_left;
@@ -42,7 +42,7 @@ struct DwPwArgs
     // pointwise stage
     const int8_t*  pw_w;        // [Co_pad][pw_wstride]
     int            pw_wstride;
-    ChanTab        pw_ct;       // rows 2, 5, 6 on the fast path (accumulators start at zero)
+    ChanTab        pw_ct;
     const int32_t* pw_corr;
     uint8_t*       y;
     int            Co;
@@ -74,7 +74,7 @@ template <int S, int P>
 inline int DwPwSmemBytes(int C)
 {
     using G = DwPwGeom<S, P>;
-    return G::TP * (C + 16) + G::SCRATCH + (C / 4) * 128;
+    return G::TP * (C + 16) + G::SCRATCH + (C / 4) * (kDwGrpDwords * 4);
 }
 
 // D: channel blocks whose halo loads are in flight (register slots); KC: k-steps per weight chunk of phase B, the next
@@ -103,7 +103,7 @@ __global__ __launch_bounds__(256) void DwPwKernel(DwPwArgs a)
     const int wave = tid >> 6;
 
     // ---- depthwise constants of all channels -> LDS ----------------------------------------------------------------
-    for (int i = tid; i < a.C * 2; i += 256)           // C/4 groups x 8 rows of 16 bytes
+    for (int i = tid; i < a.C / 4 * (kDwGrpDwords / 4); i += 256)           // rows of 16 bytes
         *reinterpret_cast<v4i*>(grp + i * 4) = *reinterpret_cast<const v4i*>(a.dw_grp + i * 4);
 
     // ---- phase A ----------------------------------------------------------------------------------------------------
@@ -166,7 +166,7 @@ __global__ __launch_bounds__(256) void DwPwKernel(DwPwArgs a)
         if (cb + D < ncb) stage_load(cb + D, jc);
 
         const uint8_t* halo = scratch + (cb & 1) * G::HALO;
-        const v4i* gc = reinterpret_cast<const v4i*>(grp + (cb * 8 + c4) * 32);   // this thread's group of 4 channels
+        const v4i* gc = reinterpret_cast<const v4i*>(grp + (cb * 8 + c4) * kDwGrpDwords);   // this thread's group of 4 channels
         const v4i w0 = gc[0], w1 = gc[1], w2 = gc[2], corr4 = gc[3];
         int acc[P][4];
 #pragma unroll
@@ -211,15 +211,12 @@ __global__ __launch_bounds__(256) void DwPwKernel(DwPwArgs a)
                 }
             }
         }
-        const float4 mp = *reinterpret_cast<const float4*>(gc + 4);
-        const float4 bp = *reinterpret_cast<const float4*>(gc + 5);
-        const float4 mm = *reinterpret_cast<const float4*>(gc + 6);
-        const float4 bm = *reinterpret_cast<const float4*>(gc + 7);
+        const Fast4 f4 = {*reinterpret_cast<const float4*>(gc + 4), *reinterpret_cast<const float4*>(gc + 5)};
         const int c = cb * 32 + c4 * 4;
 #pragma unroll
         for (int j = 0; j < P; ++j)
         {
-            const uint32_t q = Requant4Dev(acc[j][0], acc[j][1], acc[j][2], acc[j][3], mp, bp, mm, bm, a.dw_ct, nullptr, c, a.dw_rq);
+            const uint32_t q = Requant4Dev<true>(acc[j][0], acc[j][1], acc[j][2], acc[j][3], f4, a.dw_ct, c, a.dw_rq);
             *reinterpret_cast<uint32_t*>(T + (row * TW + xg * P + j) * LDT + c) = q ^ mid;
         }
     };
@@ -243,7 +240,6 @@ __global__ __launch_bounds__(256) void DwPwKernel(DwPwArgs a)
     for (int ct = wave * NC; ct < nct; ct += 4 * NC)
     {
         v16i acc[NC][TPS];
-        const v16i zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
         const int8_t* wbase = a.pw_w + static_cast<long long>(ct * 32 + frag_row) * a.pw_wstride + frag_k;
         const uint8_t* tbase = T + frag_row * LDT + frag_k;
         // weights in chunks of KC k-steps, two register slots: chunk q + 1 is on its way while chunk q is multiplied
@@ -282,7 +278,15 @@ __global__ __launch_bounds__(256) void DwPwKernel(DwPwArgs a)
 #pragma unroll
         for (int i = 0; i < NC; ++i)
 #pragma unroll
-            for (int p = 0; p < TPS; ++p) acc[i][p] = zero;
+            for (int q = 0; q < 4; ++q)
+            {
+                const v4i c4 = *reinterpret_cast<const v4i*>(a.pw_corr + (ct + i) * 32 + 8 * q + lane_c);
+#pragma unroll
+                for (int p = 0; p < TPS; ++p)
+                {
+                    acc[i][p][4 * q + 0] = c4[0]; acc[i][p][4 * q + 1] = c4[1]; acc[i][p][4 * q + 2] = c4[2]; acc[i][p][4 * q + 3] = c4[3];
+                }
+            }
         load_w(0, integral_constant<int, 0>{});
         for (int q = 0; q < nchunk; q += 2)
         {
@@ -305,12 +309,8 @@ __global__ __launch_bounds__(256) void DwPwKernel(DwPwArgs a)
                 {
                     const int cl = i * 32 + 8 * q + lane_c;
                     const int cg = ct * 32 + cl;
-                    const float4 mp = *reinterpret_cast<const float4*>(a.pw_ct.p + 2 * a.pw_ct.stride + cg);
-                    const float4 bp = *reinterpret_cast<const float4*>(a.pw_ct.p + 6 * a.pw_ct.stride + cg);
-                    const float4 mm = *reinterpret_cast<const float4*>(a.pw_ct.p + 4 * a.pw_ct.stride + cg);
-                    const float4 bm = *reinterpret_cast<const float4*>(a.pw_ct.p + 7 * a.pw_ct.stride + cg);
                     const v16i& v = acc[i][p];
-                    const uint32_t out = Requant4Dev(v[4 * q + 0], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3], mp, bp, mm, bm, a.pw_ct, a.pw_corr, cg, a.pw_rq);
+                    const uint32_t out = Requant4Any(v[4 * q + 0], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3], LoadFast4(a.pw_ct, cg), a.pw_ct, cg, a.pw_rq);
                     *reinterpret_cast<uint32_t*>(ostage + frag_row * LDO + cl) = out;
                 }
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

@@ -99,23 +99,23 @@ bool mi355x::DwPwPanelTakes(const mi355x_conv2d_s* dw, const mi355x_conv2d_s* pw
 
 namespace
 {
-// Blocks of 64 channels: 11 rows of [16][4] dwords, entry [j][e] for channel 16 e + j of the block: corr, m+, b+, m-, b-, filter taps
+// Blocks of 64 channels: kDwBlkRows rows of [16][4] dwords, entry [j][e] for channel 16 e + j of the block: corr, m, b, filter taps
 // 0..3, 4..7, 8, and those of the second halves.  Channels past the last one are all zero: a bracket that closes, some code that no
 // weight and no row sum counts.  `grp`, `second`: the plan's dw_grp and w_dot4b (or null).
 __global__ __launch_bounds__(256) void PackDwBlkKernel(const uint32_t* __restrict__ grp, const uint32_t* __restrict__ second, uint32_t* __restrict__ blk, int C, int dwords)
 {
     const int i = static_cast<int>(blockIdx.x) * 256 + static_cast<int>(threadIdx.x);
     if (i >= dwords) return;
-    const int b = i / 704, row = i % 704 / 64, c = b * 64 + i % 4 * 16 + i % 64 / 4;
+    const int b = i / (kDwBlkRows * 64), row = i % (kDwBlkRows * 64) / 64, c = b * 64 + i % 4 * 16 + i % 64 / 4;
     uint32_t v = 0;
     if (c < C)
     {
-        const uint32_t* const of = grp + (c / 4) * 32 + c % 4;         // rows of four: weights 0 .. 2, corr, m+, b+, m-, b-
-        if (row < 5) v = of[(3 + row) * 4];
+        const uint32_t* const of = grp + (c / 4) * kDwGrpDwords + c % 4;         // rows of four: weights 0 .. 2, corr, m, b
+        if (row < 3) v = of[(3 + row) * 4];
         else
-            for (int t = (row - (row < 8 ? 5 : 8)) * 4, n = 0; n < 4 && t < 9; ++t, ++n)
+            for (int t = (row - (row < 6 ? 3 : 6)) * 4, n = 0; n < 4 && t < 9; ++t, ++n)
             {
-                const uint32_t taps = row < 8 ? of[t / 3 * 4] : second ? second[c * 4 + t / 3] : 0u;
+                const uint32_t taps = row < 6 ? of[t / 3 * 4] : second ? second[c * 4 + t / 3] : 0u;
                 v |= (taps >> (8 * (t % 3)) & 0xffu) << (8 * n);
             }
     }
@@ -124,7 +124,7 @@ __global__ __launch_bounds__(256) void PackDwBlkKernel(const uint32_t* __restric
 
 int PackDwBlk(const mi355x_conv2d_s* dw, uint32_t** out)
 {
-    const int C = dw->geom.Co, dwords = (C + 63) / 64 * 704;
+    const int C = dw->geom.Co, dwords = (C + 63) / 64 * (kDwBlkRows * 64);
     hipStream_t stream;
     if (const int rc = UploadStream(&stream)) return rc;
     MI355X_HIP(hipMalloc(reinterpret_cast<void**>(out), static_cast<size_t>(dwords) * 4));

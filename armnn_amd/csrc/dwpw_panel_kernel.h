@@ -15,9 +15,11 @@
 //     1 KB; 55 bytes a clock and CU were measured for that, 14 to 20 for 128-byte rows through LDS with a wait per k-tile), the
 //     first k-steps requested ahead of the depthwise phase.  No barrier inside: two after the halo, two around the write-out.
 //   * The outputs meet in LDS and leave as 16 bytes per lane.
-// At many tiles VALU work is the largest share, most of it the requantization of both layers (25 instructions per four values): 14 x 14 x
-// 512, 64 images, 12 k of a SIMD's 27 k cycles issue VALU and 5.6 k matrix instructions, the rest of a wave's life is waits, at barriers
-// and for the weights (82 MB through the CUs' L1s).  At few tiles it is the chain of round trips.  Times against the kernel with a k-tile loop it replaces (64 images | 256): 14 x 14 x 512 -> 512
+// At many tiles VALU work is the largest share, most of it the requantization of both layers: 14 x 14 x 512, 64 images, with 25
+// instructions and a branch per four values 12 k of a SIMD's 27 k cycles issued VALU and 5.6 k matrix instructions; the rest of a
+// wave's life is waits, at barriers and for the weights (82 MB through the CUs' L1s).  (Now 23 instructions, fewer of them
+// conversions, and a branch per 16 values: a pass of MobileNetV1 at 64 images 177.3 -> 170.2 us, most of it here.)  At few tiles
+// it is the chain of round trips.  Times against the kernel with a k-tile loop it replaces (64 images | 256): 14 x 14 x 512 -> 512
 // 15.4 -> 12.8 | 54.2 -> 35.7 us, 28 x 28 x 256 -> 256 20.2 -> 17.7 | 68.9 -> 61.3, 28 x 28 x 256 -> 14 x 14 x 512 11.2 -> 10.7 | 43.1 ->
 // 34.8; against two launches, one image | eight: 14 x 14 x 512 7.6 -> 5.5 | 9.3 -> 7.5, 28 x 28 x 256 7.2 -> 4.6 | 8.6 -> 6.3.
 // Both layers' arithmetic is untouched -- exact int32 sums, the same requantization routine with the same constants -- so the
@@ -39,7 +41,7 @@ struct DwPwPanelArgs
     // depthwise 3x3, multiplier 1, C % 16 == 0
     const uint8_t*  x;
     const uint8_t*  pad16;      // 16 bytes that become the depthwise padding value under dw_xor
-    const uint32_t* dw_blk;     // constants per block of 64 channels: 11 rows of [16][4] dwords
+    const uint32_t* dw_blk;     // constants per block of 64 channels: kDwBlkRows rows of [16][4] dwords
     ChanTab         dw_ct;
     int H, W, C, Ho, Wo;
     int pad_top, pad_left;
@@ -61,6 +63,9 @@ struct DwPwPanelArgs
     Requant        pw_rq;
 };
 
+// what accumulators start from, m, b, filter taps 0 .. 3, 4 .. 7, 8, and those of the second halves
+constexpr int kDwBlkRows = 9;
+
 template <int S, int TH, int TW, int NW, int CG>
 struct DwPwPanelGeom
 {
@@ -76,9 +81,9 @@ struct DwPwPanelGeom
         const int in = (C + 63) / 64 * 4 * GP, out = PX * OP;
         return in > out ? in : out;
     }
-    // behind it the depthwise layer's constants and four rows of NCOL floats of the pointwise layer's
-    static constexpr int TB(bool u) { return u ? 2816 : 2048; }        // bytes per 64 channels
-    static constexpr int Smem(int C, bool u) { return Panel(C) + (C + 63) / 64 * TB(u) + 16 * NCOL; }
+    // behind it the depthwise layer's constants and three rows of NCOL dwords of the pointwise layer's
+    static constexpr int TB(bool u) { return (u ? kDwBlkRows : kDwBlkRows - 3) * 256; }        // bytes per 64 channels
+    static constexpr int Smem(int C, bool u) { return Panel(C) + (C + 63) / 64 * TB(u) + 12 * NCOL; }
 };
 
 // KS: k-steps of 64 channels where the instance fixes them (64 (KS - 1) < C <= 64 KS), 0: a.C decides.  U: depthwise weights in two
@@ -97,9 +102,12 @@ __global__ __launch_bounds__(64 * NW, 4) void DwPwPanelKernel(DwPwPanelArgs a)
     constexpr int WPB = KS != 0 && NW / KS >= 2 ? (NW / KS < PG ? NW / KS : PG) : 1;
     constexpr int UW = PG / WPB, UC = WPB > 1 ? UW : UW < 2 || U ? 1 : 2;
     static_assert(PG % WPB == 0 && UW % UC == 0, "whole shares");
+    // Pixel groups requantized together.  (With U the registers are full: batches of 2 and 4 spill, 57.4 against 56.4 us for a pass of
+    // 13 images at width 0.75.)
+    constexpr int PB = U ? 1 : PG < 4 ? PG : 4;
     constexpr bool EARLY = PG == 1 || (PG == 2 && !U);                      // registers for weights requested ahead of the depthwise phase
     constexpr int TB = G::TB(U);
-    constexpr int TS = KS != 0 ? (KS * (TB / 16) + G::NCOL + NT - 1) / NT : 4;      // ... and table pieces
+    constexpr int TS = KS != 0 ? (KS * (TB / 16) + G::NCOL / 4 * 3 + NT - 1) / NT : 4;      // ... and table pieces
     extern __shared__ __attribute__((aligned(16))) uint8_t panel_lds[];   // [C / 16][GP]: halo pixels, then panel pixels, of 16 bytes
 
     int b = XcdContiguousWorkItem(blockIdx.x, a.xcd_chunk);
@@ -125,13 +133,17 @@ __global__ __launch_bounds__(64 * NW, 4) void DwPwPanelKernel(DwPwPanelArgs a)
     // ---- tables ---------------------------------------------------------------------------------------------------------------------
     uint8_t* const tab = panel_lds + G::Panel(64 * steps);
     uint8_t* const ptab = tab + steps * TB;
-    const int dw_pieces = steps * (TB / 16), tab_pieces = dw_pieces + G::NCOL;
+    const int dw_pieces = steps * (TB / 16), tab_pieces = dw_pieces + G::NCOL / 4 * 3;
     auto tab_src = [&](int i) -> const void* {
-        if (i < dw_pieces) return a.dw_blk + (U ? i * 4 : (i >> 7) * 704 + (i & 127) * 4);
+        if (i < dw_pieces)
+        {
+            const int blk = i / (TB / 16);
+            return a.dw_blk + blk * (kDwBlkRows * 64) + (i - blk * (TB / 16)) * 4;
+        }
         i -= dw_pieces;
-        const int r = i / (G::NCOL / 4), c4 = (i - r * (G::NCOL / 4)) * 4;
-        const int row = U ? r + 2 : r == 0 ? 2 : r == 1 ? 6 : r == 2 ? 4 : 7;
-        return a.pw_ct.p + row * a.pw_ct.stride + min(bn * G::NCOL + c4, a.co_groups * 16 - 4);
+        const int r = i / (G::NCOL / 4), c4 = min(bn * G::NCOL + (i - r * (G::NCOL / 4)) * 4, a.co_groups * 16 - 4);
+        if (r < 2) return a.pw_ct.p + (r + 2) * a.pw_ct.stride + c4;
+        return a.pw_corr + c4;
     };
 
     // ---- the halo of the tile, all channels ---------------------------------------------------------------------------------------
@@ -216,8 +228,8 @@ __global__ __launch_bounds__(64 * NW, 4) void DwPwPanelKernel(DwPwPanelArgs a)
 #pragma unroll
             for (int m = 0; m < 3; ++m)
             {
-                w[m] = *reinterpret_cast<const v4i*>(tb + (5 + m) * 256);
-                if constexpr (U) w2[m] = *reinterpret_cast<const v4i*>(tb + (8 + m) * 256);
+                w[m] = *reinterpret_cast<const v4i*>(tb + (3 + m) * 256);
+                if constexpr (U) w2[m] = *reinterpret_cast<const v4i*>(tb + (6 + m) * 256);
             }
             // the ninth tap of the four channel groups shares one operand: lane group g reads it from channel group g
             v4i x8[UC];
@@ -250,31 +262,30 @@ __global__ __launch_bounds__(64 * NW, 4) void DwPwPanelKernel(DwPwPanelArgs a)
         };
         auto codes = [&](int blk, int u0, const v4i (&acc)[4][UC]) {
             const uint8_t* const tb = tab + blk * TB + j * 16;
-            Fast4 f;
-            f.mp = *reinterpret_cast<const float4*>(tb + 256);
-            f.bp = *reinterpret_cast<const float4*>(tb + 512);
-            f.mm = *reinterpret_cast<const float4*>(tb + 768);
-            f.bm = *reinterpret_cast<const float4*>(tb + 1024);
+            const Fast4 f[1] = {{*reinterpret_cast<const float4*>(tb + 256), *reinterpret_cast<const float4*>(tb + 512)}};
             uint8_t* const out = panel_lds + blk * (4 * GP) + (j >> 2) * GP + (16 * u0 + 4 * g) * 16 + (j & 3) * 4;
 #pragma unroll
             for (int u = 0; u < UC; ++u)
+            {
+                v4i v[4];
+                uint32_t q[4];
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    *reinterpret_cast<uint32_t*>(out + (16 * u + r) * 16) =
-                        Requant4Core(acc[0][u][r], acc[1][u][r], acc[2][u][r], acc[3][u][r], f.mp, f.bp, f.mm, f.bm, a.dw_rq,
-                                     [&](float4& m, float4& b, int4& cr) {
-                                         float mv[4], bv[4];
+                for (int r = 0; r < 4; ++r) v[r] = v4i{acc[0][u][r], acc[1][u][r], acc[2][u][r], acc[3][u][r]};
+                RequantCore<true, 4, 1>(v, q, f, a.dw_rq, [&](int, float4& m, float4& b) {
+                    float mv[4], bv[4];
 #pragma unroll
-                                         for (int e = 0; e < 4; ++e)
-                                         {
-                                             const int c = min(blk * 64 + 16 * e + j, a.C - 1);
-                                             mv[e] = a.dw_ct.p[c];
-                                             bv[e] = a.dw_ct.p[a.dw_ct.stride + c];
-                                         }
-                                         m = float4{mv[0], mv[1], mv[2], mv[3]};
-                                         b = float4{bv[0], bv[1], bv[2], bv[3]};
-                                         cr = int4{0, 0, 0, 0};
-                                     }) ^ a.mid_xor;
+                    for (int e = 0; e < 4; ++e)
+                    {
+                        const int c = min(blk * 64 + 16 * e + j, a.C - 1);
+                        mv[e] = a.dw_ct.p[c];
+                        bv[e] = a.dw_ct.p[a.dw_ct.stride + c];
+                    }
+                    m = float4{mv[0], mv[1], mv[2], mv[3]};
+                    b = float4{bv[0], bv[1], bv[2], bv[3]};
+                });
+#pragma unroll
+                for (int r = 0; r < 4; ++r) *reinterpret_cast<uint32_t*>(out + (16 * u + r) * 16) = q[r] ^ a.mid_xor;
+            }
         };
         if constexpr (WPB > 1)
         {
@@ -315,7 +326,7 @@ __global__ __launch_bounds__(64 * NW, 4) void DwPwPanelKernel(DwPwPanelArgs a)
     {
         xs[p] = 0;
 #pragma unroll
-        for (int c = 0; c < CG; ++c) acc[c][p] = v4i{0, 0, 0, 0};
+        for (int c = 0; c < CG; ++c) acc[c][p] = *reinterpret_cast<const v4i*>(ptab + (2 * G::NCOL + (wave * CG + c) * 16 + 4 * g) * 4);
     }
     const uint8_t* const pb = panel_lds + g * GP + j * 16;
     // The sum of a pixel's codes is over the channels that exist.  Those that complete the last block of 64 hold whatever the
@@ -360,27 +371,30 @@ __global__ __launch_bounds__(64 * NW, 4) void DwPwPanelKernel(DwPwPanelArgs a)
         }
     }
     __syncthreads();                                     // the panel has been read; the outputs take its place
+    WithBits(a.pw_rq, [&](auto bits) {
 #pragma unroll
     for (int c = 0; c < CG; ++c)
     {
         const uint8_t* const tc = ptab + ((wave * CG + c) * 16 + 4 * g) * 4;
-        Fast4 f;
-        f.mp = *reinterpret_cast<const float4*>(tc);
-        f.bp = *reinterpret_cast<const float4*>(tc + 4 * G::NCOL);
-        f.mm = *reinterpret_cast<const float4*>(tc + 8 * G::NCOL);
-        f.bm = *reinterpret_cast<const float4*>(tc + 12 * G::NCOL);
+        const Fast4 f = {*reinterpret_cast<const float4*>(tc), *reinterpret_cast<const float4*>(tc + 4 * G::NCOL)};
         const int cq = min((bn * NW + wave) * CG + c, a.co_groups - 1) * 16 + 4 * g;
-        v4i corr = {0, 0, 0, 0};
-        if constexpr (U) corr = *reinterpret_cast<const v4i*>(a.pw_corr + cq);
 #pragma unroll
-        for (int p = 0; p < PG; ++p)
+        for (int p0 = 0; p0 < PG; p0 += PB)
         {
-            v4i v = acc[c][p];
-            if constexpr (U) v += corr + xs[p];
-            *reinterpret_cast<uint32_t*>(panel_lds + (16 * p + j) * OP + (wave * CG + c) * 16 + 4 * g) =
-                Requant4Dev(v[0], v[1], v[2], v[3], f.mp, f.bp, f.mm, f.bm, a.pw_ct, U ? nullptr : a.pw_corr, cq, a.pw_rq);
+            v4i v[PB];
+            uint32_t out[PB];
+#pragma unroll
+            for (int i = 0; i < PB; ++i)
+            {
+                v[i] = acc[c][p0 + i];
+                if constexpr (U) v[i] += xs[p0 + i];
+            }
+            RequantPixels<decltype(bits)::value, PB>(v, out, f, a.pw_ct, cq, a.pw_rq);
+#pragma unroll
+            for (int i = 0; i < PB; ++i) *reinterpret_cast<uint32_t*>(panel_lds + (16 * (p0 + i) + j) * OP + (wave * CG + c) * 16 + 4 * g) = out[i];
         }
     }
+    });
     __syncthreads();
     const OutPtr outp = MakeOutPtr(a.y, a.y_bytes);
     constexpr int CHUNKS = NW * CG;                      // 16-byte pieces per pixel

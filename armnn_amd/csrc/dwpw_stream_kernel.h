@@ -4,15 +4,14 @@
 // Run apart, these layers are bound by memory: the tensor between them is written once and read once (112 x 112 x 32 at 64
 // images: 26 MB each way, next to 26 MB in and 51 MB out).  Here it never leaves the CU.
 //   * A block of four (or eight) waves is persistent: it keeps the pointwise weights (at most 256 x 128 bytes) and the pointwise
-//     layer's requantization rows in LDS for its whole life and walks items -- TH x TW output pixels of one image over ALL
+//     layer's constants in LDS for its whole life and walks items -- TH x TW output pixels of one image over ALL
 //     channels -- with the next item's input halo in flight (in registers) while the current one is computed.  Two barriers
 //     per item: halo staged / panel complete.
 //   * Depthwise phase: the matrix-core arithmetic of DepthwiseMfmaKernel (16 channels x 16 pixels x 4 taps per
 //     v_mfma_i32_16x16x64_i8 over diagonal weight operands kept in registers), requantized with the depthwise layer's own
 //     constants; the codes -- the bytes the separate layer would have stored, shifted to int8 where they are uint8 -- go
 //     to an LDS panel [pixel][channel].
-//   * Pointwise phase: v_mfma_i32_32x32x32_i8 over the panel and the resident weights; accumulators start at zero (the
-//     zero-point correction is part of rows 6 / 7 of the channel table), the requantized dwords pass through a wave-private
+//   * Pointwise phase: v_mfma_i32_32x32x32_i8 over the panel and the resident weights; the requantized dwords pass through a wave-private
 //     LDS area and leave as 16 bytes per lane.
 //   * Loads and stores of a wave complete in issue order and share one counter: an item's stores are issued at the start of
 //     the next iteration, ahead of that iteration's loads, so the wait for those loads covers nothing younger.
@@ -83,7 +82,7 @@ struct DwPwStreamGeom
     static constexpr int KP = C + 16;                     // bytes per panel row and per weight row in LDS
     static constexpr int PANEL = P * KP;
     static constexpr int WTS = NO * KP;
-    static constexpr int TAB = 4 * NO * 4;
+    static constexpr int TAB = 3 * NO * 4;
     static constexpr int MT = P / 32, NTL = NO / 32;      // 32 x 32 MFMA tiles of an item's output
     static constexpr bool BYN = NTL >= NW;                // a wave owns output channels (all pixels) or pixels (all channels)
     static constexpr int MTW = BYN ? MT : MT / NW;
@@ -110,6 +109,8 @@ void DwPwStreamKernel(DwPwStreamArgs a)
     constexpr int NT = G::NT, NCG = G::NCG, HR = G::HR, HC = G::HC, PITCH = G::PITCH, ROWP = G::ROWP, HALO = G::HALO;
     constexpr int CGW = G::CGW, WPC = G::WPC, UNITS = G::UNITS, KP = G::KP, MTW = G::MTW, NTW = G::NTW, LDO = G::LDO, QUADS = G::QUADS;
     constexpr int RPG = 16 / TW;
+    // pixel groups whose depthwise outputs are computed together (a pass at 64 images: 4 170.8, 2 171.3, 1 172.1 us)
+    constexpr int UB = UNITS % 4 == 0 ? 4 : UNITS % 2 == 0 ? 2 : 1;
     constexpr int CPP = C / 16;
     constexpr int NCH = HR * HC * CPP;
     constexpr int NST = (NCH + NT - 1) / NT;
@@ -131,11 +132,11 @@ void DwPwStreamKernel(DwPwStreamArgs a)
         const int row = i / CPP, part = i % CPP;
         *reinterpret_cast<v4i*>(lds + WTS0 + row * KP + part * 16) = *reinterpret_cast<const v4i*>(a.w + static_cast<long long>(row) * a.w_stride + part * 16);
     }
-    for (int i = tid; i < NO; i += NT)                  // [4][NO / 4] float4: m+, b+ (corr folded in), m-, b- (corr folded in)
+    for (int i = tid; i < NO / 4 * 3; i += NT)          // [3][NO / 4] pieces: m, b, and what the accumulators start from
     {
         const int r = i / (NO / 4), col4 = i % (NO / 4);
-        const int src_row = r == 0 ? 2 : r == 1 ? 6 : r == 2 ? 4 : 7;
-        *reinterpret_cast<float4*>(lds + TAB0 + i * 16) = *reinterpret_cast<const float4*>(a.pw_ct.p + src_row * a.pw_ct.stride + col4 * 4);
+        *reinterpret_cast<v4i*>(lds + TAB0 + i * 16) =
+            *(r < 2 ? reinterpret_cast<const v4i*>(a.pw_ct.p + (r + 2) * a.pw_ct.stride + col4 * 4) : reinterpret_cast<const v4i*>(a.pw_corr + col4 * 4));
     }
 
     // ---- staging of the input halo (as in DepthwiseMfmaKernel, all C channels) -------------------------------------------
@@ -260,18 +261,25 @@ void DwPwStreamKernel(DwPwStreamArgs a)
 #pragma unroll
         for (int i = 0; i < CGW; ++i)
 #pragma unroll
-            for (int u = 0; u < UNITS; ++u)
+            for (int u0 = 0; u0 < UNITS; u0 += UB)
             {
-                const int lo = halo + i * 16 + u * (WPC * RPG * S * ROWP);
-                const v4i b0 = *reinterpret_cast<const v4i*>(lds + lds_tap[0] + lo);
-                const v4i b1 = *reinterpret_cast<const v4i*>(lds + lds_tap[1] + lo);
-                const v4i b2 = *reinterpret_cast<const v4i*>(lds + lds_tap[2] + lo);
-                v4i acc = corr4[i];
-                acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(wa[i][0], b0, acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(wa[i][1], b1, acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(wa[i][2], b2, acc, 0, 0, 0);
-                const uint32_t q = Requant4Dev(acc[0], acc[1], acc[2], acc[3], f4[i], a.dw_ct, (cg0 + i) * 16 + 4 * g, a.dw_rq) ^ a.mid_xor;
-                *reinterpret_cast<uint32_t*>(lds + panel_write + i * 16 + u * (WPC * 16 * KP)) = q;
+                v4i acc[UB];
+                uint32_t q[UB];
+#pragma unroll
+                for (int k = 0; k < UB; ++k)
+                {
+                    const int lo = halo + i * 16 + (u0 + k) * (WPC * RPG * S * ROWP);
+                    const v4i b0 = *reinterpret_cast<const v4i*>(lds + lds_tap[0] + lo);
+                    const v4i b1 = *reinterpret_cast<const v4i*>(lds + lds_tap[1] + lo);
+                    const v4i b2 = *reinterpret_cast<const v4i*>(lds + lds_tap[2] + lo);
+                    acc[k] = corr4[i];
+                    acc[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wa[i][0], b0, acc[k], 0, 0, 0);
+                    acc[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wa[i][1], b1, acc[k], 0, 0, 0);
+                    acc[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wa[i][2], b2, acc[k], 0, 0, 0);
+                }
+                RequantPixels<true, UB>(acc, q, f4[i], a.dw_ct, (cg0 + i) * 16 + 4 * g, a.dw_rq);
+#pragma unroll
+                for (int k = 0; k < UB; ++k) *reinterpret_cast<uint32_t*>(lds + panel_write + i * 16 + (u0 + k) * (WPC * 16 * KP)) = q[k] ^ a.mid_xor;
             }
     };
     auto pointwise = [&](int b) {
@@ -279,11 +287,21 @@ void DwPwStreamKernel(DwPwStreamArgs a)
         out_base = ((w.ty * TH) * a.Wo + w.tx * TW) * NO;
         out_cols = a.Wo - w.tx * TW;
         out_n = w.n;
+        const float* tab = reinterpret_cast<const float*>(lds + TAB0);
         v16i acc[MTW][NTW];
 #pragma unroll
-        for (int mt = 0; mt < MTW; ++mt)
+        for (int nt = 0; nt < NTW; ++nt)
+        {
+            v16i init;
 #pragma unroll
-            for (int nt = 0; nt < NTW; ++nt) acc[mt][nt] = v16i{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+            for (int q = 0; q < 4; ++q)
+            {
+                const v4i c4 = *reinterpret_cast<const v4i*>(tab + 2 * NO + (n0 + nt) * 32 + 8 * q + 4 * frag_half);
+                init[4 * q + 0] = c4[0]; init[4 * q + 1] = c4[1]; init[4 * q + 2] = c4[2]; init[4 * q + 3] = c4[3];
+            }
+#pragma unroll
+            for (int mt = 0; mt < MTW; ++mt) acc[mt][nt] = init;
+        }
 #pragma unroll
         for (int ks = 0; ks < C / 32; ++ks)
         {
@@ -297,25 +315,23 @@ void DwPwStreamKernel(DwPwStreamArgs a)
 #pragma unroll
                 for (int nt = 0; nt < NTW; ++nt) acc[mt][nt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fw[nt], fa[mt], acc[mt][nt], 0, 0, 0);
         }
-        const float* tab = reinterpret_cast<const float*>(lds + TAB0);
+        WithBits(a.pw_rq, [&](auto bits) {
 #pragma unroll
         for (int nt = 0; nt < NTW; ++nt)
 #pragma unroll
             for (int q = 0; q < 4; ++q)
             {
                 const int cl = (n0 + nt) * 32 + 8 * q + 4 * frag_half;
-                const float4 mp = *reinterpret_cast<const float4*>(tab + cl);
-                const float4 bp = *reinterpret_cast<const float4*>(tab + NO + cl);
-                const float4 mm = *reinterpret_cast<const float4*>(tab + 2 * NO + cl);
-                const float4 bm = *reinterpret_cast<const float4*>(tab + 3 * NO + cl);
+                const Fast4 f = {*reinterpret_cast<const float4*>(tab + cl), *reinterpret_cast<const float4*>(tab + NO + cl)};
+                v4i v[MTW];
+                uint32_t out[MTW];
 #pragma unroll
-                for (int mt = 0; mt < MTW; ++mt)
-                {
-                    const v16i& v = acc[mt][nt];
-                    const uint32_t out = Requant4Dev(v[4 * q + 0], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3], mp, bp, mm, bm, a.pw_ct, a.pw_corr, cl, a.pw_rq);
-                    *reinterpret_cast<uint32_t*>(lds + out_write + mt * 32 * LDO + nt * 32 + 8 * q) = out;
-                }
+                for (int mt = 0; mt < MTW; ++mt) v[mt] = Quad(acc[mt][nt], q);
+                RequantPixels<decltype(bits)::value, MTW>(v, out, f, a.pw_ct, cl, a.pw_rq);
+#pragma unroll
+                for (int mt = 0; mt < MTW; ++mt) *reinterpret_cast<uint32_t*>(lds + out_write + mt * 32 * LDO + nt * 32 + 8 * q) = out[mt];
             }
+        });
     };
 
     issue(item);

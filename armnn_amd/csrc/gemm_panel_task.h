@@ -9,9 +9,8 @@
 //     operations of a wave complete in issue order on this architecture, loads and stores alike, so the wait for a ring slot
 //     counts the stores issued since as well.
 //   * No vector load sits inside the sequence: a load's result can only be awaited together with everything issued
-//     before it, which would drain the weight stream at every column tile.  So the accumulators start at zero (the
-//     zero-point correction is part of the bracket constants, rows 6 / 7 of the channel table) and the four bracket rows
-//     of all output channels are staged in LDS before the first step.
+//     before it, which would drain the weight stream at every column tile.  So what the accumulators start from and rows 2
+//     and 3 of the channel table are staged in LDS for all output channels before the first step.
 //   * LDS images, swizzle, fragment reads and MFMA shape are those of IgemmLdsTile<64, 64, 2, 2>, and the requantization
 //     bracket closes on the exact result or falls back to it: the bytes written are identical.
 #pragma once
@@ -30,7 +29,7 @@ namespace mi355x
 template <int ST, int NK>
 constexpr int GemmPanelSmemBytes(int ncol)
 {
-    return NK * 64 * 128 + ST * 64 * 128 + 64 * (64 + 16) + 4 * ncol * 4;
+    return NK * 64 * 128 + ST * 64 * 128 + 64 * (64 + 16) + 3 * ncol * 4;
 }
 constexpr int kGemmPanelMaxCols = 1024;
 
@@ -50,7 +49,7 @@ __device__ __forceinline__ void GemmPanelTask(const IgemmArgs& a, const int tm, 
     uint8_t* const panel = smem;                              // [NK][64 rows][128 B]
     uint8_t* const ring = smem + NK * BM * BK;                // [ST][64 channels][128 B]
     uint8_t* const Os = ring + ST * BN * BK;                  // [64][LDO] output bytes of one column tile
-    float* const tab = reinterpret_cast<float*>(Os + BM * LDO); // [4][ncol]: m+, b+ with corr folded in, m-, b- with corr folded in
+    float* const tab = reinterpret_cast<float*>(Os + BM * LDO); // [3][ncol]: m, b and (as integers) what the accumulators start from
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -73,17 +72,16 @@ __device__ __forceinline__ void GemmPanelTask(const IgemmArgs& a, const int tm, 
     const int tiles_n = a.tiles_n;
     const int steps = tiles_n * NK;
     const int ncol = tiles_n * BN;                             // <= the table's row stride (channels are padded to 128)
-    // the bracket rows of every output channel: requested first, written to LDS once the panel and the first weight tiles
+    // the constants of every output channel: requested first, written to LDS once the panel and the first weight tiles
     // have been requested behind them
-    constexpr int TABV = 4 * kGemmPanelMaxCols / 4 / NT;       // float4 pieces per thread at most
+    constexpr int TABV = 3 * kGemmPanelMaxCols / 4 / NT;       // float4 pieces per thread at most
     float4 tv[TABV];
 #pragma unroll
     for (int i = 0; i < TABV; ++i)
     {
-        const int e = min(tid + i * NT, ncol - 1);             // float4 index within [4][ncol / 4], clamped
+        const int e = min(tid + i * NT, ncol / 4 * 3 - 1);     // float4 index within [3][ncol / 4], clamped
         const int row = e / (ncol / 4), col4 = e - row * (ncol / 4);
-        const int src_row = row == 0 ? 2 : row == 1 ? 6 : row == 2 ? 4 : 7;
-        tv[i] = *reinterpret_cast<const float4*>(a.ct.p + src_row * a.ct.stride + col4 * 4);
+        tv[i] = *(row < 2 ? reinterpret_cast<const float4*>(a.ct.p + (row + 2) * a.ct.stride + col4 * 4) : reinterpret_cast<const float4*>(a.corr + col4 * 4));
     }
     // weights of step s = (column tile s / NK, k-tile s % NK) into ring slot `slot`
     auto load_b = [&](int s, int slot) {
@@ -107,7 +105,7 @@ __device__ __forceinline__ void GemmPanelTask(const IgemmArgs& a, const int tm, 
 
 #pragma unroll
     for (int i = 0; i < TABV; ++i)
-        if (tid + i * NT < ncol) *reinterpret_cast<float4*>(tab + (tid + i * NT) * 4) = tv[i];
+        if (tid + i * NT < ncol / 4 * 3) *reinterpret_cast<float4*>(tab + (tid + i * NT) * 4) = tv[i];
     // (the first step's barrier orders these writes before the first write-out reads them)
 
     const int lane_c = 4 * (lane >> 5);
@@ -121,7 +119,7 @@ __device__ __forceinline__ void GemmPanelTask(const IgemmArgs& a, const int tm, 
     int slot = 0;
     for (int tn = 0; tn < tiles_n; ++tn)
     {
-        v16i acc = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+        v16i acc;
 #pragma unroll
         for (int kt = 0; kt < NK; ++kt)
         {
@@ -151,6 +149,15 @@ __device__ __forceinline__ void GemmPanelTask(const IgemmArgs& a, const int tm, 
                 if (ls >= ST) ls -= ST;
                 load_b(s + ST - 1, ls);
             }
+            if (kt == 0)                         // (behind the first barrier: the table is in LDS)
+            {
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                {
+                    const v4i c4 = *reinterpret_cast<const v4i*>(tab + 2 * ncol + tn * BN + wn * 32 + 8 * q + lane_c);
+                    acc[4 * q + 0] = c4[0]; acc[4 * q + 1] = c4[1]; acc[4 * q + 2] = c4[2]; acc[4 * q + 3] = c4[3];
+                }
+            }
             const uint8_t* As = panel + kt * BM * BK;
             const uint8_t* Bs = ring + slot * BN * BK;
             v4i fa[4], fw[4];
@@ -173,12 +180,9 @@ __device__ __forceinline__ void GemmPanelTask(const IgemmArgs& a, const int tm, 
         {
             const int cl = wn * 32 + 8 * q + lane_c;
             const int c = tn * BN + cl;
-            const float4 mp = *reinterpret_cast<const float4*>(tab + c);
-            const float4 bp = *reinterpret_cast<const float4*>(tab + ncol + c);
-            const float4 mm = *reinterpret_cast<const float4*>(tab + 2 * ncol + c);
-            const float4 bm = *reinterpret_cast<const float4*>(tab + 3 * ncol + c);
-            // the rare exact path reads rows 0 / 1 and the correction from global memory (and waits for everything in flight)
-            const uint32_t out = Requant4Dev(acc[4 * q + 0], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3], mp, bp, mm, bm, a.ct, a.corr, c, a.rq);
+            const Fast4 f4 = {*reinterpret_cast<const float4*>(tab + c), *reinterpret_cast<const float4*>(tab + ncol + c)};
+            // the rare exact path reads rows 0 / 1 from global memory (and waits for everything in flight)
+            const uint32_t out = Requant4Any(acc[4 * q + 0], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3], f4, a.ct, c, a.rq);
             const int pl = wm * 32 + (lane & 31);
             *reinterpret_cast<uint32_t*>(Os + pl * LDO + cl) = out;
         }

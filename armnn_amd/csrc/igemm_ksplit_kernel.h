@@ -128,7 +128,7 @@ __global__ __launch_bounds__(256 * KG) void IgemmKSplitKernel(IgemmArgs a)
         advance(KG);
     };
 
-    // ---- accumulators: group 0 starts at the zero-point correction, the others at zero ------------------------------------
+    // ---- accumulators: group 0 starts from the plan's constants, the others at zero ------------------------------------
     const int lane_c = 4 * (lane >> 5);
     const int cbase = tn * BN + wn * 32;
     v16i acc;
@@ -209,15 +209,19 @@ __global__ __launch_bounds__(256 * KG) void IgemmKSplitKernel(IgemmArgs a)
                 const v4i p4 = part[(((g - 1) * 4 + wave) * 4 + q) * 64 + lane];
                 acc[4 * q + 0] += p4[0]; acc[4 * q + 1] += p4[1]; acc[4 * q + 2] += p4[2]; acc[4 * q + 3] += p4[3];
             }
+        const int cl = wn * 32 + lane_c;
+        v4i v[4];
+        Fast4 f[4];
+        uint32_t out[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q)
         {
-            const int cl = wn * 32 + 8 * q + lane_c;
-            const Fast4 f4 = LoadFast4(a.ct, tn * BN + cl);
-            const uint32_t out = Requant4Dev(acc[4 * q + 0], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3], f4, a.ct, tn * BN + cl, a.rq);
-            const int pl = wm * 32 + (lane & 31);
-            *reinterpret_cast<uint32_t*>(Os + pl * LDO + cl) = out;
+            v[q] = Quad(acc, q);
+            f[q] = LoadFast4(a.ct, tn * BN + cl + 8 * q);
         }
+        WithBits(a.rq, [&](auto bits) { RequantChannels<decltype(bits)::value, 4, 8>(v, out, f, a.ct, tn * BN + cl, a.rq); });
+#pragma unroll
+        for (int q = 0; q < 4; ++q) *reinterpret_cast<uint32_t*>(Os + (wm * 32 + (lane & 31)) * LDO + cl + 8 * q) = out[q];
     }
     __syncthreads();
     constexpr int CHUNKS = BN / 16;

@@ -176,7 +176,7 @@ __device__ __forceinline__ void IgemmLdsTile(const IgemmArgs& a, const int tile,
         }
     };
 
-    // ---- accumulators start at the zero-point correction ---------------------------------------------------------
+    // ---- accumulators start from the plan's constants ---------------------------------------------------------
     const int lane_c = 4 * (lane >> 5);
     const int cbase = tn * BN + wn * WTN;
     v16i acc[TC][TP];
@@ -332,6 +332,7 @@ __device__ __forceinline__ void IgemmLdsTile(const IgemmArgs& a, const int tile,
 #pragma unroll
         for (int tp = 0; tp < TP; ++tp) rowsum[tp] = (rowsum[tp] + __shfl_xor(rowsum[tp], 32) - a.rowsum_bias) * a.zw_neg;
     }
+    WithBits(a.rq, [&](auto bits) {
 #pragma unroll
     for (int tc = 0; tc < TC; ++tc)
     {
@@ -340,17 +341,16 @@ __device__ __forceinline__ void IgemmLdsTile(const IgemmArgs& a, const int tile,
         {
             const int cl = wn * WTN + tc * 32 + 8 * q + lane_c;
             const Fast4 f4 = LoadFast4(a.ct, tn * BN + cl);
+            v4i v[TP];
+            uint32_t out[TP];
 #pragma unroll
-            for (int tp = 0; tp < TP; ++tp)
-            {
-                const v16i& c = acc[tc][tp];
-                const int rt = AW ? rowsum[tp] : 0;
-                const uint32_t out = Requant4Dev(c[4 * q + 0] + rt, c[4 * q + 1] + rt, c[4 * q + 2] + rt, c[4 * q + 3] + rt, f4, a.ct, tn * BN + cl, a.rq);
-                const int pl = wm * WTM + tp * 32 + (lane & 31);
-                *reinterpret_cast<uint32_t*>(Os + pl * LDO + cl) = out;
-            }
+            for (int tp = 0; tp < TP; ++tp) v[tp] = Quad(acc[tc][tp], q) + (AW ? rowsum[tp] : 0);
+            RequantPixels<decltype(bits)::value, TP>(v, out, f4, a.ct, tn * BN + cl, a.rq);
+#pragma unroll
+            for (int tp = 0; tp < TP; ++tp) *reinterpret_cast<uint32_t*>(Os + (wm * WTM + tp * 32 + (lane & 31)) * LDO + cl) = out[tp];
         }
     }
+    });
     __syncthreads();
     after_loads();
     if (!EARLY && fuse) load_other();

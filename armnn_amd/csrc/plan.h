@@ -31,19 +31,18 @@ struct mi355x_conv2d_s
     int8_t*  w_stem   = nullptr;   // small-Ci conv on MFMA: [Co rounded up to 32][stem_kp]
     int8_t*  w_stem2  = nullptr;   // ... the second halves of weight differences that need two
     int      stem_kp  = 0;
-    uint32_t* dw_grp  = nullptr;   // depthwise 3x3: constants per group of 4 channels for the fused dw+pw kernel
+    uint32_t* dw_grp  = nullptr;   // depthwise 3x3: constants per group of 4 channels (kDwGrpDwords each: weight rows 0 .. 2, corr, m, b)
     uint32_t* w_dot4  = nullptr;   // depthwise 3x3: [C][4] dwords; small-Ci conv: [Co][Kh][RD] dwords
     uint32_t* w_dot4b = nullptr;   // depthwise 3x3 / small-Ci conv whose weight differences need two int8 halves: the second halves
     int variant = 0;               // kernel variant within an algo (see RunPlan)
     int row_dwords = 0;            // small-Ci conv: dwords per filter row
-    float*   chan     = nullptr;   // [8][Co_pad] per-channel requantization constants (rows: see ChanTab)
-    int32_t* corr     = nullptr;   // [Co_pad]  -zx' * sum_k w[c][k]
+    float*   chan     = nullptr;   // [4][Co_pad] per-channel requantization constants (rows: see ChanTab)
+    int32_t* corr     = nullptr;   // [Co_pad]  what accumulators of raw products start from: -zx' * sum_k w[c][k] + Requant::acc_base
     int K = 0, K_pad = 0, Co_pad = 0;
     int pw_blocks_per_cu = 1, pw_n_cu = 256;     // weight-stationary kernel: blocks a CU holds at once, CUs of the device
     int pw_blocks_per_cu_64 = 0;                 // ... with 64-channel slabs, where the plan's own slab is 128 (0: not prepared)
-    std::vector<float> chan_host;  // host copy, completed with the corr-folded rows once corr is known
-    std::vector<float> fast_fm, fast_fb;   // per channel: the unwidened fast-path constants and the constant half-width of the
-    std::vector<double> fast_cw;           // bracket (negative: no fast path), kept until the table is uploaded
+    std::vector<float> chan_host;  // host copy of `chan` until it is uploaded
+    long long acc_most = 0;        // no complete sum is larger than this in magnitude
     int pw_bn = 0, pw_ks = 0;      // pointwise GEMM kernel configuration (0: not applicable)
     bool bk128 = false;            // implicit GEMM walks K in 128-byte tiles
     bool k_tail = false;           // 1x1 plan whose K ends inside a 128-byte k-tile, zero padded to whole ones

@@ -29,7 +29,7 @@ struct PwArgs
 {
     const uint8_t* x;
     const int8_t*  w;        // [>= n_slabs*BN][w_stride], rows zero padded
-    ChanTab        ct;       // rows 0,1 exact; rows 2,5,6: fm, fb + corr*fm, threshold for the corr-folded form
+    ChanTab        ct;
     const int32_t* corr;
     uint8_t*       y;
     int M, K, N;
@@ -45,7 +45,7 @@ struct PwArgs
 template <int BN>
 constexpr int PwSmemBytes(int K)
 {
-    return BN * (K + 16) + 4 * 32 * (BN + 16) + 4 * BN * 4;
+    return BN * (K + 16) + 4 * 32 * (BN + 16) + 3 * BN * 4;
 }
 
 // KS = MFMA k-steps (of 32) per register chunk, K % (32 * KS) == 0;  NB = register chunks per wave (NB-1 in flight).
@@ -59,8 +59,8 @@ __global__ __launch_bounds__(256) void PwGemmKernel(PwArgs a)
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int LDW = a.K + 16;
     uint8_t* slab = smem;
-    float* cst = reinterpret_cast<float*>(smem + BN * LDW);                 // [4][BN]: the corr-folded bracket m+, bc+, m-, bc-
-    uint8_t* ostage_all = smem + BN * LDW + 4 * BN * 4;
+    float* cst = reinterpret_cast<float*>(smem + BN * LDW);                 // [3][BN]: m, b and (as integers) what the accumulators start from
+    uint8_t* ostage_all = smem + BN * LDW + 3 * BN * 4;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -95,11 +95,21 @@ __global__ __launch_bounds__(256) void PwGemmKernel(PwArgs a)
         for (int ks = 0; ks < KS; ++ks) buf[ks] = *reinterpret_cast<const v4i*>(p + ks * 32);
     };
 
-    // FIRST: the chunk opens a tile; its first MFMA takes a zero C operand instead of cleared registers
+    // FIRST: the chunk opens a tile, whose accumulators start from the plan's constants
     auto compute_chunk = [&](v4i (&buf)[KS], int ch, auto first) {
         constexpr bool FIRST = decltype(first)::value;
         const uint8_t* wbase = slab + frag_row * LDW + ch * (32 * KS) + frag_k;
-        const v16i zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+        if constexpr (FIRST)
+        {
+#pragma unroll
+            for (int tc = 0; tc < TC; ++tc)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                {
+                    const v4i c4 = *reinterpret_cast<const v4i*>(cst + 2 * BN + tc * 32 + 8 * q + 4 * (lane >> 5));
+                    acc[tc][4 * q + 0] = c4[0]; acc[tc][4 * q + 1] = c4[1]; acc[tc][4 * q + 2] = c4[2]; acc[tc][4 * q + 3] = c4[3];
+                }
+        }
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
         {
@@ -114,7 +124,7 @@ __global__ __launch_bounds__(256) void PwGemmKernel(PwArgs a)
             for (int tc = 0; tc < TC; ++tc)
             {
                 const v4i wv = *reinterpret_cast<const v4i*>(wbase + tc * 32 * LDW + ks * 32);
-                acc[tc] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wv, av, (FIRST && ks == 0) ? zero : acc[tc], 0, 0, 0);
+                acc[tc] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wv, av, acc[tc], 0, 0, 0);
             }
         }
     };
@@ -143,18 +153,19 @@ __global__ __launch_bounds__(256) void PwGemmKernel(PwArgs a)
 #pragma unroll
         for (int tc = 0; tc < TC; ++tc)
         {
+            const int cl = tc * 32 + lane_c;
+            v4i v[4];
+            Fast4 f[4];
+            uint32_t out[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q)
             {
-                const int cl = tc * 32 + 8 * q + lane_c;
-                const float4 mp = *reinterpret_cast<const float4*>(cst + cl);
-                const float4 bp = *reinterpret_cast<const float4*>(cst + BN + cl);
-                const float4 mm = *reinterpret_cast<const float4*>(cst + 2 * BN + cl);
-                const float4 bm = *reinterpret_cast<const float4*>(cst + 3 * BN + cl);
-                const uint32_t out = Requant4Dev(acc[tc][4 * q + 0] + rt, acc[tc][4 * q + 1] + rt, acc[tc][4 * q + 2] + rt, acc[tc][4 * q + 3] + rt,
-                                                 mp, bp, mm, bm, a.ct, a.corr, n0 + cl, a.rq);
-                *reinterpret_cast<uint32_t*>(ostage + frag_row * LDO + cl) = out;
+                v[q] = Quad(acc[tc], q) + rt;
+                f[q] = {*reinterpret_cast<const float4*>(cst + cl + 8 * q), *reinterpret_cast<const float4*>(cst + BN + cl + 8 * q)};
             }
+            WithBits(a.rq, [&](auto bits) { RequantChannels<decltype(bits)::value, 4, 8>(v, out, f, a.ct, n0 + cl, a.rq); });
+#pragma unroll
+            for (int q = 0; q < 4; ++q) *reinterpret_cast<uint32_t*>(ostage + frag_row * LDO + cl + 8 * q) = out[q];
         }
         // the wave reads back what its own lanes wrote: LDS operations of one wave complete in order; the fences keep
         // the compiler from moving the reads above the writes (different lanes, so no dependency it can see)
@@ -230,12 +241,10 @@ __global__ __launch_bounds__(256) void PwGemmKernel(PwArgs a)
 #pragma unroll
             for (int i = 0; i < BN / 16; ++i) *reinterpret_cast<v4i*>(slab + ((tid >> 4) + 16 * i) * LDW + c * 16) = t[i];
         }
-        for (int i = tid; i < 4 * BN; i += 256)
+        for (int i = tid; i < 3 * BN; i += 256)
         {
-            // the corr-folded bracket: m+, bc+, m-, bc-
             const int row = i / BN, c = i - row * BN;
-            const int src_row = row == 0 ? 2 : row == 1 ? 6 : row == 2 ? 4 : 7;
-            cst[i] = a.ct.p[src_row * a.ct.stride + n0 + c];
+            cst[i] = row < 2 ? a.ct.p[(row + 2) * a.ct.stride + n0 + c] : __builtin_bit_cast(float, a.corr[n0 + c]);
         }
     }
     __syncthreads();
@@ -345,7 +354,7 @@ __global__ __launch_bounds__(256) void GemvKernel(GemvArgs a)
             int v = acc[r][m];
             for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
             if (lane == 0 && n0 + r < a.N)
-                a.y[static_cast<long long>(m) * a.N + n0 + r] = static_cast<uint8_t>(Requant1FoldedDev(v, a.ct, a.corr, n0 + r, a.rq));
+                a.y[static_cast<long long>(m) * a.N + n0 + r] = static_cast<uint8_t>(Requant1Dev(v + a.corr[n0 + r], a.ct, n0 + r, a.rq));
         }
 }
 
@@ -417,11 +426,8 @@ __device__ __forceinline__ void SmallMGemmTile(const GemvArgs& a, int n0, int m0
     // accumulator group g of the 32x32 tile: channels 8 g + 4 (lane / 32) + 0..3 of row lane % 32
     const int c = n0 + 8 * wave + 4 * (lane >> 5);
     const int row = m0 + frag_row;
-    const float4 mp = *reinterpret_cast<const float4*>(a.ct.p + 2 * a.ct.stride + c);
-    const float4 bp = *reinterpret_cast<const float4*>(a.ct.p + 6 * a.ct.stride + c);
-    const float4 mm = *reinterpret_cast<const float4*>(a.ct.p + 4 * a.ct.stride + c);
-    const float4 bm = *reinterpret_cast<const float4*>(a.ct.p + 7 * a.ct.stride + c);
-    const uint32_t out = Requant4Dev(v[0], v[1], v[2], v[3], mp, bp, mm, bm, a.ct, a.corr, c, a.rq);
+    const v4i corr = *reinterpret_cast<const v4i*>(a.corr + c);
+    const uint32_t out = Requant4Any(v[0] + corr[0], v[1] + corr[1], v[2] + corr[2], v[3] + corr[3], LoadFast4(a.ct, c), a.ct, c, a.rq);
     if constexpr (THROUGH)
     {
         // Bytes written through one by one are slow, and rows of N bytes start anywhere: the tile meets in LDS (in `part`,

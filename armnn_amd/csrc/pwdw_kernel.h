@@ -46,7 +46,7 @@ struct PwDwArgs
     int tiles_n;                // C / 64
     int total_blocks, xcd_chunk;
     // depthwise stage
-    const uint32_t* dw_grp;     // [C/4][8][4] dwords per group of 4 channels: w row 0, w row 1, w row 2, corr, m+, b+, m-, b-
+    const uint32_t* dw_grp;     // per group of 4 channels, kDwGrpDwords: rows of four, w row 0, w row 1, w row 2, corr, m, b
     ChanTab         dw_ct;
     Requant         dw_rq;
     uint32_t        dw_xor;     // 0x80808080 when the intermediate tensor is uint8: T holds the signed-shifted codes
@@ -202,15 +202,13 @@ __global__ __launch_bounds__(64 * NW) void PwDwKernel(PwDwArgs a)
     // ---- depthwise constants of this thread's 4 channels, requested before the GEMM's tiles ---------------------------
     const int c4 = tid & 15;
     v4i w0 = {}, w1 = {}, w2 = {}, corr4 = {};
-    float4 dmp = {}, dbp = {}, dmm = {}, dbm = {};
+    Fast4 df4 = {};
     if constexpr (!POOL)
     {
-        const v4i* gc = reinterpret_cast<const v4i*>(a.dw_grp + (tn * (BN / 4) + c4) * 32);
+        const v4i* gc = reinterpret_cast<const v4i*>(a.dw_grp + (tn * (BN / 4) + c4) * kDwGrpDwords);
         w0 = gc[0]; w1 = gc[1]; w2 = gc[2]; corr4 = gc[3];
-        dmp = *reinterpret_cast<const float4*>(gc + 4);
-        dbp = *reinterpret_cast<const float4*>(gc + 5);
-        dmm = *reinterpret_cast<const float4*>(gc + 6);
-        dbm = *reinterpret_cast<const float4*>(gc + 7);
+        df4.m = *reinterpret_cast<const float4*>(gc + 4);
+        df4.b = *reinterpret_cast<const float4*>(gc + 5);
     }
 
     const int nk = a.K_pad / BK;
@@ -268,7 +266,7 @@ __global__ __launch_bounds__(64 * NW) void PwDwKernel(PwDwArgs a)
                 const int cg = cbase + 8 * q + lane_c;
                 const Fast4 f4 = LoadFast4(a.pw_ct, cg);
                 const v16i& v = acc[tp];
-                const uint32_t out = Requant4Dev(v[4 * q + 0], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3], f4, a.pw_ct, cg, a.pw_rq);
+                const uint32_t out = Requant4Any(v[4 * q + 0], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3], f4, a.pw_ct, cg, a.pw_rq);
                 if (inside) *reinterpret_cast<uint32_t*>(cell + 8 * q) = POOL ? out : out ^ a.dw_xor;
             }
         }
@@ -367,7 +365,7 @@ __global__ __launch_bounds__(64 * NW) void PwDwKernel(PwDwArgs a)
 #pragma unroll
         for (int j = 0; j < 2; ++j)
         {
-            const uint32_t q = Requant4Dev(o[j][0], o[j][1], o[j][2], o[j][3], dmp, dbp, dmm, dbm, a.dw_ct, nullptr, cglob, a.dw_rq);
+            const uint32_t q = Requant4Dev<true>(o[j][0], o[j][1], o[j][2], o[j][3], df4, a.dw_ct, cglob, a.dw_rq);
             const int ox = xg * 2 + j;
             if (ox < a.Wo) *reinterpret_cast<uint32_t*>(yrow + static_cast<long long>(ox) * a.C) = q;
         }

@@ -97,6 +97,10 @@ __global__ __launch_bounds__(256, KB <= 256 ? 4 : 3) void RowPanelKernel(IgemmAr
 #pragma unroll
     for (int r = 0; r < RD; ++r)
         if (r < steps) load_weights(r, r);
+    // (what the accumulators start from)
+    v4i corr[CG];
+#pragma unroll
+    for (int c = 0; c < CG; ++c) corr[c] = *reinterpret_cast<const v4i*>(a.corr + cgrp[c] * 16 + 4 * g);
     // ---- the Addition's other input ---------------------------------------------------------------------------------------------
     v4i other[NP];
     const bool fuse = a.res != nullptr;
@@ -116,7 +120,7 @@ __global__ __launch_bounds__(256, KB <= 256 ? 4 : 3) void RowPanelKernel(IgemmAr
     {
         xs[p] = 0;
 #pragma unroll
-        for (int c = 0; c < CG; ++c) acc[c][p] = v4i{0, 0, 0, 0};
+        for (int c = 0; c < CG; ++c) acc[c][p] = corr[c];
     }
     const uint8_t* const pb = row_lds + g * GP + j * 16;
     for (int k0 = 0; k0 < a.Ci; k0 += KB)
@@ -168,27 +172,25 @@ __global__ __launch_bounds__(256, KB <= 256 ? 4 : 3) void RowPanelKernel(IgemmAr
     for (int c = 0; c < CG; ++c)
     {
         const int cq = cgrp[c] * 16 + 4 * g;
-        f[c].mp = *reinterpret_cast<const float4*>(a.ct.p + 2 * a.ct.stride + cq);
-        f[c].bp = *reinterpret_cast<const float4*>(a.ct.p + (AW ? 3 : 6) * a.ct.stride + cq);
-        f[c].mm = *reinterpret_cast<const float4*>(a.ct.p + 4 * a.ct.stride + cq);
-        f[c].bm = *reinterpret_cast<const float4*>(a.ct.p + (AW ? 5 : 7) * a.ct.stride + cq);
+        f[c] = LoadFast4(a.ct, cq);
     }
     __syncthreads();                                     // the rows have been read; the outputs take their place
+    WithBits(a.rq, [&](auto bits) {
 #pragma unroll
     for (int c = 0; c < CG; ++c)
     {
         const int cq = cgrp[c] * 16 + 4 * g;
-        v4i corr = {0, 0, 0, 0};
-        if constexpr (AW) corr = *reinterpret_cast<const v4i*>(a.corr + cq);
-#pragma unroll
-        for (int p = 0; p < PG; ++p)
+        uint32_t out[PG];
+        if constexpr (AW)
         {
-            v4i v = acc[c][p];
-            if constexpr (AW) v += corr + xs[p];
-            *reinterpret_cast<uint32_t*>(row_lds + (16 * p + j) * OP + (wave * CG + c) * 16 + 4 * g) =
-                Requant4Dev(v[0], v[1], v[2], v[3], f[c].mp, f[c].bp, f[c].mm, f[c].bm, a.ct, AW ? nullptr : a.corr, cq, a.rq);
+#pragma unroll
+            for (int p = 0; p < PG; ++p) acc[c][p] += xs[p];
         }
+        RequantPixels<decltype(bits)::value, PG>(acc[c], out, f[c], a.ct, cq, a.rq);
+#pragma unroll
+        for (int p = 0; p < PG; ++p) *reinterpret_cast<uint32_t*>(row_lds + (16 * p + j) * OP + (wave * CG + c) * 16 + 4 * g) = out[p];
     }
+    });
     __syncthreads();
     const OutPtr outp = MakeOutPtr(a.y, static_cast<long long>(a.M) * a.Co);
 #pragma unroll

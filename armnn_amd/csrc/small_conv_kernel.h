@@ -203,7 +203,7 @@ __global__ __launch_bounds__(256) void SmallConvKernel(IgemmArgs a)
             // what the bytes beyond K added are padding values
             v += (total - (steps * 64 - a.Kh * a.Kw * a.Ci) * static_cast<int>(static_cast<int8_t>(a.pad_word & 0xffu))) * a.zw_neg;
         }
-        stage[pg * 16 + j][cg * 4 + g] = Requant4Dev(v[0], v[1], v[2], v[3], f4, a.ct, cq, a.rq);
+        stage[pg * 16 + j][cg * 4 + g] = Requant4Any(v[0], v[1], v[2], v[3], f4, a.ct, cq, a.rq);
     }
     __syncthreads();
     if (wave == 0 && om < a.M && c0 < a.Co)

@@ -1,0 +1,80 @@
+"""The requantization's fast path over every sum a layer can meet, against the reference's own sequence (a division per value).
+
+A value's bytes come from a bracket around the reference's fp32 value and, where the bracket does not close, from that sequence.
+With two channels of full-range codes and weights 127 and 1 the sums of a 1x1 layer are all the integers of a range, so that
+each channel's scale and bias meet each of them."""
+import numpy as np
+import pytest
+
+from armnn_amd import shim
+from armnn_amd.tensor import DataType, QTensor, TensorInfo
+
+pytestmark = pytest.mark.gpu
+S8, U8 = DataType.QAsymmS8, DataType.QAsymmU8
+
+
+def _fast_and_exact(run):
+    fast = run()
+    shim.set_option("exact_division_epilogue", 1)
+    try:
+        exact = run()
+    finally:
+        shim.set_option("exact_division_epilogue", 0)
+    return fast, exact
+
+
+def _scales(kind, channels):
+    rng = np.random.default_rng(7)
+    if kind == "general":
+        return rng.uniform(0.002, 0.02, channels)
+    if kind == "powers_of_two":             # sums sit exactly on half-integers
+        return 2.0 ** -rng.integers(4, 12, channels)
+    if kind == "ratios":                    # ... now and then
+        return rng.choice([0.047, 0.02, 0.0235, 0.01], channels) / rng.choice([1, 2, 3, 8], channels)
+    if kind == "steps_of_codes":            # a code and more per step of the sum
+        return rng.uniform(0.05, 40.0, channels)
+    return rng.uniform(1e-9, 1e-7, channels)    # one code for all sums
+
+
+@pytest.mark.parametrize("clamp", [False, True], ids=["type_range", "clamp_inside"])
+@pytest.mark.parametrize("out", [(S8, -128), (U8, 3), (S8, 21)], ids=["s8", "u8", "s8_offset"])
+@pytest.mark.parametrize("kind", ["general", "powers_of_two", "ratios", "steps_of_codes", "one_code"])
+@pytest.mark.parametrize("ci", [16, 32, 256])
+def test_every_sum_of_a_range(kind, ci, out, clamp):
+    channels = 64
+    codes = np.arange(-128, 128, dtype=np.int8)
+    x = np.zeros((1, 256, 256, ci), np.int8)
+    x[0, :, :, 0], x[0, :, :, 1] = codes[:, None], codes[None, :]
+    w = np.zeros((channels, 1, 1, ci), np.int8)
+    w[:, 0, 0, 0], w[:, 0, 0, 1] = 127, 1
+    scales = _scales(kind, channels).astype(np.float32)
+    b = np.random.default_rng(11).integers(-9000, 9000, channels).astype(np.int32)
+    b[::5] = 0
+    xq = QTensor(TensorInfo(x.shape, S8, (0.5,), 0), x)
+    wq = QTensor(TensorInfo(w.shape, DataType.QSymmS8, tuple(scales), 0, 0), w)
+    bq = QTensor(TensorInfo((channels,), DataType.Signed32, tuple(np.float32(0.5) * scales), 0, 0), b)
+    info = TensorInfo((1, 256, 256, channels), out[0], (0.25,), out[1])
+    act = dict(activation=shim.ACT_BOUNDED_RELU, act_a=20.0, act_b=-1.5) if clamp else {}
+    fast, exact = _fast_and_exact(lambda: shim.conv2d(xq, wq, bq, info, **act).data)
+    print(f"{kind} {ci}: {shim.last_kernel()}, {len(np.unique(exact))} codes", flush=True)
+    np.testing.assert_array_equal(fast, exact)
+
+
+@pytest.mark.parametrize("scale", [1e-6, 2e-5, 6.2e-5, 1e-4, 3e-3])
+@pytest.mark.parametrize("m", [1, 40, 300])
+def test_sums_beyond_two_to_the_22nd(m, scale):
+    """Sums up to 1.3e8, where the bits of a raised accumulator no longer step in ones; with the small scales codes there are not
+    saturated, and the sums are converted."""
+    k, o = 4096, 128
+    rng = np.random.default_rng(m)
+    # rows whose codes and channels whose weights lean to one side more or less: sums of every size
+    x = np.clip(rng.integers(-128, 128, (m, k)) + np.linspace(-255, 255, m)[:, None], -128, 127).astype(np.int8)
+    w = np.clip(rng.integers(-127, 128, (o, k)) + np.linspace(-254, 254, o)[:, None], -127, 127).astype(np.int8)
+    scales = np.full(o, scale, np.float32) * np.linspace(0.5, 1.5, o).astype(np.float32)
+    xq = QTensor(TensorInfo((m, k), S8, (1.0,), -3), x)
+    wq = QTensor(TensorInfo((o, k), DataType.QSymmS8, tuple(scales), 0, 0), w)
+    bq = QTensor(TensorInfo((o,), DataType.Signed32, tuple(scales), 0, 0), rng.integers(-90000, 90000, o).astype(np.int32))
+    info = TensorInfo((m, o), S8, (1.0,), 5)
+    fast, exact = _fast_and_exact(lambda: shim.fully_connected(xq, wq, bq, info).data)
+    print(f"{m} rows, scale {scale}: {shim.last_kernel()}, {len(np.unique(exact))} codes", flush=True)
+    np.testing.assert_array_equal(fast, exact)
