@@ -32,7 +32,7 @@ constexpr int BigGemmSmemBytes()
 {
     constexpr int stages = ST * (BM + BN) * 128;
     constexpr int out = BM * (BN + 16);
-    return (stages > out ? stages : out) + 2 * BN * 4;       // + the block's slice of the per-channel table
+    return (stages > out ? stages : out) + 4 * BN * 4;       // + the block's slice of the per-channel table
 }
 
 // 2 x 2 waves, wave tile (BM / 2) x (BN / 2).  Needs Ci % 128 == 0 (a k-tile is 128 bytes of one filter tap) and
@@ -252,20 +252,20 @@ __global__ __launch_bounds__(256) void BigGemmKernel(IgemmArgs a, int xcd_rows)
     constexpr int LAST = (KS - 1) & 1;           // fragment buffer of a tile's last k-step
     constexpr int PRE = NM / 4;                  // MFMAs of the last k-step issued ahead of the barrier
 
-    // ---- the block's slice of the per-channel table (rows 2 and 3, BN channels) goes to LDS behind
+    // ---- the block's slice of the per-channel table (BN channels) goes to LDS behind
     // the stages: with one wave per SIMD nothing would hide the epilogue's table reads from global memory, one round trip
     // per channel quad.  The rare exact path reads its two rows from global memory.
     constexpr int TAB = (ST * STAGE > BM * LDO ? ST * STAGE : BM * LDO);
     float* tab_lds = reinterpret_cast<float*>(smem + TAB);
     {
-        constexpr int N4 = 2 * BN / 4;                     // float4 pieces
+        constexpr int N4 = 4 * BN / 4;                     // float4 pieces
         v4i piece[(N4 + 255) / 256];
 #pragma unroll
         for (int i = 0; i < (N4 + 255) / 256; ++i)
         {
             const int e = i * 256 + tid;
             const int row = e / (BN / 4), col = e - row * (BN / 4);
-            if (e < N4) piece[i] = *reinterpret_cast<const v4i*>(a.ct.p + static_cast<long long>(row + 2) * a.ct.stride + tn * BN + col * 4);
+            if (e < N4) piece[i] = *reinterpret_cast<const v4i*>(a.ct.p + static_cast<long long>(row) * a.ct.stride + tn * BN + col * 4);
         }
         // ---- prologue: ST tiles requested behind the table reads (older requests complete first) ...
 #pragma unroll
@@ -363,12 +363,12 @@ __global__ __launch_bounds__(256) void BigGemmKernel(IgemmArgs a, int xcd_rows)
         for (int q = 0; q < 4; ++q)
         {
             const int cl = wn * WTN + tc * 32 + 8 * q + lane_c;
-            const Fast4 f4 = {*reinterpret_cast<const float4*>(tab_lds + cl), *reinterpret_cast<const float4*>(tab_lds + BN + cl)};
+            const Fast4 f4 = {*reinterpret_cast<const float4*>(tab_lds + 2 * BN + cl), *reinterpret_cast<const float4*>(tab_lds + 3 * BN + cl)};
             v4i v[TP];
             uint32_t out[TP];
 #pragma unroll
             for (int tp = 0; tp < TP; ++tp) v[tp] = Quad(acc[tc][tp], q) + (AW ? rowsum[tp] : 0);
-            RequantPixels<decltype(bits)::value, TP>(v, out, f4, a.ct, tn * BN + cl, a.rq);
+            RequantPixels<decltype(bits)::value, TP>(v, out, f4, ChanTab{tab_lds, BN}, cl, a.rq);
 #pragma unroll
             for (int tp = 0; tp < TP; ++tp) *reinterpret_cast<uint32_t*>(Os + (wm * WTM + tp * 32 + (lane & 31)) * LDO + cl) = out[tp];
         }

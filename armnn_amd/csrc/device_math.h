@@ -159,9 +159,10 @@ __device__ __forceinline__ uint32_t HighBytes4(U16x2 v01, U16x2 v23)
 
 // N times four values -> N packed dwords; their constants: f[n], or f[0] for all.
 // The N are independent chains of arithmetic with one test at their end, so that a wave has all of them to issue from: a test
-// per four values is a branch, which the compiler moves nothing across.  When some lane of the wave has a byte that differs between
-// the two sides, the wave redoes that position of those four with the reference's sequence on every lane (always right, and
-// cheaper than sorting out which lanes need it); load_exact(n, mult, biasf) supplies rows 0 and 1 of the table.  The constants are
+// per four values is a branch, which the compiler moves nothing across.  Where some lane of the wave has a byte that differs between
+// the two sides, values are redone with the reference's sequence; load_exact(n, mult, biasf) supplies rows 0 and 1 of the table for
+// that.  It happens to one batch of four in six, and the waves of a block wait for one another soon after: kernels of many
+// values have those rows in LDS (from L2, 1.5 k cycles, a pass of MobileNetV1 at 64 images took 5 % longer).  The constants are
 // finite (the host checks them and the accumulator range), so no NaN reaches a conversion.
 template <bool BITS, int N, int NF, typename LoadExact>
 __device__ __forceinline__ void RequantCore(const v4i (&acc)[N], uint32_t (&out)[N], const Fast4 (&f)[NF], const Requant& rq, LoadExact load_exact)
@@ -196,26 +197,31 @@ __device__ __forceinline__ void RequantCore(const v4i (&acc)[N], uint32_t (&out)
     if (__builtin_expect(__builtin_amdgcn_ballot_w64(any != 0u) != 0, 0))
     {
         constexpr int base = BITS ? kAccBaseBits : 0;
-        // usually one value of the wave's 256 N is flagged: only its position is redone (on every lane: the exact result is
-        // always the right one)
 #pragma unroll
         for (int n = 0; n < N; ++n)
         {
             if (N > 1 && __builtin_amdgcn_ballot_w64(differ[n] != 0u) == 0) continue;
             float4 m, b;
             load_exact(n, m, b);
-            const float ms[4] = {m.x, m.y, m.z, m.w}, bs[4] = {b.x, b.y, b.z, b.w};
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                if (__builtin_amdgcn_ballot_w64((differ[n] & (0xffu << (8 * k))) != 0u) != 0)
-                    out[n] = (out[n] & ~(0xffu << (8 * k))) | ((static_cast<uint32_t>(RequantExactDev(acc[n][k] - base, ms[k], bs[k], rq) + rq.pk_bias) & 0xffu) << (8 * k));
+            // every lane redoes its first flagged position (any position where none is: the exact result is always the right one)
+            do
+            {
+                const uint32_t d = differ[n];
+                const bool upper = (d & 0xffffu) == 0u, odd = ((upper ? d >> 16 : d) & 0xffu) == 0u;
+                const int sum = upper ? (odd ? acc[n][3] : acc[n][2]) : (odd ? acc[n][1] : acc[n][0]);
+                const float mult = upper ? (odd ? m.w : m.z) : (odd ? m.y : m.x), biasf = upper ? (odd ? b.w : b.z) : (odd ? b.y : b.x);
+                const uint32_t mask = 0xffu << ((upper ? 16 : 0) + (odd ? 8 : 0));
+                const uint32_t code = static_cast<uint32_t>(RequantExactDev(sum - base, mult, biasf, rq) + rq.pk_bias) & 0xffu;
+                out[n] = (out[n] & ~mask) | (code * 0x01010101u & mask);
+                differ[n] = d & ~mask;
+            } while (__builtin_amdgcn_ballot_w64(differ[n] != 0u) != 0);
         }
     }
 #pragma unroll
     for (int n = 0; n < N; ++n) out[n] ^= rq.pk_xor;
 }
 
-// N pixels, channels c .. c + 3 of each
+// N pixels, channels c .. c + 3 of each.  `ct`: the table, or rows 0 and 1 of it (a copy in LDS).
 template <bool BITS, int N>
 __device__ __forceinline__ void RequantPixels(const v4i (&acc)[N], uint32_t (&out)[N], const Fast4& f, const ChanTab& ct, int c, const Requant& rq)
 {

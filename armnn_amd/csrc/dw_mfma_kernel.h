@@ -66,7 +66,8 @@ struct DwMfmaTile
     static constexpr int ROWS_READ = ((UNITS * WPC * (16 / TW)) - 1) * S + 3;
     static constexpr int HALO = (ROWS_READ > HR ? ROWS_READ : HR) * ROWP;   // one of the two halo buffers
     static constexpr int OUT = NW * QUADS * 1024;        // the waves' output areas: 4 pixel groups x 16 pixels x 16 bytes each
-    static constexpr int SMEM = 2 * HALO + OUT;
+    static constexpr int EXACT = NW * 128;               // mult and biasf of each wave's 16 channels
+    static constexpr int SMEM = 2 * HALO + OUT + EXACT;
 };
 
 // floor(b / d) for b * d < 2^32 with rcp = ceil(2^32 / d)
@@ -190,6 +191,7 @@ __global__ __launch_bounds__((DwMfmaTile<S, CB, TH, TW>::NT)) void DepthwiseMfma
     const int y_lane = ((pg0 * RPG + rj) * a.Wo + cj) * a.C + cg * 16 + g * y_pg;
     const int image_bytes = a.Ho * a.Wo * a.C;   // (the host checks that an image stays below 2 GiB)
 
+    const int exact = 2 * G::HALO + G::OUT + wave * 128;      // [mult, biasf][16 channels], the wave's own
     v4i wa[3], wb[3], corr4;
     Fast4 f4;
     int cur_cb = -1;
@@ -213,6 +215,7 @@ __global__ __launch_bounds__((DwMfmaTile<S, CB, TH, TW>::NT)) void DepthwiseMfma
         const int cq = c0 + 4 * g;               // the four channels this lane requantizes
         corr4 = *reinterpret_cast<const v4i*>(a.corr + cq);
         f4 = LoadFast4(a.ct, cq);
+        if (j < 2) *reinterpret_cast<float4*>(dw_mfma_lds + exact + j * 64 + g * 16) = *reinterpret_cast<const float4*>(a.ct.p + j * a.ct.stride + cq);
     };
     // Stores go through a buffer descriptor of the item's image: a lane whose pixel lies right of the image or whose channels
     // do not exist gets an offset past the descriptor's size and a row below the image runs past it by itself, so the
@@ -234,7 +237,6 @@ __global__ __launch_bounds__((DwMfmaTile<S, CB, TH, TW>::NT)) void DepthwiseMfma
     auto compute = [&](int b, int halo) {
         const Where w = decode(b);
         if (w.cb != cur_cb) { constants(w.cb); cur_cb = w.cb; }
-        const int cq = w.cb * CB + cg * 16 + 4 * g;
         const bool lane_ok = w.tx * TW + cj < a.Wo && w.cb * CB + cg * 16 < a.C;
         out_y0 = lane_ok ? y_lane + ((w.ty * TH) * a.Wo + w.tx * TW) * a.C + w.cb * CB : static_cast<int>(0x80000000u);
         out_n = w.n;
@@ -261,7 +263,7 @@ __global__ __launch_bounds__((DwMfmaTile<S, CB, TH, TW>::NT)) void DepthwiseMfma
                 }
             }
             uint32_t out[UB];
-            RequantPixels<true, UB>(acc, out, f4, a.ct, cq, a.rq);
+            RequantPixels<true, UB>(acc, out, f4, ChanTab{reinterpret_cast<const float*>(dw_mfma_lds + exact), 16}, 4 * g, a.rq);
 #pragma unroll
             for (int i = 0; i < UB; ++i)
                 if (u0 + i < UNITS) *reinterpret_cast<uint32_t*>(dw_mfma_lds + out_write + ((u0 + i) >> 2) * 1024 + ((u0 + i) & 3) * 256) = out[i];

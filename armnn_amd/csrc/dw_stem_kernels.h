@@ -537,7 +537,7 @@ __global__ __launch_bounds__(256) void SmallCiMfmaKernel(SmallCiArgs a)
     constexpr int NDWP = KH * RD;                 // patch dwords per pixel
     constexpr int KST = (NDWP + 7) / 8;           // MFMA k-steps of 32 bytes
     __shared__ __attribute__((aligned(16))) uint32_t tile[SmallCiTile<KH, TH>::DWORDS];
-    __shared__ __attribute__((aligned(16))) float cst[3][NT * 32];      // m, b and (as integers) what the accumulators start from
+    __shared__ __attribute__((aligned(16))) float cst[5][NT * 32];      // m, b, (as integers) what the accumulators start from, mult, biasf
 
     int b = blockIdx.x;
     const int tx = b % a.tiles_x; b /= a.tiles_x;
@@ -547,10 +547,10 @@ __global__ __launch_bounds__(256) void SmallCiMfmaKernel(SmallCiArgs a)
     const int S = a.stride;
     int iy_org, ix_org, mis;
     StageSmallCiHalo<KH, TH>(a, tile, tx, ty, n, tid, iy_org, ix_org, mis);
-    for (int i = tid; i < 3 * NT * 32; i += 256)
+    for (int i = tid; i < 5 * NT * 32; i += 256)
     {
         const int row = i / (NT * 32), c = i - row * (NT * 32);
-        cst[row][c] = row < 2 ? a.ct.p[(row + 2) * a.ct.stride + c] : __builtin_bit_cast(float, a.corr[c]);
+        cst[row][c] = row == 2 ? __builtin_bit_cast(float, a.corr[c]) : a.ct.p[(row < 2 ? row + 2 : row - 3) * a.ct.stride + c];
     }
 
     const int lane = tid & 63, wave = tid >> 6;
@@ -633,7 +633,7 @@ __global__ __launch_bounds__(256) void SmallCiMfmaKernel(SmallCiArgs a)
                 q4[qd] = Quad(acc, qd);
                 f[qd] = {*reinterpret_cast<const float4*>(&cst[0][cl + 8 * qd]), *reinterpret_cast<const float4*>(&cst[1][cl + 8 * qd])};
             }
-            WithBits(a.rq, [&](auto bits) { RequantChannels<decltype(bits)::value, 4, 8>(q4, o, f, a.ct, cl, a.rq); });
+            WithBits(a.rq, [&](auto bits) { RequantChannels<decltype(bits)::value, 4, 8>(q4, o, f, ChanTab{cst[3], NT * 32}, cl, a.rq); });
             // lane and lane + 32 hold interleaved 4-channel groups of one pixel; trading two dwords gives each of them
             // 16 contiguous channels (the low lane 0..15, the high lane 16..31) and one 16-byte store
             const uint32_t r0 = __shfl_xor(half ? o[0] : o[2], 32);

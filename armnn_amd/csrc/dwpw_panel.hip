@@ -19,7 +19,6 @@ int LaunchT(const mi355x_conv2d_s* dw, const mi355x_conv2d_s* pw, uint32_t batch
     const auto rcp = [](int d) { return static_cast<uint32_t>(((1ull << 32) + static_cast<uint32_t>(d) - 1) / static_cast<uint32_t>(d)); };
     DwPwPanelArgs a;
     a.x = static_cast<const uint8_t*>(x); a.pad16 = dw->pad16; a.dw_blk = dw->dw_blk.load(std::memory_order_acquire);
-    a.dw_ct = ChanTab{dw->chan, dw->Co_pad};
     a.H = g.H; a.W = g.W; a.C = g.Co; a.Ho = g.Ho; a.Wo = g.Wo;
     a.pad_top = g.pad_top; a.pad_left = g.pad_left;
     a.tiles_x = (g.Wo + TW - 1) / TW; a.tiles_y = (g.Ho + TH - 1) / TH;
@@ -99,10 +98,11 @@ bool mi355x::DwPwPanelTakes(const mi355x_conv2d_s* dw, const mi355x_conv2d_s* pw
 
 namespace
 {
-// Blocks of 64 channels: kDwBlkRows rows of [16][4] dwords, entry [j][e] for channel 16 e + j of the block: corr, m, b, filter taps
+// Blocks of 64 channels: kDwBlkRows rows of [16][4] dwords, entry [j][e] for channel 16 e + j of the block: corr, m, b, mult, biasf, filter taps
 // 0..3, 4..7, 8, and those of the second halves.  Channels past the last one are all zero: a bracket that closes, some code that no
-// weight and no row sum counts.  `grp`, `second`: the plan's dw_grp and w_dot4b (or null).
-__global__ __launch_bounds__(256) void PackDwBlkKernel(const uint32_t* __restrict__ grp, const uint32_t* __restrict__ second, uint32_t* __restrict__ blk, int C, int dwords)
+// weight and no row sum counts.  `grp`, `chan`, `second`: the plan's dw_grp, chan
+// and w_dot4b (or null).
+__global__ __launch_bounds__(256) void PackDwBlkKernel(const uint32_t* __restrict__ grp, const float* __restrict__ chan, int stride, const uint32_t* __restrict__ second, uint32_t* __restrict__ blk, int C, int dwords)
 {
     const int i = static_cast<int>(blockIdx.x) * 256 + static_cast<int>(threadIdx.x);
     if (i >= dwords) return;
@@ -112,10 +112,11 @@ __global__ __launch_bounds__(256) void PackDwBlkKernel(const uint32_t* __restric
     {
         const uint32_t* const of = grp + (c / 4) * kDwGrpDwords + c % 4;         // rows of four: weights 0 .. 2, corr, m, b
         if (row < 3) v = of[(3 + row) * 4];
+        else if (row < 5) v = __builtin_bit_cast(uint32_t, chan[(row - 3) * stride + c]);
         else
-            for (int t = (row - (row < 6 ? 3 : 6)) * 4, n = 0; n < 4 && t < 9; ++t, ++n)
+            for (int t = (row - (row < 8 ? 5 : 8)) * 4, n = 0; n < 4 && t < 9; ++t, ++n)
             {
-                const uint32_t taps = row < 6 ? of[t / 3 * 4] : second ? second[c * 4 + t / 3] : 0u;
+                const uint32_t taps = row < 8 ? of[t / 3 * 4] : second ? second[c * 4 + t / 3] : 0u;
                 v |= (taps >> (8 * (t % 3)) & 0xffu) << (8 * n);
             }
     }
@@ -128,7 +129,7 @@ int PackDwBlk(const mi355x_conv2d_s* dw, uint32_t** out)
     hipStream_t stream;
     if (const int rc = UploadStream(&stream)) return rc;
     MI355X_HIP(hipMalloc(reinterpret_cast<void**>(out), static_cast<size_t>(dwords) * 4));
-    hipLaunchKernelGGL(PackDwBlkKernel, dim3(static_cast<unsigned>((dwords + 255) / 256)), dim3(256), 0, stream, dw->dw_grp, dw->w_dot4b, *out, C, dwords);
+    hipLaunchKernelGGL(PackDwBlkKernel, dim3(static_cast<unsigned>((dwords + 255) / 256)), dim3(256), 0, stream, dw->dw_grp, dw->chan, dw->Co_pad, dw->w_dot4b, *out, C, dwords);
     MI355X_HIP(hipGetLastError());
     MI355X_HIP(hipStreamSynchronize(stream));
     return 0;

@@ -42,7 +42,6 @@ struct DwPwPanelArgs
     const uint8_t*  x;
     const uint8_t*  pad16;      // 16 bytes that become the depthwise padding value under dw_xor
     const uint32_t* dw_blk;     // constants per block of 64 channels: kDwBlkRows rows of [16][4] dwords
-    ChanTab         dw_ct;
     int H, W, C, Ho, Wo;
     int pad_top, pad_left;
     int tiles_x, tiles_y, nb;   // nb: blocks per tile (output channels / (16 NW CG), rounded up)
@@ -63,8 +62,8 @@ struct DwPwPanelArgs
     Requant        pw_rq;
 };
 
-// what accumulators start from, m, b, filter taps 0 .. 3, 4 .. 7, 8, and those of the second halves
-constexpr int kDwBlkRows = 9;
+// what accumulators start from, m, b, mult, biasf, filter taps 0 .. 3, 4 .. 7, 8, and those of the second halves
+constexpr int kDwBlkRows = 11;
 
 template <int S, int TH, int TW, int NW, int CG>
 struct DwPwPanelGeom
@@ -81,9 +80,9 @@ struct DwPwPanelGeom
         const int in = (C + 63) / 64 * 4 * GP, out = PX * OP;
         return in > out ? in : out;
     }
-    // behind it the depthwise layer's constants and three rows of NCOL dwords of the pointwise layer's
+    // behind it the depthwise layer's constants and five rows of NCOL dwords of the pointwise layer's
     static constexpr int TB(bool u) { return (u ? kDwBlkRows : kDwBlkRows - 3) * 256; }        // bytes per 64 channels
-    static constexpr int Smem(int C, bool u) { return Panel(C) + (C + 63) / 64 * TB(u) + 12 * NCOL; }
+    static constexpr int Smem(int C, bool u) { return Panel(C) + (C + 63) / 64 * TB(u) + 20 * NCOL; }
 };
 
 // KS: k-steps of 64 channels where the instance fixes them (64 (KS - 1) < C <= 64 KS), 0: a.C decides.  U: depthwise weights in two
@@ -107,7 +106,7 @@ __global__ __launch_bounds__(64 * NW, 4) void DwPwPanelKernel(DwPwPanelArgs a)
     constexpr int PB = U ? 1 : PG < 4 ? PG : 4;
     constexpr bool EARLY = PG == 1 || (PG == 2 && !U);                      // registers for weights requested ahead of the depthwise phase
     constexpr int TB = G::TB(U);
-    constexpr int TS = KS != 0 ? (KS * (TB / 16) + G::NCOL / 4 * 3 + NT - 1) / NT : 4;      // ... and table pieces
+    constexpr int TS = KS != 0 ? (KS * (TB / 16) + G::NCOL / 4 * 5 + NT - 1) / NT : 4;      // ... and table pieces
     extern __shared__ __attribute__((aligned(16))) uint8_t panel_lds[];   // [C / 16][GP]: halo pixels, then panel pixels, of 16 bytes
 
     int b = XcdContiguousWorkItem(blockIdx.x, a.xcd_chunk);
@@ -133,7 +132,7 @@ __global__ __launch_bounds__(64 * NW, 4) void DwPwPanelKernel(DwPwPanelArgs a)
     // ---- tables ---------------------------------------------------------------------------------------------------------------------
     uint8_t* const tab = panel_lds + G::Panel(64 * steps);
     uint8_t* const ptab = tab + steps * TB;
-    const int dw_pieces = steps * (TB / 16), tab_pieces = dw_pieces + G::NCOL / 4 * 3;
+    const int dw_pieces = steps * (TB / 16), tab_pieces = dw_pieces + G::NCOL / 4 * 5;
     auto tab_src = [&](int i) -> const void* {
         if (i < dw_pieces)
         {
@@ -142,8 +141,8 @@ __global__ __launch_bounds__(64 * NW, 4) void DwPwPanelKernel(DwPwPanelArgs a)
         }
         i -= dw_pieces;
         const int r = i / (G::NCOL / 4), c4 = min(bn * G::NCOL + (i - r * (G::NCOL / 4)) * 4, a.co_groups * 16 - 4);
-        if (r < 2) return a.pw_ct.p + (r + 2) * a.pw_ct.stride + c4;
-        return a.pw_corr + c4;
+        if (r == 2) return a.pw_corr + c4;
+        return a.pw_ct.p + (r < 2 ? r + 2 : r - 3) * a.pw_ct.stride + c4;        // m, b, ., mult, biasf
     };
 
     // ---- the halo of the tile, all channels ---------------------------------------------------------------------------------------
@@ -228,8 +227,8 @@ __global__ __launch_bounds__(64 * NW, 4) void DwPwPanelKernel(DwPwPanelArgs a)
 #pragma unroll
             for (int m = 0; m < 3; ++m)
             {
-                w[m] = *reinterpret_cast<const v4i*>(tb + (3 + m) * 256);
-                if constexpr (U) w2[m] = *reinterpret_cast<const v4i*>(tb + (6 + m) * 256);
+                w[m] = *reinterpret_cast<const v4i*>(tb + (5 + m) * 256);
+                if constexpr (U) w2[m] = *reinterpret_cast<const v4i*>(tb + (8 + m) * 256);
             }
             // the ninth tap of the four channel groups shares one operand: lane group g reads it from channel group g
             v4i x8[UC];
@@ -272,16 +271,8 @@ __global__ __launch_bounds__(64 * NW, 4) void DwPwPanelKernel(DwPwPanelArgs a)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) v[r] = v4i{acc[0][u][r], acc[1][u][r], acc[2][u][r], acc[3][u][r]};
                 RequantCore<true, 4, 1>(v, q, f, a.dw_rq, [&](int, float4& m, float4& b) {
-                    float mv[4], bv[4];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                    {
-                        const int c = min(blk * 64 + 16 * e + j, a.C - 1);
-                        mv[e] = a.dw_ct.p[c];
-                        bv[e] = a.dw_ct.p[a.dw_ct.stride + c];
-                    }
-                    m = float4{mv[0], mv[1], mv[2], mv[3]};
-                    b = float4{bv[0], bv[1], bv[2], bv[3]};
+                    m = *reinterpret_cast<const float4*>(tb + 768);
+                    b = *reinterpret_cast<const float4*>(tb + 1024);
                 });
 #pragma unroll
                 for (int r = 0; r < 4; ++r) *reinterpret_cast<uint32_t*>(out + (16 * u + r) * 16) = q[r] ^ a.mid_xor;
@@ -377,7 +368,7 @@ __global__ __launch_bounds__(64 * NW, 4) void DwPwPanelKernel(DwPwPanelArgs a)
     {
         const uint8_t* const tc = ptab + ((wave * CG + c) * 16 + 4 * g) * 4;
         const Fast4 f = {*reinterpret_cast<const float4*>(tc), *reinterpret_cast<const float4*>(tc + 4 * G::NCOL)};
-        const int cq = min((bn * NW + wave) * CG + c, a.co_groups - 1) * 16 + 4 * g;
+        const ChanTab exact{reinterpret_cast<const float*>(tc) + 3 * G::NCOL, G::NCOL};
 #pragma unroll
         for (int p0 = 0; p0 < PG; p0 += PB)
         {
@@ -389,7 +380,7 @@ __global__ __launch_bounds__(64 * NW, 4) void DwPwPanelKernel(DwPwPanelArgs a)
                 v[i] = acc[c][p0 + i];
                 if constexpr (U) v[i] += xs[p0 + i];
             }
-            RequantPixels<decltype(bits)::value, PB>(v, out, f, a.pw_ct, cq, a.pw_rq);
+            RequantPixels<decltype(bits)::value, PB>(v, out, f, exact, 0, a.pw_rq);
 #pragma unroll
             for (int i = 0; i < PB; ++i) *reinterpret_cast<uint32_t*>(panel_lds + (16 * (p0 + i) + j) * OP + (wave * CG + c) * 16 + 4 * g) = out[i];
         }

@@ -82,7 +82,7 @@ struct DwPwStreamGeom
     static constexpr int KP = C + 16;                     // bytes per panel row and per weight row in LDS
     static constexpr int PANEL = P * KP;
     static constexpr int WTS = NO * KP;
-    static constexpr int TAB = 3 * NO * 4;
+    static constexpr int TAB = 5 * NO * 4 + 2 * C * 4;    // the pointwise layer's m, b, start values, mult, biasf; the depthwise layer's mult, biasf
     static constexpr int MT = P / 32, NTL = NO / 32;      // 32 x 32 MFMA tiles of an item's output
     static constexpr bool BYN = NTL >= NW;                // a wave owns output channels (all pixels) or pixels (all channels)
     static constexpr int MTW = BYN ? MT : MT / NW;
@@ -132,12 +132,15 @@ void DwPwStreamKernel(DwPwStreamArgs a)
         const int row = i / CPP, part = i % CPP;
         *reinterpret_cast<v4i*>(lds + WTS0 + row * KP + part * 16) = *reinterpret_cast<const v4i*>(a.w + static_cast<long long>(row) * a.w_stride + part * 16);
     }
-    for (int i = tid; i < NO / 4 * 3; i += NT)          // [3][NO / 4] pieces: m, b, and what the accumulators start from
+    for (int i = tid; i < NO / 4 * 5; i += NT)
     {
         const int r = i / (NO / 4), col4 = i % (NO / 4);
         *reinterpret_cast<v4i*>(lds + TAB0 + i * 16) =
-            *(r < 2 ? reinterpret_cast<const v4i*>(a.pw_ct.p + (r + 2) * a.pw_ct.stride + col4 * 4) : reinterpret_cast<const v4i*>(a.pw_corr + col4 * 4));
+            *(r == 2 ? reinterpret_cast<const v4i*>(a.pw_corr + col4 * 4) : reinterpret_cast<const v4i*>(a.pw_ct.p + (r < 2 ? r + 2 : r - 3) * a.pw_ct.stride + col4 * 4));
     }
+    for (int i = tid; i < C / 2; i += NT)
+        *reinterpret_cast<v4i*>(lds + TAB0 + 5 * NO * 4 + i * 16) = *reinterpret_cast<const v4i*>(a.dw_ct.p + i / (C / 4) * a.dw_ct.stride + i % (C / 4) * 4);
+    const ChanTab pw_exact{reinterpret_cast<const float*>(lds + TAB0) + 3 * NO, NO}, dw_exact{reinterpret_cast<const float*>(lds + TAB0) + 5 * NO, C};
 
     // ---- staging of the input halo (as in DepthwiseMfmaKernel, all C channels) -------------------------------------------
     const int dxm = static_cast<int>(a.dw_xor);
@@ -277,7 +280,7 @@ void DwPwStreamKernel(DwPwStreamArgs a)
                     acc[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wa[i][1], b1, acc[k], 0, 0, 0);
                     acc[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wa[i][2], b2, acc[k], 0, 0, 0);
                 }
-                RequantPixels<true, UB>(acc, q, f4[i], a.dw_ct, (cg0 + i) * 16 + 4 * g, a.dw_rq);
+                RequantPixels<true, UB>(acc, q, f4[i], dw_exact, (cg0 + i) * 16 + 4 * g, a.dw_rq);
 #pragma unroll
                 for (int k = 0; k < UB; ++k) *reinterpret_cast<uint32_t*>(lds + panel_write + i * 16 + (u0 + k) * (WPC * 16 * KP)) = q[k] ^ a.mid_xor;
             }
@@ -327,7 +330,7 @@ void DwPwStreamKernel(DwPwStreamArgs a)
                 uint32_t out[MTW];
 #pragma unroll
                 for (int mt = 0; mt < MTW; ++mt) v[mt] = Quad(acc[mt][nt], q);
-                RequantPixels<decltype(bits)::value, MTW>(v, out, f, a.pw_ct, cl, a.pw_rq);
+                RequantPixels<decltype(bits)::value, MTW>(v, out, f, pw_exact, cl, a.pw_rq);
 #pragma unroll
                 for (int mt = 0; mt < MTW; ++mt) *reinterpret_cast<uint32_t*>(lds + out_write + mt * 32 * LDO + nt * 32 + 8 * q) = out[mt];
             }

@@ -60,7 +60,7 @@ constexpr int HaloSmemBytes(int hp)
     constexpr int stages = ST * BN * 128;
     constexpr int out = MF * 32 * (BN + 16);
     const int work = HaloTileBytes<CI>(hp) + stages;
-    return (work > out ? work : out) + 2 * BN * 4;
+    return (work > out ? work : out) + 4 * BN * 4;
 }
 
 // WM x WN = 4 waves; a wave owns TP 32-pixel fragments and 32 output channels: block tile (32 * WM * TP) pixels x
@@ -84,7 +84,7 @@ __global__ __launch_bounds__(256) void HaloConvKernel(HaloArgs a)
     uint8_t* halo = smem;
     uint8_t* wst = smem + HaloTileBytes<CI>(a.HP);
     const int work = HaloTileBytes<CI>(a.HP) + ST * WSTAGE;
-    float* tab_lds = reinterpret_cast<float*>(smem + (work > MF * 32 * LDO ? work : MF * 32 * LDO));   // rows 2 and 3 of the channel table, BN channels
+    float* tab_lds = reinterpret_cast<float*>(smem + (work > MF * 32 * LDO ? work : MF * 32 * LDO));   // the channel table, BN channels
 
     const int nblocks = a.tiles_m * a.tiles_n;
     const int per_xcd = (nblocks + 7) >> 3;
@@ -121,9 +121,9 @@ __global__ __launch_bounds__(256) void HaloConvKernel(HaloArgs a)
         }
     }
 
-    // ---- rows 2 and 3 of the channel table go to LDS: the epilogue then waits for no global load ---------------------
+    // ---- the channel table goes to LDS: the epilogue then waits for no global load ---------------------
     v4i tab_piece = {0, 0, 0, 0};
-    if (tid < BN / 2) tab_piece = *reinterpret_cast<const v4i*>(a.ct.p + static_cast<long long>((tid / (BN / 4)) + 2) * a.ct.stride + tn * BN + (tid % (BN / 4)) * 4);
+    if (tid < BN) tab_piece = *reinterpret_cast<const v4i*>(a.ct.p + static_cast<long long>(tid / (BN / 4)) * a.ct.stride + tn * BN + (tid % (BN / 4)) * 4);
 
     // ---- weights: lane fetches row (lane >> 3) of each 8-row group, the chunk whose slot is (lane & 7) ---------------------
     const int lrow = lane >> 3;
@@ -217,7 +217,7 @@ __global__ __launch_bounds__(256) void HaloConvKernel(HaloArgs a)
 #pragma unroll
     for (int s = 0; s < ST - 1; ++s)
         if (s < nk) load_w(s, s);
-    if (tid < BN / 2) *reinterpret_cast<v4i*>(tab_lds + tid * 4) = tab_piece;      // visible to all after the first barrier below
+    if (tid < BN) *reinterpret_cast<v4i*>(tab_lds + tid * 4) = tab_piece;      // visible to all after the first barrier below
     int stage = 0;
     for (int kt = 0; kt < nk; ++kt)
     {
@@ -245,12 +245,12 @@ __global__ __launch_bounds__(256) void HaloConvKernel(HaloArgs a)
         for (int q = 0; q < 4; ++q)
         {
             const int cq = cl + 8 * q + lane_c;
-            const Fast4 f4 = {*reinterpret_cast<const float4*>(tab_lds + cq), *reinterpret_cast<const float4*>(tab_lds + BN + cq)};
+            const Fast4 f4 = {*reinterpret_cast<const float4*>(tab_lds + 2 * BN + cq), *reinterpret_cast<const float4*>(tab_lds + 3 * BN + cq)};
             v4i v[TP];
             uint32_t out[TP];
 #pragma unroll
             for (int tp = 0; tp < TP; ++tp) v[tp] = Quad(acc[tp], q);
-            RequantPixels<decltype(bits)::value, TP>(v, out, f4, a.ct, tn * BN + cq, a.rq);
+            RequantPixels<decltype(bits)::value, TP>(v, out, f4, ChanTab{tab_lds, BN}, cq, a.rq);
 #pragma unroll
             for (int tp = 0; tp < TP; ++tp) *reinterpret_cast<uint32_t*>(Os + ((wm * TP + tp) * 32 + (lane & 31)) * LDO + cl + 8 * q + lane_c) = out[tp];
         }

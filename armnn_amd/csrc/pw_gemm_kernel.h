@@ -45,7 +45,7 @@ struct PwArgs
 template <int BN>
 constexpr int PwSmemBytes(int K)
 {
-    return BN * (K + 16) + 4 * 32 * (BN + 16) + 3 * BN * 4;
+    return BN * (K + 16) + 4 * 32 * (BN + 16) + 5 * BN * 4;
 }
 
 // KS = MFMA k-steps (of 32) per register chunk, K % (32 * KS) == 0;  NB = register chunks per wave (NB-1 in flight).
@@ -59,8 +59,8 @@ __global__ __launch_bounds__(256) void PwGemmKernel(PwArgs a)
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int LDW = a.K + 16;
     uint8_t* slab = smem;
-    float* cst = reinterpret_cast<float*>(smem + BN * LDW);                 // [3][BN]: m, b and (as integers) what the accumulators start from
-    uint8_t* ostage_all = smem + BN * LDW + 3 * BN * 4;
+    float* cst = reinterpret_cast<float*>(smem + BN * LDW);                 // [5][BN]: m, b, (as integers) what the accumulators start from, mult, biasf
+    uint8_t* ostage_all = smem + BN * LDW + 5 * BN * 4;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -163,7 +163,7 @@ __global__ __launch_bounds__(256) void PwGemmKernel(PwArgs a)
                 v[q] = Quad(acc[tc], q) + rt;
                 f[q] = {*reinterpret_cast<const float4*>(cst + cl + 8 * q), *reinterpret_cast<const float4*>(cst + BN + cl + 8 * q)};
             }
-            WithBits(a.rq, [&](auto bits) { RequantChannels<decltype(bits)::value, 4, 8>(v, out, f, a.ct, n0 + cl, a.rq); });
+            WithBits(a.rq, [&](auto bits) { RequantChannels<decltype(bits)::value, 4, 8>(v, out, f, ChanTab{cst + 3 * BN, BN}, cl, a.rq); });
 #pragma unroll
             for (int q = 0; q < 4; ++q) *reinterpret_cast<uint32_t*>(ostage + frag_row * LDO + cl + 8 * q) = out[q];
         }
@@ -241,10 +241,10 @@ __global__ __launch_bounds__(256) void PwGemmKernel(PwArgs a)
 #pragma unroll
             for (int i = 0; i < BN / 16; ++i) *reinterpret_cast<v4i*>(slab + ((tid >> 4) + 16 * i) * LDW + c * 16) = t[i];
         }
-        for (int i = tid; i < 3 * BN; i += 256)
+        for (int i = tid; i < 5 * BN; i += 256)
         {
             const int row = i / BN, c = i - row * BN;
-            cst[i] = row < 2 ? a.ct.p[(row + 2) * a.ct.stride + n0 + c] : __builtin_bit_cast(float, a.corr[n0 + c]);
+            cst[i] = row == 2 ? __builtin_bit_cast(float, a.corr[n0 + c]) : a.ct.p[(row < 2 ? row + 2 : row - 3) * a.ct.stride + n0 + c];
         }
     }
     __syncthreads();

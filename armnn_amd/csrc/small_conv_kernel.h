@@ -110,7 +110,8 @@ __global__ __launch_bounds__(256) void SmallConvKernel(IgemmArgs a)
     const int cg = wave >> 1, pg = wave & 1;
     const int cq = tn * 32 + cg * 16 + 4 * g;
     const v4i corr4 = *reinterpret_cast<const v4i*>(a.corr + cq);
-    const Fast4 f4 = LoadFast4(a.ct, cq);
+    const Fast4 f4[1] = {LoadFast4(a.ct, cq)};
+    const float4 mult = *reinterpret_cast<const float4*>(a.ct.p + cq), biasf = *reinterpret_cast<const float4*>(a.ct.p + a.ct.stride + cq);
     v4i acc[2][2];                                       // [channel group][pixel group]
 #pragma unroll
     for (int c = 0; c < 2; ++c)
@@ -203,7 +204,10 @@ __global__ __launch_bounds__(256) void SmallConvKernel(IgemmArgs a)
             // what the bytes beyond K added are padding values
             v += (total - (steps * 64 - a.Kh * a.Kw * a.Ci) * static_cast<int>(static_cast<int8_t>(a.pad_word & 0xffu))) * a.zw_neg;
         }
-        stage[pg * 16 + j][cg * 4 + g] = Requant4Any(v[0], v[1], v[2], v[3], f4, a.ct, cq, a.rq);
+        const v4i sums[1] = {v};
+        uint32_t out[1];
+        WithBits(a.rq, [&](auto bits) { RequantCore<decltype(bits)::value, 1, 1>(sums, out, f4, a.rq, [&](int, float4& m, float4& b) { m = mult; b = biasf; }); });
+        stage[pg * 16 + j][cg * 4 + g] = out[0];
     }
     __syncthreads();
     if (wave == 0 && om < a.M && c0 < a.Co)
