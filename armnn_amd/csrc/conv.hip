@@ -1469,8 +1469,8 @@ int PwDwCheck(const mi355x_conv2d_s* pw, const mi355x_conv2d_s* dw, PwDwShape* s
 template <int MF, int S>
 int LaunchPwDwT(const PwDwArgs& a, hipStream_t stream)
 {
-    constexpr int smem = PwDwStageBytes<MF, kPwDwStages>(), NW = PwDwWavesFor(MF);
-    static_assert(smem <= 160 * 1024 && smem == PwDwSmemFor(MF), "LDS of one CU");
+    constexpr int smem = PwDwStageBytes<MF, kPwDwStages>() + kPwDwTab, NW = PwDwWavesFor(MF);
+    static_assert(smem <= 160 * 1024 && smem == PwDwSmemFor(MF) + kPwDwTab, "LDS of one CU");
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&PwDwKernel<MF, kPwDwStages, S, NW>),
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, smem);
     MI355X_HIP(attr);
@@ -1541,7 +1541,7 @@ int LaunchPwPoolT(const mi355x_conv2d_s* pw, const mi355x_pool2d_desc* pool, uin
     a.pool_rq = MakeRequant(pool->output, MI355X_ACT_NONE, 0.0f, 0.0f);
     a.pool_is_max = pool->pool_type == 0;
     a.y = static_cast<uint8_t*>(y);
-    constexpr int smem = PwDwStageBytes<MF, kPwDwStages>(), NW = PwDwWavesFor(MF);
+    constexpr int smem = PwDwStageBytes<MF, kPwDwStages>() + kPwDwTab, NW = PwDwWavesFor(MF);
     static_assert(MF * 32 * kPwDwPitch <= smem, "the intermediate tile reuses the GEMM's stages");
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&PwDwKernel<MF, kPwDwStages, 1, NW, true>),
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, smem);

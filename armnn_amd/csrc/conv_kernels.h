@@ -254,7 +254,7 @@ template <int BM, int BN, int BK>
 constexpr int IgemmSmemBytes()
 {
     constexpr int stage = (BM + BN) * (BK + 16);
-    constexpr int out = BM * (BN + 16);
+    constexpr int out = BM * (BN + 16) + 16 * BN;        // the output tile and the block's slice of the channel table
     return 2 * stage > out ? 2 * stage : out;
 }
 
@@ -439,6 +439,9 @@ __global__ __launch_bounds__(256) void IgemmKernel(IgemmArgs a)
         for (int tp = 0; tp < TP; ++tp) acc[tc][tp] = init;
     }
 
+    // the block's slice of the channel table, BN channels: it goes to LDS when the stages have been read
+    v4i tab_piece = {0, 0, 0, 0};
+    if (tid < BN) tab_piece = *reinterpret_cast<const v4i*>(a.ct.p + static_cast<long long>(tid / (BN / 4)) * a.ct.stride + tn * BN + tid % (BN / 4) * 4);
     const int nk = a.k_tiles != 0 ? a.k_tiles : a.K_pad / BK;
     const int frag_row = lane & 31;
     const int frag_k = (lane >> 5) * 16;
@@ -501,6 +504,9 @@ __global__ __launch_bounds__(256) void IgemmKernel(IgemmArgs a)
 
     // ---- epilogue: requantize, pack 4 channels per dword, stage the byte tile in LDS ---------------------
     uint8_t* Os = smem;   // all reads of the stage buffers are behind the loop's final barrier
+    float* const tab_lds = reinterpret_cast<float*>(smem + BM * (BN + 16));
+    if (tid < BN) *reinterpret_cast<v4i*>(tab_lds + tid * 4) = tab_piece;
+    __syncthreads();
     if constexpr (AW)
     {
         // lanes l and l ^ 32 hold the two halves of every k-slice of pixel (l & 31)
@@ -515,12 +521,12 @@ __global__ __launch_bounds__(256) void IgemmKernel(IgemmArgs a)
         for (int q = 0; q < 4; ++q)
         {
             const int cl = wn * WTN + tc * 32 + 8 * q + lane_c;           // channel within the block tile
-            const Fast4 f4 = LoadFast4(a.ct, tn * BN + cl);
+            const Fast4 f4 = {*reinterpret_cast<const float4*>(tab_lds + 2 * BN + cl), *reinterpret_cast<const float4*>(tab_lds + 3 * BN + cl)};
             v4i v[TP];
             uint32_t out[TP];
 #pragma unroll
             for (int tp = 0; tp < TP; ++tp) v[tp] = Quad(acc[tc][tp], q) + (AW ? rowsum[tp] : 0);
-            RequantPixels<decltype(bits)::value, TP>(v, out, f4, a.ct, tn * BN + cl, a.rq);
+            RequantPixels<decltype(bits)::value, TP>(v, out, f4, ChanTab{tab_lds, BN}, cl, a.rq);
 #pragma unroll
             for (int tp = 0; tp < TP; ++tp) *reinterpret_cast<uint32_t*>(Os + (wm * WTM + tp * 32 + (lane & 31)) * LDO + cl) = out[tp];
         }

@@ -40,7 +40,7 @@ __global__ __launch_bounds__(256 * KG) void IgemmKSplitKernel(IgemmArgs a)
     constexpr int STAGE = (BM + BN) * BK;
     constexpr int LDO = BN + 16;
     constexpr int POFF = 8192;                   // partial tiles start behind the output staging area
-    static_assert(BM * LDO <= POFF, "output staging fits in front of the partial tiles");
+    static_assert(BM * LDO + 16 * BN <= POFF, "output staging and the slice of the channel table fit in front of the partial tiles");
     typedef __attribute__((address_space(3))) void* LdsPtr;
     typedef const __attribute__((address_space(1))) void* GlobalPtr;
 
@@ -141,6 +141,9 @@ __global__ __launch_bounds__(256 * KG) void IgemmKSplitKernel(IgemmArgs a)
     }
 
     const int nk = a.K_pad / BK;
+    // the block's slice of the channel table: it goes to LDS when the stages have been read
+    v4i tab_piece = {0, 0, 0, 0};
+    if (tid < BN) tab_piece = *reinterpret_cast<const v4i*>(a.ct.p + static_cast<long long>(tid / (BN / 4)) * a.ct.stride + tn * BN + tid % (BN / 4) * 4);
     const int nkg = grp < nk ? (nk - grp + KG - 1) / KG : 0;     // k-tiles of this group
     const int iters = (nk + KG - 1) / KG;                        // the same for every group: barriers are block-wide
     const int frag_row = lane & 31;
@@ -189,6 +192,8 @@ __global__ __launch_bounds__(256 * KG) void IgemmKSplitKernel(IgemmArgs a)
     }
     __syncthreads();
 
+    float* const tab_lds = reinterpret_cast<float*>(smem + BM * LDO);
+    if (tid < BN) *reinterpret_cast<v4i*>(tab_lds + tid * 4) = tab_piece;
     // ---- the groups' partial tiles meet in LDS; group 0 adds them in the order 1, 2, ... -------------------------------------
     v4i* part = reinterpret_cast<v4i*>(smem + POFF);
     if (grp > 0)
@@ -217,9 +222,9 @@ __global__ __launch_bounds__(256 * KG) void IgemmKSplitKernel(IgemmArgs a)
         for (int q = 0; q < 4; ++q)
         {
             v[q] = Quad(acc, q);
-            f[q] = LoadFast4(a.ct, tn * BN + cl + 8 * q);
+            f[q] = {*reinterpret_cast<const float4*>(tab_lds + 2 * BN + cl + 8 * q), *reinterpret_cast<const float4*>(tab_lds + 3 * BN + cl + 8 * q)};
         }
-        WithBits(a.rq, [&](auto bits) { RequantChannels<decltype(bits)::value, 4, 8>(v, out, f, a.ct, tn * BN + cl, a.rq); });
+        WithBits(a.rq, [&](auto bits) { RequantChannels<decltype(bits)::value, 4, 8>(v, out, f, ChanTab{tab_lds, BN}, cl, a.rq); });
 #pragma unroll
         for (int q = 0; q < 4; ++q) *reinterpret_cast<uint32_t*>(Os + (wm * 32 + (lane & 31)) * LDO + cl + 8 * q) = out[q];
     }

@@ -28,7 +28,7 @@ template <int BM, int BN, int ST>
 constexpr int IgemmLdsSmemBytes()
 {
     constexpr int stages = ST * (BM + BN) * 128;
-    constexpr int out = BM * (BN + 16);
+    constexpr int out = BM * (BN + 16) + 16 * BN;        // the output tile and the block's slice of the channel table
     return stages > out ? stages : out;
 }
 
@@ -197,6 +197,11 @@ __device__ __forceinline__ void IgemmLdsTile(const IgemmArgs& a, const int tile,
         for (int tp = 0; tp < TP; ++tp) acc[tc][tp] = init;
     }
 
+    // the block's slice of the channel table, BN channels: it goes to LDS when the stages have been read
+    static_assert(BN <= NT, "one piece per thread");
+    v4i tab_piece = {0, 0, 0, 0};
+    if (tid < BN) tab_piece = *reinterpret_cast<const v4i*>(a.ct.p + static_cast<long long>(tid / (BN / 4)) * a.ct.stride + tn * BN + tid % (BN / 4) * 4);
+
     const int nk = a.K_pad / BK;
     const int frag_row = lane & 31;
     const int frag_half = lane >> 5;
@@ -306,6 +311,8 @@ __device__ __forceinline__ void IgemmLdsTile(const IgemmArgs& a, const int tile,
 
     // ---- epilogue: requantize, pack 4 channels per dword, stage the byte tile in LDS, coalesced write-out -----------
     uint8_t* Os = smem;
+    float* const tab_lds = reinterpret_cast<float*>(smem + BM * (BN + 16));
+    if (tid < BN) *reinterpret_cast<v4i*>(tab_lds + tid * 4) = tab_piece;
     constexpr int CHUNKS = BN / 16;
     constexpr int ROWS_PER_PASS = NT / CHUNKS;
     constexpr int NP = (BM + ROWS_PER_PASS - 1) / ROWS_PER_PASS;   // 16-byte pieces a thread writes
@@ -327,6 +334,7 @@ __device__ __forceinline__ void IgemmLdsTile(const IgemmArgs& a, const int tile,
         }
     };
     if (EARLY && fuse) load_other();
+    __syncthreads();
     if constexpr (AW)
     {
 #pragma unroll
@@ -340,12 +348,12 @@ __device__ __forceinline__ void IgemmLdsTile(const IgemmArgs& a, const int tile,
         for (int q = 0; q < 4; ++q)
         {
             const int cl = wn * WTN + tc * 32 + 8 * q + lane_c;
-            const Fast4 f4 = LoadFast4(a.ct, tn * BN + cl);
+            const Fast4 f4 = {*reinterpret_cast<const float4*>(tab_lds + 2 * BN + cl), *reinterpret_cast<const float4*>(tab_lds + 3 * BN + cl)};
             v4i v[TP];
             uint32_t out[TP];
 #pragma unroll
             for (int tp = 0; tp < TP; ++tp) v[tp] = Quad(acc[tc][tp], q) + (AW ? rowsum[tp] : 0);
-            RequantPixels<decltype(bits)::value, TP>(v, out, f4, a.ct, tn * BN + cl, a.rq);
+            RequantPixels<decltype(bits)::value, TP>(v, out, f4, ChanTab{tab_lds, BN}, cl, a.rq);
 #pragma unroll
             for (int tp = 0; tp < TP; ++tp) *reinterpret_cast<uint32_t*>(Os + (wm * WTM + tp * 32 + (lane & 31)) * LDO + cl) = out[tp];
         }

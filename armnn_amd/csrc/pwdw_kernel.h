@@ -70,6 +70,8 @@ constexpr int PwDwStageBytes()
     return ST * (MF * 32 + kPwDwBN) * 128;
 }
 
+constexpr int kPwDwTab = 16 * kPwDwBN;           // behind the stages: the block's slice of the 1x1 layer's channel table
+
 // s_waitcnt vmcnt(n) for a wave-uniform run-time n: the instruction takes an immediate, so the even counts a k-tile
 // pipeline produces are enumerated and anything else waits for the next smaller one (stricter, never wrong).
 __device__ __forceinline__ void WaitVmcntAtMost(int n)
@@ -211,6 +213,11 @@ __global__ __launch_bounds__(64 * NW) void PwDwKernel(PwDwArgs a)
         df4.b = *reinterpret_cast<const float4*>(gc + 5);
     }
 
+    float* const tab_lds = reinterpret_cast<float*>(smem + ST * STAGE);
+    static_assert(BN == 64, "one load instruction");
+    if (wave == 0)       // (ahead of the tiles: there when the first of them is)
+        __builtin_amdgcn_global_load_lds((GlobalPtr)(a.pw_ct.p + lane / (BN / 4) * a.pw_ct.stride + tn * BN + lane % (BN / 4) * 4), (LdsPtr)(tab_lds), 16, 0, 0);
+
     const int nk = a.K_pad / BK;
 #pragma unroll
     for (int s = 0; s < ST - 1; ++s)
@@ -260,15 +267,20 @@ __global__ __launch_bounds__(64 * NW) void PwDwKernel(PwDwArgs a)
                 inside = hy < a.HR && hx < a.HC;
                 cell = T + ((g * a.HR + hy) * a.HC + hx) * PITCH + tc * 32 + lane_c;
             }
+            const int cl = tc * 32 + lane_c;
+            v4i v[4];
+            Fast4 pf[4];
+            uint32_t out[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q)
             {
-                const int cg = cbase + 8 * q + lane_c;
-                const Fast4 f4 = LoadFast4(a.pw_ct, cg);
-                const v16i& v = acc[tp];
-                const uint32_t out = Requant4Any(v[4 * q + 0], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3], f4, a.pw_ct, cg, a.pw_rq);
-                if (inside) *reinterpret_cast<uint32_t*>(cell + 8 * q) = POOL ? out : out ^ a.dw_xor;
+                v[q] = Quad(acc[tp], q);
+                pf[q] = {*reinterpret_cast<const float4*>(tab_lds + 2 * BN + cl + 8 * q), *reinterpret_cast<const float4*>(tab_lds + 3 * BN + cl + 8 * q)};
             }
+            WithBits(a.pw_rq, [&](auto bits) { RequantChannels<decltype(bits)::value, 4, 8>(v, out, pf, ChanTab{tab_lds, BN}, cl, a.pw_rq); });
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (inside) *reinterpret_cast<uint32_t*>(cell + 8 * q) = POOL ? out[q] : out[q] ^ a.dw_xor;
         }
     }
     __syncthreads();

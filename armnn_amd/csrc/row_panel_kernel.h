@@ -29,7 +29,7 @@ template <int CG>
 constexpr int RowPanelSmem(int K)
 {
     const int in = ((K < kRowPanelK ? K : kRowPanelK) + 63) / 64 * 4 * kRowPanelGp, out = 64 * (64 * CG + 16);
-    return in > out ? in : out;
+    return (in > out ? in : out) + 16 * 64 * CG;         // + the block's slice of the channel table
 }
 
 // a.w in operand order (PackFragKernel); a.tiles_n = ceil(Co / (64 CG)), a.tiles_m = ceil(M / 64).  a.res: an Addition behind.
@@ -84,6 +84,10 @@ __global__ __launch_bounds__(256, KB <= 256 ? 4 : 3) void RowPanelKernel(IgemmAr
         // pieces that complete the last k-step: their weights are zero, and with AW they must not count either
         for (int i = tid + pr * 64; i < (pr + 3) / 4 * 4 * 64; i += NT) *reinterpret_cast<v4i*>(row_lds + (i >> 6) * GP + (i & 63) * 16) = v4i{0, 0, 0, 0};
     };
+    // the block's slice of the channel table (channels past the last one: some other channel's, nothing is stored)
+    float* const tab_lds = reinterpret_cast<float*>(row_lds + RowPanelSmem<CG>(a.Ci) - 16 * NCOL);
+    v4i tab_piece = {0, 0, 0, 0};
+    if (tid < NCOL) tab_piece = *reinterpret_cast<const v4i*>(a.ct.p + tid / (NCOL / 4) * a.ct.stride + min(bn * NCOL + tid % (NCOL / 4) * 4, co_groups * 16 - 4));
     load_rows(0);
     // ---- weights of the wave's CG groups of output channels -----------------------------------------------------------------------
     int cgrp[CG];
@@ -127,6 +131,7 @@ __global__ __launch_bounds__(256, KB <= 256 ? 4 : 3) void RowPanelKernel(IgemmAr
     {
         if (k0 != 0) __syncthreads();                    // the rows before have been read
         store_rows(k0);
+        if (k0 == 0 && tid < NCOL) *reinterpret_cast<v4i*>(tab_lds + tid * 4) = tab_piece;
         __syncthreads();
         const bool more = k0 + KB < a.Ci;
         if (more) load_rows(k0 + KB);
@@ -167,26 +172,20 @@ __global__ __launch_bounds__(256, KB <= 256 ? 4 : 3) void RowPanelKernel(IgemmAr
             xs[p] *= a.zw_neg;
         }
     }
-    Fast4 f[CG];
-#pragma unroll
-    for (int c = 0; c < CG; ++c)
-    {
-        const int cq = cgrp[c] * 16 + 4 * g;
-        f[c] = LoadFast4(a.ct, cq);
-    }
     __syncthreads();                                     // the rows have been read; the outputs take their place
     WithBits(a.rq, [&](auto bits) {
 #pragma unroll
     for (int c = 0; c < CG; ++c)
     {
-        const int cq = cgrp[c] * 16 + 4 * g;
+        const int cl = (wave * CG + c) * 16 + 4 * g;
+        const Fast4 f = {*reinterpret_cast<const float4*>(tab_lds + 2 * NCOL + cl), *reinterpret_cast<const float4*>(tab_lds + 3 * NCOL + cl)};
         uint32_t out[PG];
         if constexpr (AW)
         {
 #pragma unroll
             for (int p = 0; p < PG; ++p) acc[c][p] += xs[p];
         }
-        RequantPixels<decltype(bits)::value, PG>(acc[c], out, f[c], a.ct, cq, a.rq);
+        RequantPixels<decltype(bits)::value, PG>(acc[c], out, f, ChanTab{tab_lds, NCOL}, cl, a.rq);
 #pragma unroll
         for (int p = 0; p < PG; ++p) *reinterpret_cast<uint32_t*>(row_lds + (16 * p + j) * OP + (wave * CG + c) * 16 + 4 * g) = out[p];
     }
