@@ -99,6 +99,8 @@ struct Requant
     int32_t  pk_full;       // the clamp is 0..255: the instruction's own saturation does it
     // Convolution / FullyConnected epilogue (device_math.h), per plan
     float    two_c;              // width of the bracket
+    int32_t  all_fast;           // every channel has a fast path
+    float    half_offset_f;      // 0.5 + offset + pk_bias
     int32_t  acc_base;           // kAccBaseBits where the bits of an accumulator are a float, else 0: sums are raised by this much
     uint32_t pk_lo2, pk_hi2;     // the clamp, for two codes at a time in 16 bits each
 };

@@ -459,16 +459,21 @@ void FinishTable(mi355x_conv2d_s* p, std::vector<int32_t>& corr)
     const double most_t = std::max(std::fabs(257.5 - zp), std::fabs(-1.5 - zp));
     std::vector<uint8_t> fast(Co, 0);
     bool bits = p->acc_most < (1ll << 29);
+    bool all_fast = s_out > 0x1p-90 && s_out < 0x1p90;       // (SettleDev: nothing near the ends of fp32)
     double c_codes = 1024.0 * u;                      // (enough to tell p from q anywhere)
     for (int c = 0; c < Co; ++c)
     {
         const double fm = static_cast<double>(tab[c]) / s_out, fb = static_cast<double>(tab[CP + c]) / s_out, bias = std::fabs(fb);
-        // Half-width in codes: the reference converts the sum (sums beyond 2^24 round), multiplies, adds the bias and divides, the first
-        // two on values of up to |t| + |bias| codes, the others of up to |t|; here a conversion and m round |t| + |bias|, b rounds
-        // |bias| + |offset'| + 1, and p and q round on a scale where 256 codes are 1 (128 each).  1.05 for the second order.
-        const double w = 1.05 * u * (2.0 * (most_t + bias) + 2.0 * most_t + 2.0 * (most_t + bias) + bias + std::fabs(zp) + 1.0 + 256.0);
-        fast[c] = p->rq.fast_ok != 0 && std::isfinite(fm) && std::isfinite(fb) && (fm == 0.0 || (std::isnormal(tab[c]) && std::isnormal(static_cast<float>(fm * unit)))) &&
+        // Half-width in codes: the reference multiplies, adds the bias and divides, on values of up to |t| + |bias|, |t| and |t| codes (1.02
+        // for the second order); both sides convert the sum, which rounds from 2^24 on; m and b are off by what they are off; p and
+        // q round on a scale where 256 codes are 1 (128 each).
+        const double m = fm * unit, b = (256.0 * (fb + zp + 0.5) - 0.5) / 65535.0, reach = most_t + bias;
+        const double m_off = m != 0.0 ? std::fabs(static_cast<double>(static_cast<float>(m)) / m - 1.0) * reach : 0.0;
+        const double w = u * (1.02 * (reach + 2.0 * most_t) + (reach >= 16777216.0 * std::fabs(fm) ? 2.04 * reach : 0.0) + 256.0) + m_off +
+                         0.5 * std::ldexp(1.0, std::ilogb(std::fabs(b) + 0.001) - 23) / unit;
+        fast[c] = p->rq.fast_ok != 0 && std::isfinite(fm) && std::isfinite(fb) && (fm == 0.0 || (std::isnormal(tab[c]) && std::isnormal(static_cast<float>(m)))) &&
                   w < 0.0625 && static_cast<double>(p->acc_most) * std::fabs(fm) < 268435456.0;
+        all_fast &= fast[c] != 0;
         if (!fast[c]) continue;
         c_codes = std::max(c_codes, w);
         // where the steps are not ones, codes must be saturated
@@ -484,6 +489,7 @@ void FinishTable(mi355x_conv2d_s* p, std::vector<int32_t>& corr)
         tab[3 * CP + c] = static_cast<float>((256.0 * code - 0.5) / 65535.0 + c_x);
     }
     p->rq.two_c = std::nextafterf(static_cast<float>(2.0 * c_x), 1.0f);
+    p->rq.all_fast = all_fast ? 1 : 0;
     p->rq.acc_base = bits ? kAccBaseBits : 0;
     for (int32_t& v : corr) v += p->rq.acc_base;
 }

@@ -149,6 +149,24 @@ __device__ __forceinline__ float AccValue(int acc)
     else return static_cast<float>(acc);
 }
 
+// Which of codes k - 1 and k (unsigned bytes, before the activation's clamp) a value has that the bracket puts into one of them; k
+// when `open` is 0.
+//   f is the reference's fp32 value, h = k - 0.5 - offset' the half-integer in question.  fl(f / s_out) >= h exactly if f / s_out >= h -
+//   d with d half the distance from |h| to the float below it (h - d is a tie that rounds to h, whose mantissa is even), and
+//   fl(f / s_out) > h for negative h exactly if f / s_out > h + d; rounding half away from zero asks for the first where h is
+//   positive, for the second where it is negative.  f - h s_out has few bits and is exact in the fma, d s_out is a shift: the
+//   division's result is known without the division.
+__device__ __forceinline__ int SettleDev(float sum, float mult, float biasf, int k, uint32_t open, const Requant& rq)
+{
+    const float f = __fadd_rn(__fmul_rn(sum, mult), biasf);
+    const float h = static_cast<float>(k) - rq.half_offset_f;
+    const float r = __fmaf_rn(-h, rq.out_scale, f);
+    const uint32_t below = (__builtin_bit_cast(uint32_t, fabsf(h)) - 1u) & 0x7f800000u;         // 2^exponent of the float below |h|
+    const float ds = __fmul_rn(__fmul_rn(__builtin_bit_cast(float, below), 0x1p-24f), rq.out_scale);
+    const bool up = h > 0.0f ? r >= -ds : r > ds;
+    return k - (open != 0u && !up ? 1 : 0);
+}
+
 typedef unsigned short U16x2 __attribute__((ext_vector_type(2)));
 
 // the high bytes of four 16-bit values -> one dword
@@ -182,6 +200,32 @@ __device__ __forceinline__ void RequantCore(const v4i (&acc)[N], uint32_t (&out)
         differ[n] = out[n] ^ HighBytes4(lo01, lo23);
         any |= differ[n];
     }
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(any != 0u) != 0, 0))
+    {
+        constexpr int base = BITS ? kAccBaseBits : 0;
+#pragma unroll
+        for (int n = 0; n < N; ++n)
+        {
+            if (N > 1 && __builtin_amdgcn_ballot_w64(differ[n] != 0u) == 0) continue;
+            float4 m, b;
+            load_exact(n, m, b);
+            // every lane redoes its first flagged position (any position where none is: the result is always the right one)
+            do
+            {
+                const uint32_t d = differ[n];
+                const bool upper = (d & 0xffffu) == 0u, odd = ((upper ? d >> 16 : d) & 0xffu) == 0u;
+                const int sum = upper ? (odd ? acc[n][3] : acc[n][2]) : (odd ? acc[n][1] : acc[n][0]);
+                const float mult = upper ? (odd ? m.w : m.z) : (odd ? m.y : m.x), biasf = upper ? (odd ? b.w : b.z) : (odd ? b.y : b.x);
+                const int shift = (upper ? 16 : 0) + (odd ? 8 : 0);
+                const uint32_t mask = 0xffu << shift;
+                int code;
+                if (rq.all_fast) code = SettleDev(AccValue<BITS>(sum), mult, biasf, static_cast<int>((out[n] >> shift) & 0xffu), d & mask, rq);
+                else code = RequantExactDev(sum - base, mult, biasf, rq) + rq.pk_bias;
+                out[n] = (out[n] & ~mask) | (static_cast<uint32_t>(code) << shift);
+                differ[n] = d & ~mask;
+            } while (__builtin_amdgcn_ballot_w64(differ[n] != 0u) != 0);
+        }
+    }
     if (!rq.pk_full)
     {
         // the clamp, two codes at a time
@@ -192,29 +236,6 @@ __device__ __forceinline__ void RequantCore(const v4i (&acc)[N], uint32_t (&out)
             const U16x2 even = __builtin_elementwise_min(__builtin_elementwise_max(__builtin_bit_cast(U16x2, out[n] & 0x00ff00ffu), least), most);
             const U16x2 odd = __builtin_elementwise_min(__builtin_elementwise_max(__builtin_bit_cast(U16x2, (out[n] >> 8) & 0x00ff00ffu), least), most);
             out[n] = __builtin_bit_cast(uint32_t, even) | (__builtin_bit_cast(uint32_t, odd) << 8);
-        }
-    }
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(any != 0u) != 0, 0))
-    {
-        constexpr int base = BITS ? kAccBaseBits : 0;
-#pragma unroll
-        for (int n = 0; n < N; ++n)
-        {
-            if (N > 1 && __builtin_amdgcn_ballot_w64(differ[n] != 0u) == 0) continue;
-            float4 m, b;
-            load_exact(n, m, b);
-            // every lane redoes its first flagged position (any position where none is: the exact result is always the right one)
-            do
-            {
-                const uint32_t d = differ[n];
-                const bool upper = (d & 0xffffu) == 0u, odd = ((upper ? d >> 16 : d) & 0xffu) == 0u;
-                const int sum = upper ? (odd ? acc[n][3] : acc[n][2]) : (odd ? acc[n][1] : acc[n][0]);
-                const float mult = upper ? (odd ? m.w : m.z) : (odd ? m.y : m.x), biasf = upper ? (odd ? b.w : b.z) : (odd ? b.y : b.x);
-                const uint32_t mask = 0xffu << ((upper ? 16 : 0) + (odd ? 8 : 0));
-                const uint32_t code = static_cast<uint32_t>(RequantExactDev(sum - base, mult, biasf, rq) + rq.pk_bias) & 0xffu;
-                out[n] = (out[n] & ~mask) | (code * 0x01010101u & mask);
-                differ[n] = d & ~mask;
-            } while (__builtin_amdgcn_ballot_w64(differ[n] != 0u) != 0);
         }
     }
 #pragma unroll

@@ -129,6 +129,8 @@ Requant MakeRequant(const mi355x_quant& out, int32_t activation, float a, float 
     rq.fast_ok = !GlobalOptions().exact_division_epilogue && std::isnormal(rq.inv_scale) && std::isnormal(out.scale) && out.offset >= -255 && out.offset <= 255 &&
                  rq.act_lo <= rq.act_hi;
     rq.two_c = 0.0f;
+    rq.all_fast = 0;
+    rq.half_offset_f = 0.5f + static_cast<float>(out.offset + rq.pk_bias);
     rq.acc_base = 0;
     rq.pk_lo2 = static_cast<uint32_t>(rq.act_lo + rq.pk_bias) * 0x00010001u;
     rq.pk_hi2 = static_cast<uint32_t>(rq.act_hi + rq.pk_bias) * 0x00010001u;
