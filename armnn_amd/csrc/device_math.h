@@ -180,8 +180,10 @@ __device__ __forceinline__ uint32_t HighBytes4(U16x2 v01, U16x2 v23)
 // per four values is a branch, which the compiler moves nothing across.  Where some lane of the wave has a byte that differs between
 // the two sides, values are redone with the reference's sequence; load_exact(n, mult, biasf) supplies rows 0 and 1 of the table for
 // that.  It happens to one batch of four in six, and the waves of a block wait for one another soon after: kernels of many
-// values have those rows in LDS (from L2, 1.5 k cycles, a pass of MobileNetV1 at 64 images took 5 % longer).  The constants are
-// finite (the host checks them and the accumulator range), so no NaN reaches a conversion.
+// values have those rows in LDS (from L2, 1.5 k cycles, a pass of MobileNetV1 at 64 images took 5 % longer).  One copy of that code
+// serves the batch, each lane choosing among the N (a copy for each of the N: 161.0 against 158.7 us at 64 images, 584 against 572
+// at 256; the instructions are cold when they are wanted).  The constants are finite (the host checks them and the accumulator
+// range), so no NaN reaches a conversion.
 template <bool BITS, int N, int NF, typename LoadExact>
 __device__ __forceinline__ void RequantCore(const v4i (&acc)[N], uint32_t (&out)[N], const Fast4 (&f)[NF], const Requant& rq, LoadExact load_exact)
 {
@@ -203,28 +205,40 @@ __device__ __forceinline__ void RequantCore(const v4i (&acc)[N], uint32_t (&out)
     if (__builtin_expect(__builtin_amdgcn_ballot_w64(any != 0u) != 0, 0))
     {
         constexpr int base = BITS ? kAccBaseBits : 0;
-#pragma unroll
-        for (int n = 0; n < N; ++n)
+        // every lane redoes its first flagged value (some value where none is: the result is always the right one)
+        do
         {
-            if (N > 1 && __builtin_amdgcn_ballot_w64(differ[n] != 0u) == 0) continue;
-            float4 m, b;
-            load_exact(n, m, b);
-            // every lane redoes its first flagged position (any position where none is: the result is always the right one)
-            do
+            int s0 = acc[N - 1][0], s1 = acc[N - 1][1], s2 = acc[N - 1][2], s3 = acc[N - 1][3], which = N - 1;
+            uint32_t d = differ[N - 1], o = out[N - 1];
+#pragma unroll
+            for (int n = N - 2; n >= 0; --n)
             {
-                const uint32_t d = differ[n];
-                const bool upper = (d & 0xffffu) == 0u, odd = ((upper ? d >> 16 : d) & 0xffu) == 0u;
-                const int sum = upper ? (odd ? acc[n][3] : acc[n][2]) : (odd ? acc[n][1] : acc[n][0]);
-                const float mult = upper ? (odd ? m.w : m.z) : (odd ? m.y : m.x), biasf = upper ? (odd ? b.w : b.z) : (odd ? b.y : b.x);
-                const int shift = (upper ? 16 : 0) + (odd ? 8 : 0);
-                const uint32_t mask = 0xffu << shift;
-                int code;
-                if (rq.all_fast) code = SettleDev(AccValue<BITS>(sum), mult, biasf, static_cast<int>((out[n] >> shift) & 0xffu), d & mask, rq);
-                else code = RequantExactDev(sum - base, mult, biasf, rq) + rq.pk_bias;
-                out[n] = (out[n] & ~mask) | (static_cast<uint32_t>(code) << shift);
-                differ[n] = d & ~mask;
-            } while (__builtin_amdgcn_ballot_w64(differ[n] != 0u) != 0);
-        }
+                const int a0 = acc[n][0], a1 = acc[n][1], a2 = acc[n][2], a3 = acc[n][3];
+                const uint32_t dn = differ[n], on = out[n];
+                const bool take = dn != 0u;
+                s0 = take ? a0 : s0; s1 = take ? a1 : s1; s2 = take ? a2 : s2; s3 = take ? a3 : s3;
+                d = take ? dn : d; o = take ? on : o; which = take ? n : which;
+            }
+            float4 m, b;
+            load_exact(which, m, b);
+            const bool upper = (d & 0xffffu) == 0u, odd = ((upper ? d >> 16 : d) & 0xffu) == 0u;
+            const int sum = upper ? (odd ? s3 : s2) : (odd ? s1 : s0);
+            const float mult = upper ? (odd ? m.w : m.z) : (odd ? m.y : m.x), biasf = upper ? (odd ? b.w : b.z) : (odd ? b.y : b.x);
+            const int shift = (upper ? 16 : 0) + (odd ? 8 : 0);
+            const uint32_t mask = 0xffu << shift;
+            int code;
+            if (rq.all_fast) code = SettleDev(AccValue<BITS>(sum), mult, biasf, static_cast<int>((o >> shift) & 0xffu), d & mask, rq);
+            else code = RequantExactDev(sum - base, mult, biasf, rq) + rq.pk_bias;
+            o = (o & ~mask) | (static_cast<uint32_t>(code) << shift);
+            any = 0u;
+#pragma unroll
+            for (int n = 0; n < N; ++n)
+            {
+                out[n] = which == n ? o : out[n];
+                differ[n] = which == n ? d & ~mask : differ[n];
+                any |= differ[n];
+            }
+        } while (__builtin_amdgcn_ballot_w64(any != 0u) != 0);
     }
     if (!rq.pk_full)
     {
