@@ -1338,7 +1338,7 @@ int LaunchDwPw(const mi355x_conv2d_s* dw, const mi355x_conv2d_s* pw, uint32_t ba
     return 0;
 }
 
-// ---- depthwise 3x3 + pointwise for the wide, shallow front layers: persistent blocks, pointwise weights resident in LDS -----
+// ---- depthwise 3x3 + pointwise for the wide, shallow front layers: persistent blocks, pointwise weights resident in registers -----
 // which: 1 = stride 1, 32 -> 64 channels; 2 = stride 2, 64 -> 128; 3 = stride 1, 128 -> 128; 4 = stride 2, 128 -> 256 (eight
 // waves: its weights and halo leave room for one block per CU); 0 when the pair does not fit
 int DwPwStreamShape(const mi355x_conv2d_s* dw, const mi355x_conv2d_s* pw)

@@ -3,16 +3,19 @@
 //
 // Run apart, these layers are bound by memory: the tensor between them is written once and read once (112 x 112 x 32 at 64
 // images: 26 MB each way, next to 26 MB in and 51 MB out).  Here it never leaves the CU.
-//   * A block of four (or eight) waves is persistent: it keeps the pointwise weights (at most 256 x 128 bytes) and the pointwise
-//     layer's constants in LDS for its whole life and walks items -- TH x TW output pixels of one image over ALL
-//     channels -- with the next item's input halo in flight (in registers) while the current one is computed.  Two barriers
-//     per item: halo staged / panel complete.
+//   * A block of four (or eight) waves is persistent: its waves keep the pointwise weights and both layers' constants in registers for
+//     their whole life and walk items -- TH x TW output pixels of one image over ALL channels -- with the next item's input
+//     halo in flight (in registers) while the current one is computed.  Two barriers per item: halo staged / panel complete.
 //   * Depthwise phase: the matrix-core arithmetic of DepthwiseMfmaKernel (16 channels x 16 pixels x 4 taps per
 //     v_mfma_i32_16x16x64_i8 over diagonal weight operands kept in registers), requantized with the depthwise layer's own
 //     constants; the codes -- the bytes the separate layer would have stored, shifted to int8 where they are uint8 -- go
 //     to an LDS panel [pixel][channel].
-//   * Pointwise phase: v_mfma_i32_32x32x32_i8 over the panel and the resident weights; the requantized dwords pass through a wave-private
-//     LDS area and leave as 16 bytes per lane.
+//   * Pointwise phase: a wave owns 64 output channels of its share of the pixels, as 16 x 16 results with pixels as rows; column j of the
+//     four results of 16 pixels is channel 4 j + result, so that a lane holds channels 4 j .. 4 j + 3 of four pixels, always the
+//     same four channels: weights (8 to 32 registers) and constants stay where they are.  (With channels as rows, 32 x 32, a wave
+//     read weights and constants again for every item, a third of the LDS traffic; a pass of
+//     MobileNetV1 at 64 images 160.7 -> 158.0 us, at 256 576 -> 569.5.)  The requantized dwords pass
+//     through a wave-private LDS area and leave as 16 bytes per lane.
 //   * Loads and stores of a wave complete in issue order and share one counter: an item's stores are issued at the start of
 //     the next iteration, ahead of that iteration's loads, so the wait for those loads covers nothing younger.
 //   * Stores go through a buffer descriptor of the item's image: a pixel right of the image gets an offset past the
@@ -81,21 +84,21 @@ struct DwPwStreamGeom
     static constexpr int HALO = HR * ROWP;                // the halo buffer
     static constexpr int KP = C + 16;                     // bytes per panel row and per weight row in LDS
     static constexpr int PANEL = P * KP;
-    static constexpr int WTS = NO * KP;
-    static constexpr int TAB = 5 * NO * 4 + 2 * C * 4;    // the pointwise layer's m, b, start values, mult, biasf; the depthwise layer's mult, biasf
-    static constexpr int MT = P / 32, NTL = NO / 32;      // 32 x 32 MFMA tiles of an item's output
-    static constexpr bool BYN = NTL >= NW;                // a wave owns output channels (all pixels) or pixels (all channels)
-    static constexpr int MTW = BYN ? MT : MT / NW;
-    static constexpr int NTW = BYN ? NTL / NW : NTL;
-    static_assert(MTW == 2, "a wave's output area is 64 pixels deep");
-    static constexpr int SC = NTW * 32;                   // channels a wave writes per pixel
-    static constexpr int LDO = SC + 16;
-    static constexpr int OUT = NW * 64 * LDO;
-    static constexpr int QUADS = 64 * (SC / 16) / 64;     // 16-byte stores per lane and item
-    static constexpr int SMEM = HALO + PANEL + WTS + TAB + OUT;
+    static constexpr int TAB = 2 * NO * 4 + 2 * C * 4;    // mult and biasf of both layers
+    static constexpr int WN = NO / 64, WM = NW / WN;      // waves side by side over channels and pixels
+    static_assert(NW % WN == 0 && P % (16 * WM) == 0, "whole shares");
+    static constexpr int PXW = P / WM, MT = PXW / 16;     // a wave's pixels, in groups of 16
+    static constexpr int KB = C >= 64 ? 64 : 32, KST = C / KB;     // bytes of K per MFMA
+    static constexpr int LDO = 64 + 16;
+    static constexpr int OUT = NW * PXW * LDO;
+    static constexpr int QUADS = PXW * 4 / 64;            // 16-byte stores per lane and item
+    static constexpr int SMEM = HALO + PANEL + TAB + OUT;
     // Blocks per CU that LDS allows; the register budget follows it (a few spilled registers cost less than the third block
     // gains: 112 x 112 x 32 -> 64 at 64 images 29.5 us with two blocks, 24.4 with three).
-    static constexpr int BLOCKS = 160 * 1024 / SMEM >= 3 ? 3 : 160 * 1024 / SMEM >= 2 ? 2 : 1;
+    // (With 128 channels the weights and constants alone take 60 registers: a third block of four waves would spill 88, a second of
+    // eight took a launch of one image from 6.2 to 12.1 us.)
+    static constexpr int FIT = 160 * 1024 / SMEM, MOST = C <= 64 ? 3 : NWAVES == 4 ? 2 : 1;
+    static constexpr int BLOCKS = FIT >= MOST ? MOST : FIT >= 1 ? FIT : 1;
     static constexpr int WAVES_PER_SIMD = BLOCKS * NW / 4;
 };
 
@@ -107,7 +110,7 @@ void DwPwStreamKernel(DwPwStreamArgs a)
     using G = DwPwStreamGeom<S, C, NO, TH, TW, NWAVES>;
     constexpr int NW = G::NW;
     constexpr int NT = G::NT, NCG = G::NCG, HR = G::HR, HC = G::HC, PITCH = G::PITCH, ROWP = G::ROWP, HALO = G::HALO;
-    constexpr int CGW = G::CGW, WPC = G::WPC, UNITS = G::UNITS, KP = G::KP, MTW = G::MTW, NTW = G::NTW, LDO = G::LDO, QUADS = G::QUADS;
+    constexpr int CGW = G::CGW, WPC = G::WPC, UNITS = G::UNITS, KP = G::KP, LDO = G::LDO, QUADS = G::QUADS;
     constexpr int RPG = 16 / TW;
     // pixel groups whose depthwise outputs are computed together (a pass at 64 images: 4 170.8, 2 171.3, 1 172.1 us)
     constexpr int UB = UNITS % 4 == 0 ? 4 : UNITS % 2 == 0 ? 2 : 1;
@@ -116,7 +119,7 @@ void DwPwStreamKernel(DwPwStreamArgs a)
     constexpr int NST = (NCH + NT - 1) / NT;
     extern __shared__ __attribute__((aligned(16))) uint8_t dwpw_stream_lds[];
     uint8_t* const lds = dwpw_stream_lds;
-    constexpr int PANEL0 = HALO, WTS0 = PANEL0 + G::PANEL, TAB0 = WTS0 + G::WTS, OUT0 = TAB0 + G::TAB;
+    constexpr int PANEL0 = HALO, TAB0 = PANEL0 + G::PANEL, OUT0 = TAB0 + G::TAB;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
@@ -126,21 +129,12 @@ void DwPwStreamKernel(DwPwStreamArgs a)
     int item = xcd * a.xcd_chunk + static_cast<int>(blockIdx.x >> 3);
     if (item >= item_end) return;
 
-    // ---- resident constants of the pointwise layer -------------------------------------------------------------------------
-    for (int i = tid; i < NO * CPP; i += NT)
-    {
-        const int row = i / CPP, part = i % CPP;
-        *reinterpret_cast<v4i*>(lds + WTS0 + row * KP + part * 16) = *reinterpret_cast<const v4i*>(a.w + static_cast<long long>(row) * a.w_stride + part * 16);
-    }
-    for (int i = tid; i < NO / 4 * 5; i += NT)
-    {
-        const int r = i / (NO / 4), col4 = i % (NO / 4);
-        *reinterpret_cast<v4i*>(lds + TAB0 + i * 16) =
-            *(r == 2 ? reinterpret_cast<const v4i*>(a.pw_corr + col4 * 4) : reinterpret_cast<const v4i*>(a.pw_ct.p + (r < 2 ? r + 2 : r - 3) * a.pw_ct.stride + col4 * 4));
-    }
+    // ---- what the exact path reads of both layers' tables ------------------------------------------------------------------
+    for (int i = tid; i < NO / 2; i += NT)
+        *reinterpret_cast<v4i*>(lds + TAB0 + i * 16) = *reinterpret_cast<const v4i*>(a.pw_ct.p + i / (NO / 4) * a.pw_ct.stride + i % (NO / 4) * 4);
     for (int i = tid; i < C / 2; i += NT)
-        *reinterpret_cast<v4i*>(lds + TAB0 + 5 * NO * 4 + i * 16) = *reinterpret_cast<const v4i*>(a.dw_ct.p + i / (C / 4) * a.dw_ct.stride + i % (C / 4) * 4);
-    const ChanTab pw_exact{reinterpret_cast<const float*>(lds + TAB0) + 3 * NO, NO}, dw_exact{reinterpret_cast<const float*>(lds + TAB0) + 5 * NO, C};
+        *reinterpret_cast<v4i*>(lds + TAB0 + 2 * NO * 4 + i * 16) = *reinterpret_cast<const v4i*>(a.dw_ct.p + i / (C / 4) * a.dw_ct.stride + i % (C / 4) * 4);
+    const ChanTab pw_exact{reinterpret_cast<const float*>(lds + TAB0), NO}, dw_exact{reinterpret_cast<const float*>(lds + TAB0) + 2 * NO, C};
 
     // ---- staging of the input halo (as in DepthwiseMfmaKernel, all C channels) -------------------------------------------
     const int dxm = static_cast<int>(a.dw_xor);
@@ -189,6 +183,9 @@ void DwPwStreamKernel(DwPwStreamArgs a)
             if (st_lds[k] >= 0) *reinterpret_cast<v4i*>(lds + halo + st_lds[k]) = st[k] ^ dxm;
     };
 
+    // The first item's halo is requested ahead of the constants: it is wanted first, and loads arrive in the order of their requests.
+    issue(item);
+
     // ---- depthwise roles: lane (j, g): pixel j of a group of 16 and tap slot g as an operand, channel quad g as a result --
     const int j = lane & 15, g = lane >> 4;
     const int rj = j / TW, cj = j % TW;
@@ -228,24 +225,35 @@ void DwPwStreamKernel(DwPwStreamArgs a)
     // the codes of pixel (pg0 + u WPC) 16 + j, channels (cg0 + i) 16 + 4 g ..: one dword of the panel
     const int panel_write = PANEL0 + (pg0 * 16 + j) * KP + cg0 * 16 + 4 * g;
 
-    // ---- pointwise roles: wave owns 32 x 32 tiles [m0, m0 + MTW) x [n0, n0 + NTW) of the item's P x NO output -------------
-    const int m0 = G::BYN ? 0 : wave * MTW;
-    const int n0 = G::BYN ? wave * NTW : 0;
-    const int frag_row = lane & 31, frag_half = lane >> 5;
-    const int a_frag = PANEL0 + (m0 * 32 + frag_row) * KP + frag_half * 16;
-    const int b_frag = WTS0 + (n0 * 32 + frag_row) * KP + frag_half * 16;
-    // the wave's output area [64 pixels][LDO]; lane writes dwords at (pixel frag_row of tile mt, channels 8 q + 4 frag_half of tile nt)
-    const int out_area = OUT0 + wave * 64 * LDO;
-    const int out_write = out_area + frag_row * LDO + 4 * frag_half;
-    // 16-byte pieces of that area: piece id = k 64 + lane -> (pixel id / PPP, part id % PPP).  64 / PPP pixels per store
-    // instruction are whole tile rows, so a lane keeps its column and part; only the row moves with k.
-    constexpr int PPP = G::SC / 16;
-    constexpr int RPS = 64 / PPP / TW;                     // tile rows per store instruction
-    static_assert((64 / PPP) % TW == 0, "whole tile rows per store instruction");
-    const int sr0 = lane / PPP, part0 = lane % PPP;
-    const int y_col = (m0 * 32 + sr0) % TW;
+    // ---- pointwise roles: the wave's pixels [px0, px0 + PXW) and channels [n0, n0 + 64); lane (j, g): operand row or column j, bytes of K
+    // by g; as a result channels n0 + 4 j .. + 3 of pixels 4 g .. 4 g + 3 of a group of 16 ----------------------------------
+    constexpr int WN = G::WN, PXW = G::PXW, MT = G::MT, KB = G::KB, KST = G::KST, KL = KB / 4;    // KL: a lane's bytes of K
+    const int px0 = wave / WN * PXW, n0 = wave % WN * 64;
+    typedef typename std::conditional<KB == 64, v4i, long>::type KVec;
+    KVec pw[KST][4];
+    v4i pw_init[4];
+    Fast4 pf;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+    {
+#pragma unroll
+        for (int ks = 0; ks < KST; ++ks)
+            pw[ks][t] = *reinterpret_cast<const KVec*>(a.w + static_cast<long long>(n0 + 4 * j + t) * a.w_stride + ks * KB + g * KL);
+        const int c = a.pw_corr[n0 + 4 * j + t];
+        pw_init[t] = v4i{c, c, c, c};
+    }
+    pf = LoadFast4(a.pw_ct, n0 + 4 * j);
+    const int a_frag = PANEL0 + (px0 + j) * KP + g * KL;
+    // the wave's output area [PXW pixels][LDO]
+    const int out_area = OUT0 + wave * PXW * LDO;
+    const int out_write = out_area + 4 * g * LDO + 4 * j;
+    // 16-byte pieces of that area: piece id = k 64 + lane -> (pixel id / 4, part id % 4).  16 pixels per store instruction are whole
+    // tile rows, so a lane keeps its column and part; only the row moves with k.
+    constexpr int RPS = 16 / TW;                           // tile rows per store instruction
+    const int sr0 = lane / 4, part0 = lane % 4;
+    const int y_col = sr0 % TW;
     const int out_read = out_area + sr0 * LDO + part0 * 16;
-    const int y_lane = (((m0 * 32 + sr0) / TW) * a.Wo + y_col) * NO + n0 * 32 + part0 * 16;
+    const int y_lane = (((px0 + sr0) / TW) * a.Wo + y_col) * NO + n0 + part0 * 16;
     const int y_step = RPS * a.Wo * NO;
     const int image_bytes = a.Ho * a.Wo * NO;
 
@@ -255,7 +263,7 @@ void DwPwStreamKernel(DwPwStreamArgs a)
 #pragma unroll
         for (int k = 0; k < QUADS; ++k)
         {
-            const v4i v = *reinterpret_cast<const v4i*>(lds + out_read + k * (64 / PPP) * LDO);
+            const v4i v = *reinterpret_cast<const v4i*>(lds + out_read + k * 16 * LDO);
             const int yo = y_col < out_cols ? out_base + y_lane + k * y_step : static_cast<int>(0x80000000u);
             __builtin_amdgcn_raw_buffer_store_b128(v, yrsrc, yo, 0, 0);
         }
@@ -290,54 +298,33 @@ void DwPwStreamKernel(DwPwStreamArgs a)
         out_base = ((w.ty * TH) * a.Wo + w.tx * TW) * NO;
         out_cols = a.Wo - w.tx * TW;
         out_n = w.n;
-        const float* tab = reinterpret_cast<const float*>(lds + TAB0);
-        v16i acc[MTW][NTW];
-#pragma unroll
-        for (int nt = 0; nt < NTW; ++nt)
-        {
-            v16i init;
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-            {
-                const v4i c4 = *reinterpret_cast<const v4i*>(tab + 2 * NO + (n0 + nt) * 32 + 8 * q + 4 * frag_half);
-                init[4 * q + 0] = c4[0]; init[4 * q + 1] = c4[1]; init[4 * q + 2] = c4[2]; init[4 * q + 3] = c4[3];
-            }
-#pragma unroll
-            for (int mt = 0; mt < MTW; ++mt) acc[mt][nt] = init;
-        }
-#pragma unroll
-        for (int ks = 0; ks < C / 32; ++ks)
-        {
-            v4i fa[MTW], fw[NTW];
-#pragma unroll
-            for (int mt = 0; mt < MTW; ++mt) fa[mt] = *reinterpret_cast<const v4i*>(lds + a_frag + mt * 32 * KP + ks * 32);
-#pragma unroll
-            for (int nt = 0; nt < NTW; ++nt) fw[nt] = *reinterpret_cast<const v4i*>(lds + b_frag + nt * 32 * KP + ks * 32);
-#pragma unroll
-            for (int mt = 0; mt < MTW; ++mt)
-#pragma unroll
-                for (int nt = 0; nt < NTW; ++nt) acc[mt][nt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fw[nt], fa[mt], acc[mt][nt], 0, 0, 0);
-        }
         WithBits(a.pw_rq, [&](auto bits) {
 #pragma unroll
-        for (int nt = 0; nt < NTW; ++nt)
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
+            for (int mt = 0; mt < MT; ++mt)
             {
-                const int cl = (n0 + nt) * 32 + 8 * q + 4 * frag_half;
-                const Fast4 f = {*reinterpret_cast<const float4*>(tab + cl), *reinterpret_cast<const float4*>(tab + NO + cl)};
-                v4i v[MTW];
-                uint32_t out[MTW];
+                v4i acc[4];
 #pragma unroll
-                for (int mt = 0; mt < MTW; ++mt) v[mt] = Quad(acc[mt][nt], q);
-                RequantPixels<decltype(bits)::value, MTW>(v, out, f, pw_exact, cl, a.pw_rq);
+                for (int ks = 0; ks < KST; ++ks)
+                {
+                    const KVec x = *reinterpret_cast<const KVec*>(lds + a_frag + mt * 16 * KP + ks * KB);
 #pragma unroll
-                for (int mt = 0; mt < MTW; ++mt) *reinterpret_cast<uint32_t*>(lds + out_write + mt * 32 * LDO + nt * 32 + 8 * q) = out[mt];
+                    for (int t = 0; t < 4; ++t)
+                    {
+                        if constexpr (KB == 64) acc[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x, pw[ks][t], ks == 0 ? pw_init[t] : acc[t], 0, 0, 0);
+                        else acc[t] = __builtin_amdgcn_mfma_i32_16x16x32_i8(x, pw[ks][t], ks == 0 ? pw_init[t] : acc[t], 0, 0, 0);
+                    }
+                }
+                v4i v[4];
+                uint32_t out[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[r] = v4i{acc[0][r], acc[1][r], acc[2][r], acc[3][r]};
+                RequantPixels<decltype(bits)::value, 4>(v, out, pf, pw_exact, n0 + 4 * j, a.pw_rq);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) *reinterpret_cast<uint32_t*>(lds + out_write + (mt * 16 + r) * LDO) = out[r];
             }
         });
     };
 
-    issue(item);
     while (true)
     {
         // (one halo buffer: its readers, the depthwise phase of the item before, all passed that item's second barrier)
