@@ -8,6 +8,7 @@
 #include "dwpw_panel.h"
 #include "dwpw_stream_kernel.h"
 #include "pwdw_kernel.h"
+#include "stem_rgb_kernel.h"
 #include "pool_softmax_items.h"
 #include "igemm_ksplit_kernel.h"
 #include "pw_gemm_kernel.h"
@@ -411,6 +412,23 @@ int BuildPlan(const mi355x_conv2d_desc& d, const void* weights_host, const mi355
                 if (int rc = Upload(reinterpret_cast<void**>(&p->w_stem2), wm.data(), wm.size())) return rc;
             }
             p->stem_kp = kp;
+            // Three channels at stride 2, filter rows of up to eight (3x3: four) pixels: the kernel over pixels of four bytes.  Two halves of
+            // a 7x7 filter would take 128 registers of weights.
+            if (Ci == 3 && d.stride_x == 2 && ((Kh == 3 && Kw <= 4) || (Kh == 7 && Kw <= 8 && stem_fits)))
+            {
+                const int row = StemRgbRow(Kh), k = StemRgbK(Kh);
+                for (int half = 0; half < (stem_fits ? 1 : 2); ++half)
+                {
+                    const uint32_t* const src = half == 0 ? wp.data() : wp2.data();
+                    std::vector<int8_t> wr(static_cast<size_t>(rows) * k, 0);
+                    for (int c = 0; c < Co; ++c)
+                        for (int r = 0; r < Kh; ++r)
+                            for (int bidx = 0; bidx < row_bytes; ++bidx)
+                                wr[static_cast<size_t>(c) * k + r * row + bidx / 3 * 4 + bidx % 3] =
+                                    static_cast<int8_t>(src[(static_cast<size_t>(c) * Kh + r) * RD + bidx / 4] >> (8 * (bidx % 4)));
+                    if (int rc = Upload(reinterpret_cast<void**>(half == 0 ? &p->w_rgb : &p->w_rgb2), wr.data(), wr.size())) return rc;
+                }
+            }
         }
         char buf[96];
         snprintf(buf, sizeof(buf), "smallci_dot4_lds %dx%dx%d stride %u, tile 32x16", Kh, Kw, Ci, d.stride_x);
@@ -1192,6 +1210,19 @@ int RunPlan(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, hi
                 nbm = static_cast<long long>(batch) * a.tiles_x * a.tiles_y;
             }
             const dim3 gridm(static_cast<unsigned>(nbm));
+            if (p->w_rgb && static_cast<long long>(batch) * g.H * g.W * 3 >= 12)
+            {
+                a.w_rgb = p->w_rgb; a.w_rgb2 = p->w_rgb2;
+                NoteKernel("StemRgbKernel<%d, %d, %d, %s>", g.Kh, g.Co <= 32 ? 1 : 2, th8 ? 8 : 16, BoolName(p->w_rgb2 != nullptr));
+                const auto kernel = g.Kh == 3 ? (p->w_rgb2 ? (g.Co <= 32 ? StemRgbKernel<3, 1, 16, true> : StemRgbKernel<3, 2, 16, true>)
+                                                 : th8     ? (g.Co <= 32 ? StemRgbKernel<3, 1, 8> : StemRgbKernel<3, 2, 8>)
+                                                           : (g.Co <= 32 ? StemRgbKernel<3, 1, 16> : StemRgbKernel<3, 2, 16>))
+                                              : (th8 ? (g.Co <= 32 ? StemRgbKernel<7, 1, 8> : StemRgbKernel<7, 2, 8>)
+                                                     : (g.Co <= 32 ? StemRgbKernel<7, 1, 16> : StemRgbKernel<7, 2, 16>));
+                hipLaunchKernelGGL(kernel, gridm, dim3(256), 0, stream, a);
+                MI355X_HIP(hipGetLastError());
+                return 0;
+            }
             NoteKernel("SmallCiMfmaKernel<%d, %d, %d, %d, %s>", g.Kh, g.Kh == 3 ? 3 : 6, g.Co <= 32 ? 1 : 2, th8 ? 8 : 16, BoolName(p->w_stem2 != nullptr));
             if (th8)
             {

@@ -288,6 +288,8 @@ struct SmallCiArgs
     const int8_t* w_mfma;     // MFMA variant: [Co rounded up to 32][kp] bytes, a filter's rows as RD dwords each, zero padded
     const int8_t* w_mfma2;    // W2: the second halves, same layout
     int kp;                   // bytes per weight row of w_mfma (multiple of 32)
+    const int8_t* w_rgb;      // StemRgbKernel: [32 or 64 channels][StemRgbK] bytes
+    const int8_t* w_rgb2;     // W2: the second halves, same layout
     Requant rq;
 };
 

@@ -31,6 +31,8 @@ struct mi355x_conv2d_s
     int8_t*  w_stem   = nullptr;   // small-Ci conv on MFMA: [Co rounded up to 32][stem_kp]
     int8_t*  w_stem2  = nullptr;   // ... the second halves of weight differences that need two
     int      stem_kp  = 0;
+    int8_t*  w_rgb    = nullptr;   // three-channel stem at stride 2: weights as StemRgbKernel reads them
+    int8_t*  w_rgb2   = nullptr;   // ... and second halves
     uint32_t* dw_grp  = nullptr;   // depthwise 3x3: constants per group of 4 channels (kDwGrpDwords each: weight rows 0 .. 2, corr, m, b)
     uint32_t* w_dot4  = nullptr;   // depthwise 3x3: [C][4] dwords; small-Ci conv: [Co][Kh][RD] dwords
     uint32_t* w_dot4b = nullptr;   // depthwise 3x3 / small-Ci conv whose weight differences need two int8 halves: the second halves
@@ -69,6 +71,8 @@ struct mi355x_conv2d_s
         (void)hipFree(w_panel);
         (void)hipFree(w_stem);
         (void)hipFree(w_stem2);
+        (void)hipFree(w_rgb);
+        (void)hipFree(w_rgb2);
         (void)hipFree(w_dot4);
         (void)hipFree(w_dot4b);
         (void)hipFree(chan);
