@@ -375,7 +375,7 @@ __device__ __forceinline__ void IgemmLdsTile(const IgemmArgs& a, const int tile,
                 if (r < BM && m < a.M)
                 {
                     v4i ov = *reinterpret_cast<const v4i*>(Os + r * LDO + oc * 16);
-                    if (fuse) ov = AddResidual16(ov, other[i], a.add);
+                    if (fuse) ov = AddQuantize16Dev(ov, other[i], a.add);
                     StoreOut16(outp, static_cast<long long>(m) * a.Co + c0, ov);
                 }
             }

@@ -320,20 +320,16 @@ __global__ __launch_bounds__(64) void GlobalPoolSmallKernel(PoolArgs p, QIn qin,
 }
 
 // 16 elements per thread, 16-byte loads and stores
-template <bool CLAMP>
-__global__ __launch_bounds__(256) void AddVec16Kernel(AddFuse f, const v4u* __restrict__ x0,
-                                                      const v4u* __restrict__ x1, v4u* __restrict__ y, size_t n16)
+__global__ __launch_bounds__(256) void AddVec16Kernel(AddFuse f, const StoreVec4* __restrict__ x0,
+                                                      const StoreVec4* __restrict__ x1, StoreVec4* __restrict__ y, size_t n16)
 {
     const OutPtr outp = MakeOutPtr(reinterpret_cast<uint8_t*>(y), static_cast<long long>(n16) * 16);
     size_t i = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
     const size_t stride = static_cast<size_t>(gridDim.x) * 256;
     for (; i < n16; i += stride)
     {
-        const v4u a = x0[i], b = x1[i];
-        v4u o;
-#pragma unroll
-        for (int d = 0; d < 4; ++d) o[d] = AddQuantize4Dev<CLAMP>(a[d], b[d], f);
-        StoreOut16(outp, static_cast<long long>(i) * 16, StoreVec4{static_cast<int>(o[0]), static_cast<int>(o[1]), static_cast<int>(o[2]), static_cast<int>(o[3])});
+        const StoreVec4 a = x0[i], b = x1[i];
+        StoreOut16(outp, static_cast<long long>(i) * 16, AddQuantize16Dev(a, b, f));
     }
 }
 
@@ -564,12 +560,8 @@ int mi355x_add_run(size_t n, const mi355x_quant* in0_q, const mi355x_quant* in1_
     {
         NoteKernel("AddVec16Kernel");
         const AddFuse f = MakeAddFuse(*in0_q, *in1_q, *out_q, activation, a, b);
-        if (f.rq.pk_full)
-            hipLaunchKernelGGL(AddVec16Kernel<false>, dim3(GridFor(n / 16)), dim3(256), 0, ToHip(stream), f,
-                               static_cast<const v4u*>(input0_dev), static_cast<const v4u*>(input1_dev), static_cast<v4u*>(output_dev), n / 16);
-        else
-            hipLaunchKernelGGL(AddVec16Kernel<true>, dim3(GridFor(n / 16)), dim3(256), 0, ToHip(stream), f,
-                               static_cast<const v4u*>(input0_dev), static_cast<const v4u*>(input1_dev), static_cast<v4u*>(output_dev), n / 16);
+        hipLaunchKernelGGL(AddVec16Kernel, dim3(GridFor(n / 16)), dim3(256), 0, ToHip(stream), f,
+                           static_cast<const StoreVec4*>(input0_dev), static_cast<const StoreVec4*>(input1_dev), static_cast<StoreVec4*>(output_dev), n / 16);
     }
     else
     {

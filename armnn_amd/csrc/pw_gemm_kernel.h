@@ -183,7 +183,7 @@ __global__ __launch_bounds__(256) void PwGemmKernel(PwArgs a)
                 const int c0 = n0 + cc * 16;
                 if (row < a.M && c0 < a.N)
                     StoreOut16(outp, static_cast<long long>(row) * a.N + c0,
-                               AddResidual16(*reinterpret_cast<const v4i*>(ostage + r * LDO + cc * 16), other[i], a.add));
+                               AddQuantize16Dev(*reinterpret_cast<const v4i*>(ostage + r * LDO + cc * 16), other[i], a.add));
             }
         }
         else if ((a.N & 15) == 0)

@@ -200,7 +200,7 @@ __global__ __launch_bounds__(256, KB <= 256 ? 4 : 3) void RowPanelKernel(IgemmAr
         if (m < a.M && c0 < a.Co)
         {
             v4i v = *reinterpret_cast<const v4i*>(row_lds + r * OP + chunk * 16);
-            if (fuse) v = AddResidual16(v, other[i], a.add);
+            if (fuse) v = AddQuantize16Dev(v, other[i], a.add);
             StoreOut16(outp, static_cast<long long>(m) * a.Co + c0, v);
         }
     }

@@ -214,7 +214,7 @@ __global__ __launch_bounds__(256) void SmallConvKernel(IgemmArgs a)
     {
         v4i v = *reinterpret_cast<const v4i*>(&stage[orow][(lane & 1) * 4]);
         const long long at = static_cast<long long>(om) * a.Co + c0;
-        if (fuse) v = AddResidual16(v, other, a.add);
+        if (fuse) v = AddQuantize16Dev(v, other, a.add);
         if (a.vec_out) StoreOut16(MakeOutPtr(a.y, static_cast<long long>(a.M) * a.Co), at, v);
         else StoreRagged16(a.y + at, v, a.Co - c0);
     }
