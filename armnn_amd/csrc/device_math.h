@@ -307,14 +307,19 @@ __device__ __forceinline__ void WithBits(const Requant& rq, F write_out)
     else write_out(std::false_type{});
 }
 
-// one channel (scalar kernels): the same bracket
-__device__ __forceinline__ int Requant1Dev(int acc, const ChanTab& ct, int c, const Requant& rq)
+// one channel (scalar kernels): the same bracket.  m, b: rows 2 and 3 of the table at channel c
+__device__ __forceinline__ int Requant1Dev(int acc, float m, float b, const ChanTab& ct, int c, const Requant& rq)
 {
-    const float p = __fmaf_rn(rq.acc_base != 0 ? AccValue<true>(acc) : AccValue<false>(acc), ct.p[2 * ct.stride + c], ct.p[3 * ct.stride + c]);
+    const float p = __fmaf_rn(rq.acc_base != 0 ? AccValue<true>(acc) : AccValue<false>(acc), m, b);
     const U16x2 v = __builtin_amdgcn_cvt_pknorm_u16(p, __fsub_rn(p, rq.two_c));
     const int hi = v.x >> 8, lo = v.y >> 8;
     if (__builtin_expect(hi != lo, 0)) return RequantExactDev(acc - rq.acc_base, ct.p[c], ct.p[ct.stride + c], rq);
     return min(max(hi - rq.pk_bias, rq.act_lo), rq.act_hi);
+}
+
+__device__ __forceinline__ int Requant1Dev(int acc, const ChanTab& ct, int c, const Requant& rq)
+{
+    return Requant1Dev(acc, ct.p[2 * ct.stride + c], ct.p[3 * ct.stride + c], ct, c, rq);
 }
 
 // value already in float (pooling, add, ...): reciprocal fast path with the exact fallback near ties.

@@ -9,9 +9,8 @@
 //   The epilogue requantizes 4 channels at a time, stages the 32 x BN byte tile in the wave's private LDS area and
 //   writes it with 16-byte row-contiguous stores.
 //
-//   Zero points: uint8 activations are xor-ed with 0x80 in registers; acc = sum x' w, and the per-channel constant
-//   corr[n] = -zx' * sum_k w[n][k] is folded into the requantization constants (rows 5/6 of the channel table) on
-//   the fast path and added to the accumulator on the exact path.
+//   Zero points: uint8 activations are xor-ed with 0x80 in registers; acc = sum x' w, and accumulators start from the plan's
+//   corr[n] = -zx' * sum_k w[n][k] (and Requant::acc_base).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -281,6 +280,13 @@ __global__ __launch_bounds__(256) void PwGemmKernel(PwArgs a)
 // FullyConnected / pointwise layers with at most 4 GEMM rows (batch-1 inference): a matrix-vector product bound by
 // streaming the weights once from HBM.  A wave owns 4 output channels at a time; its 64 lanes split K in 16-byte
 // chunks (one coalesced 1 KB load per weight row and step), multiply with v_dot4 and reduce across the wave.
+// MR: rows of a wave, one or two; three and four rows make two groups of blocks.  What such a launch takes beyond an empty one's 2.7 us
+// is mostly instructions, each executed once or twice and fetched from L2 for that: with four rows to a wave there was twice the
+// products and exchanges, and a layer of 64 x 10 took 5.1 us where it now takes 2.8.  For the same reason the sums are exchanged by
+// halves and requantized side by side in the lanes that end up with them (one after the other in lane 0 before: 0.8 us more at one row), and
+// the loads of up to four steps go out together (a branch on the zero point stood between them: 0.4 us).
+// Before -> here: 4096 x 4096 at one row 4.7 -> 3.4 us = 4.9 TB/s, two 6.2 -> 4.0, three 7.7 -> 5.0, four 9.1 -> 5.0; 1024 -> 1001 3.5 -> 2.6
+// and, four rows, 7.3 -> 3.0; 2048 -> 1001 3.8 -> 2.65; 4032 -> 155, four rows, 10.0 -> 3.5.
 struct GemvArgs
 {
     const uint8_t* x;        // [M][K]
@@ -290,8 +296,8 @@ struct GemvArgs
     uint8_t*       y;        // [M][N]
     int M, K, N, w_stride;
     uint32_t xor_mask;
-    int zw_neg;              // minus the zero point of the stored int8 weights; when not 0 every row's activations are summed
-                             // as well and zw_neg times that sum joins the row's accumulators
+    int zw_neg;              // minus the zero point of the stored int8 weights: zw_neg times the sum of a row's activations joins the
+                             // row's accumulators
     Requant rq;
 };
 
@@ -301,9 +307,17 @@ __global__ __launch_bounds__(256) void GemvKernel(GemvArgs a)
     constexpr int R = 4;
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
-    const int n0 = (static_cast<int>(blockIdx.x) * 4 + wave) * R;
+    // the groups of rows of the same 16 channels run on one XCD, one behind the other: its L2 has the weights for the second
+    const int b = static_cast<int>(blockIdx.x), groups = MR == 1 ? 1 : (a.M + MR - 1) / MR;       // (MR = 1: a single row)
+    const int m0 = groups == 1 ? 0 : (b >> 3) % groups * MR, block = groups == 1 ? b : (b >> 3) / groups * 8 + (b & 7);
+    const int n0 = (block * 4 + wave) * R;
     if (n0 >= a.N) return;
     const int xm = static_cast<int>(a.xor_mask);
+    // the sum this lane requantizes in the end, channel rank % R of row rank / R; its constants are requested ahead of the weights
+    constexpr int RANKS = R * MR;
+    const int rank = lane / (64 / RANKS), r_own = rank % R, c_own = min(n0 + r_own, a.N - 1);
+    const int start = a.corr[c_own];
+    const float fm = a.ct.p[2 * a.ct.stride + c_own], fb = a.ct.p[3 * a.ct.stride + c_own];
     int acc[R][MR], xs[MR];
 #pragma unroll
     for (int r = 0; r < R; ++r)
@@ -311,51 +325,72 @@ __global__ __launch_bounds__(256) void GemvKernel(GemvArgs a)
         for (int m = 0; m < MR; ++m) acc[r][m] = 0;
 #pragma unroll
     for (int m = 0; m < MR; ++m) xs[m] = 0;
-    const int chunks = a.K >> 4;
+    const int chunks = a.K >> 4, steps = (chunks + 63) >> 6;
     const int8_t* wrow = a.w + static_cast<long long>(n0) * a.w_stride;
-#pragma unroll 4
-    for (int j = lane; j < chunks; j += 64)
-    {
-        v4i xv[MR];
+    // UN steps of 64 chunks, all of their loads requested before the first is used; a lane past the last chunk reads that one again and
+    // counts it for nothing.  The rows' sums are taken whether the weights have a zero point or not: a branch here would
+    // stand between the steps' loads.
+    auto walk = [&](int s0, auto un) {
+        constexpr int UN = decltype(un)::value;
+        v4i xv[UN][MR], wv[UN][R];
 #pragma unroll
-        for (int m = 0; m < MR; ++m) xv[m] = *reinterpret_cast<const v4i*>(a.x + static_cast<long long>(m) * a.K + j * 16) ^ xm;
-        if (a.zw_neg != 0)       // uniform
+        for (int u = 0; u < UN; ++u)
         {
+            const int j = min((s0 + u) * 64 + lane, chunks - 1) * 16;
+#pragma unroll
+            for (int r = 0; r < R; ++r) wv[u][r] = *reinterpret_cast<const v4i*>(wrow + static_cast<long long>(r) * a.w_stride + j);
+#pragma unroll
+            for (int m = 0; m < MR; ++m) xv[u][m] = *reinterpret_cast<const v4i*>(a.x + static_cast<long long>(min(m0 + m, a.M - 1)) * a.K + j);
+        }
+#pragma unroll
+        for (int u = 0; u < UN; ++u)
+        {
+            const int counts = (s0 + u) * 64 + lane < chunks ? -1 : 0;
 #pragma unroll
             for (int m = 0; m < MR; ++m)
+            {
+                const v4i x = (xv[u][m] ^ xm) & counts;
 #pragma unroll
-                for (int d = 0; d < 4; ++d) xs[m] = __builtin_amdgcn_sdot4(xv[m][d], 0x01010101, xs[m], false);
+                for (int d = 0; d < 4; ++d)
+                {
+                    xs[m] = __builtin_amdgcn_sdot4(x[d], 0x01010101, xs[m], false);
+#pragma unroll
+                    for (int r = 0; r < R; ++r) acc[r][m] = __builtin_amdgcn_sdot4(x[d], wv[u][r][d], acc[r][m], false);
+                }
+            }
         }
+    };
+    int s0 = 0;
+    for (; s0 + 4 <= steps; s0 += 4) walk(s0, std::integral_constant<int, 4>{});
+    if (s0 + 2 <= steps) { walk(s0, std::integral_constant<int, 2>{}); s0 += 2; }
+    if (s0 < steps) walk(s0, std::integral_constant<int, 1>{});
 #pragma unroll
-        for (int r = 0; r < R; ++r)
-        {
-            const v4i wv = *reinterpret_cast<const v4i*>(wrow + static_cast<long long>(r) * a.w_stride + j * 16);
+    for (int m = 0; m < MR; ++m)
 #pragma unroll
-            for (int m = 0; m < MR; ++m)
+        for (int r = 0; r < R; ++r) acc[r][m] += xs[m] * a.zw_neg;       // joins every channel's sum, lane by lane
+    // The sums meet by halves: a lane keeps one half of its values and gives the other away, so that each exchange is over half as
+    // many, and every lane ends with one of the sums, value RANK of them, which it requantizes
+    int v[RANKS];
 #pragma unroll
-                for (int d = 0; d < 4; ++d) acc[r][m] = __builtin_amdgcn_sdot4(xv[m][d], wv[d], acc[r][m], false);
-        }
-    }
-    if (a.zw_neg != 0)
+    for (int i = 0; i < RANKS; ++i) v[i] = acc[i % R][i / R];
+#pragma unroll
+    for (int half = RANKS / 2, o = 32; o > 0; o >>= 1, half >>= 1)
     {
-#pragma unroll
-        for (int m = 0; m < MR; ++m)
+        if (half > 0)
         {
-            xs[m] *= a.zw_neg;           // joins every channel's sum below, lane by lane
+            const bool upper = (lane & o) != 0;
 #pragma unroll
-            for (int r = 0; r < R; ++r) acc[r][m] += xs[m];
+            for (int i = 0; i < half; ++i)
+            {
+                const int keep = upper ? v[i + half] : v[i], give = upper ? v[i] : v[i + half];
+                v[i] = keep + __shfl_xor(give, o);
+            }
         }
+        else v[0] += __shfl_xor(v[0], o);
     }
-#pragma unroll
-    for (int r = 0; r < R; ++r)
-#pragma unroll
-        for (int m = 0; m < MR; ++m)
-        {
-            int v = acc[r][m];
-            for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-            if (lane == 0 && n0 + r < a.N)
-                a.y[static_cast<long long>(m) * a.N + n0 + r] = static_cast<uint8_t>(Requant1Dev(v + a.corr[n0 + r], a.ct, n0 + r, a.rq));
-        }
+    const int row = m0 + rank / R;
+    if ((lane & (64 / RANKS - 1)) == 0 && row < a.M && n0 + r_own < a.N)
+        a.y[static_cast<long long>(row) * a.N + n0 + r_own] = static_cast<uint8_t>(Requant1Dev(v[0] + start, fm, fb, a.ct, c_own, a.rq));
 }
 
 // ---------------------------------------------------------------------------------------------------------------
