@@ -6,9 +6,9 @@
 //   * The outputs meet in LDS and leave as 16 bytes per lane, with an Addition behind the layer on the way, whose other input was
 //     requested at the start.
 // Four waves per SIMD (128 registers) are what hides the round trips: the same kernel at 144 registers took 7.0 us where it takes
-// 5.3.  The largest share of a launch is the CU's L1, at two clocks a line: 64 rows and 128 rows of weights per 128 bytes of K, at 28 x 28
-// x 128 -> 512 6.4 k accesses per CU, 13 k of the launch's 18 k clocks; over 56 x 56 x 256 -> 64 the rows' way from memory is (4.1 TB/s,
-// 910 clocks a request).  With the Addition the write-out's VALU work comes on top.  Before -> here, 32 images unless said: 28 x 28 x 128 -> 512 14.8 -> 8.3 us, 14 x 14 x 256 -> 1024
+// 5.3.  What takes the time is waiting (54 % of a wave's life) and the CU's L1, at two clocks a line: 64 rows and 128 rows of weights per 128 bytes
+// of K, at 28 x 28 x 128 -> 512 4.1 k accesses per CU, 8 k of the launch's 18 k clocks; over 56 x 56 x 256 -> 64 the rows' way from memory is
+// (3.9 TB/s, 840 clocks a request).  With the Addition the write-out's VALU work comes on top.  Before -> here, 32 images unless said: 28 x 28 x 128 -> 512 14.8 -> 8.3 us, 14 x 14 x 256 -> 1024
 // 9.4 -> 6.7, 56 x 56 x 256 -> 64 18.1 -> 9.7, 56 x 56 x 256 -> 512 52.7 -> 33.1, 56 x 56 x 48 -> 96 (16 images) 7.4 -> 5.1.
 #pragma once
 
