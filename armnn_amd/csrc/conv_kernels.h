@@ -242,6 +242,10 @@ struct IgemmArgs
     int rowsum_bias;        // (K_pad - K) * zx': what the bytes beyond K add to a row sum
     int k_tiles = 0;        // IgemmKernel: k-tiles to walk where they are fewer than K_pad holds
     int vec_out = 0;        // IgemmKernel: output rows are whole, aligned 16-byte pieces
+    // SmallConvKernel: where each of the four waves starts in K (first k-step, and the filter tap and byte of it that begins there), and
+    // the reciprocals that decode a pixel, 2^32 / Wo and / Ho rounded up (0: the sizes are beyond them)
+    struct { int step, ky, kx, ci; } wave_k[5] = {};
+    uint32_t wo_magic = 0, ho_magic = 0;
     Requant rq;
     const uint8_t* res = nullptr;   // direct-to-LDS kernel: the other input of an Addition fused into the write-out ([M][Co]), or null
     AddFuse add;

@@ -119,6 +119,18 @@ int mi355x::LaunchSmallConv(const mi355x_conv2d_s* p, uint32_t batch, const void
         a.Ck = p->ragged_ck;
         a.x_last16 = a.x + static_cast<long long>(batch) * p->geom.H * p->geom.W * p->geom.Ci - 16;
     }
+    const int tap_bytes = rg ? a.Ck : a.Ci, steps = (a.Kh * a.Kw * tap_bytes + 63) / 64;
+    for (int w = 0; w <= 4; ++w)
+    {
+        const int step = steps * w / 4, tap = step * 64 / tap_bytes;
+        a.wave_k[w] = {step, tap / a.Kw, tap % a.Kw, step * 64 % tap_bytes};
+    }
+    // x * ceil(2^32 / d) / 2^32 is x / d rounded down as long as x d < 2^32
+    if (static_cast<long long>(a.M) * std::max(a.Wo, a.Ho) < 0x100000000ll)
+    {
+        a.wo_magic = static_cast<uint32_t>(0x100000000ull / a.Wo + (0x100000000ull % a.Wo != 0));
+        a.ho_magic = static_cast<uint32_t>(0x100000000ull / a.Ho + (0x100000000ull % a.Ho != 0));
+    }
     NoteKernel("SmallConvKernel<%s, %s>", BoolName(aw), BoolName(rg));
     const auto kernel = aw ? (rg ? SmallConvKernel<true, true> : SmallConvKernel<true, false>) : (rg ? SmallConvKernel<false, true> : SmallConvKernel<false, false>);
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, stream, a);

@@ -8,11 +8,14 @@
 //     its way after a quarter as many round trips and no LDS staging or barrier lies in between;
 //   * the partial tiles meet in LDS, where the waves add them up in a fixed order, requantize four channels per lane, and
 //     one wave writes the tile in 16-byte pieces (with a following Addition on the way, if there is one).
-// What is left is latency: waves wait 63 % of their cycles (3 x 3 over 14 x 14 x 256, one image), and of the 14 k cycles of a block the
+// What is left is latency: waves wait 59 % of their cycles (3 x 3 over 14 x 14 x 256, one image), and of the 13 k cycles of a block the
 // CU's address unit, which takes an instruction's cache lines one after the other, is busy for 4.3 k.  Hence v_mfma_i32_16x16x64_i8,
 // whose activation operand is 16 pixels x 64 contiguous bytes (32x32x32: 32 pixels x 32), and weights stored in operand order
 // (PackFragKernel), so that a wave's weight load is one run of 1 KB instead of 32 rows.
-// Launches back to back, before -> here (one image unless said): 3 x 3 over 28 x 28 x 128 7.2 -> 4.5 us, 14 x 14 x 256 9.1 ->
+// The other part of a launch is instructions that are fetched to be executed once or twice: with the pixels' divisions as multiplications
+// by reciprocals, each wave's start in K from the host and no loop in the walk over taps of 64 bytes and more, 3 x 3 layers take 0.25 us
+// less (28 x 28 x 128 4.83 -> 4.55, 14 x 14 x 256 5.82 -> 5.53, 7 x 7 x 512 7.70 -> 7.48, 56 x 56 x 64 3.93 -> 3.70), ResNet-50 116.2 -> 115.7.
+// Launches back to back, against the larger tiles (one image unless said): 3 x 3 over 28 x 28 x 128 7.2 -> 4.5 us, 14 x 14 x 256 9.1 ->
 // 5.5, 7 x 7 x 512 13.3 -> 7.4, 56 x 56 x 64 5.9 -> 3.7, 28 x 28 x 96 7.2 -> 3.8; 1 x 1 over 14 x 14 x 1024 -> 256 5.7 -> 4.0, 28 x 28 x
 // 128 -> 256 5.6 -> 3.1; FullyConnected 4096 -> 4096 of 64 rows 12.9 -> 9.6.  An empty kernel takes 2.75 us in such a row.
 #pragma once
@@ -83,10 +86,11 @@ __global__ __launch_bounds__(256) void SmallConvKernel(IgemmArgs a)
         if (a.unit) { n = 0; oy = 0; ox = m; }
         else
         {
-            ox = m % a.Wo;
-            const int t = m / a.Wo;
-            oy = t % a.Ho;
-            n = t / a.Ho;
+            // (a divisor of 1 has no reciprocal in 32 bits)
+            const int t = a.Wo == 1 ? m : a.wo_magic != 0 ? static_cast<int>(__umulhi(static_cast<uint32_t>(m), a.wo_magic)) : m / a.Wo;
+            ox = m - t * a.Wo;
+            n = a.Ho == 1 ? t : a.ho_magic != 0 ? static_cast<int>(__umulhi(static_cast<uint32_t>(t), a.ho_magic)) : t / a.Ho;
+            oy = t - n * a.Ho;
         }
         iy0[p] = oy * a.stride_y - a.pad_top;
         ix0[p] = ox * a.stride_x - a.pad_left;
@@ -95,17 +99,32 @@ __global__ __launch_bounds__(256) void SmallConvKernel(IgemmArgs a)
     // this wave's k-steps of 64 bytes
     const int tap_bytes = RG ? a.Ck : a.Ci;
     const int steps = (a.Kh * a.Kw * tap_bytes + 63) >> 6;
-    const int s0 = steps * wave / NW, s1 = steps * (wave + 1) / NW;
+    const int uw = __builtin_amdgcn_readfirstlane(wave);
+    const int s0 = a.wave_k[uw].step, s1 = a.wave_k[uw + 1].step;
     const int8_t* wp = a.w + static_cast<long long>(2 * tn) * steps * 1024 + lane * 16;
     const long long w_next = static_cast<long long>(steps) * 1024;       // the tile's second group of 16 channels
     // the lane's chunk: filter tap and channel, advanced by 64 bytes per step
-    int ci = s0 * 64 + g * 16, ky, kx;
-    {
-        const int tap = ci / tap_bytes;
-        ci -= tap * tap_bytes;
-        ky = tap / a.Kw;
-        kx = tap - ky * a.Kw;
-    }
+    int ci = a.wave_k[uw].ci + g * 16, ky = a.wave_k[uw].ky, kx = a.wave_k[uw].kx;
+    // 64 bytes on: past the tap's end at most once where a tap has 64 bytes (uniform; a loop here is branches for every step)
+    const bool wide = tap_bytes >= 64;
+    auto wrap = [&] {
+        if (wide)
+        {
+            const bool over = ci >= tap_bytes;
+            ci -= over ? tap_bytes : 0;
+            kx += over ? 1 : 0;
+            const bool row = kx == a.Kw;
+            kx = row ? 0 : kx;
+            ky += row ? 1 : 0;
+            return;
+        }
+        while (ci >= tap_bytes)
+        {
+            ci -= tap_bytes;
+            if (++kx == a.Kw) { kx = 0; ++ky; }
+        }
+    };
+    wrap();
     // what this wave will requantize with (wave 2 c + p finishes channel group c of pixel group p), requested ahead of the operands
     const int cg = wave >> 1, pg = wave & 1;
     const int cq = tn * 32 + cg * 16 + 4 * g;
@@ -147,11 +166,7 @@ __global__ __launch_bounds__(256) void SmallConvKernel(IgemmArgs a)
             wv[u][0] = *reinterpret_cast<const v4i*>(ws);
             wv[u][1] = *reinterpret_cast<const v4i*>(ws + w_next);
             ci += 64;
-            while (ci >= tap_bytes)
-            {
-                ci -= tap_bytes;
-                if (++kx == a.Kw) { kx = 0; ++ky; }
-            }
+            wrap();
         }
 #pragma unroll
         for (int u = 0; u < U; ++u)
