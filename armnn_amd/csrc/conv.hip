@@ -1,5 +1,6 @@
 // Convolution2d / DepthwiseConvolution2d / FullyConnected entry points of the C ABI: plan creation
 // (constant re-layout, per-channel requantization constants, kernel selection) and launches.
+#include "bracket.h"
 #include "common.h"
 #include "conv_kernels.h"
 #include "dw_stem_kernels.h"
@@ -123,15 +124,37 @@ int BuildPlan(const mi355x_conv2d_desc& d, const void* weights_host, const mi355
         const long long xmax = g.in_u8 ? std::max(std::abs(0 - g.zx), std::abs(255 - g.zx)) : std::max(std::abs(-128 - g.zx), std::abs(127 - g.zx));
         const size_t nw = static_cast<size_t>(d.depthwise ? 1 : Co) * Kh * Kw * (d.depthwise ? Co : Ci);
         const uint8_t* wb = static_cast<const uint8_t*>(weights_host);
-        long long wmax = 0;
-        for (size_t i = 0; i < nw; ++i)
+        const int flip = g.w_u8 ? 0 : 0x80;
+        // each channel's weights: [Co][K], or [Kh * Kw][Co] in a depthwise layer
+        const size_t per_row = d.depthwise ? static_cast<size_t>(Co) : static_cast<size_t>(p->K);
+        std::vector<double>& most = p->chan_most;
+        most.assign(Co, 0.0);
+        int wmax = 0;
+        for (size_t i = 0; i < nw; i += per_row)
         {
-            const int wv = g.w_u8 ? static_cast<int>(wb[i]) : static_cast<int>(static_cast<int8_t>(wb[i]));
-            wmax = std::max<long long>(wmax, std::abs(wv - g.zw));
+            if (d.depthwise)
+                for (int c = 0; c < Co; ++c)
+                {
+                    const int v = std::abs((wb[i + c] ^ flip) - flip - g.zw);
+                    wmax = std::max(wmax, v);
+                    most[c] += v;
+                }
+            else
+            {
+                long long sum = 0;
+                for (size_t k = 0; k < per_row; ++k)
+                {
+                    const int v = std::abs((wb[i + k] ^ flip) - flip - g.zw);
+                    wmax = std::max(wmax, v);
+                    sum += v;
+                }
+                most[i / per_row] = static_cast<double>(sum);
+            }
         }
+        for (double& v : most) v *= static_cast<double>(xmax);
         p->acc_most = static_cast<long long>(p->K) * xmax * wmax;
         if (p->acc_most >= (1ll << 31))
-            return SetError(MI355X_ERR_UNSUPPORTED, "%d taps of up to %lld x %lld could overflow the 32-bit accumulator", p->K, xmax, wmax);
+            return SetError(MI355X_ERR_UNSUPPORTED, "%d taps of up to %lld x %lld could overflow the 32-bit accumulator", p->K, xmax, static_cast<long long>(wmax));
     }
     p->Co_pad = (Co + 127) / 128 * 128;
     // K is padded to the implicit GEMM's k-tile.  128-byte tiles pay when a row chunk is one whole cache line, i.e. when
@@ -455,60 +478,23 @@ int BuildPlan(const mi355x_conv2d_desc& d, const void* weights_host, const mi355
         p->info = d.depthwise ? "direct_depthwise" : "direct_conv";
     }
     if (int rc = Upload(reinterpret_cast<void**>(&p->chan), p->chan_host.data(), p->chan_host.size() * sizeof(float))) return rc;
-    p->chan_host.clear();
-    p->chan_host.shrink_to_fit();
+    p->chan_host = std::vector<float>();
+    p->chan_most = std::vector<double>();
     return 0;
 }
 
 // Rows 2 and 3 of the channel table, Requant::two_c and Requant::acc_base; `corr` (may be empty), the zero-point correction, becomes
-// what accumulators of raw products start from.  What the bracket encloses is told in device_math.h.
+// what accumulators of raw products start from.
 void FinishTable(mi355x_conv2d_s* p, std::vector<int32_t>& corr)
 {
-    constexpr double u = 1.0 / 16777216.0;            // unit roundoff of fp32
-    constexpr double unit = 256.0 / 65535.0;          // a code on the scale of m and b
-    constexpr double whole = 1 << 22;                 // 1.5 * 2^23 + sum steps in ones up to here
     const mi355x_conv2d_desc& d = p->d;
-    const int CP = p->Co_pad, Co = static_cast<int>(d.out_c);
-    std::vector<float>& tab = p->chan_host;
-    const double s_out = d.output.scale;
-    // the fast path works 128 codes higher for signed outputs (Requant::pk_bias), so that is its offset
-    const double zp = d.output.offset + p->rq.pk_bias;
-    // |t - offset'| of a value that is not saturated
-    const double most_t = std::max(std::fabs(257.5 - zp), std::fabs(-1.5 - zp));
-    std::vector<uint8_t> fast(Co, 0);
-    bool bits = p->acc_most < (1ll << 29);
-    bool all_fast = s_out > 0x1p-90 && s_out < 0x1p90;       // (SettleDev: nothing near the ends of fp32)
-    double c_codes = 1024.0 * u;                      // (enough to tell p from q anywhere)
-    for (int c = 0; c < Co; ++c)
-    {
-        const double fm = static_cast<double>(tab[c]) / s_out, fb = static_cast<double>(tab[CP + c]) / s_out, bias = std::fabs(fb);
-        // Half-width in codes: the reference multiplies, adds the bias and divides, on values of up to |t| + |bias|, |t| and |t| codes (1.02
-        // for the second order); both sides convert the sum, which rounds from 2^24 on; m and b are off by what they are off; p and
-        // q round on a scale where 256 codes are 1 (128 each).
-        const double m = fm * unit, b = (256.0 * (fb + zp + 0.5) - 0.5) / 65535.0, reach = most_t + bias;
-        const double m_off = m != 0.0 ? std::fabs(static_cast<double>(static_cast<float>(m)) / m - 1.0) * reach : 0.0;
-        const double w = u * (1.02 * (reach + 2.0 * most_t) + (reach >= 16777216.0 * std::fabs(fm) ? 2.04 * reach : 0.0) + 256.0) + m_off +
-                         0.5 * std::ldexp(1.0, std::ilogb(std::fabs(b) + 0.001) - 23) / unit;
-        fast[c] = p->rq.fast_ok != 0 && std::isfinite(fm) && std::isfinite(fb) && (fm == 0.0 || (std::isnormal(tab[c]) && std::isnormal(static_cast<float>(m)))) &&
-                  w < 0.0625 && static_cast<double>(p->acc_most) * std::fabs(fm) < 268435456.0;
-        all_fast &= fast[c] != 0;
-        if (!fast[c]) continue;
-        c_codes = std::max(c_codes, w);
-        // where the steps are not ones, codes must be saturated
-        if (static_cast<double>(p->acc_most) > whole && whole * std::fabs(fm) - std::fabs(fb + zp) < 300.0) bits = false;
-    }
-    const double c_x = c_codes * unit;
-    for (int c = 0; c < Co; ++c)
-    {
-        const double fm = static_cast<double>(tab[c]) / s_out, fb = static_cast<double>(tab[CP + c]) / s_out;
-        // (a channel without a fast path: a byte's edge whatever the sum, p gives 128 and q 127)
-        const double code = fast[c] ? fb + zp + 0.5 : 128.0;
-        tab[2 * CP + c] = fast[c] ? static_cast<float>(fm * unit) : 0.0f;
-        tab[3 * CP + c] = static_cast<float>((256.0 * code - 0.5) / 65535.0 + c_x);
-    }
-    p->rq.two_c = std::nextafterf(static_cast<float>(2.0 * c_x), 1.0f);
-    p->rq.all_fast = all_fast ? 1 : 0;
-    p->rq.acc_base = bits ? kAccBaseBits : 0;
+    const int CP = p->Co_pad;
+    float* const tab = p->chan_host.data();
+    const Bracket k = ChooseBracket(tab, tab + CP, p->chan_most.data(), static_cast<int>(d.out_c), d.output.scale, d.output.offset + p->rq.pk_bias, p->rq.fast_ok != 0,
+                                    static_cast<double>(p->acc_most), tab + 2 * CP, tab + 3 * CP);
+    p->rq.two_c = k.two_c;
+    p->rq.all_fast = k.all_fast ? 1 : 0;
+    p->rq.acc_base = k.bits ? kAccBaseBits : 0;
     for (int32_t& v : corr) v += p->rq.acc_base;
 }
 

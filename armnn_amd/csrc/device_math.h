@@ -37,7 +37,7 @@ __device__ __forceinline__ int RequantExactDev(int acc, float mult, float biasf,
     return QuantizeDev(__fadd_rn(__fmul_rn(static_cast<float>(acc), mult), biasf), rq);
 }
 
-// Per-channel constants, four rows of `stride` floats, built on the host (conv.hip, FinishTable):
+// Per-channel constants, four rows of `stride` floats, built on the host (bracket.h):
 //   row 0 mult   s_in * s_w[c]                      row 1 biasf  float(bias[c]) * s_b[c]
 //   row 2 m, row 3 b   the fast path (below)
 // A kernel's accumulators start from the plan's `corr` array (or get it added before the requantization): the zero-point
@@ -60,7 +60,7 @@ __device__ __forceinline__ v4i Quad(const v16i& v, int q)
 //   per instruction: rint(65535 x), saturated to 0 .. 65535) leaves the code in the high byte of its 16 bits,
 //       65535 x = 256 (t + 0.5) - 0.5,
 //   so that x crosses from one high byte to the next where t is a half-integer.  The host chooses c above every rounding on both
-//   sides (the reference's four; those of m, b, the conversion, the fma and the subtraction: FinishTable has the sum), so that
+//   sides (the reference's four; those of m, b, the conversion, the fma and the subtraction: bracket.h has the sum), so that
 //       p = fma(float(acc), m, b)  and  q = p - 2c     enclose the reference's x:   q < x(t) < p.
 //   When both give the same high byte, t -- strictly between them -- rounds to that code under any tie rule, the reference's
 //   half-away-from-zero included.  Values whose two bytes differ (about two in 10^4) are recomputed with the reference's own
@@ -245,9 +245,9 @@ __device__ __forceinline__ void RequantCore(const v4i (&acc)[N], uint32_t (&out)
             const float mult = upper ? (odd ? m.w : m.z) : (odd ? m.y : m.x), biasf = upper ? (odd ? b.w : b.z) : (odd ? b.y : b.x);
             const int shift = (upper ? 16 : 0) + (odd ? 8 : 0);
             const uint32_t mask = 0xffu << shift;
-            int code;
-            if (rq.all_fast) code = SettleDev(AccValue<BITS>(sum), mult, biasf, static_cast<int>((o >> shift) & 0xffu), d & mask, rq);
-            else code = RequantExactDev(sum - base, mult, biasf, rq) + rq.pk_bias;
+            int code = SettleDev(static_cast<float>(sum - base), mult, biasf, static_cast<int>((o >> shift) & 0xffu), d & mask, rq);
+            // bytes 128 and 127: a channel without a fast path (or a value between these two codes, which either way settles)
+            if (!rq.all_fast && (d & mask) == mask) code = RequantExactDev(sum - base, mult, biasf, rq) + rq.pk_bias;
             o = (o & ~mask) | (static_cast<uint32_t>(code) << shift);
             any = 0u;
 #pragma unroll

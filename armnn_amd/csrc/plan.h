@@ -44,6 +44,7 @@ struct mi355x_conv2d_s
     int pw_blocks_per_cu = 1, pw_n_cu = 256;     // weight-stationary kernel: blocks a CU holds at once, CUs of the device
     int pw_blocks_per_cu_64 = 0;                 // ... with 64-channel slabs, where the plan's own slab is 128 (0: not prepared)
     std::vector<float> chan_host;  // host copy of `chan` until it is uploaded
+    std::vector<double> chan_most; // each channel's most, until then
     long long acc_most = 0;        // no complete sum is larger than this in magnitude
     int pw_bn = 0, pw_ks = 0;      // pointwise GEMM kernel configuration (0: not applicable)
     bool bk128 = false;            // implicit GEMM walks K in 128-byte tiles

@@ -78,3 +78,40 @@ def test_sums_beyond_two_to_the_22nd(m, scale):
     fast, exact = _fast_and_exact(lambda: shim.fully_connected(xq, wq, bq, info).data)
     print(f"{m} rows, scale {scale}: {shim.last_kernel()}, {len(np.unique(exact))} codes", flush=True)
     np.testing.assert_array_equal(fast, exact)
+
+
+@pytest.mark.parametrize("layer", ["conv1x1", "conv3x3", "depthwise", "classifier", "few_rows", "stem"])
+@pytest.mark.parametrize("odd", ["no_weights", "smallest_scale", "always_least", "always_most", "wide", "no_fast_path"])
+def test_an_odd_channel_among_others(odd, layer):
+    """Channels 5 and 40 are dead, saturated, uncertain over many codes or outside the fast path; the others are as usual."""
+    n, h, ci, co, k = {"conv1x1": (2, 28, 64, 128, 1), "conv3x3": (2, 20, 64, 64, 3), "depthwise": (2, 30, 64, 64, 3),
+                       "classifier": (1, 40, 1024, 72, 1), "few_rows": (1, 1, 512, 64, 1), "stem": (1, 33, 3, 64, 3)}[layer]
+    dw = layer == "depthwise"
+    rng = np.random.default_rng(17)
+    taps = k * k * (1 if dw else ci)
+    w = np.clip(np.rint(rng.standard_normal((1, k, k, co) if dw else (co, k, k, ci)) * 30), -127, 127).astype(np.int8)
+    scales = (rng.uniform(0.002, 0.02, co) / np.sqrt(taps) * 3).astype(np.float32)
+    b = np.rint(rng.standard_normal(co) * 500).astype(np.int32)
+    for c in (5, 40):
+        if odd == "no_weights":
+            (w[..., c] if dw else w[c])[...] = 0
+            scales[c], b[c] = 1.2e-38, 2 ** 31 - 1
+        elif odd == "smallest_scale":
+            scales[c], b[c] = 1.2e-38, 3
+        elif odd == "always_least":
+            b[c] = int(-3e4 / scales[c])
+        elif odd == "always_most":
+            b[c] = int(3e4 / scales[c])
+        elif odd == "wide":                       # a bias that some sums take back
+            scales[c], b[c] = 0.4, int(-0.3 * 127 * 64 * np.sqrt(taps))
+        else:                                     # sums of more codes than the fast path allows
+            scales[c], b[c] = 3e7, 12
+    stride = 2 if layer == "stem" else 1
+    ho = -(-h // stride)
+    xq = QTensor(TensorInfo((n, h, h, ci), S8, (0.0235,), -3), rng.integers(-128, 128, (n, h, h, ci)).astype(np.int8))
+    wq = QTensor(TensorInfo(w.shape, DataType.QSymmS8, tuple(scales), 0, 3 if dw else 0), w)
+    bq = QTensor(TensorInfo((co,), DataType.Signed32, tuple(np.float32(0.0235) * scales), 0, 0), b)
+    info = TensorInfo((n, ho, ho, co), S8, (0.0235,), -20)
+    fast, exact = _fast_and_exact(lambda: shim.conv2d(xq, wq, bq, info, pad_top=k // 2, pad_left=k // 2, stride_x=stride, stride_y=stride, depthwise=dw).data)
+    print(f"{odd} {layer}: {shim.last_kernel()}, {len(np.unique(exact))} codes, of channel 5 {len(np.unique(exact[..., 5]))}", flush=True)
+    np.testing.assert_array_equal(fast, exact)
