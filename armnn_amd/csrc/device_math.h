@@ -57,7 +57,8 @@ __device__ __forceinline__ v4i Quad(const v16i& v, int q)
 // Fast path with an exact fallback.
 //   t = float(acc) * mult / s_out + biasf / s_out + offset' is the reference's value before rounding, with its roundings (offset': 128
 //   higher for signed outputs, codes as unsigned bytes).  The fast path works on a scale on which v_cvt_pknorm_u16_f32 (two values
-//   per instruction: rint(65535 x), saturated to 0 .. 65535) leaves the code in the high byte of its 16 bits,
+//   per instruction: rint(65535 x), saturated to 0 .. 65535 -- exactly, for every float: peaks.hip has the check) leaves the code in
+//   the high byte of its 16 bits,
 //       65535 x = 256 (t + 0.5) - 0.5,
 //   so that x crosses from one high byte to the next where t is a half-integer.  The host chooses c above every rounding on both
 //   sides (the reference's four; those of m, b, the conversion, the fma and the subtraction: bracket.h has the sum), so that

@@ -3,7 +3,8 @@
 //   * the same with the operands read from LDS every step (2 + 4 fragments per 8 MFMAs, as a GEMM wave tile does):
 //     the clock the device sustains with the matrix cores and LDS busy together is lower, and so is this rate;
 //   * HBM copy rate: 16-byte loads and stores over buffers far larger than the caches.
-// Measurement support for the benchmark scripts; not part of the inference ABI.
+// And one property that the requantization rests on (device_math.h): what v_cvt_pknorm_u16_f32 makes of every float.
+// Measurement support for the benchmark scripts and tests; not part of the inference ABI.
 #include <hip/hip_runtime.h>
 #include <cstdint>
 
@@ -133,6 +134,27 @@ __global__ __launch_bounds__(256) void ReadKernel(const v4i* __restrict__ src, s
     }
     for (; i < n16; i += stride) acc ^= src[i];
     if ((acc[0] ^ acc[1] ^ acc[2] ^ acc[3]) == 0x12345678) sink[0] = 1;
+}
+
+// Every float but NaN, on both sides of the conversion, against rint(65535 x) in 64 bits, saturated to 0 .. 65535.  bad[0]: how many
+// differ, bad[1]: the bits of one that does.
+__global__ __launch_bounds__(256) void PkNormKernel(unsigned int* bad)
+{
+    const uint64_t threads = static_cast<uint64_t>(gridDim.x) * 256;
+    for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x; i < (1ull << 32); i += threads)
+    {
+        const uint32_t bits = static_cast<uint32_t>(i);
+        if ((bits & 0x7fffffffu) > 0x7f800000u) continue;
+        const float x = __builtin_bit_cast(float, bits);
+        const double v = __builtin_rint(65535.0 * static_cast<double>(x));        // 16 + 24 bits: exact before rint
+        const uint32_t want = v < 0.0 ? 0u : v > 65535.0 ? 65535u : static_cast<uint32_t>(v);
+        const uint32_t got = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pknorm_u16(x, x));
+        if (got != (want | want << 16))
+        {
+            atomicAdd(&bad[0], 1u);
+            bad[1] = bits;
+        }
+    }
 }
 
 struct Events
@@ -295,6 +317,25 @@ int mi355x_peak_hbm_copy(size_t bytes, double* bytes_per_s)
     }
     (void)hipFree(src);
     (void)hipFree(dst);
+    return rc;
+}
+
+// How many floats v_cvt_pknorm_u16_f32 converts to something else than rint(65535 x) saturated to 0 .. 65535, and the bits of one of them.
+int mi355x_check_pknorm(unsigned int* wrong, unsigned int* example)
+{
+    if (!wrong || !example) return 1;
+    unsigned int* bad = nullptr;
+    unsigned int host[2] = {0u, 0u};
+    if (hipMalloc(&bad, sizeof(host)) != hipSuccess) return 2;
+    int rc = hipMemcpy(bad, host, sizeof(host), hipMemcpyHostToDevice) == hipSuccess ? 0 : 2;
+    if (rc == 0)
+    {
+        hipLaunchKernelGGL(PkNormKernel, dim3(4096), dim3(256), 0, nullptr, bad);
+        if (hipGetLastError() != hipSuccess || hipMemcpy(host, bad, sizeof(host), hipMemcpyDeviceToHost) != hipSuccess) rc = 2;
+    }
+    (void)hipFree(bad);
+    *wrong = host[0];
+    *example = host[1];
     return rc;
 }
 } // extern "C"

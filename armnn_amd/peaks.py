@@ -9,10 +9,26 @@ import os
 _LIB = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "libmi355x_peaks.so")
 
 
-def measure(copy_bytes: int = 1 << 30) -> dict:
+def _load():
     if not os.path.exists(_LIB):
         raise RuntimeError(f"{_LIB} is missing: build it with `make -C armnn_amd/csrc`")
-    lib = C.CDLL(_LIB)
+    return C.CDLL(_LIB)
+
+
+def pknorm_mismatches() -> tuple:
+    """(number, bits of one) of the floats that v_cvt_pknorm_u16_f32 converts to something else than rint(65535 x) saturated to
+    0 .. 65535: the requantization's bracket counts on there being none."""
+    lib = _load()
+    lib.mi355x_check_pknorm.argtypes = [C.POINTER(C.c_uint), C.POINTER(C.c_uint)]
+    wrong, example = C.c_uint(), C.c_uint()
+    rc = lib.mi355x_check_pknorm(C.byref(wrong), C.byref(example))
+    if rc != 0:
+        raise RuntimeError(f"mi355x_check_pknorm failed ({rc})")
+    return wrong.value, example.value
+
+
+def measure(copy_bytes: int = 1 << 30) -> dict:
+    lib = _load()
     lib.mi355x_peak_mfma_i8.argtypes = [C.c_int, C.POINTER(C.c_double)]
     lib.mi355x_peak_hbm_copy.argtypes = [C.c_size_t, C.POINTER(C.c_double)]
     lib.mi355x_peak_hbm_read.argtypes = [C.c_size_t, C.POINTER(C.c_double)]

@@ -6,7 +6,7 @@ each channel's scale and bias meet each of them."""
 import numpy as np
 import pytest
 
-from armnn_amd import shim
+from armnn_amd import peaks, shim
 from armnn_amd.tensor import DataType, QTensor, TensorInfo
 
 pytestmark = pytest.mark.gpu
@@ -34,6 +34,13 @@ def _scales(kind, channels):
     if kind == "steps_of_codes":            # a code and more per step of the sum
         return rng.uniform(0.05, 40.0, channels)
     return rng.uniform(1e-9, 1e-7, channels)    # one code for all sums
+
+
+def test_the_conversion_is_exact_for_every_float():
+    """The bracket has no term for v_cvt_pknorm_u16_f32: it has to be rint(65535 x), saturated, for all 2^32 floats but NaN."""
+    shim.Device()
+    wrong, example = peaks.pknorm_mismatches()
+    assert wrong == 0, f"{wrong} floats, {example:#010x} among them"
 
 
 @pytest.mark.parametrize("clamp", [False, True], ids=["type_range", "clamp_inside"])
