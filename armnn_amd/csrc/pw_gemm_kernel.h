@@ -285,8 +285,10 @@ __global__ __launch_bounds__(256) void PwGemmKernel(PwArgs a)
 // products and exchanges, and a layer of 64 x 10 took 5.1 us where it now takes 2.8.  For the same reason the sums are exchanged by
 // halves and requantized side by side in the lanes that end up with them (one after the other in lane 0 before: 0.8 us more at one row), and
 // the loads of up to four steps go out together (a branch on the zero point stood between them: 0.4 us).
-// Before -> here: 4096 x 4096 at one row 4.7 -> 3.4 us = 4.9 TB/s, two 6.2 -> 4.0, three 7.7 -> 5.0, four 9.1 -> 5.0; 1024 -> 1001 3.5 -> 2.6
-// and, four rows, 7.3 -> 3.0; 2048 -> 1001 3.8 -> 2.65; 4032 -> 155, four rows, 10.0 -> 3.5.
+// Before -> here, us a launch of a replayed graph, the same weights each time (an XCD's share is in its L2) and weights that come from HBM:
+// 4096 x 4096 at one row 4.6 -> 3.2 and 7.5 -> 5.6 (3.0 TB/s), two 6.0 -> 3.8 and 8.8 -> 6.1, three 7.3 -> 4.7 and 10.1 -> 6.7, four
+// 8.9 -> 4.8 and 11.5 -> 6.8; 1024 -> 1001 3.05 -> 2.1 and 4.4 -> 3.0, four rows 6.7 -> 2.8 and 7.9 -> 3.6; 4032 -> 155, four rows, 9.5 -> 3.3
+// and 10.6 -> 3.9.
 struct GemvArgs
 {
     const uint8_t* x;        // [M][K]
