@@ -254,7 +254,7 @@ __global__ __launch_bounds__(256) void BigGemmKernel(IgemmArgs a, int xcd_rows)
 
     // ---- the block's slice of the per-channel table (BN channels) goes to LDS behind
     // the stages: with one wave per SIMD nothing would hide the epilogue's table reads from global memory, one round trip
-    // per channel quad.  The rare exact path reads its two rows from global memory.
+    // per channel quad.  Values that the bracket leaves open are settled from its first two rows.
     constexpr int TAB = (ST * STAGE > BM * LDO ? ST * STAGE : BM * LDO);
     float* tab_lds = reinterpret_cast<float*>(smem + TAB);
     {

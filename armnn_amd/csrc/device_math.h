@@ -157,6 +157,9 @@ __device__ __forceinline__ float AccValue(int acc)
 //   fl(f / s_out) > h for negative h exactly if f / s_out > h + d; rounding half away from zero asks for the first where h is
 //   positive, for the second where it is negative.  f - h s_out has few bits and is exact in the fma, d s_out is a shift: the
 //   division's result is known without the division.
+//   Against the division in its place, MobileNetV1 at one image 35.4 against 35.8 us, at 64 155.5 against 156.3, at 256 544 against 542; the 3x3
+//   layer 64 x 56 x 56 x 64 14.1 against 13.9.  (A bracket whose width bounds the constants' roundings instead of taking them as
+//   they are, 35.7, 156.8, 547 and 14.2.)
 __device__ __forceinline__ int SettleDev(float sum, float mult, float biasf, int k, uint32_t open, const Requant& rq)
 {
     const float f = __fadd_rn(__fmul_rn(sum, mult), biasf);

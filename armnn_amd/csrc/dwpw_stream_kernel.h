@@ -60,7 +60,7 @@ struct DwPwStreamArgs
 };
 
 // S: depthwise stride; C: channels between the layers; NO: output channels; TH x TW: output pixels per item; NWAVES: 4 or
-// 8 waves per block (8 where the weights and the halo leave room for one block per CU only)
+// 8 waves per block (8 for 256 output channels: two to each 64 of them)
 template <int S, int C, int NO, int TH, int TW, int NWAVES = 4>
 struct DwPwStreamGeom
 {
@@ -70,7 +70,7 @@ struct DwPwStreamGeom
     static constexpr int NW = NWAVES, NT = 64 * NW;
     static constexpr int NCG = C / 16;
     static constexpr int P = TH * TW;                     // pixels per item
-    static_assert(P % 64 == 0, "whole 32-pixel MFMA tiles, two per wave at least");
+    static_assert(P % 64 == 0, "groups of 16 pixels, shared evenly by four waves");
     static constexpr int NPG = P / 16;
     static constexpr int CGW = NCG > NW ? NCG / NW : 1;  // channel groups per wave
     static constexpr int WPC = NCG < NW ? NW / NCG : 1;  // waves sharing a channel group (they split the pixel groups)
@@ -82,7 +82,7 @@ struct DwPwStreamGeom
     static constexpr int ROWP_RAW = HC * PITCH;
     static constexpr int ROWP = (TW == 8 && S == 1) ? ((ROWP_RAW + 127) / 256 * 256 + 128) : ROWP_RAW;
     static constexpr int HALO = HR * ROWP;                // the halo buffer
-    static constexpr int KP = C + 16;                     // bytes per panel row and per weight row in LDS
+    static constexpr int KP = C + 16;                     // bytes per panel row
     static constexpr int PANEL = P * KP;
     static constexpr int TAB = 2 * NO * 4 + 2 * C * 4;    // mult and biasf of both layers
     static constexpr int WN = NO / 64, WM = NW / WN;      // waves side by side over channels and pixels
