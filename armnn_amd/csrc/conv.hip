@@ -12,6 +12,7 @@
 #include "stem_rgb_kernel.h"
 #include "pool_softmax_items.h"
 #include "igemm_ksplit_kernel.h"
+#include "igemm_tile.h"
 #include "pw_gemm_kernel.h"
 #include "igemm.h"
 #include "igemm_lds_kernel.h"
@@ -629,6 +630,7 @@ int LaunchIgemmLdsT(const mi355x_conv2d_s* p, uint32_t batch, const void* x, voi
     bool unit_fast = false;
     if (const int rc = FillIgemmLdsArgs(p, BM, BN, batch, x, y, &a, &unit_fast)) return rc;
     const ConvGeom& g = p->geom;
+    if (a.tiles_n * BN > p->Co_pad) return SetError(MI355X_ERR_UNSUPPORTED, "implicit GEMM: %d padded channels are not whole %d-wide tiles", p->Co_pad, BN);
     if (t_pending_add && (g.Co & 15) == 0)
     {
         a.res = t_pending_add->other;
@@ -1098,14 +1100,8 @@ int RunPlan(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, hi
         // in flight to hide global-load latency, so problems that would yield few large tiles take 64x64 tiles
         // (4x the blocks, 8 waves/SIMD).
         const long long M = static_cast<long long>(batch) * g.Ho * g.Wo;
-        const long long big = ((M + 127) / 128) * ((g.Co + 127) / 128);
-        // tile: 64x64 while the 128-wide tiling would leave CUs idle; k-tile: 128 bytes whenever K was padded to it
-        const bool bk128 = p->bk128;
-        // 256x256 tiles (16 waves) halve the operand traffic per output once they alone fill three quarters of the CUs
-        const long long huge = ((M + 255) / 256) * ((g.Co + 255) / 256);
-        const int tile = p->tile_override ? p->tile_override
-                       : gemm_instead ? 96
-                       : big < 400 ? 64 : (huge >= 192 && g.Co >= 256) ? 512 : 128;
+        const bool bk128 = p->bk128;                  // k-tile: 128 bytes whenever K was padded to it
+        const int tile = IgemmTile(p->tile_override, gemm_instead, M, g.Co, p->Co_pad);
         // channel counts that are multiples of 128: k-tiles go from global memory straight into LDS
         const int lds_stages = p->opt_igemm_lds;
         if (lds_stages != 0 && ((bk128 && (g.Ci % 128) == 0) || (p->k_tail && p->tile_override == 0)))
