@@ -1558,7 +1558,7 @@ int LaunchPwPoolT(const mi355x_conv2d_s* pw, const mi355x_pool2d_desc* pool, uin
     a.pool_is_max = pool->pool_type == 0;
     a.y = static_cast<uint8_t*>(y);
     constexpr int smem = PwDwStageBytes<MF, kPwDwStages>() + kPwDwTab, NW = PwDwWavesFor(MF);
-    static_assert(MF * 32 * kPwDwPitch <= smem, "the intermediate tile reuses the GEMM's stages");
+    static_assert(MF * 32 * kPwDwPitch <= smem - kPwDwTab, "the intermediate tile reuses the GEMM's stages and leaves the table behind them");
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&PwDwKernel<MF, kPwDwStages, 1, NW, true>),
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, smem);
     MI355X_HIP(attr);
