@@ -1,7 +1,7 @@
 """Three-channel stems at stride 2 through AUTO against the plain kernel, bit for bit.
 
 Sizes are where the kernel's twelve-byte loads and its tiles can go wrong: images whose first and last pixels end the tensor, fewer pixels
-than a load or a tile, every width modulo 4, filters narrower and wider than their operand rows allow, output channels around 32 and
+than a load or a tile, tiles of 8 and of 16 rows, every width modulo 4, filters narrower and wider than their operand rows allow, output channels around 32 and
 64, two halves of the weights."""
 import numpy as np
 import pytest
@@ -27,8 +27,10 @@ STEMS = [
     ("7x7_valid_60", dict(n=1, h=9, w=35, co=60, kh=7, kw=7, padding="valid"), True),
     ("7x8", dict(n=1, h=17, w=33, co=64, kh=7, kw=8), True),
     ("7x5_wide_padding", dict(n=2, h=8, w=5, co=48, kh=7, kw=5, padding=(6, 5, 4, 4)), True),
-    ("7x7_tiles_of_16_rows", dict(n=20, h=130, w=200, co=64, kh=7, kw=7), True),
-    ("3x3_tiles_of_16_rows", dict(n=24, h=130, w=260, co=32, kh=3, kw=3), True),
+    ("7x7_tiles_of_16_rows", dict(n=40, h=130, w=200, co=64, kh=7, kw=7), True),     # (768 tiles of 16 rows or more; the last has one)
+    ("7x7_tiles_of_16_rows_32", dict(n=40, h=130, w=200, co=32, kh=7, kw=7), True),
+    ("3x3_tiles_of_16_rows", dict(n=32, h=130, w=260, co=32, kh=3, kw=3), True),
+    ("3x3_tiles_of_16_rows_64", dict(n=32, h=130, w=260, co=64, kh=3, kw=3), True),
 ]
 
 
@@ -45,4 +47,8 @@ def test_rgb_stems(name, kw, taken, weights, in_u8):
     kernel = shim.last_kernel()
     print(f"{name}: {kernel}", flush=True)
     assert kernel.startswith("StemRgbKernel") == (taken and (weights == "per_axis" or kw["kh"] == 3))
+    if kernel.startswith("StemRgbKernel"):
+        halves = weights == "two_halves"                  # always in tiles of 16 rows
+        rows = 16 if halves or "16_rows" in name else 8
+        assert kernel == f"StemRgbKernel<{kw['kh']}, {1 if kw['co'] <= 32 else 2}, {rows}, {'true' if halves else 'false'}>"
     np.testing.assert_array_equal(got.data, shim.conv2d(c.x, c.w, c.b, c.out_info, algo=shim.ALGO_DIRECT, **kwargs).data)
