@@ -249,7 +249,9 @@ __device__ __forceinline__ void RequantCore(const v4i (&acc)[N], uint32_t (&out)
             const float mult = upper ? (odd ? m.w : m.z) : (odd ? m.y : m.x), biasf = upper ? (odd ? b.w : b.z) : (odd ? b.y : b.x);
             const int shift = (upper ? 16 : 0) + (odd ? 8 : 0);
             const uint32_t mask = 0xffu << shift;
-            int code = SettleDev(static_cast<float>(sum - base), mult, biasf, static_cast<int>((o >> shift) & 0xffu), d & mask, rq);
+            // (AccValue, and not the conversion of sum - base, 0.8 us of 120 in FullyConnected 8192 x 4096 x 4096: beyond 2^22, where the bits are
+            // not the sum, a value is open only if its channel's slope is so small that neither moves its bias)
+            int code = SettleDev(AccValue<BITS>(sum), mult, biasf, static_cast<int>((o >> shift) & 0xffu), d & mask, rq);
             // bytes 128 and 127: a channel without a fast path (or a value between these two codes, which either way settles)
             if (!rq.all_fast && (d & mask) == mask) code = RequantExactDev(sum - base, mult, biasf, rq) + rq.pk_bias;
             o = (o & ~mask) | (static_cast<uint32_t>(code) << shift);

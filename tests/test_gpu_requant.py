@@ -87,6 +87,26 @@ def test_sums_beyond_two_to_the_22nd(m, scale):
     np.testing.assert_array_equal(fast, exact)
 
 
+@pytest.mark.parametrize("m", [1, 40, 300])
+def test_sums_beyond_two_to_the_22nd_of_channels_with_the_smallest_scale(m):
+    """Such a channel's values are its bias, here a half-integer number of codes, so that all of them are settled one by one, from
+    accumulators whose bits are not the sum.  The other channels are saturated beyond 2^22."""
+    k, o = 4096, 128
+    rng = np.random.default_rng(m)
+    x = np.clip(rng.integers(-128, 128, (m, k)) + np.linspace(-255, 255, m)[:, None], -128, 127).astype(np.int8)
+    w = np.clip(rng.integers(-127, 128, (o, k)) + np.linspace(-254, 254, o)[:, None], -127, 127).astype(np.int8)
+    scales = np.full(o, 3e-3, np.float32)
+    scales[::2] = np.float32(1.2e-38)
+    b = rng.integers(-260, 260, o).astype(np.int32) * 2 + 1
+    xq = QTensor(TensorInfo((m, k), S8, (1.0,), -3), x)
+    wq = QTensor(TensorInfo((o, k), DataType.QSymmS8, tuple(scales), 0, 0), w)
+    bq = QTensor(TensorInfo((o,), DataType.Signed32, (0.5,) * o, 0, 0), b)
+    info = TensorInfo((m, o), S8, (1.0,), 5)
+    fast, exact = _fast_and_exact(lambda: shim.fully_connected(xq, wq, bq, info).data)
+    print(f"{m} rows: {shim.last_kernel()}, {len(np.unique(exact))} codes", flush=True)
+    np.testing.assert_array_equal(fast, exact)
+
+
 @pytest.mark.parametrize("layer", ["conv1x1", "conv3x3", "depthwise", "classifier", "few_rows", "stem"])
 @pytest.mark.parametrize("odd", ["no_weights", "smallest_scale", "always_least", "always_most", "wide", "no_fast_path"])
 def test_an_odd_channel_among_others(odd, layer):
