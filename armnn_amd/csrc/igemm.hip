@@ -131,8 +131,11 @@ int mi355x::LaunchSmallConv(const mi355x_conv2d_s* p, uint32_t batch, const void
         a.wo_magic = static_cast<uint32_t>(0x100000000ull / a.Wo + (0x100000000ull % a.Wo != 0));
         a.ho_magic = static_cast<uint32_t>(0x100000000ull / a.Ho + (0x100000000ull % a.Ho != 0));
     }
-    NoteKernel("SmallConvKernel<%s, %s>", BoolName(aw), BoolName(rg));
-    const auto kernel = aw ? (rg ? SmallConvKernel<true, true> : SmallConvKernel<true, false>) : (rg ? SmallConvKernel<false, true> : SmallConvKernel<false, false>);
+    const bool whole = !rg && a.Ci % 64 == 0;
+    NoteKernel("SmallConvKernel<%s, %s, %s>", BoolName(aw), BoolName(rg), BoolName(whole));
+    const auto kernel = rg      ? (aw ? SmallConvKernel<true, true, false> : SmallConvKernel<false, true, false>)
+                        : whole ? (aw ? SmallConvKernel<true, false, true> : SmallConvKernel<false, false, true>)
+                                : (aw ? SmallConvKernel<true, false, false> : SmallConvKernel<false, false, false>);
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, stream, a);
     MI355X_HIP(hipGetLastError());
     return 0;

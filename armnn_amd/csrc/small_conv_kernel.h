@@ -12,9 +12,13 @@
 // CU's address unit, which takes an instruction's cache lines one after the other, is busy for 4.3 k.  Hence v_mfma_i32_16x16x64_i8,
 // whose activation operand is 16 pixels x 64 contiguous bytes (32x32x32: 32 pixels x 32), and weights stored in operand order
 // (PackFragKernel), so that a wave's weight load is one run of 1 KB instead of 32 rows.
-// The other part of a launch is instructions that are fetched to be executed once or twice: with the pixels' divisions as multiplications
-// by reciprocals, each wave's start in K from the host and no loop in the walk over taps of 64 bytes and more, 3 x 3 layers take 0.25 us
-// less (28 x 28 x 128 4.83 -> 4.55, 14 x 14 x 256 5.82 -> 5.53, 7 x 7 x 512 7.70 -> 7.48, 56 x 56 x 64 3.93 -> 3.70), ResNet-50 116.2 -> 115.7.
+// The other part of a launch is instructions that are fetched to be executed once or twice: pixels are decoded with reciprocals and a
+// wave's start in K comes from the host.  With the divisions -> here, us: launched one by one 28 x 28 x 128 4.78 -> 4.53, 14 x 14 x 256 5.78
+// -> 5.50, 7 x 7 x 512 7.70 -> 7.48, 56 x 56 x 64 3.87 -> 3.68; from a graph of 120, three sets of tensors in turn, 4.21 -> 4.18, 5.25 -> 5.19, 7.18 ->
+// 7.20, 3.33 -> 3.29, FullyConnected of 64 rows 4096 -> 4096 9.20 -> 8.80.  From such a graph layers whose channels are no multiple of 64, with
+// the divisions -> walking taps by selects -> here: 3 x 3 over 14 x 14 x 144, two images 3.80 -> 3.90 -> 3.71, 5 x 5 to 128 channels at stride 2
+// over 16 x 16, four images, from 272 7.83 -> 8.28 -> 7.46, from 496 15.7 -> 16.3 -> 15.2; no multiple of 16, 3 x 3 over 14 x 14 x 72 3.50 -> 3.62 ->
+// 3.40, 12 x 12 x 300 5.78 -> 6.14 -> 5.69.
 // Launches back to back, against the larger tiles (one image unless said): 3 x 3 over 28 x 28 x 128 7.2 -> 4.5 us, 14 x 14 x 256 9.1 ->
 // 5.5, 7 x 7 x 512 13.3 -> 7.4, 56 x 56 x 64 5.9 -> 3.7, 28 x 28 x 96 7.2 -> 3.8; 1 x 1 over 14 x 14 x 1024 -> 256 5.7 -> 4.0, 28 x 28 x
 // 128 -> 256 5.6 -> 3.1; FullyConnected 4096 -> 4096 of 64 rows 12.9 -> 9.6.  An empty kernel takes 2.75 us in such a row.
@@ -58,10 +62,11 @@ static __global__ __launch_bounds__(256) void PackFragKernel(const int8_t* __res
 }
 
 // a.w in PackFragKernel's order.  AW: the weights have a zero point (row sums beside the products); RG: Ci is no multiple of
-// 16; both as in IgemmKernel.  a.tiles_n = ceil(Co / 32), a.tiles_m = ceil(M / 32); one tile per block.
-template <bool AW, bool RG>
+// 16; both as in IgemmKernel.  WHOLE: Ci is a multiple of 64, a filter tap whole k-steps.  a.tiles_n = ceil(Co / 32), a.tiles_m = ceil(M / 32); one tile per block.
+template <bool AW, bool RG, bool WHOLE>
 __global__ __launch_bounds__(256) void SmallConvKernel(IgemmArgs a)
 {
+    static_assert(!(RG && WHOLE), "channels that are no multiple of 16 make no whole k-steps");
     constexpr int NW = 4;                                // (8 and 16 waves were slower: more instructions for the same lines)
     __shared__ __attribute__((aligned(16))) v4i part[NW][4][64];
     __shared__ int rowpart[NW][2][64];
@@ -100,15 +105,33 @@ __global__ __launch_bounds__(256) void SmallConvKernel(IgemmArgs a)
     const int tap_bytes = RG ? a.Ck : a.Ci;
     const int steps = (a.Kh * a.Kw * tap_bytes + 63) >> 6;
     const int uw = __builtin_amdgcn_readfirstlane(wave);
-    const int s0 = a.wave_k[uw].step, s1 = a.wave_k[uw + 1].step;
+    const int s0 = RG ? steps * uw / NW : a.wave_k[uw].step, s1 = RG ? steps * (uw + 1) / NW : a.wave_k[uw + 1].step;
     const int8_t* wp = a.w + static_cast<long long>(2 * tn) * steps * 1024 + lane * 16;
     const long long w_next = static_cast<long long>(steps) * 1024;       // the tile's second group of 16 channels
-    // the lane's chunk: filter tap and channel, advanced by 64 bytes per step
-    int ci = a.wave_k[uw].ci + g * 16, ky = a.wave_k[uw].ky, kx = a.wave_k[uw].kx;
-    // 64 bytes on: past the tap's end at most once where a tap has 64 bytes (uniform; a loop here is branches for every step)
+    // the lane's chunk: filter tap and channel, advanced by 64 bytes per step.  Where the wave starts comes from the host, 0.05 to 0.1 us less
+    // than dividing for it -- but 0.02 to 0.2 more in most of the RG layers, whose lanes then have to walk to their own start
+    int ci, ky, kx;
+    if constexpr (RG)
+    {
+        ci = s0 * 64 + g * 16;
+        const int tap = ci / tap_bytes;
+        ci -= tap * tap_bytes;
+        ky = tap / a.Kw;
+        kx = tap - ky * a.Kw;
+    }
+    else
+    {
+        ci = a.wave_k[uw].ci + g * 16;
+        ky = a.wave_k[uw].ky;
+        kx = a.wave_k[uw].kx;
+    }
+    // WHOLE walks by selects.  (`wide` always holds there: a branch between the steps, without which the compiler mixes their loads and a
+    // launch takes 2 % longer.)  By itself such a launch would be faster with the loop, 3 x 3 over 14 x 14 x 256 5.07 against 5.20 us, but not beside
+    // others: ResNet-50, 192 x 192, two images, three networks in turn, 118.9 with selects, 119.7 with the loop.  In the other layers the
+    // selects, which need a tap's offset anew for every step, cost up to a tenth (below).
     const bool wide = tap_bytes >= 64;
     auto wrap = [&] {
-        if (wide)
+        if (WHOLE && wide)
         {
             const bool over = ci >= tap_bytes;
             ci -= over ? tap_bytes : 0;
@@ -124,13 +147,16 @@ __global__ __launch_bounds__(256) void SmallConvKernel(IgemmArgs a)
             if (++kx == a.Kw) { kx = 0; ++ky; }
         }
     };
-    wrap();
-    // what this wave will requantize with (wave 2 c + p finishes channel group c of pixel group p), requested ahead of the operands
+    if constexpr (!RG) wrap();
+    // what this wave will requantize with (wave 2 c + p finishes channel group c of pixel group p), requested ahead of the operands (RG: rows 0
+    // and 1 of the table when a value asks for them, 0.02 to 0.1 us less)
     const int cg = wave >> 1, pg = wave & 1;
     const int cq = tn * 32 + cg * 16 + 4 * g;
     const v4i corr4 = *reinterpret_cast<const v4i*>(a.corr + cq);
     const Fast4 f4[1] = {LoadFast4(a.ct, cq)};
-    const float4 mult = *reinterpret_cast<const float4*>(a.ct.p + cq), biasf = *reinterpret_cast<const float4*>(a.ct.p + a.ct.stride + cq);
+    const auto exact_row = [&](int r) { return *reinterpret_cast<const float4*>(a.ct.p + r * a.ct.stride + cq); };
+    float4 mult = {}, biasf = {};
+    if constexpr (!RG) { mult = exact_row(0); biasf = exact_row(1); }
     v4i acc[2][2];                                       // [channel group][pixel group]
 #pragma unroll
     for (int c = 0; c < 2; ++c)
@@ -221,7 +247,9 @@ __global__ __launch_bounds__(256) void SmallConvKernel(IgemmArgs a)
         }
         const v4i sums[1] = {v};
         uint32_t out[1];
-        WithBits(a.rq, [&](auto bits) { RequantCore<decltype(bits)::value, 1, 1>(sums, out, f4, a.rq, [&](int, float4& m, float4& b) { m = mult; b = biasf; }); });
+        WithBits(a.rq, [&](auto bits) {
+            RequantCore<decltype(bits)::value, 1, 1>(sums, out, f4, a.rq, [&](int, float4& m, float4& b) { m = RG ? exact_row(0) : mult; b = RG ? exact_row(1) : biasf; });
+        });
         stage[pg * 16 + j][cg * 4 + g] = out[0];
     }
     __syncthreads();

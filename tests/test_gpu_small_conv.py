@@ -63,3 +63,19 @@ def test_few_rows_with_an_addition_behind(n, h, ci, co, k):
     dev.synchronize()
     assert kernel.startswith("SmallConvKernel<" if ci % 128 == 0 else "Add"), kernel
     np.testing.assert_array_equal(both.download(info.shape, numpy_dtype(S8)), want.data)
+
+
+@pytest.mark.parametrize("zw", [0, 93], ids=["symmetric", "zero_point"])
+@pytest.mark.parametrize("ci,k,walk", [(16, 5, "false, false"), (48, 3, "false, false"), (64, 3, "false, true"), (112, 5, "false, false"), (192, 3, "false, true"),
+                                       (272, 5, "false, false"), (320, 5, "false, true"), (24, 5, "true, false"), (72, 3, "true, false"), (250, 5, "true, false")])
+def test_walks_over_the_taps(ci, k, walk, zw):
+    """Taps of whole steps of 64 bytes, of other multiples of 16 and of any size, shorter and longer than a step, each wave's start inside
+    a tap or at one's end."""
+    wq = dict(w_dtype=U8, w_offset=zw, per_axis=False) if zw else {}
+    c = cases.make_conv_case("walk", 53000 + ci + zw, n=2, h=9, w=7, ci=ci, co=36, kh=k, kw=k, out_offset=-20, act=cases.RELU6, **wq)
+    kwargs = dict(activation=c.act[0], act_a=c.act[1], act_b=c.act[2], **c.params)
+    got = shim.conv2d(c.x, c.w, c.b, c.out_info, **kwargs)
+    kernel = shim.last_kernel()
+    print(ci, k, kernel, flush=True)
+    assert kernel == f"SmallConvKernel<{'true' if zw else 'false'}, {walk}>"
+    np.testing.assert_array_equal(got.data, shim.conv2d(c.x, c.w, c.b, c.out_info, algo=shim.ALGO_DIRECT, **kwargs).data)
