@@ -101,7 +101,8 @@ int  mi355x_abi_version(void);
  *   (identical bytes; lets tests compare the two).
  *   "igemm_tile" = 0 | 64 | 96 | 128 | 256 | 512: plans created while it is set run on the LDS-tiled implicit-GEMM
  *   kernel with 64x64, 128x64, 128x128, 256x128 or 256x256 tiles instead of the automatic choice (the two largest only
- *   where the direct-to-LDS kernel applies; identical bytes; tests and tuning).  Further values force the other MFMA
+ *   where the direct-to-LDS kernel applies, and 256x256 only where the output channels rounded up to 128 are a multiple of
+ *   256; identical bytes; tests and tuning).  Further values force the other MFMA
  *   kernels where their shape rules allow them: 2256 | 2128 | 1256 the large-tile GEMM at 256x256, 256x128, 128x256;
  *   2064 | 4064 64x64 tiles with K split over 2 or 4 groups of waves inside the block; 3000 | 3001 the convolution that
  *   keeps its input tile resident in on-chip memory (3001: half-height tiles).
