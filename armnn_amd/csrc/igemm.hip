@@ -131,7 +131,8 @@ int mi355x::LaunchSmallConv(const mi355x_conv2d_s* p, uint32_t batch, const void
         a.wo_magic = static_cast<uint32_t>(0x100000000ull / a.Wo + (0x100000000ull % a.Wo != 0));
         a.ho_magic = static_cast<uint32_t>(0x100000000ull / a.Ho + (0x100000000ull % a.Ho != 0));
     }
-    const bool whole = !rg && a.Ci % 64 == 0;
+    // (5 x 5 filters take the loop, from a graph 256 channels 9.45 -> 9.31 us, 512 16.6 -> 16.2; smaller ones the selects: small_conv_kernel.h)
+    const bool whole = !rg && a.Ci % 64 == 0 && a.Kh * a.Kw <= 9;
     NoteKernel("SmallConvKernel<%s, %s, %s>", BoolName(aw), BoolName(rg), BoolName(whole));
     const auto kernel = rg      ? (aw ? SmallConvKernel<true, true, false> : SmallConvKernel<false, true, false>)
                         : whole ? (aw ? SmallConvKernel<true, false, true> : SmallConvKernel<false, false, true>)

@@ -62,7 +62,7 @@ static __global__ __launch_bounds__(256) void PackFragKernel(const int8_t* __res
 }
 
 // a.w in PackFragKernel's order.  AW: the weights have a zero point (row sums beside the products); RG: Ci is no multiple of
-// 16; both as in IgemmKernel.  WHOLE: Ci is a multiple of 64, a filter tap whole k-steps.  a.tiles_n = ceil(Co / 32), a.tiles_m = ceil(M / 32); one tile per block.
+// 16; both as in IgemmKernel.  WHOLE: Ci is a multiple of 64, a filter tap whole k-steps (LaunchSmallConv has the rule).  a.tiles_n = ceil(Co / 32), a.tiles_m = ceil(M / 32); one tile per block.
 template <bool AW, bool RG, bool WHOLE>
 __global__ __launch_bounds__(256) void SmallConvKernel(IgemmArgs a)
 {
