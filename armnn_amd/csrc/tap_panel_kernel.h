@@ -126,14 +126,7 @@ __device__ __forceinline__ void TapPanelBlock(const TapPanelArgs& t)
         const int n = DivByInvariant(r, a.Ho, a.ho_magic);
         const int iy = (r - n * a.Ho) * a.stride_y - a.pad_top, ix = (m - r * a.Wo) * a.stride_x - a.pad_left;
         first[e] = (n * a.H + iy) * a.W + ix;
-        if (a.dil_x == 1 && a.dil_y == 1)
-        {
-            // columns lo .. hi - 1 of the filter, the same in rows lo .. hi - 1
-            const int xl = min(max(-ix, 0), a.Kw), xh = min(max(a.W - ix, 0), a.Kw), yl = min(max(-iy, 0), a.Kh), yh = min(max(a.H - iy, 0), a.Kh);
-            const uint32_t cols = (1u << xh) - (1u << xl);
-            const uint32_t rows = t.tap_rows & static_cast<uint32_t>((1ull << (yh * a.Kw)) - (1ull << (yl * a.Kw)));
-            taps[e] = xh > xl && yh > yl ? cols * rows : 0u;
-        }
+        if (a.dil_x == 1 && a.dil_y == 1) taps[e] = TapsInside(iy, ix, a.H, a.W, a.Kh, a.Kw, t.tap_rows);
         else
         {
             uint32_t cols = 0u;

@@ -2,6 +2,7 @@
 #pragma once
 
 #include <algorithm>
+#include <cstdint>
 
 namespace mi355x
 {
@@ -32,6 +33,17 @@ constexpr int PieceInside(int i, int lo, int hi)
 {
     const int upper = i < hi ? i : hi;
     return upper > lo ? upper : lo;
+}
+
+// Taps, bit ky Kw + kx, that lie inside an H x W image for the output whose first tap is at (iy, ix), for filters of up to 32 taps without dilation:
+// columns lo .. hi - 1 of the filter, the same in rows lo .. hi - 1.  tap_rows: bits 0, Kw, 2 Kw, ... (Kh - 1) Kw.
+constexpr uint32_t TapsInside(int iy, int ix, int H, int W, int Kh, int Kw, uint32_t tap_rows)
+{
+    const auto within = [](int v, int most) { return v < 0 ? 0 : v < most ? v : most; };
+    const int xl = within(-ix, Kw), xh = within(W - ix, Kw), yl = within(-iy, Kh), yh = within(H - iy, Kh);
+    const uint32_t cols = static_cast<uint32_t>((1ull << xh) - (1ull << xl));      // (xh is 32 in a row of 32 taps)
+    const uint32_t rows = tap_rows & static_cast<uint32_t>((1ull << (yh * Kw)) - (1ull << (yl * Kw)));
+    return xh > xl && yh > yl ? cols * rows : 0u;
 }
 
 } // namespace mi355x

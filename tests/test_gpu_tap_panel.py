@@ -72,6 +72,46 @@ def test_runs_hold_what_their_taps_read(tmp_path):
     assert r.returncode == 0, r.stdout
 
 
+# every filter of up to 32 taps, its window anywhere around images narrower and wider than it: each bit against the definition
+MASK_PROGRAM = r"""
+#include "tap_panel_run.h"
+#include <cstdio>
+int main()
+{
+    long windows = 0, bad = 0;
+    for (int Kh = 1; Kh <= 32; ++Kh)
+        for (int Kw = 1; Kh * Kw <= 32; ++Kw)
+        {
+            uint32_t tap_rows = 0;
+            for (int ky = 0; ky < Kh; ++ky) tap_rows |= 1u << (ky * Kw);
+            for (int H : {1, 2, 5, 32, 40})
+                for (int W : {1, 3, 7, 31, 32, 33, 64})
+                    for (int iy = -Kh - 1; iy <= H + 1; ++iy)
+                        for (int ix = -Kw - 1; ix <= W + 1; ++ix)
+                        {
+                            uint32_t want = 0;
+                            for (int ky = 0; ky < Kh; ++ky)
+                                for (int kx = 0; kx < Kw; ++kx)
+                                    if (iy + ky >= 0 && iy + ky < H && ix + kx >= 0 && ix + kx < W) want |= 1u << (ky * Kw + kx);
+                            bad += mi355x::TapsInside(iy, ix, H, W, Kh, Kw, tap_rows) != want;
+                            ++windows;
+                        }
+        }
+    std::printf("%ld windows, %ld wrong masks\n", windows, bad);
+    return bad != 0;
+}
+"""
+
+
+def test_masks_of_the_taps_inside_an_image(tmp_path):
+    src, exe = tmp_path / "mask.cpp", tmp_path / "mask"
+    src.write_text(MASK_PROGRAM)
+    subprocess.run(["g++", "-O2", "-std=c++17", "-fsanitize=shift", "-fno-sanitize-recover=shift", "-Wall", "-Werror",
+                    f"-I{os.path.join(ROOT, 'armnn_amd', 'csrc')}", str(src), "-o", str(exe)], check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
 LAYERS = [
     ("one_pixel_c64", dict(n=1, h=1, w=1, ci=64, co=16)),
     ("31_pixels_c80_co33", dict(n=1, h=1, w=31, ci=80, co=33)),
@@ -87,6 +127,10 @@ LAYERS = [
     ("filter_1x7_c80", dict(n=2, h=5, w=12, ci=80, co=64, kh=1, kw=7)),
     ("first_row_in_the_padding_c192", dict(n=1, h=9, w=200, ci=192, co=32, kh=1, kw=3, stride=(2, 2), padding=(1, 0, 1, 1))),
     ("first_row_in_the_padding_ragged_c200", dict(n=1, h=9, w=200, ci=200, co=17, kh=1, kw=3, stride=(2, 2), padding=(1, 0, 1, 1))),
+    ("32_taps_in_a_row_c64", dict(n=2, h=3, w=70, ci=64, co=32, kh=1, kw=32)),
+    ("32_taps_in_a_row_ragged_c72", dict(n=1, h=2, w=45, ci=72, co=17, kh=1, kw=32)),
+    ("32_taps_in_a_column_c80", dict(n=1, h=40, w=3, ci=80, co=32, kh=32, kw=1)),
+    ("filter_4x8_c64", dict(n=2, h=9, w=11, ci=64, co=48, kh=4, kw=8)),
     ("one_tap_c64", dict(n=3, h=7, w=5, ci=64, co=130, kh=1, kw=1)),
     ("one_tap_c1040", dict(n=65, h=1, w=1, ci=1040, co=33, kh=1, kw=1)),
     ("one_tap_ragged_c50", dict(n=1, h=3, w=43, ci=50, co=17, kh=1, kw=1)),
