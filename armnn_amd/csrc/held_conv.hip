@@ -41,10 +41,10 @@ template <int HS, bool BITS>
 int LaunchT(const HeldConvArgs& t, int smem, hipStream_t stream)
 {
     typedef void (*Kernel)(HeldConvArgs);
-    const Kernel kernel = HaloConvKernel<64, kWaves, HS, BITS>;
+    const Kernel kernel = HeldConvKernel<kWaves, HS, BITS>;
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kBlockLds);
     MI355X_HIP(attr);
-    NoteKernel("HaloConvKernel<64, %d, %d, %s>", kWaves, HS, BoolName(BITS));
+    NoteKernel("HeldConvKernel<%d, %d, %s>", kWaves, HS, BoolName(BITS));
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((t.blocks + 7) / 8 * 8)), dim3(Geom::NT), smem, stream, t);
     MI355X_HIP(hipGetLastError());
     return 0;

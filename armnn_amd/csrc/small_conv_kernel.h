@@ -1,5 +1,5 @@
-// Convolutions and FullyConnected layers with few output rows: a block owns 32 rows x 32 channels and its waves split K.  (Layers of many taps over
-// whole k-steps take the form with a panel, tap_panel_kernel.h.)
+// Convolutions and FullyConnected layers with few output rows: a block owns 32 rows x 32 channels and its waves split K.  (Filters of nine taps and more over many
+// whole k-steps take TapPanelKernel, tap_panel_kernel.h.)
 //
 // A layer of one or a few small images gives the 64 x 64 tiles of IgemmLdsKernel too few blocks, each of which then walks
 // its whole K one k-tile and one barrier at a time: at one image a 3 x 3 layer of ResNet-50 over 14 x 14 x 256 is 16 blocks

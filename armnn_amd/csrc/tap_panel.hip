@@ -52,11 +52,8 @@ Account TileAccount(const mi355x_conv2d_s* p, long long M, int steps)
     return {static_cast<double>(blocks / slots) * round(resident) + round((blocks % slots + 255) / 256), blocks * share / 256.0, resident == 1 && blocks > 256};
 }
 
-hipError_t LargeLds(void (*kernel)(TapPanelArgs)) { return hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes); }
-
-// `few`: the launch is of SmallConvKernel's sizes
 template <int KG, int BM, int BN, bool AW, bool RG, bool WHOLE>
-int LaunchT(const mi355x_conv2d_s* p, bool few, uint32_t batch, const void* x, void* y, const uint8_t* res, const AddFuse* add, hipStream_t stream)
+int LaunchT(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, const uint8_t* res, const AddFuse* add, hipStream_t stream)
 {
     using T = TapTile<KG, BM, BN>;
     using G = typename T::Geom;
@@ -95,56 +92,15 @@ int LaunchT(const mi355x_conv2d_s* p, bool few, uint32_t batch, const void* x, v
         const int step = steps * w / KG, tap = step * 64 / tap_bytes;
         t.wave_k[w] = {step, tap / a.Kw, tap % a.Kw, step * 64 % tap_bytes};
     }
-    typedef void (*Kernel)(TapPanelArgs);
-    const auto launch = [&](Kernel kernel) -> int {
-        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((nblocks + 7) / 8 * 8)), dim3(64 * T::WAVES), smem, stream, t);
-        MI355X_HIP(hipGetLastError());
-        return 0;
-    };
-    if constexpr (KG == 4 && BM == 32 && BN == 32 && WHOLE)
-    {
-        if (few)
-        {
-            const bool nine = g.Kh * g.Kw <= 9;
-            static const hipError_t attr9 = LargeLds(static_cast<Kernel>(SmallConvKernel<AW, false, true>)), attr = LargeLds(static_cast<Kernel>(SmallConvKernel<AW, false, false>));
-            MI355X_HIP(attr9);
-            MI355X_HIP(attr);
-            NoteKernel("SmallConvKernel<%s, false, %s>", BoolName(AW), BoolName(nine));
-            return launch(nine ? static_cast<Kernel>(SmallConvKernel<AW, false, true>) : static_cast<Kernel>(SmallConvKernel<AW, false, false>));
-        }
-    }
-    if constexpr (BM == 32)
-    {
-        const Kernel kernel = IgemmKSplitKernel<KG, BM, BN, AW, RG, WHOLE>;
-        static const hipError_t attr = LargeLds(kernel);
-        MI355X_HIP(attr);
-        NoteKernel("IgemmKSplitKernel<%d, %d, %d, %s, %s, %s>", KG, BM, BN, BoolName(AW), BoolName(RG), BoolName(WHOLE));
-        return launch(kernel);
-    }
-    else
-    {
-        if constexpr (WHOLE)
-        {
-            if (g.Ci % 128 == 0)
-            {
-                const Kernel kernel = IgemmLdsKernel<BM, BN, T::WM, T::WN, KG, AW>;
-                static const hipError_t attr = LargeLds(kernel);
-                MI355X_HIP(attr);
-                NoteKernel("IgemmLdsKernel<%d, %d, %d, %d, %d, %s>", BM, BN, T::WM, T::WN, KG, BoolName(AW));
-                return launch(kernel);
-            }
-        }
-        const Kernel kernel = IgemmKernel<BM, BN, T::WM, T::WN, KG, WHOLE, AW, RG>;
-        static const hipError_t attr = LargeLds(kernel);
-        MI355X_HIP(attr);
-        NoteKernel("IgemmKernel<%d, %d, %d, %d, %d, %s, %s, %s>", BM, BN, T::WM, T::WN, KG, BoolName(WHOLE), BoolName(AW), BoolName(RG));
-        return launch(kernel);
-    }
+    const auto kernel = TapPanelKernel<KG, BM, BN, AW, RG, WHOLE>;
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
+    MI355X_HIP(attr);
+    NoteKernel("TapPanelKernel<%d, %d, %d, %s, %s, %s>", KG, BM, BN, BoolName(AW), BoolName(RG), BoolName(WHOLE));
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((nblocks + 7) / 8 * 8)), dim3(64 * T::WAVES), smem, stream, t);
+    MI355X_HIP(hipGetLastError());
+    return 0;
 }
-} // namespace
 
-namespace
-{
 bool Unit(const ConvGeom& g)
 {
     return g.Kh == 1 && g.Kw == 1 && g.stride_x == 1 && g.stride_y == 1 && g.pad_top == 0 && g.pad_left == 0 && g.Ho == g.H && g.Wo == g.W;
@@ -217,29 +173,27 @@ int mi355x::TapPanelTile(const mi355x_conv2d_s* p, uint32_t batch)
 }
 
 template <int KG, int BM, int BN>
-static int LaunchTile(const mi355x_conv2d_s* p, bool few, uint32_t batch, const void* x, void* y, const uint8_t* res, const AddFuse* add, hipStream_t stream)
+static int LaunchTile(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, const uint8_t* res, const AddFuse* add, hipStream_t stream)
 {
     const bool aw = p->zw_neg != 0;
     if (p->ragged_ck != 0)
-        return aw ? LaunchT<KG, BM, BN, true, true, false>(p, few, batch, x, y, res, add, stream) : LaunchT<KG, BM, BN, false, true, false>(p, few, batch, x, y, res, add, stream);
+        return aw ? LaunchT<KG, BM, BN, true, true, false>(p, batch, x, y, res, add, stream) : LaunchT<KG, BM, BN, false, true, false>(p, batch, x, y, res, add, stream);
     if (p->geom.Ci % 64 != 0)
-        return aw ? LaunchT<KG, BM, BN, true, false, false>(p, few, batch, x, y, res, add, stream) : LaunchT<KG, BM, BN, false, false, false>(p, few, batch, x, y, res, add, stream);
-    return aw ? LaunchT<KG, BM, BN, true, false, true>(p, few, batch, x, y, res, add, stream) : LaunchT<KG, BM, BN, false, false, true>(p, few, batch, x, y, res, add, stream);
+        return aw ? LaunchT<KG, BM, BN, true, false, false>(p, batch, x, y, res, add, stream) : LaunchT<KG, BM, BN, false, false, false>(p, batch, x, y, res, add, stream);
+    return aw ? LaunchT<KG, BM, BN, true, false, true>(p, batch, x, y, res, add, stream) : LaunchT<KG, BM, BN, false, false, true>(p, batch, x, y, res, add, stream);
 }
 
 int mi355x::LaunchTapPanel(const mi355x_conv2d_s* p, int tile, uint32_t batch, const void* x, void* y, const uint8_t* res, const AddFuse* add, hipStream_t stream)
 {
-    const long long rows = static_cast<long long>(batch) * p->geom.Ho * p->geom.Wo;
-    const bool few = (rows + 31) / 32 * ((p->geom.Co + 31) / 32) <= kSmallConvMostTiles;
     switch (tile)
     {
-    case 0: return LaunchTile<4, 32, 32>(p, few, batch, x, y, res, add, stream);
-    case 1: return LaunchTile<4, 32, 64>(p, few, batch, x, y, res, add, stream);
-    case 2: return LaunchTile<2, 64, 64>(p, few, batch, x, y, res, add, stream);
-    case 3: return LaunchTile<2, 128, 64>(p, few, batch, x, y, res, add, stream);
-    case 4: return LaunchTile<1, 128, 64>(p, few, batch, x, y, res, add, stream);
-    case 5: return LaunchTile<1, 64, 64>(p, few, batch, x, y, res, add, stream);
-    case 6: return LaunchTile<2, 64, 128>(p, few, batch, x, y, res, add, stream);
-    default: return LaunchTile<2, 32, 64>(p, few, batch, x, y, res, add, stream);
+    case 0: return LaunchTile<4, 32, 32>(p, batch, x, y, res, add, stream);
+    case 1: return LaunchTile<4, 32, 64>(p, batch, x, y, res, add, stream);
+    case 2: return LaunchTile<2, 64, 64>(p, batch, x, y, res, add, stream);
+    case 3: return LaunchTile<2, 128, 64>(p, batch, x, y, res, add, stream);
+    case 4: return LaunchTile<1, 128, 64>(p, batch, x, y, res, add, stream);
+    case 5: return LaunchTile<1, 64, 64>(p, batch, x, y, res, add, stream);
+    case 6: return LaunchTile<2, 64, 128>(p, batch, x, y, res, add, stream);
+    default: return LaunchTile<2, 32, 64>(p, batch, x, y, res, add, stream);
     }
 }

@@ -460,40 +460,12 @@ __device__ __forceinline__ void TapPanelBlock(const TapPanelArgs& t)
     }
 }
 
-// ---- the kernels: each family's form with a panel ------------------------------------------------------------------------------------------
-// 32 pixels: K split over two or four waves
+// KG, BM, BN: one of TapTile's.
 template <int KG, int BM, int BN, bool AW, bool RG, bool WHOLE>
-__global__ __launch_bounds__((64 * TapTile<KG, BM, BN>::WAVES), (TapTile<KG, BM, BN>::WAVES_PER_SIMD)) void IgemmKSplitKernel(TapPanelArgs t)
+__global__ __launch_bounds__((64 * TapTile<KG, BM, BN>::WAVES), (TapTile<KG, BM, BN>::WAVES_PER_SIMD)) void TapPanelKernel(TapPanelArgs t)
 {
     using T = TapTile<KG, BM, BN>;
     TapPanelBlock<T::WM, T::WN, KG, T::CG, T::PG, T::RD, AW, RG, WHOLE>(t);
-}
-
-// more, over channels that are a multiple of 128
-template <int BM, int BN, int WM, int WN, int KG, bool AW>
-__global__ __launch_bounds__((64 * WM * WN * KG), (TapTile<KG, BM, BN>::WAVES_PER_SIMD)) void IgemmLdsKernel(TapPanelArgs t)
-{
-    using T = TapTile<KG, BM, BN>;
-    static_assert(WM == T::WM && WN == T::WN, "the tile's waves");
-    TapPanelBlock<WM, WN, KG, T::CG, T::PG, T::RD, AW, false, true>(t);
-}
-
-// ... and over others; UT: a multiple of 64
-template <int BM, int BN, int WM, int WN, int KG, bool UT, bool AW, bool RG>
-__global__ __launch_bounds__((64 * WM * WN * KG), (TapTile<KG, BM, BN>::WAVES_PER_SIMD)) void IgemmKernel(TapPanelArgs t)
-{
-    using T = TapTile<KG, BM, BN>;
-    static_assert(WM == T::WM && WN == T::WN, "the tile's waves");
-    TapPanelBlock<WM, WN, KG, T::CG, T::PG, T::RD, AW, RG, UT>(t);
-}
-
-// few rows, channels that are a multiple of 64; NINE: filters of up to nine taps (the form without a panel walks them in another way)
-template <bool AW, bool RG, bool NINE>
-__global__ __launch_bounds__(256, 4) void SmallConvKernel(TapPanelArgs t)
-{
-    static_assert(!RG, "whole k-steps");
-    using T = TapTile<4, 32, 32>;
-    TapPanelBlock<T::WM, T::WN, 4, T::CG, T::PG, T::RD, AW, false, true>(t);
 }
 
 } // namespace mi355x

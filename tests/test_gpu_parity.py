@@ -211,15 +211,18 @@ def test_k_split_over_wave_groups_gives_the_same_bytes():
             print(f"{c.name} tile {tile}: {got.data.size} outputs, {kernel}", flush=True)
             assert kernel.startswith("IgemmKSplitKernel<%d" % (tile // 1000)), kernel
             np.testing.assert_array_equal(got.data, want.data, err_msg=f"{c.name} tile {tile}")
-    # the automatic choice: ResNet-50's 3x3 layers of the last two stages at 16 images, FullyConnected-like 1x1 with K = 2048
-    auto = [(cases.make_conv_case("ks_auto_7x7_c512", 831, n=16, h=7, w=7, ci=512, co=512, act=cases.RELU), 4),
-            (cases.make_conv_case("ks_auto_14x14_c256", 832, n=16, h=14, w=14, ci=256, co=256, act=cases.RELU), 2),
-            (cases.make_conv_case("ks_auto_7x7_c2048_1x1", 833, n=16, h=7, w=7, ci=2048, co=512, kh=1, kw=1, act=cases.RELU), 4)]
-    for c, groups in auto:
+    # the automatic choice: 1x1 projections at stride 2 over 2048 channels; filters of several taps, and stretches of 1x1 layers at stride 1, hold their
+    # input pixels in LDS
+    auto = [(cases.make_conv_case("ks_auto_14x14_c2048_s2", 834, n=16, h=14, w=14, ci=2048, co=512, kh=1, kw=1, stride=(2, 2), act=cases.RELU), "IgemmKSplitKernel<4, 2, "),
+            (cases.make_conv_case("ks_auto_14x14_c2048_s2_32_images", 835, n=32, h=14, w=14, ci=2048, co=512, kh=1, kw=1, stride=(2, 2), act=cases.RELU), "IgemmKSplitKernel<2, "),
+            (cases.make_conv_case("ks_auto_7x7_c512", 831, n=16, h=7, w=7, ci=512, co=512, act=cases.RELU), "TapPanelKernel<4, 32, 64, "),
+            (cases.make_conv_case("ks_auto_14x14_c256", 832, n=16, h=14, w=14, ci=256, co=256, act=cases.RELU), "TapPanelKernel<2, 32, 64, "),
+            (cases.make_conv_case("ks_auto_7x7_c2048_1x1", 833, n=16, h=7, w=7, ci=2048, co=512, kh=1, kw=1, act=cases.RELU), "TapPanelKernel<4, 32, 64, ")]
+    for c, expected in auto:
         got = _gpu_conv(c, shim.ALGO_AUTO)
         kernel = shim.last_kernel()
         print(f"{c.name}: {kernel}", flush=True)
-        assert kernel.startswith("IgemmKSplitKernel<%d" % groups), kernel
+        assert kernel.startswith(expected), kernel
         np.testing.assert_array_equal(got.data, _gpu_conv(c, shim.ALGO_DIRECT).data, err_msg=c.name)
 
 
@@ -255,9 +258,11 @@ def test_resident_tile_convolution_gives_the_same_bytes():
                 assert kernel.startswith("HaloConvKernel<64, 2, 2, 2,"), kernel
             np.testing.assert_array_equal(got.data, want.data, err_msg=f"{c.name} tile {tile} {kernel}")
         print(f"{c.name}: {want.data.size} outputs, {kernel}", flush=True)
-    # 16 images of 56 x 56 make 224 blocks: the automatic choice
-    shim.conv2d(cs[0].x, cs[0].w, cs[0].b, cs[0].out_info, activation=cs[0].act[0], act_a=cs[0].act[1], act_b=cs[0].act[2], **cs[0].params)
-    assert shim.last_kernel().startswith("HaloConvKernel<"), shim.last_kernel()
+    # 16 images of 56 x 56 make 224 blocks: the automatic choice for fewer than nine taps (nine stay in the waves' registers)
+    for c, kernel in ((cases.make_conv_case("halo_c64_2x2_56", 811, n=16, h=56, w=56, ci=64, co=64, kh=2, kw=2, act=cases.RELU6), "HaloConvKernel<"), (cs[0], "HeldConvKernel<")):
+        got = _gpu_conv(c, shim.ALGO_AUTO)
+        assert shim.last_kernel().startswith(kernel), shim.last_kernel()
+        np.testing.assert_array_equal(got.data, _gpu_conv(c, shim.ALGO_DIRECT).data, err_msg=c.name)
     # a forced implicit-GEMM tile keeps the same layers on the other kernels, which must agree as well
     c = cs[0]
     shim.set_option("igemm_tile", 128)
@@ -417,14 +422,18 @@ def test_pointwise_slab_widths_give_the_same_bytes():
 
 
 def test_plans_told_that_they_share_the_device_pick_small_blocks_and_give_the_same_bytes():
-    """mi355x_conv2d_set_concurrency(plan, 2): the 3x3 convolution over 64 channels leaves the kernel that keeps its input
-    tile in LDS for the implicit GEMM with 128x64 tiles, and the 3x3 convolution over 256 channels at 14x14 leaves the
-    K split over two wave groups for plain 64x64 blocks; the four-group split of the smallest launches stays; a 1x1
+    """mi355x_conv2d_set_concurrency(plan, 2): the 2x2 convolution over 64 channels leaves the kernel that keeps its input
+    tile in LDS for the implicit GEMM with 128x64 tiles, the 3x3 one the kernel with its weights in registers for one with a run of pixels in LDS; the
+    3x3 convolution over 256 channels at 14x14 takes a larger tile of that kernel, the one over 512 at 7x7 the same; a strided 1x1 convolution over 2048
+    channels leaves the K split over two wave groups for plain 64x64 blocks; the four-group split of the smallest launches stays; a 1x1
     convolution over 128 channels takes 64-channel weight slabs instead of 128-channel ones (over 64 channels it has them
     anyway).  Same bytes as alone, and as the direct kernel."""
-    picks = [(cases.make_conv_case("shared_3x3_c64_56", 841, n=16, h=56, w=56, ci=64, co=64, act=cases.RELU), "HaloConvKernel<64", "IgemmKernel<128, 64"),
-             (cases.make_conv_case("shared_3x3_c256_14", 842, n=16, h=14, w=14, ci=256, co=256, act=cases.RELU), "IgemmKSplitKernel<2", "IgemmLdsKernel<64, 64"),
-             (cases.make_conv_case("shared_3x3_c512_7", 843, n=16, h=7, w=7, ci=512, co=512, act=cases.RELU), "IgemmKSplitKernel<4", "IgemmKSplitKernel<4"),
+    picks = [(cases.make_conv_case("shared_2x2_c64_56", 847, n=16, h=56, w=56, ci=64, co=64, kh=2, kw=2, act=cases.RELU), "HaloConvKernel<64", "IgemmKernel<128, 64"),
+             (cases.make_conv_case("shared_3x3_c64_56", 841, n=16, h=56, w=56, ci=64, co=64, act=cases.RELU), "HeldConvKernel<", "TapPanelKernel<1, 128, 64"),
+             (cases.make_conv_case("shared_3x3_c256_14", 842, n=16, h=14, w=14, ci=256, co=256, act=cases.RELU), "TapPanelKernel<2, 32, 64", "TapPanelKernel<2, 64, 64"),
+             (cases.make_conv_case("shared_3x3_c512_7", 843, n=16, h=7, w=7, ci=512, co=512, act=cases.RELU), "TapPanelKernel<4, 32, 64", "TapPanelKernel<4, 32, 64"),
+             (cases.make_conv_case("shared_1x1_c2048_s2_32", 848, n=32, h=14, w=14, ci=2048, co=512, kh=1, kw=1, stride=(2, 2), act=cases.RELU), "IgemmKSplitKernel<2", "IgemmLdsKernel<64, 64"),
+             (cases.make_conv_case("shared_1x1_c2048_s2_16", 849, n=16, h=14, w=14, ci=2048, co=512, kh=1, kw=1, stride=(2, 2), act=cases.RELU), "IgemmKSplitKernel<4", "IgemmKSplitKernel<4"),
              (cases.make_conv_case("shared_1x1_k128_co512", 845, n=3, h=28, w=28, ci=128, co=512, kh=1, kw=1, act=cases.RELU), "PwGemmKernel<128, 4", "PwGemmKernel<64, 4"),
              (cases.make_conv_case("shared_1x1_k64_co256", 846, n=2, h=56, w=56, ci=64, co=256, kh=1, kw=1), "PwGemmKernel<64, 2", "PwGemmKernel<64, 2"),
              (cases.make_conv_case("shared_3x3_c64_small", 844, n=1, h=20, w=20, ci=64, co=64, act=cases.RELU6), None, None)]

@@ -40,15 +40,17 @@ def test_few_rows(port, name, kw, in_u8, zw):
     got = shim.conv2d(c.x, c.w, c.b, c.out_info, **kwargs)
     kernel = shim.last_kernel()
     print(f"{name}: {kernel}", flush=True)
-    assert kernel.startswith("SmallConvKernel<") or c.out_info.num_elements // c.out_info.shape[-1] <= 4, kernel
+    panel = "7x7_c512_3x3" == name                       # many whole k-steps: the form with a panel
+    assert kernel.startswith("TapPanelKernel<" if panel else "SmallConvKernel<") or c.out_info.num_elements // c.out_info.shape[-1] <= 4, kernel
     np.testing.assert_array_equal(got.data, shim.conv2d(c.x, c.w, c.b, c.out_info, algo=shim.ALGO_DIRECT, **kwargs).data)
     want = port.activation(port.conv2d(c.x, c.w, c.b, c.out_info, **c.params), c.out_info, *c.act)
     mx, exact = lsb_diff(got.data, want.data)
     assert mx <= 1 and exact >= 0.99, (mx, exact)
 
 
-@pytest.mark.parametrize("n,h,ci,co,k", [(1, 14, 256, 1024, 1), (1, 7, 512, 2048, 1), (1, 9, 128, 48, 3), (1, 9, 64, 48, 3)])
-def test_few_rows_with_an_addition_behind(n, h, ci, co, k):
+@pytest.mark.parametrize("n,h,ci,co,k,expected", [(1, 14, 256, 1024, 1, "SmallConvKernel<"), (1, 7, 512, 2048, 1, "SmallConvKernel<"), (1, 9, 128, 48, 2, "SmallConvKernel<"),
+                                                  (1, 9, 64, 48, 3, "Add"), (1, 9, 128, 48, 3, "TapPanelKernel<")])
+def test_few_rows_with_an_addition_behind(n, h, ci, co, k, expected):
     c = cases.make_conv_case("add", 52000 + co + k, n=n, h=h, w=h, ci=ci, co=co, kh=k, kw=k, in_scale=0.0235, out_scale=0.1, out_offset=3)
     info = TensorInfo(c.out_info.shape, S8, (0.1,), -128)
     other = QTensor(info, synth.uniform_int(52, info.shape, -128, 127, np.int64))
@@ -61,21 +63,24 @@ def test_few_rows_with_an_addition_behind(n, h, ci, co, k):
     plan.run_add(n, xd.ptr, od.ptr, info, info, both.ptr, activation=shim.ACT_RELU)
     kernel = shim.last_kernel()
     dev.synchronize()
-    assert kernel.startswith("SmallConvKernel<" if ci % 128 == 0 else "Add"), kernel
+    assert kernel.startswith(expected), kernel
     np.testing.assert_array_equal(both.download(info.shape, numpy_dtype(S8)), want.data)
 
 
 @pytest.mark.parametrize("zw", [0, 93], ids=["symmetric", "zero_point"])
-@pytest.mark.parametrize("ci,k,walk", [(16, 5, "false, false"), (48, 3, "false, false"), (64, 3, "false, true"), (112, 5, "false, false"), (192, 3, "false, true"),
-                                       (272, 5, "false, false"), (320, 5, "false, false"), (320, 1, "false, true"), (24, 5, "true, false"), (72, 3, "true, false"), (250, 5, "true, false")])
-def test_walks_over_the_taps(ci, k, walk, zw):
+@pytest.mark.parametrize("ci,k,stride,walk", [
+    (16, 5, 1, "false, false"), (48, 3, 1, "false, false"), (64, 3, 1, "false, true"), (112, 5, 1, "false, false"), (192, 3, 2, "false, true"), (272, 5, 1, "false, false"),
+    (64, 4, 1, "false, false"), (128, 5, 2, "false, false"), (320, 1, 1, "false, true"), (24, 5, 1, "true, false"), (72, 3, 1, "true, false"), (250, 5, 1, "true, false"),
+    (192, 3, 1, None), (320, 5, 1, None)])
+def test_walks_over_the_taps(ci, k, stride, walk, zw):
     """Taps of whole steps of 64 bytes, of other multiples of 16 and of any size, shorter and longer than a step, each wave's start inside
-    a tap or at one's end."""
+    a tap or at one's end.  Many whole k-steps at stride 1 take the form with a panel."""
     wq = dict(w_dtype=U8, w_offset=zw, per_axis=False) if zw else {}
-    c = cases.make_conv_case("walk", 53000 + ci + zw, n=2, h=9, w=7, ci=ci, co=36, kh=k, kw=k, out_offset=-20, act=cases.RELU6, **wq)
+    c = cases.make_conv_case("walk", 53000 + ci + zw, n=2, h=9, w=7, ci=ci, co=36, kh=k, kw=k, stride=(stride, stride), out_offset=-20, act=cases.RELU6, **wq)
     kwargs = dict(activation=c.act[0], act_a=c.act[1], act_b=c.act[2], **c.params)
     got = shim.conv2d(c.x, c.w, c.b, c.out_info, **kwargs)
     kernel = shim.last_kernel()
     print(ci, k, kernel, flush=True)
-    assert kernel == f"SmallConvKernel<{'true' if zw else 'false'}, {walk}>"
+    aw = "true" if zw else "false"
+    assert kernel == (f"SmallConvKernel<{aw}, {walk}>" if walk else f"TapPanelKernel<4, 32, 32, {aw}, false, true>")
     np.testing.assert_array_equal(got.data, shim.conv2d(c.x, c.w, c.b, c.out_info, algo=shim.ALGO_DIRECT, **kwargs).data)

@@ -156,17 +156,19 @@ def test_tiles_give_the_plain_kernels_bytes(name, kw, in_u8, zw):
         finally:
             shim.set_option("igemm_tile", 0)
         print(kernel, flush=True)
-        assert kernel.startswith(("IgemmKSplitKernel<", "IgemmLdsKernel<", "IgemmKernel<", "SmallConvKernel<")) and kernel.count(",") in (2, 5, 7), kernel
+        assert kernel.startswith("TapPanelKernel<"), kernel
         np.testing.assert_array_equal(got.data, want, err_msg=f"{tile} {kernel}")
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n,h,ci,co,k,stride,kernel", [
-    (16, 14, 256, 256, 3, 1, "IgemmKSplitKernel<2, 32, 64, false, false, true>"), (9, 28, 72, 96, 3, 1, "IgemmKSplitKernel<2, 32, 64, false, true, false>"), (16, 28, 128, 128, 3, 1, "IgemmLdsKernel<64, "),
-    (24, 33, 152, 64, 3, 1, "IgemmKernel<"), (40, 28, 64, 200, 5, 2, "IgemmKernel<"), (20, 9, 384, 48, 5, 1, "SmallConvKernel<false, false, false>"),
-    (300, 1, 1024, 1001, 1, 1, "IgemmKSplitKernel<4, 32, 64, false, false, true>"), (120, 1, 1040, 3001, 1, 1, "IgemmKSplitKernel<4, 32, 64, false, false, false>"),
-    (1, 28, 128, 512, 1, 1, "IgemmKSplitKernel<2, 32, 64, false, false, true>"), (1, 56, 96, 130, 1, 1, "IgemmKSplitKernel<2, 32, 64, false, false, false>")])
-def test_launches_that_choose_a_tile(n, h, ci, co, k, stride, kernel):
+@pytest.mark.parametrize("n,h,ci,co,k,stride,alone,shared", [
+    (16, 14, 256, 256, 3, 1, "2, 32, 64, false, false, true", "2, 64, 64, false, false, true"), (9, 28, 72, 96, 3, 1, "2, 32, 64, false, true, false", "2, 64, 64, false, true, false"),
+    (16, 28, 128, 128, 3, 1, "2, 64, 128, false, false, true", "2, 64, 64, false, false, true"), (24, 33, 152, 64, 3, 1, "2, 64, 64, false, true, false", "2, 64, 64, false, true, false"),
+    (40, 28, 64, 200, 5, 2, "2, 64, 128, false, false, true", "1, 64, 64, false, false, true"), (16, 56, 64, 64, 3, 1, None, "1, 128, 64, false, false, true"),
+    (16, 7, 512, 512, 3, 1, "4, 32, 64, false, false, true", "4, 32, 64, false, false, true"), (20, 9, 384, 48, 5, 1, "4, 32, 32, false, false, true", "4, 32, 32, false, false, true"),
+    (300, 1, 1024, 1001, 1, 1, "4, 32, 64, false, false, true", "4, 32, 64, false, false, true"), (120, 1, 1040, 3001, 1, 1, "4, 32, 64, false, false, false", "4, 32, 64, false, false, false"),
+    (1, 28, 128, 512, 1, 1, "2, 32, 64, false, false, true", "2, 32, 64, false, false, true"), (1, 56, 96, 130, 1, 1, "2, 32, 64, false, false, false", "2, 32, 64, false, false, false")])
+def test_launches_that_choose_a_tile(n, h, ci, co, k, stride, alone, shared):
     """The automatic choice, with and without launches beside it, on first use inside a captured graph as well."""
     c = cases.make_conv_case("auto", 98000 + ci, n=n, h=h, w=h, ci=ci, co=co, kh=k, kw=k, stride=(stride, stride), act=cases.RELU)
     kwargs = dict(activation=c.act[0], act_a=c.act[1], act_b=c.act[2], **c.params)
@@ -180,9 +182,9 @@ def test_launches_that_choose_a_tile(n, h, ci, co, k, stride, kernel):
         dev.graph_begin(stream)
         plan.run(n, x.ptr, y.ptr, stream)
         graph = dev.graph_end(stream)
-        if lanes == 1:
-            print(shim.last_kernel(), flush=True)
-            assert shim.last_kernel().startswith(kernel), shim.last_kernel()
+        kernel, tile = shim.last_kernel(), alone if lanes == 1 else shared
+        print(lanes, kernel, flush=True)
+        assert kernel == f"TapPanelKernel<{tile}>" if tile else not kernel.startswith("TapPanelKernel<"), kernel
         for _ in range(3):
             y.upload(blank)
             dev.graph_launch(graph, stream)
@@ -193,16 +195,18 @@ def test_launches_that_choose_a_tile(n, h, ci, co, k, stride, kernel):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n,ci", [(16, 128), (2, 128), (16, 80)])
-def test_an_addition_behind(n, ci):
-    c = cases.make_conv_case("add", 99000 + ci + n, n=n, h=14, w=14, ci=ci, co=48, in_scale=0.0235, out_scale=0.1, out_offset=3)
+@pytest.mark.parametrize("n,ci,co,kernel", [(16, 128, 48, "TapPanelKernel<"), (2, 128, 48, "TapPanelKernel<"), (40, 80, 48, "TapPanelKernel<"), (16, 128, 40, "Add")])
+def test_an_addition_behind(n, ci, co, kernel):
+    c = cases.make_conv_case("add", 99000 + ci + n, n=n, h=14, w=14, ci=ci, co=co, in_scale=0.0235, out_scale=0.1, out_offset=3)
     info = TensorInfo(c.out_info.shape, S8, (0.1,), -128)
     other = QTensor(info, synth.uniform_int(52, info.shape, -128, 127, np.int64))
     plan = shim.Conv2dPlan(c.x.info, c.w, c.b, c.out_info, **c.params)
     xd, od = shim.DeviceBuffer(c.x.data.nbytes).upload(c.x.data), shim.DeviceBuffer(other.data.nbytes).upload(other.data)
     mid, both = shim.DeviceBuffer(other.data.nbytes), shim.DeviceBuffer(other.data.nbytes)
     plan.run(n, xd.ptr, mid.ptr)
+    assert shim.last_kernel().startswith("TapPanelKernel<"), shim.last_kernel()
     want = shim.add(QTensor(c.out_info, mid.download(info.shape, numpy_dtype(S8))), other, info, activation=shim.ACT_RELU)
     plan.run_add(n, xd.ptr, od.ptr, info, info, both.ptr, activation=shim.ACT_RELU)
+    assert shim.last_kernel().startswith(kernel), shim.last_kernel()      # "Add": channels that are no whole pieces leave it a launch of its own
     shim.Device().synchronize()
     np.testing.assert_array_equal(both.download(info.shape, numpy_dtype(S8)), want.data)
