@@ -11,7 +11,7 @@ using namespace mi355x;
 
 namespace
 {
-constexpr int kWaves = 4, kSlots = 512, kFewPieces = 4, kMostPieces = 10, kBlockLds = 80 * 1024;
+constexpr int kWaves = 4, kSlots = 512, kFewPieces = 4, kMostPieces = 10, kBlockLds = 80 * 1024, kMostRunPerOutput = 4;
 using Geom = HeldConvGeom<kWaves>;
 
 TapWindow Window(const ConvGeom& g) { return {g.H, g.W, g.Ho, g.Wo, g.Kh, g.Kw, g.stride_y, g.stride_x, g.dil_y, g.dil_x}; }
@@ -72,7 +72,15 @@ bool mi355x::HeldConvPays(const mi355x_conv2d_s* p, uint32_t batch)
     // block starts.  Tiles of one pixel x 64 channels: 12.8 k 5.35 us against 5.05 and 5.19 against 4.66, 18.0 k 5.27 against 5.30, 18.8 k 5.28 against 5.80,
     // 23.1 k 5.34 against 5.39; with long runs 25.1 k 5.84 against 5.78, 40.0 k 6.57 against 6.92.
     const long long M = static_cast<long long>(batch) * g.Ho * g.Wo, tiles = M * ((g.Co + 63) / 64);
-    return tiles >= 18000 && (tiles >= 32000 || Pitch(g, M, GroupsOfBlock(p, M)) / 16 * 4 <= kFewPieces * Geom::NT);
+    if (tiles < 18000) return false;
+    const int groups = GroupsOfBlock(p, M);
+    if (tiles < 32000 && Pitch(g, M, groups) / 16 * 4 > kFewPieces * Geom::NT) return false;
+    // Wide rows, tall filters and wide dilations leave a block few outputs beside the pixels that their other taps read, and a launch rounds of blocks
+    // that each fetch both the run and the weights.  A launch of one round stays ahead (one image of 224 x 224, 5.0 pixels of a run per output, 7.3 us against 8.5, 2
+    // of 94 x 94 dilated by 2, 5.8 pixels, 6.8 against 7.5).  In several it does up to four pixels per output (3 images of 224 x 224, 3.8 pixels, 14.2 against
+    // 15.2; 3 of 240 x 240, 4.8 pixels, 17.6 against 16.9, of 256 x 256, 6.4 pixels, 22.1 against 18.7; 300 x 300, 19.8 pixels, 23.9 against 10.4).
+    const long long slots = std::max(1, kSlots / ((g.Co + 63) / 64));
+    return groups * slots >= (M + 15) / 16 || TapRun(Window(g), M, groups * 16) <= kMostRunPerOutput * 16 * groups;
 }
 
 int mi355x::LaunchHeldConv(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, hipStream_t stream)
