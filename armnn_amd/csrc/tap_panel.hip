@@ -4,6 +4,7 @@
 
 #include "common.h"
 #include "igemm.h"
+#include "igemm_tile.h"
 #include "tap_panel_kernel.h"
 #include "tap_panel_run.h"
 
@@ -24,18 +25,20 @@ int PanelPitch(const ConvGeom& g, long long M, int pixels)
 
 // What a launch on a tile takes, in clocks: from its start to its end, and of all 256 CUs together, per CU.  Negative: the tile does not fit.
 // alone_in_turns: a CU holds one block at a time and gets several.
-struct Account { double span, work; bool alone_in_turns; };
+// us: microseconds of the launch by itself.  bringing: the panel's share of its blocks' work.
+struct Account { double span, work, us, bringing; bool alone_in_turns; };
 
 // A block takes 4900 clocks of round trips and set-up, 6.6 for the pieces a lane brings to the panel, and for each k-step a wave takes 16 per matrix
 // instruction and 130 beside them; partial tiles cost 43 per four results and further wave of K.  Blocks of a CU overlap until its SIMDs are full of
 // matrix instructions, write-out (90), partial tiles and the panel.  Fitted to 60 layers of 3x3 and 5x5 taps, strides 1 and 2, 16 to 512
 // channels and over 392 tiles of 32 x 32, each on six to eight tiles: spans are 14 % off, but the tile with the least one takes 1.3 % longer than the best.
+// The microseconds are a sum of the same parts fitted to 508 layers with filters of 2 to 32 taps and dilations 1 to 6 as well: 10 % off.
 template <int KG, int BM, int BN>
 Account TileAccount(const mi355x_conv2d_s* p, long long M, int steps)
 {
     using T = TapTile<KG, BM, BN>;
     using G = typename T::Geom;
-    constexpr Account none = {-1.0, -1.0, false};
+    constexpr Account none = {-1.0, -1.0, 0.0, 0.0, false};
     const ConvGeom& g = p->geom;
     if (p->Co_pad % BN != 0) return none;
     const double panel = static_cast<double>((p->ragged_ck ? p->ragged_ck : g.Ci) / 16) * PanelPitch(g, M, BM);
@@ -49,7 +52,33 @@ Account TileAccount(const mi355x_conv2d_s* p, long long M, int steps)
     const double share = kPerSimd * (k * kMfma + 90.0 + kPartial) + bring;
     const auto round = [&](long long blocks) { return blocks == 0 ? 0.0 : std::max(block, blocks * share + 4900.0); };
     const long long blocks = (M + BM - 1) / BM * ((g.Co + BN - 1) / BN), slots = 256ll * resident;
-    return {static_cast<double>(blocks / slots) * round(resident) + round((blocks % slots + 255) / 256), blocks * share / 256.0, resident == 1 && blocks > 256};
+    const double rounds = static_cast<double>((blocks + slots - 1) / slots), per_cu = blocks / 256.0, mfma = k * T::CG * T::PG;
+    const double us = 2.53 + rounds * (1.37 + 0.0156 * mfma + 0.0518 * k + 3.02e-5 * panel / kPerSimd) + per_cu * (kPerSimd * (0.0112 * mfma + 0.13) + 4.65e-6 * panel);
+    return {static_cast<double>(blocks / slots) * round(resident) + round((blocks % slots + 255) / 256), blocks * share / 256.0, us, bring / share, resident == 1 && blocks > 256};
+}
+
+// Whether 256-row tiles of one wave per SIMD, `columns` channels wide, fill the chip (RunPlan gives them such launches).
+bool Fill256Rows(const mi355x_conv2d_s* p, long long M, int columns) { return p->Co_pad % columns == 0 && (M + 255) / 256 * (p->Co_pad / columns) >= 224; }
+
+// Microseconds that a launch of over kSmallConvMostTiles tiles takes on the kernels which walk k-tiles and read pixels per tap, wherever the taps are: a line for each
+// tile, fitted to 530 layers of 3 to 32 taps, 16 to 1024 channels and dilations 1 to 6, 10 % off.
+double TiledUs(const mi355x_conv2d_s* p, long long M)
+{
+    struct Line { int bm, bn, bk; double launch, k_tile, k_tile_of_round, round; };      // a round: 256 blocks
+    const ConvGeom& g = p->geom;
+    const int K = g.Kh * g.Kw * (p->ragged_ck ? p->ragged_ck : g.Ci);
+    const auto us = [&](const Line& l) {
+        const double rounds = static_cast<double>((M + l.bm - 1) / l.bm * ((g.Co + l.bn - 1) / l.bn)) / 256.0, k_tiles = (K + l.bk - 1) / l.bk;
+        return l.launch + k_tiles * (l.k_tile + rounds * l.k_tile_of_round) + rounds * l.round;
+    };
+    if (g.Ci % 128 == 0)
+    {
+        if (Fill256Rows(p, M, 256) || Fill256Rows(p, M, 128)) return us({256, 128, 128, 9.06, 0.0, 0.729, 12.4});
+        const bool one_round = (M + 63) / 64 * ((g.Co + 63) / 64) <= 256;                // three stages of k-tiles
+        return us({64, 64, 128, one_round ? 3.01 : 1.71, 0.29, 0.145, 1.11});
+    }
+    if (IgemmTile(0, false, M, g.Co, p->Co_pad) == 64) return us({64, 64, 64, 2.37, 0.308, 0.0647, 0.57});
+    return g.Co <= 64 ? us({128, 64, 64, 2.45, 0.23, 0.183, 0.82}) : us({128, 128, 64, 3.71, 0.09, 0.31, 1.48});
 }
 
 template <int KG, int BM, int BN, bool AW, bool RG, bool WHOLE>
@@ -145,12 +174,21 @@ int mi355x::TapPanelTile(const mi355x_conv2d_s* p, uint32_t batch)
         // us, 7 x 7 x 512 7.26 -> 5.40, 28 x 28 x 128 4.27 -> 4.03, eight images 14 x 14 x 256 7.66 -> 5.0, 5 x 5 over 9 x 9 x 384, 20 images, 12.2 -> 8.2; but 56 x
         // 56 x 64 3.37 against 3.85, and taps that are no whole k-steps 0.85 to 0.95 of the rate.  At stride 2 the panel has four times
         // the pixels: from 512 channels on (7.60 -> 7.20; 256 5.35 against 5.40, 128 4.54 against 4.80).
-        if (tiles <= kSmallConvMostTiles) return p->ragged_ck == 0 && g.Ci % 64 == 0 && steps >= (g.stride_x * g.stride_y == 1 ? 18 : 63) ? 0 : -1;
+        // It has to serve nine taps or more (2 x 2 over 24 x 24 x 448 4.58 us against 5.01, 1 x 7 over 15 x 15 x 192 4.32 against 4.57), and be short beside
+        // its outputs and k-steps: input pixels per output of up to nine (18 k-steps: 11 x 138 x 128 9.7 and 4.44 against 4.98, 36: 56 x 56 x 256 dilated by
+        // 2 8.1 and 8.06 -> 7.11, by 4 15.2 and 8.07 against 15.2), or twelve from 63 k-steps on (46 x 46 x 192 under 5 x 5 at stride 2 10.7 and 7.9 -> 7.3, 10 x 10
+        // x 320 under 32 x 1 13.8 and 9.9 against 11.4; 32 k-steps under 32 x 1 33 and 4.59 against 6.48).  Under dilated filters of more taps a lane first
+        // finds out, tap by tap, which of them are inside (36 x 36 x 64 under 1 x 32 4.33 against 5.55).
+        if (tiles <= kSmallConvMostTiles)
+        {
+            const int taps = g.Kh * g.Kw;
+            const bool pays = p->ragged_ck == 0 && g.Ci % 64 == 0 && steps >= (g.stride_x * g.stride_y == 1 ? 18 : 63) && taps >= 9 && (taps == 9 || (g.dil_x == 1 && g.dil_y == 1));
+            return pays && TapRun(Window(g), M, 32) <= 32 * (steps >= 63 ? 12 : 9) ? 0 : -1;
+        }
         // 256-row tiles of one wave per SIMD that fill the chip, where they are as wide (28 x 28 x 512, 32 images, 62.7 us here, 63.3 there, and 59
         // against 55 beside other launches) or the panel has four times the pixels, at
         // stride 2 (56 x 56 x 256 to 512 channels, 32 images, 57 us against 50, 120 x 120 x 128 to 256, eight, 17.9 against 19.2); elsewhere 80 us there are 63 here
-        const long long rows256 = (M + 255) / 256;
-        if (g.Ci % 128 == 0 && ((p->Co_pad % 256 == 0 && rows256 * (p->Co_pad / 256) >= 224) || (g.stride_x * g.stride_y > 1 && rows256 * (p->Co_pad / 128) >= 224))) return -1;
+        if (g.Ci % 128 == 0 && (Fill256Rows(p, M, 256) || (g.stride_x * g.stride_y > 1 && Fill256Rows(p, M, 128)))) return -1;
         // 64 channels at stride 1 that the kernel with weights in registers does not take (held_conv.hip): the resident-tile kernel, whose weights pass LDS, from
         // the size on where all its blocks are busy (56 x 56 to 64 channels, 32 and 64 images 9.7 and 15.4 us against 9.9 and 15.6; eight 6.0 against 5.6),
         // unless other launches share the device
@@ -169,6 +207,12 @@ int mi355x::TapPanelTile(const mi355x_conv2d_s* p, uint32_t batch)
     // Panels of a wide stride that fill a CU's LDS by themselves, one after the other: 28 x 28 x 512 at stride 2, 64 images 85 us here and 41 on 128 x
     // 128 tiles, 16 images 27.9 and 23, eight 15.4 and 17; 112 x 112 x 256 to 64 channels, eight images, 21 and 14.
     if (best >= 0 && p->tile_override == 0 && g.stride_x * g.stride_y > 1 && accounts[best].alone_in_turns) return -1;
+    // Wide rows, tall filters and wide dilations: where a good part of a block's work is to bring its run, kernels that read pixels per tap may be faster, by their
+    // account (160 x 160 x 64 under 9 x 1, two images, 8.4 us against 16.3; 148 x 148 x 64 dilated by 6 7.6 against 18.2; 224 x 224 x 256 to 64 channels 19.4 against
+    // 27.4, to 256 51 against 65; but 112 x 112 x 448 to 48 21.9 -> 12.4, 93 x 93 x 192 to 32, two images, 11.9 -> 6.9).  Of 342 layers above the small tiles
+    // 72 took over 3 % longer here than there, up to 4.3 times; with the line four do, three of them by 5 %, one by a third, and of 330 layers that it was not drawn from
+    // seven, by up to 15 %.
+    if (best >= 0 && p->tile_override == 0 && accounts[best].bringing >= 0.37 && accounts[best].us > 0.95 * TiledUs(p, M)) return -1;
     return best;
 }
 

@@ -195,6 +195,21 @@ def test_launches_that_choose_a_tile(n, h, ci, co, k, stride, alone, shared):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,h,ci,co,kh,kw,dilation,kernel", [
+    (2, 160, 64, 64, 9, 1, 1, "IgemmKernel<128, 64, "), (2, 148, 64, 32, 3, 3, 6, "IgemmKernel<64, 64, "), (1, 224, 256, 64, 3, 3, 1, "IgemmLdsKernel<64, 64, "),
+    (2, 56, 64, 64, 32, 1, 1, "SmallConvKernel<"), (2, 56, 256, 64, 3, 3, 4, "SmallConvKernel<"), (1, 24, 448, 288, 2, 2, 1, "SmallConvKernel<"),
+    (2, 93, 192, 32, 3, 3, 1, "TapPanelKernel<"), (2, 56, 256, 64, 3, 3, 2, "TapPanelKernel<")])
+def test_launches_whose_runs_are_long_for_their_outputs(n, h, ci, co, kh, kw, dilation, kernel):
+    """They leave the panel to kernels that read pixels per tap, unless those take longer all the same."""
+    c = cases.make_conv_case("long", 98500 + ci, n=n, h=h, w=h, ci=ci, co=co, kh=kh, kw=kw, dilation=(dilation, dilation), act=cases.RELU)
+    kwargs = dict(activation=c.act[0], act_a=c.act[1], act_b=c.act[2], **c.params)
+    got = shim.conv2d(c.x, c.w, c.b, c.out_info, **kwargs)
+    print(shim.last_kernel(), flush=True)
+    assert shim.last_kernel().startswith(kernel), shim.last_kernel()
+    np.testing.assert_array_equal(got.data, shim.conv2d(c.x, c.w, c.b, c.out_info, algo=shim.ALGO_DIRECT, **kwargs).data)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n,ci,co,kernel", [(16, 128, 48, "TapPanelKernel<"), (2, 128, 48, "TapPanelKernel<"), (40, 80, 48, "TapPanelKernel<"), (16, 128, 40, "Add")])
 def test_an_addition_behind(n, ci, co, kernel):
     c = cases.make_conv_case("add", 99000 + ci + n, n=n, h=14, w=14, ci=ci, co=co, in_scale=0.0235, out_scale=0.1, out_offset=3)
