@@ -11,7 +11,7 @@ using namespace mi355x;
 
 namespace
 {
-constexpr int kWaves = 4, kSlots = 512, kFewPieces = 4, kMostPieces = 10, kBlockLds = 80 * 1024, kMostRunPerOutput = 4;
+constexpr int kWaves = 4, kSlots = 512, kFewPieces = 4, kMostPieces = 10, kBlockLds = 80 * 1024;
 using Geom = HeldConvGeom<kWaves>;
 
 TapWindow Window(const ConvGeom& g) { return {g.H, g.W, g.Ho, g.Wo, g.Kh, g.Kw, g.stride_y, g.stride_x, g.dil_y, g.dil_x}; }
@@ -77,10 +77,11 @@ bool mi355x::HeldConvPays(const mi355x_conv2d_s* p, uint32_t batch)
     if (tiles < 32000 && Pitch(g, M, groups) / 16 * 4 > kFewPieces * Geom::NT) return false;
     // Wide rows, tall filters and wide dilations leave a block few outputs beside the pixels that their other taps read, and a launch rounds of blocks
     // that each fetch both the run and the weights.  A launch of one round stays ahead (one image of 224 x 224, 5.0 pixels of a run per output, 7.3 us against 8.5, 2
-    // of 94 x 94 dilated by 2, 5.8 pixels, 6.8 against 7.5).  In several it does up to four pixels per output (3 images of 224 x 224, 3.8 pixels, 14.2 against
-    // 15.2; 3 of 240 x 240, 4.8 pixels, 17.6 against 16.9, of 256 x 256, 6.4 pixels, 22.1 against 18.7; 300 x 300, 19.8 pixels, 23.9 against 10.4).
+    // of 94 x 94 dilated by 2, 5.8 pixels, 6.8 against 7.5).  In several it does up to five pixels per output (3 images of 208 x 208, 4.3 pixels, 12.5 against 16.3, of
+    // 240 x 240, 4.8 pixels, 17.4 against 18.3, of 256 x 256, 6.4 pixels, 22.1 against 18.7; 300 x 300, 19.8 pixels, 23.9 against 10.4), to over 128 channels, whose tiles
+    // of 64 each fetch the run, up to four (224 x 224 to 192 channels, 3.8 pixels, 14.4 against 14.8; to 256, 4.1 pixels, 19.7 against 15.4).
     const long long slots = std::max(1, kSlots / ((g.Co + 63) / 64));
-    return groups * slots >= (M + 15) / 16 || TapRun(Window(g), M, groups * 16) <= kMostRunPerOutput * 16 * groups;
+    return groups * slots >= (M + 15) / 16 || TapRun(Window(g), M, groups * 16) <= (g.Co <= 128 ? 5 : 4) * 16 * groups;
 }
 
 int mi355x::LaunchHeldConv(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, hipStream_t stream)

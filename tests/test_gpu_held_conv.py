@@ -44,7 +44,7 @@ def test_weights_in_registers_give_the_plain_kernels_bytes(name, kw, in_u8):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("n,h,co,taken", [(6, 56, 64, "4"), (32, 56, 64, "10"), (40, 28, 192, "4"), (3, 56, 64, None), (1, 112, 128, None), (6, 56, 65, None),
-                                             (1, 208, 64, "10"), (3, 150, 64, "10"), (3, 240, 64, None), (1, 300, 64, None)])
+                                             (1, 208, 64, "10"), (3, 150, 64, "10"), (3, 208, 64, "10"), (1, 224, 256, None), (3, 256, 64, None), (1, 300, 64, None)])
 def test_launches_that_choose_it(n, h, co, taken):
     """... but not where rows are so wide that several rounds of blocks would each fetch a long run for few outputs."""
     c = cases.make_conv_case("auto", 96100 + n, n=n, h=h, w=h, ci=64, co=co, act=cases.RELU)
