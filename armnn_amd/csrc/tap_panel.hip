@@ -162,7 +162,16 @@ int mi355x::TapPanelTile(const mi355x_conv2d_s* p, uint32_t batch)
         // 1x1 layers, two stretches between other kernels.  Over 256 tiles of 32 x 32, which SmallConvKernel runs in a second round of one per CU, 32 x 64
         // tiles of eight waves are half as many (300 rows 768 -> 1024 4.57 -> 4.21 us, 1024 -> 1024 5.54 -> 4.48, 2048 -> 1024 7.78 -> 5.69; 400 rows 2048 ->
         // 1001 8.36 -> 6.43; 512 rows 2048 -> 1024 8.36 -> 7.38, but 1024 -> 1024 5.26 against 5.40, 64 rows 2048 -> 4096, 256 tiles, 6.04 against 6.45).
-        if (steps >= 12 && tiles > 256 && tiles <= (steps >= 32 ? 512 : 448)) return 1;
+        // From 28 k-steps on that is so for all layers (of 320 drawn ones 0.66 to 1.04 of the time), and over kSmallConvMostTiles, where the other side is a larger tile
+        // (1107 rows 736 -> 384 6.13 -> 4.84).  Below, of those whose steps lie whole in the channels, if few of the 64 columns are idle (0.74 to 1.07; 2977 rows
+        // 1344 -> 96 4.96 against 5.29, 1690 rows 1088 -> 144 4.90 against 5.38); the others, whose steps find their place anew each, at few rows, whose
+        // weights outweigh them by far, from 16 k-steps or a good part of a second round on (85 rows 1488 -> 3004 0.79 of the time, 76 rows 1136 -> 3417 0.86, 157
+        // rows 912 -> 2447, 385 tiles, 0.85; but 96 rows 880 -> 2874, 270 tiles, 4.35 against 4.79, 612 rows 1232 -> 432 4.74 against 5.28).
+        if (tiles > 256 && tiles <= (steps >= 32 ? 512 : 448) && steps >= 12)
+        {
+            const bool whole = p->ragged_ck == 0 && g.Ci % 64 == 0;
+            if (steps >= 28 || tiles > kSmallConvMostTiles || (whole ? (g.Co + 63) / 64 * 20 <= 11 * columns : M <= 256 && (steps >= 16 || tiles >= 364))) return 1;
+        }
         // Layers whose weights the persistent kernel keeps in LDS: that takes a launch 5.2 us whatever its size (28 x 28 x 128 -> 512, one image
         // 5.23 -> 3.48, two 5.30 -> 3.79; 40 x 40 x 96 -> 288 5.52 -> 3.62); over 64 channels it takes 3.80 against 3.71 here, over 32 3.77 against 3.80.
         return p->pw_bn != 0 && !p->pw_forced && g.Ci > 64 && tiles > kSmallConvMostTiles && tiles <= 1024 ? 7 : -1;

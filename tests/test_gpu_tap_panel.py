@@ -167,6 +167,8 @@ def test_tiles_give_the_plain_kernels_bytes(name, kw, in_u8, zw):
     (40, 28, 64, 200, 5, 2, "2, 64, 128, false, false, true", "1, 64, 64, false, false, true"), (16, 56, 64, 64, 3, 1, None, "1, 128, 64, false, false, true"),
     (16, 7, 512, 512, 3, 1, "4, 32, 64, false, false, true", "4, 32, 64, false, false, true"), (20, 9, 384, 48, 5, 1, "4, 32, 32, false, false, true", "4, 32, 32, false, false, true"),
     (300, 1, 1024, 1001, 1, 1, "4, 32, 64, false, false, true", "4, 32, 64, false, false, true"), (120, 1, 1040, 3001, 1, 1, "4, 32, 64, false, false, false", "4, 32, 64, false, false, false"),
+    (612, 1, 1232, 432, 1, 1, None, None), (1690, 1, 1088, 144, 1, 1, None, None), (85, 1, 1488, 3004, 1, 1, "4, 32, 64, false, false, false", "4, 32, 64, false, false, false"),
+    (755, 1, 1848, 397, 1, 1, "4, 32, 64, false, true, false", "4, 32, 64, false, true, false"),
     (1, 28, 128, 512, 1, 1, "2, 32, 64, false, false, true", "2, 32, 64, false, false, true"), (1, 56, 96, 130, 1, 1, "2, 32, 64, false, false, false", "2, 32, 64, false, false, false")])
 def test_launches_that_choose_a_tile(n, h, ci, co, k, stride, alone, shared):
     """The automatic choice, with and without launches beside it, on first use inside a captured graph as well."""
