@@ -113,6 +113,10 @@ int LaunchT(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, co
     t.by_columns = static_cast<long long>(p->Co_pad) * p->K_pad > 2 * in_pixels * g.Ci && nblocks * a.tiles_m < (1ll << 32);
     t.minor = t.by_columns ? a.tiles_m : a.tiles_n;
     t.rcp_minor = reciprocal(t.minor);
+    if (g.Kh == 1) a.dil_y = 1;                          // (one row has none, whatever the descriptor says: the kernel counts its reach in taps)
+    if (g.Kw == 1) a.dil_x = 1;
+    t.rcp_dy = reciprocal(a.dil_y);
+    t.rcp_dx = reciprocal(a.dil_x);
     a.wo_magic = reciprocal(a.Wo);
     a.ho_magic = reciprocal(a.Ho);
     const int steps = (a.Kh * a.Kw * tap_bytes + 63) / 64;
@@ -186,12 +190,13 @@ int mi355x::TapPanelTile(const mi355x_conv2d_s* p, uint32_t batch)
         // It has to serve nine taps or more (2 x 2 over 24 x 24 x 448 4.58 us against 5.01, 1 x 7 over 15 x 15 x 192 4.32 against 4.57), and be short beside
         // its outputs and k-steps: input pixels per output of up to nine (18 k-steps: 11 x 138 x 128 9.7 and 4.44 against 4.98, 36: 56 x 56 x 256 dilated by
         // 2 8.1 and 8.06 -> 7.11, by 4 15.2 and 8.07 against 15.2), or twelve from 63 k-steps on (46 x 46 x 192 under 5 x 5 at stride 2 10.7 and 7.9 -> 7.3, 10 x 10
-        // x 320 under 32 x 1 13.8 and 9.9 against 11.4; 32 k-steps under 32 x 1 33 and 4.59 against 6.48).  Under dilated filters of more taps a lane first
-        // finds out, tap by tap, which of them are inside (36 x 36 x 64 under 1 x 32 4.33 against 5.55).
+        // x 320 under 32 x 1 13.8 and 9.9 against 11.4; 32 k-steps under 32 x 1 33 and 4.59 against 6.48).
+        // Dilated filters from a second round of tiles on (8 x 36 x 36 x 128 under 4 x 4 7.0 -> 5.8, 39 x 39 x 192 under 5 x 5, three images, 9.4 -> 8.2; below it 18 x 18
+        // x 64 under 5 x 5, four images, 4.20 against 4.72, 34 x 34 x 192 under 4 x 4 5.08 against 6.06).
         if (tiles <= kSmallConvMostTiles)
         {
-            const int taps = g.Kh * g.Kw;
-            const bool pays = p->ragged_ck == 0 && g.Ci % 64 == 0 && steps >= (g.stride_x * g.stride_y == 1 ? 18 : 63) && taps >= 9 && (taps == 9 || (g.dil_x == 1 && g.dil_y == 1));
+            const bool pays = p->ragged_ck == 0 && g.Ci % 64 == 0 && steps >= (g.stride_x * g.stride_y == 1 ? 18 : 63) && g.Kh * g.Kw >= 9 &&
+                              ((g.dil_x == 1 && g.dil_y == 1) || tiles > 256);
             return pays && TapRun(Window(g), M, 32) <= 32 * (steps >= 63 ? 12 : 9) ? 0 : -1;
         }
         // 256-row tiles of one wave per SIMD that fill the chip, where they are as wide (28 x 28 x 512, 32 images, 62.7 us here, 63.3 there, and 59

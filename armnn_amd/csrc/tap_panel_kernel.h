@@ -38,6 +38,7 @@ struct TapPanelArgs
     int panel_bytes;                // of all channels
     uint32_t tap_rows;              // bits 0, Kw, 2 Kw, ... (Kh - 1) Kw
     uint32_t rcp_pr, rcp_minor;     // ceil(2^32 / d) of the 16-byte pieces per pixel and of minor
+    uint32_t rcp_dy, rcp_dx;        // ... and of the dilations
     struct { int step, ky, kx, ci; } wave_k[5];     // where each share of K starts: k-step, and the filter tap and byte of it that begins there
     int minor, by_columns;          // the faster index of a tile is its row, of tiles_m, or its column, of tiles_n
 };
@@ -126,14 +127,11 @@ __device__ __forceinline__ void TapPanelBlock(const TapPanelArgs& t)
         const int n = DivByInvariant(r, a.Ho, a.ho_magic);
         const int iy = (r - n * a.Ho) * a.stride_y - a.pad_top, ix = (m - r * a.Wo) * a.stride_x - a.pad_left;
         first[e] = (n * a.H + iy) * a.W + ix;
-        if (a.dil_x == 1 && a.dil_y == 1) taps[e] = TapsInside(iy, ix, a.H, a.W, a.Kh, a.Kw, t.tap_rows);
-        else
-        {
-            uint32_t cols = 0u;
-            for (int kx = 0; kx < a.Kw; ++kx) cols |= static_cast<unsigned>(ix + kx * a.dil_x) < static_cast<unsigned>(a.W) ? 1u << kx : 0u;
-            taps[e] = 0u;
-            for (int ky = 0; ky < a.Kh; ++ky) taps[e] |= static_cast<unsigned>(iy + ky * a.dil_y) < static_cast<unsigned>(a.H) ? cols << (ky * a.Kw) : 0u;
-        }
+        const auto itself = [](int v) { return v; };
+        taps[e] = a.dil_x == 1 && a.dil_y == 1
+                      ? TapsInside(iy, ix, a.H, a.W, a.Kh, a.Kw, 1, 1, t.tap_rows, itself, itself)
+                      : TapsInside(iy, ix, a.H, a.W, a.Kh, a.Kw, a.dil_y, a.dil_x, t.tap_rows, [&](int v) { return DivByInvariant(v, a.dil_y, t.rcp_dy); },
+                                   [&](int v) { return DivByInvariant(v, a.dil_x, t.rcp_dx); });
     }
     // first taps of the block's first and last pixel
     int base, last;

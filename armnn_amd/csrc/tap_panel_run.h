@@ -35,12 +35,15 @@ constexpr int PieceInside(int i, int lo, int hi)
     return upper > lo ? upper : lo;
 }
 
-// Taps, bit ky Kw + kx, that lie inside an H x W image for the output whose first tap is at (iy, ix), for filters of up to 32 taps without dilation:
-// columns lo .. hi - 1 of the filter, the same in rows lo .. hi - 1.  tap_rows: bits 0, Kw, 2 Kw, ... (Kh - 1) Kw.
-constexpr uint32_t TapsInside(int iy, int ix, int H, int W, int Kh, int Kw, uint32_t tap_rows)
+// Taps, bit ky Kw + kx, that lie inside an H x W image for the output whose first tap is at (iy, ix), for filters of up to 32 taps, dy rows and dx columns
+// apart: columns lo .. hi - 1 of the filter, the same in rows lo .. hi - 1.  tap_rows: bits 0, Kw, 2 Kw, ... (Kh - 1) Kw.  by_dy, by_dx: an integer up to (K + 1)
+// d of the axis divided by d.
+template <class DivY, class DivX>
+constexpr uint32_t TapsInside(int iy, int ix, int H, int W, int Kh, int Kw, int dy, int dx, uint32_t tap_rows, DivY by_dy, DivX by_dx)
 {
-    const auto within = [](int v, int most) { return v < 0 ? 0 : v < most ? v : most; };
-    const int xl = within(-ix, Kw), xh = within(W - ix, Kw), yl = within(-iy, Kh), yh = within(H - iy, Kh);
+    // pixels 0 .. v of an axis, of the filter's at most, and one step of it less a pixel
+    const auto reach = [](int v, int K, int d) { return (v < 0 ? 0 : v < K * d ? v : K * d) + d - 1; };
+    const int xl = by_dx(reach(-ix, Kw, dx)), xh = by_dx(reach(W - ix, Kw, dx)), yl = by_dy(reach(-iy, Kh, dy)), yh = by_dy(reach(H - iy, Kh, dy));
     const uint32_t cols = static_cast<uint32_t>((1ull << xh) - (1ull << xl));      // (xh is 32 in a row of 32 taps)
     const uint32_t rows = tap_rows & static_cast<uint32_t>((1ull << (yh * Kw)) - (1ull << (yl * Kw)));
     return xh > xl && yh > yl ? cols * rows : 0u;

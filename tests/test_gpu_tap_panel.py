@@ -76,6 +76,18 @@ def test_runs_hold_what_their_taps_read(tmp_path):
 MASK_PROGRAM = r"""
 #include "tap_panel_run.h"
 #include <cstdio>
+#include <cstdlib>
+// the kernel's division: a multiplication by ceil(2^32 / d)
+struct Div
+{
+    int d, K;
+    int operator()(int v) const
+    {
+        if (v < 0 || v > (K + 1) * d) std::abort();
+        const uint32_t rcp = static_cast<uint32_t>((0x100000000ull + d - 1) / d);
+        return d == 1 ? v : static_cast<int>(static_cast<uint64_t>(v) * rcp >> 32);
+    }
+};
 int main()
 {
     long windows = 0, bad = 0;
@@ -84,18 +96,22 @@ int main()
         {
             uint32_t tap_rows = 0;
             for (int ky = 0; ky < Kh; ++ky) tap_rows |= 1u << (ky * Kw);
-            for (int H : {1, 2, 5, 32, 40})
+            for (int H : {1, 2, 5, 33, 40})
                 for (int W : {1, 3, 7, 31, 32, 33, 64})
-                    for (int iy = -Kh - 1; iy <= H + 1; ++iy)
-                        for (int ix = -Kw - 1; ix <= W + 1; ++ix)
-                        {
-                            uint32_t want = 0;
-                            for (int ky = 0; ky < Kh; ++ky)
-                                for (int kx = 0; kx < Kw; ++kx)
-                                    if (iy + ky >= 0 && iy + ky < H && ix + kx >= 0 && ix + kx < W) want |= 1u << (ky * Kw + kx);
-                            bad += mi355x::TapsInside(iy, ix, H, W, Kh, Kw, tap_rows) != want;
-                            ++windows;
-                        }
+                    for (int d : {1, 2, 3, 7})
+                    {
+                        const int dy = d, dx = d == 3 ? 2 : d;
+                        for (int iy = -(Kh - 1) * dy - 2; iy <= H + 1; iy += H < 33 || iy % 5 ? 1 : 2)
+                            for (int ix = -(Kw - 1) * dx - 2; ix <= W + 1; ++ix)
+                            {
+                                uint32_t want = 0;
+                                for (int ky = 0; ky < Kh; ++ky)
+                                    for (int kx = 0; kx < Kw; ++kx)
+                                        if (iy + ky * dy >= 0 && iy + ky * dy < H && ix + kx * dx >= 0 && ix + kx * dx < W) want |= 1u << (ky * Kw + kx);
+                                bad += mi355x::TapsInside(iy, ix, H, W, Kh, Kw, dy, dx, tap_rows, Div{dy, Kh}, Div{dx, Kw}) != want;
+                                ++windows;
+                            }
+                    }
         }
     std::printf("%ld windows, %ld wrong masks\n", windows, bad);
     return bad != 0;
@@ -200,6 +216,7 @@ def test_launches_that_choose_a_tile(n, h, ci, co, k, stride, alone, shared):
 @pytest.mark.parametrize("n,h,ci,co,kh,kw,dilation,kernel", [
     (2, 160, 64, 64, 9, 1, 1, "IgemmKernel<128, 64, "), (2, 148, 64, 32, 3, 3, 6, "IgemmKernel<64, 64, "), (1, 224, 256, 64, 3, 3, 1, "IgemmLdsKernel<64, 64, "),
     (2, 56, 64, 64, 32, 1, 1, "SmallConvKernel<"), (2, 56, 256, 64, 3, 3, 4, "SmallConvKernel<"), (1, 24, 448, 288, 2, 2, 1, "SmallConvKernel<"),
+    (4, 18, 64, 48, 5, 5, 3, "SmallConvKernel<"), (8, 36, 128, 16, 4, 4, 2, "TapPanelKernel<"), (5, 26, 128, 100, 4, 7, 3, "TapPanelKernel<"),
     (2, 93, 192, 32, 3, 3, 1, "TapPanelKernel<"), (2, 56, 256, 64, 3, 3, 2, "TapPanelKernel<")])
 def test_launches_whose_runs_are_long_for_their_outputs(n, h, ci, co, kh, kw, dilation, kernel):
     """They leave the panel to kernels that read pixels per tap, unless those take longer all the same."""
