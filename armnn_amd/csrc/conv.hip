@@ -982,6 +982,23 @@ int LaunchDwMfma(const mi355x_conv2d_s* p, Dw3x3Args a, hipStream_t stream)
     return 0;
 }
 
+// Groups of the kernel with weights in registers (0: not that one) and tile of the one with a panel (-1: not that one) for a launch.  Up to eight tiles are accounted
+// for, 80 to 760 ns on the host: the plan keeps the last answer, one word with what it was given for.
+struct RunChoice { int held_groups, tile; };
+
+RunChoice ChooseRun(const mi355x_conv2d_s* p, uint32_t batch)
+{
+    // bits 0 - 3: tile + 1, 4 - 14: groups, 15: there is an answer, 16 - 47: batch, 48: beside other launches
+    const uint64_t asked = 1ull << 15 | static_cast<uint64_t>(batch) << 16 | static_cast<uint64_t>(p->concurrency > 1) << 48;
+    uint64_t kept = p->run_choice.load(std::memory_order_relaxed);
+    if ((kept & ~0x7fffull) != asked)
+    {
+        kept = asked | static_cast<uint64_t>(HeldConvGroups(p, batch)) << 4 | static_cast<uint64_t>(TapPanelTile(p, batch) + 1);
+        p->run_choice.store(kept, std::memory_order_relaxed);
+    }
+    return {static_cast<int>(kept >> 4 & 0x7ff), static_cast<int>(kept & 15) - 1};
+}
+
 int RunPlan(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, hipStream_t stream)
 {
     if (!p) return SetError(MI355X_ERR_INVALID_ARGUMENT, "plan is null");
@@ -1031,18 +1048,17 @@ int RunPlan(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, hi
                 return LaunchRowPanel(p, batch, x, y, res, res ? &t_pending_add->fuse : nullptr, stream);
             }
         }
-        // Nine taps over 64 channels at many rows: weights in registers (HeldConvPays has the line)
-        if (!t_pending_add && p->opt_igemm_lds != 0 && (p->tile_override == 5009 || p->tile_override == 0) && HeldConvTakes(p, batch, y) &&
-            (p->tile_override == 5009 || HeldConvPays(p, batch)))
-            return LaunchHeldConv(p, batch, x, y, stream);
-        // A run of input pixels in LDS, weights from L2, for filters of several taps and some launches of one (TapPanelTile has the lines)
-        if (p->opt_igemm_lds != 0 && (p->tile_override == 0 || p->tile_override >= 5000))
+        // Nine taps over 64 channels at many rows: weights in registers (held_conv.hip has the lines).  A run of input pixels in LDS, weights from L2, for
+        // filters of several taps and some launches of one (TapPanelTile has the lines).
+        if (p->w_frag && p->opt_igemm_lds != 0 && (p->tile_override == 0 || p->tile_override >= 5000))
         {
-            if (const int t = TapPanelTile(p, batch); t >= 0)
+            const RunChoice c = ChooseRun(p, batch);
+            if (c.held_groups != 0 && !t_pending_add) return LaunchHeldConv(p, c.held_groups, batch, x, y, stream);
+            if (c.tile >= 0)
             {
                 const uint8_t* res = nullptr;
                 if (t_pending_add && (g.Co & 15) == 0) { res = t_pending_add->other; t_pending_add->taken = true; }
-                return LaunchTapPanel(p, t, batch, x, y, res, res ? &t_pending_add->fuse : nullptr, stream);
+                return LaunchTapPanel(p, c.tile, batch, x, y, res, res ? &t_pending_add->fuse : nullptr, stream);
             }
         }
         // Few rows: 32 x 32 tiles whose waves split K (small_conv_kernel.h), while they number at most what 14 x 14 x 256 makes at 8

@@ -6,12 +6,11 @@
 namespace mi355x
 {
 
-// Whether the kernel can run a launch of a MI355X_ALGO_MFMA plan.
-bool HeldConvTakes(const mi355x_conv2d_s* p, uint32_t batch, const void* y);
+// The groups of 16 outputs that a block of a launch of a MI355X_ALGO_MFMA plan works on (1 to 1024; tensors aligned to 16 bytes); 0 where the kernel does not
+// take the launch or another one is faster.
+int HeldConvGroups(const mi355x_conv2d_s* p, uint32_t batch);
 
-// ... and whether it is the fastest (a plan that it can run).
-bool HeldConvPays(const mi355x_conv2d_s* p, uint32_t batch);
-
-int LaunchHeldConv(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, hipStream_t stream);
+// `groups`: of HeldConvGroups.
+int LaunchHeldConv(const mi355x_conv2d_s* p, int groups, uint32_t batch, const void* x, void* y, hipStream_t stream);
 
 } // namespace mi355x

@@ -53,6 +53,8 @@ struct mi355x_conv2d_s
     bool halo_ok = false;          // shape fits the resident-tile kernel (weights without a zero point are checked at launch)
     unsigned concurrency = 1;      // launches of the plan's network that run side by side (mi355x_conv2d_set_concurrency)
     int tile_override = 0;         // 0: choose the MFMA tile per launch; 64 / 96 (= 128x64) / 128: the "igemm_tile" option at plan creation
+    // Which kernel with a run of input pixels the last launch got, if any, and the batch and lanes that it was chosen for (ChooseRun, conv.hip)
+    mutable std::atomic<uint64_t> run_choice{0};
     int opt_xcd_cols = 0;
     int opt_igemm_lds = 2, opt_dw_rows = 0, opt_dw_cb = 0, opt_dw_mfma = 1, opt_stem_dot4 = 0;     // the other process-wide options, as they stood at plan creation
                                    // (launches read the plan, never the mutable globals: plans may run on any host thread)

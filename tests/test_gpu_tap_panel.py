@@ -244,3 +244,30 @@ def test_an_addition_behind(n, ci, co, kernel):
     assert shim.last_kernel().startswith(kernel), shim.last_kernel()      # "Add": channels that are no whole pieces leave it a launch of its own
     shim.Device().synchronize()
     np.testing.assert_array_equal(both.download(info.shape, numpy_dtype(S8)), want.data)
+
+
+@pytest.mark.gpu
+def test_a_plans_choice_follows_batch_and_lanes():
+    """What a plan keeps of its last choice is for that batch and those lanes alone."""
+    c = cases.make_conv_case("kept", 99500, n=64, h=14, w=14, ci=64, co=256, act=cases.RELU)
+    kwargs = dict(activation=c.act[0], act_a=c.act[1], act_b=c.act[2], **c.params)
+    want = shim.conv2d(c.x, c.w, c.b, c.out_info, algo=shim.ALGO_DIRECT, **kwargs).data
+    x, y = shim.DeviceBuffer(c.x.data.nbytes).upload(c.x.data), shim.DeviceBuffer(want.nbytes)
+    dev = shim.Device()
+
+    def run(plan, n, lanes):
+        plan.set_concurrency(lanes)
+        y.upload(np.zeros_like(want))
+        plan.run(n, x.ptr, y.ptr)
+        kernel = shim.last_kernel()
+        dev.synchronize()
+        np.testing.assert_array_equal(y.download(want.shape, want.dtype)[:n], want[:n], err_msg=f"{n} {lanes} {kernel}")
+        return kernel
+
+    calls = [(n, lanes) for n in (64, 1, 16, 7) for lanes in (1, 2)]
+    fresh = {call: run(shim.Conv2dPlan(c.x.info, c.w, c.b, c.out_info, **kwargs), *call) for call in calls}
+    print(fresh, flush=True)
+    assert len(set(fresh.values())) >= 4 and fresh[64, 1].startswith("HeldConvKernel<") and fresh[64, 2].startswith("TapPanelKernel<")
+    plan = shim.Conv2dPlan(c.x.info, c.w, c.b, c.out_info, **kwargs)
+    for call in calls + calls[::-1] + calls[::3] + calls[:1] * 2:
+        assert run(plan, *call) == fresh[call], call
