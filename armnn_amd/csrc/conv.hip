@@ -313,8 +313,12 @@ int BuildPlan(const mi355x_conv2d_desc& d, const void* weights_host, const mi355
         else
             snprintf(buf, sizeof(buf), "igemm_mfma_i8_32x32x32 tiles 128x128|128x64|64x64 x%d K=%d", p->bk128 ? 128 : 64, p->K);
         p->info = buf;
+        // (what a launch gets depends on its size: RunPlan; callers keep 127 characters)
+        const bool runs = p->w_frag && Kh * Kw > 1 && p->opt_igemm_lds != 0 && TapPanelTakes(p);
         if (p->zw_neg != 0) p->info += ", weight zero point by row sums";
-        else if (p->halo_ok) p->info += "; launches of 192 or more row tiles: input tile resident in LDS for all taps";
+        else if (HeldConvTakes(p) && runs) p->info += "; weights in registers or input pixels in LDS where faster";
+        else if (runs) p->info += "; input pixels in LDS for all taps where faster";
+        else if (p->halo_ok && p->opt_igemm_lds != 0) p->info += "; from 192 row tiles on input tile in LDS for all taps";
     }
     else if (algo == MI355X_ALGO_DEPTHWISE && dw3_ok)
     {
@@ -1062,11 +1066,12 @@ int RunPlan(const mi355x_conv2d_s* p, uint32_t batch, const void* x, void* y, hi
             }
         }
         // Few rows: 32 x 32 tiles whose waves split K (small_conv_kernel.h), while they number at most what 14 x 14 x 256 makes at 8
-        // images.  Tiles run in rounds of one per CU, and a round takes its time whole: 14 x 14 x 256, 3 x 3, 248 tiles 6.1 us, 344 to
-        // 496 8.5 to 8.8, 592 11.1, where the larger tiles take 9.0 to 9.3 for all of them.  So the line belongs between one round and
+        // images.  Tiles run in rounds of one per CU (1x1 over 848 to 912 channels, 256 rows at most: 257 to 270 tiles 4.3 to 4.4 us, 320 4.8 to 5.1, 385 5.5 to 5.8, where
+        // the larger tiles take 5.9 to 6.7 from 396 to 440).  So the line belongs between one round and
         // two, and inside the second it decides little: there the small tiles take 0.94 to 0.97 of the others' time over 512 and
         // 1024 channels, 0.6 over 72, 96 and 128, and 0.98 to 1.06 in 1x1 layers of 2048 to 4096.  Where the layer has a weight slab (at
-        // most 128 input channels, 1x1) from 128 tiles on: 128 -> 256 at 28 x 28, 200 tiles, 5.6 -> 3.1 us.
+        // most 128 input channels, 1x1) from 128 tiles on: 128 -> 256 at 28 x 28, 200 tiles, 5.6 -> 3.1 us.  Filters of nine taps and more over many whole k-steps
+        // have left for the kernel above.
         const long long small_tiles = (rows + 31) / 32 * ((g.Co + 31) / 32);
         if (p->w_frag && p->tile_override == 0 && small_tiles <= kSmallConvMostTiles && (!p->pw_bn || small_tiles >= kSmallConvLeastSlabTiles))
         {

@@ -6,6 +6,9 @@
 namespace mi355x
 {
 
+// Whether the kernel can run launches of a MI355X_ALGO_MFMA plan with w_frag.
+bool HeldConvTakes(const mi355x_conv2d_s* p);
+
 // The groups of 16 outputs that a block of a launch of a MI355X_ALGO_MFMA plan works on (1 to 1024; tensors aligned to 16 bytes); 0 where the kernel does not
 // take the launch or another one is faster.
 int HeldConvGroups(const mi355x_conv2d_s* p, uint32_t batch);

@@ -43,8 +43,7 @@ bool Takes(const mi355x_conv2d_s* p, uint32_t batch)
     const ConvGeom& g = p->geom;
     const long long M = static_cast<long long>(batch) * g.Ho * g.Wo, in_pixels = static_cast<long long>(batch) * g.H * g.W;
     // (pixels are decoded with reciprocals, and a pixel's number in a run stands above its taps' bits)
-    return p->w_frag && g.Ci == 64 && g.Kh * g.Kw == kHeldTaps && (g.Co & 15) == 0 && p->zw_neg == 0 && TapsInOrder(Window(g)) &&
-           M <= (1ll << 27) && in_pixels <= (1ll << 27) && M * std::max(g.Wo, g.Ho) < (1ll << 32) &&
+    return p->w_frag && HeldConvTakes(p) && M <= (1ll << 27) && in_pixels <= (1ll << 27) && M * std::max(g.Wo, g.Ho) < (1ll << 32) &&
            (M + 15) / 16 * ((g.Co + 63) / 64) * ((g.Co + 63) / 64) < (1ll << 31) && Fits(g, M, 1);
 }
 
@@ -84,6 +83,12 @@ int LaunchT(const HeldConvArgs& t, int smem, hipStream_t stream)
     return 0;
 }
 } // namespace
+
+bool mi355x::HeldConvTakes(const mi355x_conv2d_s* p)
+{
+    const ConvGeom& g = p->geom;
+    return g.Ci == 64 && g.Kh * g.Kw == kHeldTaps && (g.Co & 15) == 0 && p->zw_neg == 0 && TapsInOrder(Window(g));
+}
 
 int mi355x::HeldConvGroups(const mi355x_conv2d_s* p, uint32_t batch)
 {

@@ -247,6 +247,17 @@ def test_an_addition_behind(n, ci, co, kernel):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("ci,co,k,zw,text", [(64, 64, 3, 0, "; weights in registers or input pixels in LDS where faster"), (64, 65, 3, 0, "; input pixels in LDS for all taps where faster"),
+                                             (128, 64, 3, 0, "; input pixels in LDS for all taps where faster"), (128, 64, 3, 93, ", weight zero point by row sums"), (64, 64, 2, 0, "; from 192 row tiles on input tile in LDS for all taps"),
+                                             (16, 64, 3, 0, ""), (256, 64, 1, 0, "")])
+def test_what_a_plan_says_of_its_launches(ci, co, k, zw, text):
+    wq = dict(w_dtype=U8, w_offset=zw, per_axis=False) if zw else {}
+    c = cases.make_conv_case("info", 99600 + ci, n=1, h=8, w=8, ci=ci, co=co, kh=k, kw=k, **wq)
+    info = shim.Conv2dPlan(c.x.info, c.w, c.b, c.out_info, **c.params).algo()[1]
+    assert len(info) < 127 and info.endswith(text) and (text or "in LDS" not in info), info
+
+
+@pytest.mark.gpu
 def test_a_plans_choice_follows_batch_and_lanes():
     """What a plan keeps of its last choice is for that batch and those lanes alone."""
     c = cases.make_conv_case("kept", 99500, n=64, h=14, w=14, ci=64, co=256, act=cases.RELU)
