@@ -51,7 +51,7 @@ struct ChanTab
 // The first BYTES of the kernel's arguments come to the scalar cache in one round trip.  The compiler loads an argument where it is first
 // used, and a launch finds that cache empty: one line of 64 bytes after the other, each waited for ahead of the loads of tensors behind
 // it.  Passes, three networks in turn: ResNet-50 at one image 115.5 -> 112.8 us (alone 310 -> 297), at 32 images 412 -> 403.6, MobileNetV1 at one
-// image 35.7 -> 34.8 (alone 113 -> 107), at 64 155 -> 154.3; launches, three sets of tensors in turn: FullyConnected 4096 -> 4096 of one row 4.48 -> 4.30,
+// image 35.7 -> 34.8 (alone 113 -> 107), at 64 the same; launches, three sets of tensors in turn: FullyConnected 4096 -> 4096 of one row 4.48 -> 4.30,
 // 3 x 3 over 64 x 56 x 56 x 64 14.09 -> 13.86, 1 x 1 over 32 x 28 x 28 x 128 -> 512 7.69 -> 7.59.  Not in IgemmKernel, whose launches took 0.05 us longer with it.
 template <int BYTES>
 __device__ __forceinline__ void FetchArgs()
