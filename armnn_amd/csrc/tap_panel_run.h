@@ -41,8 +41,9 @@ constexpr int PieceInside(int i, int lo, int hi)
 template <class DivY, class DivX>
 constexpr uint32_t TapsInside(int iy, int ix, int H, int W, int Kh, int Kw, int dy, int dx, uint32_t tap_rows, DivY by_dy, DivX by_dx)
 {
-    // pixels 0 .. v of an axis, of the filter's at most, and one step of it less a pixel
-    const auto reach = [](int v, int K, int d) { return (v < 0 ? 0 : v < K * d ? v : K * d) + d - 1; };
+    // pixels 0 .. v of an axis, of the filter's at most, and one step of it less a pixel (a maximum and a minimum: with comparisons and selects launches took
+    // up to 0.13 us longer, 5 x 5 over 16 x 28 x 28 x 64 10.89 -> 10.76, 3 x 3 over 16 x 14 x 14 x 256 6.40 -> 6.33)
+    const auto reach = [](int v, int K, int d) { return std::min(std::max(v, 0), K * d) + d - 1; };
     const int xl = by_dx(reach(-ix, Kw, dx)), xh = by_dx(reach(W - ix, Kw, dx)), yl = by_dy(reach(-iy, Kh, dy)), yh = by_dy(reach(H - iy, Kh, dy));
     const uint32_t cols = static_cast<uint32_t>((1ull << xh) - (1ull << xl));      // (xh is 32 in a row of 32 taps)
     const uint32_t rows = tap_rows & static_cast<uint32_t>((1ull << (yh * Kw)) - (1ull << (yl * Kw)));
